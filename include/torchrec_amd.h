@@ -351,7 +351,6 @@ int tra_mch_remap_keys(const void* values, int64_t n, const void* offsets, int32
                        const int64_t* const* mapping, const int64_t* table_size,
                        const int64_t* miss_id, void* out, void* stream);
 
-/* Measurement ------------------------------------------------------------- */
 /* Column regroup of pooled outputs ------------------------------------------- */
 /* Copies num_blocks column blocks between row-major matrices of `rows` rows:
  * block k is width[k] elements of every row, read at src[k] with row stride
@@ -365,6 +364,17 @@ int tra_regroup_columns(const void* const* src, const int64_t* src_stride, void*
                         const int64_t* dst_stride, const int32_t* width, int32_t num_blocks,
                         int64_t rows, int32_t elem_bytes, void* stream);
 
+/* The same from whole tensors and a description that does not change from call
+ * to call: `blocks` is a HOST array of num_blocks x 5 int32 {source tensor,
+ * first source column, destination tensor, first destination column, width},
+ * src / dst HOST arrays of num_src / num_dst device pointers with their row
+ * strides in elements.  A block must lie inside its tensors' row strides. */
+int tra_regroup_tensors(const void* const* src, const int64_t* src_stride, int32_t num_src,
+                        void* const* dst, const int64_t* dst_stride, int32_t num_dst,
+                        const int32_t* blocks, int32_t num_blocks, int64_t rows,
+                        int32_t elem_bytes, void* stream);
+
+/* Measurement ------------------------------------------------------------- */
 /* Streaming device-to-device copy of `bytes` bytes (a multiple of 16, 16-byte
  * aligned pointers) by a kernel named tra_copy_kernel.  A copy of known size
  * under the same hardware counters calibrates FETCH_SIZE / WRITE_SIZE readings

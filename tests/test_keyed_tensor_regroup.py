@@ -79,6 +79,22 @@ def test_regroup_kernel_against_slicing(dtype):
     assert torch.equal(got[0], torch.cat([wide[:, 40:60], wide[:, 10:40]], 1))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("unit", [1, 2, 4, 8])  # fp16 columns per vector of 2, 4, 8, 16 bytes
+@pytest.mark.parametrize("rows", [1, 3, 513, 2049, 16387])  # 1, 4 and 16 rows per thread, and remainders
+def test_regroup_kernel_tiles(rows, unit):
+    """Edges of the kernel's row and column tiles: one column vector, one more than a tile of 256."""
+    dev = torch.device("cuda:0")
+    for widths in ([unit], [unit * 256, unit], [unit * 40] * 13):
+        keys = [f"k{i}" for i in range(len(widths))]
+        # a pad column of one unit keeps the source rows aligned to the unit and no more
+        wide = torch.randint(0, 2**15, (rows, sum(widths) + unit), device=dev, dtype=torch.int16).view(torch.float16)
+        kt = KeyedTensor(keys=keys, length_per_key=widths, values=wide[:, unit:])
+        groups = [keys[::-1], keys[:1]]
+        for g, w in zip(regroup_kts([kt], groups), _regroup_keyed_tensors([kt], groups)):
+            assert torch.equal(g.view(torch.int16), w.view(torch.int16))
+
+
 @pytest.mark.parametrize("dev", DEVICES)
 def test_kt_regroup_as_dict_module(dev):
     """torchrec/modules/tests/test_regroup.py: same result as the static method,

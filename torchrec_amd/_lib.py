@@ -48,6 +48,7 @@ EXPORTED_SYMBOLS = [
     "tra_mch_remap",
     "tra_mch_remap_keys",
     "tra_regroup_columns",
+    "tra_regroup_tensors",
     "tra_copy_bytes",
 ]
 
@@ -127,6 +128,10 @@ def lib() -> ctypes.CDLL:
             ctypes.POINTER(vp), ctypes.POINTER(i64), ctypes.POINTER(vp), ctypes.POINTER(i64), ctypes.POINTER(i32),
             i32, i64, i32, vp,
         ]
+        l.tra_regroup_tensors.argtypes = [
+            ctypes.POINTER(vp), ctypes.POINTER(i64), i32, ctypes.POINTER(vp), ctypes.POINTER(i64), i32,
+            vp, i32, i64, i32, vp,
+        ]
         l.tra_copy_bytes.argtypes = [vp, vp, i64, vp]
         _lib = l
     return _lib
@@ -144,6 +149,30 @@ def forward_lengths_entry():
         return l.tra_tbe_forward_lengths
     _fastcall.bind(ctypes.cast(l.tra_tbe_forward_lengths, ctypes.c_void_p).value)
     return _fastcall.forward_lengths
+
+
+def regroup_entry(fast: bool = True):
+    """``tra_regroup_tensors`` as a callable ``(src, src_stride, dst, dst_stride, blocks, num_blocks, rows,
+    elem_bytes, stream)`` of lists of integers and integers: through the extension module when it is
+    there (at most 64 tensors on a side), else (or with ``fast=False``) through ctypes."""
+    l = lib()
+    try:
+        from torchrec_amd import _fastcall
+    except ImportError:
+        fast = False
+    if not fast:
+        vp, i64 = ctypes.c_void_p, ctypes.c_int64
+
+        def call(src, src_stride, dst, dst_stride, blocks, num_blocks, rows, elem_bytes, stream):
+            ns, nd = len(src), len(dst)
+            return l.tra_regroup_tensors(
+                (vp * ns)(*src), (i64 * ns)(*src_stride), ns, (vp * nd)(*dst), (i64 * nd)(*dst_stride), nd,
+                blocks, num_blocks, rows, elem_bytes, stream,
+            )
+
+        return call
+    _fastcall.bind_regroup(ctypes.cast(l.tra_regroup_tensors, ctypes.c_void_p).value)
+    return _fastcall.regroup_tensors
 
 
 def check(rc: int) -> None:

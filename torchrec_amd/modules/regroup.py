@@ -8,7 +8,7 @@ from typing import Dict, List, Optional
 import torch
 
 from torchrec_amd.modules.embedding_configs import data_type_to_dtype
-from torchrec_amd.sparse.jagged_tensor import KeyedTensor, _regroup_plan, regroup_kts
+from torchrec_amd.sparse.jagged_tensor import _regroup_layout, _regroup_plan, KeyedTensor, regroup_kts
 from torchrec_amd.types import DataType
 
 
@@ -30,6 +30,8 @@ class KTRegroupAsDict(torch.nn.Module):
         self._multi_device = multi_device
         self._is_inited = False
         self._plan = None
+        self._layout = None
+        self._layout = None
 
     def embedding_cast(self, embs: List[torch.Tensor]) -> List[torch.Tensor]:
         if self._emb_dtype is None:
@@ -46,14 +48,16 @@ class KTRegroupAsDict(torch.nn.Module):
                         raise RuntimeError(f"Duplicate key {key} found in KeyedTensors, undefined behavior")
                     seen.add(key)
             self._plan = _regroup_plan(keyed_tensors, self._groups)
+            self._layout = _regroup_layout(self._plan)
             self._is_inited = True
         if self._emb_dtype is not None:
             keyed_tensors = [
                 KeyedTensor(keys=kt.keys(), length_per_key=kt.length_per_key(), values=v, key_dim=kt.key_dim())
                 for kt, v in zip(keyed_tensors, self.embedding_cast([kt.values() for kt in keyed_tensors]))
             ]
-        return dict(zip(self._keys, regroup_kts(keyed_tensors, self._groups, plan=self._plan)))
+        return dict(zip(self._keys, regroup_kts(keyed_tensors, self._groups, self._plan, self._layout)))
 
     def clear_cache(self) -> None:
         self._is_inited = False
         self._plan = None
+        self._layout = None

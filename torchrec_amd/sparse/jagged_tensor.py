@@ -15,11 +15,13 @@ permutation run in the HIP kernels behind ``torchrec_amd.ops``.
 """
 from __future__ import annotations
 
+import ctypes
+from array import array
 from typing import Dict, List, Optional, Tuple, Union
 
 import torch
 
-from torchrec_amd import ops
+from torchrec_amd import _lib, ops
 
 
 def _cumsum(o: List[int]) -> List[int]:
@@ -667,54 +669,66 @@ def _regroup_keyed_tensors(keyed_tensors: List[KeyedTensor], groups: List[List[s
     return out
 
 
-def regroup_kts(keyed_tensors: List[KeyedTensor], groups: List[List[str]], plan=None) -> List[torch.Tensor]:
+_REGROUP = None  # the library's tra_regroup_tensors, bound on first use
+
+
+def _regroup_layout(plan):
+    """A ``_regroup_plan`` as ``tra_regroup_tensors`` reads it: (number of blocks, their int32
+    description, width of every group)."""
+    blocks: List[int] = []
+    widths = []
+    for g, group in enumerate(plan):
+        col_out = 0
+        for t, col, w in group:
+            blocks += (t, col, g, col_out, w)
+            col_out += w
+        widths.append(col_out)
+    return len(blocks) // 5, array("i", blocks), widths
+
+
+def regroup_kts(
+    keyed_tensors: List[KeyedTensor], groups: List[List[str]], plan=None, layout=None
+) -> List[torch.Tensor]:
     """KeyedTensor.regroup (jagged_tensor.py:209-239).  Two-dimensional fp16 / bf16 /
     fp32 tensors on the GPU (the pooled lookup's outputs) are regrouped by one
     launch of the column-copy kernel for all groups; anything else by slicing.
     ``plan`` is a ``_regroup_plan`` result kept by a caller whose key layout does
-    not change."""
-    first = keyed_tensors[0].values()
-    on_gpu = (
-        first.device.type == "cuda"
-        and keyed_tensors[0].key_dim() == 1
-        and all(
-            kt.values().dim() == 2 and kt.key_dim() == 1 and kt.values().dtype == first.dtype
-            and kt.values().device == first.device and kt.values().stride(1) == 1
-            and kt.values().shape[0] == first.shape[0]
-            for kt in keyed_tensors
-        )
-        and first.element_size() in (2, 4)
-    )
+    not change, ``layout`` the ``_regroup_layout`` of it."""
+    first = keyed_tensors[0]._values
+    dtype, dev = first.dtype, first.device
+    esz = first.element_size()
+    rows = first.shape[0] if first.dim() else 0
+    on_gpu = dev.type == "cuda" and (esz == 2 or esz == 4)
+    src, src_stride = [], []
+    if on_gpu:
+        di = first.get_device()
+        for kt in keyed_tensors:
+            v = kt._values
+            if kt._key_dim == 1 and v.dim() == 2 and v.dtype is dtype and v.get_device() == di and v.shape[0] == rows:
+                stride, step = v.stride()
+                if step == 1:
+                    src.append(v.data_ptr())
+                    src_stride.append(stride)
+                    continue
+            on_gpu = False
+            break
     if not on_gpu:
         return _regroup_keyed_tensors(keyed_tensors, groups)
-    import ctypes
-
-    from torchrec_amd import _lib
-
-    if plan is None:
-        plan = _regroup_plan(keyed_tensors, groups)
-    rows, esz = first.shape[0], first.element_size()
-    outs = [torch.empty((rows, sum(w for _, _, w in blocks)), dtype=first.dtype, device=first.device) for blocks in plan]
-    src, src_stride, dst, dst_stride, width = [], [], [], [], []
-    for blocks, out in zip(plan, outs):
-        col_out = 0
-        for t, col, w in blocks:
-            v = keyed_tensors[t].values()
-            src.append(v.data_ptr() + col * esz)
-            src_stride.append(v.stride(0))
-            dst.append(out.data_ptr() + col_out * esz)
-            dst_stride.append(out.stride(0) if out.shape[1] else 1)
-            width.append(w)
-            col_out += w
-    n = len(src)
-    if n and rows:
-        vp, i64, i32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32
-        _lib.check(
-            _lib.lib().tra_regroup_columns(
-                (vp * n)(*src), (i64 * n)(*src_stride), (vp * n)(*dst), (i64 * n)(*dst_stride), (i32 * n)(*width),
-                n, rows, esz, _lib.current_stream(first.device),
-            )
+    if layout is None:
+        layout = _regroup_layout(plan if plan is not None else _regroup_plan(keyed_tensors, groups))
+    n_blocks, blocks, widths = layout
+    outs = [torch.empty(rows, w, dtype=dtype, device=dev) for w in widths]
+    if n_blocks and rows:
+        global _REGROUP
+        if _REGROUP is None:
+            _REGROUP = _lib.regroup_entry()
+        call = _REGROUP if len(src) <= 64 and len(outs) <= 64 else _lib.regroup_entry(fast=False)
+        rc = call(
+            src, src_stride, [o.data_ptr() for o in outs], widths, blocks.buffer_info()[0], n_blocks, rows, esz,
+            _lib.current_stream(dev),
         )
+        if rc != 0:
+            _lib.check(rc)
     return outs
 
 
