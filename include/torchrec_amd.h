@@ -304,6 +304,12 @@ int tra_bucketize_scatter(const void* offsets, const void* indices,
  * with scale/bias moved to the row header. */
 int tra_quantize_rows(const float* in, int64_t rows, int32_t dim, int32_t bits,
                       uint8_t* out, int32_t row_bytes, void* stream);
+/* The same for a whole table of a store that has not been cleared: every byte
+ * between a row's payload and the next row, and `tail_bytes` bytes behind the
+ * last row, are written as zero.  `in` 16-byte aligned, rows of whole dwords. */
+int tra_quantize_rows_padded(const float* in, int64_t rows, int32_t dim, int32_t bits,
+                             uint8_t* out, int32_t row_stride, int64_t tail_bytes,
+                             void* stream);
 /* Same input, fbgemm's own output format: [rows, dim*bits/8 + 4] with the
  * fp16 scale/bias at the END of each row. */
 int tra_quantize_rows_sbhalf(const float* in, int64_t rows, int32_t dim,

@@ -302,3 +302,26 @@ def test_quantize_rows_odd_dims(bits):
         want = O.quantize_sbhalf(w, bits)
         got = ops.FloatOrHalfToFusedNBitRowwiseQuantizedSBHalf(torch.from_numpy(w).to(DEV), bits).cpu().numpy()
         assert np.array_equal(got, want), (bits, dim, int((got != want).sum()))
+
+
+@pytest.mark.parametrize("bits,dim", [(8, 4), (8, 36), (8, 128), (8, 512), (8, 520), (4, 8), (4, 40), (4, 128), (4, 512),
+                                      (4, 520), (2, 16), (2, 112), (2, 1040)])
+@pytest.mark.parametrize("rows,extra,tail", [(1, 0, 0), (3, 12, 60), (257, 28, 4), (1030, 4, 252)])
+def test_quantize_rows_padded_bytes(bits, dim, rows, extra, tail):
+    """Whole rows of a store that held other bytes: header, payload and zeros, and nothing behind the tail.  The dims
+    are one lane, lanes that are no power of two, a full wave, and more than a wave of lanes."""
+    from torchrec_amd import _lib
+
+    payload = dim * bits // 8
+    stride = 4 + payload + extra
+    w = np.random.default_rng(rows * dim).normal(0, 0.1, (rows, dim)).astype(np.float32)
+    out = torch.full((rows * stride + tail + 64,), 0xAB, dtype=torch.uint8, device=DEV)
+    src = torch.from_numpy(w).to(DEV)
+    _lib.check(_lib.lib().tra_quantize_rows_padded(
+        src.data_ptr(), rows, dim, bits, out.data_ptr(), stride, tail, _lib.current_stream(DEV)))
+    got = out.cpu().numpy()
+    want = O.quantize_sbhalf(w, bits)
+    table = got[: rows * stride].reshape(rows, stride)
+    assert np.array_equal(table[:, :4], want[:, payload:]) and np.array_equal(table[:, 4 : 4 + payload], want[:, :payload])
+    assert not table[:, 4 + payload :].any() and not got[rows * stride : rows * stride + tail].any()
+    assert (got[rows * stride + tail :] == 0xAB).all()

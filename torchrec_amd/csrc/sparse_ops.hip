@@ -10,6 +10,11 @@
 
 namespace tra {
 
+// (native vectors: an array of HIP's uint4 objects is kept in scratch memory, which doubled the regroup kernel's time)
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 16;
 constexpr int kScanTile = kScanThreads * kScanItems;
@@ -432,6 +437,42 @@ __global__ __launch_bounds__(kWalkThreads) void bucketize_scatter_wave_kernel(
 // FloatOrHalfToFusedNBitRowwiseQuantizedSBHalf: min/max, bias = fp16(min),
 // scale = fp16((max - bias) / (2^bits - 1)), q = clamp(rint((x - bias) * (1/scale))).
 // header_first: TBE row [scale][bias][payload]; otherwise fbgemm's trailer row.
+// A row's header dword (fp16 scale, fp16 bias) from its extremes, with the bias
+// and the reciprocal scale its elements are quantized by.
+template <int BITS>
+__device__ __forceinline__ uint32_t row_header(float mn, float mx, float& bias, float& inv) {
+  constexpr int kQMax = (1 << BITS) - 1;
+  const __half bias_h = __float2half_rn(mn);
+  bias = __half2float(bias_h);
+  const float range = mx - bias;
+  float scale = range == 0.0f ? 1.0f : range / (float)kQMax;
+  scale = __half2float(__float2half_rn(scale));
+  if (scale == 0.0f) scale = 1.0f;
+  inv = 1.0f / scale;
+  if (__builtin_isinf(inv)) {
+    scale = 1.0f;
+    inv = 1.0f;
+  }
+  return (uint32_t)__half_as_ushort(__float2half_rn(scale)) | ((uint32_t)__half_as_ushort(bias_h) << 16);
+}
+
+// DPL output dwords from their elements.
+template <int BITS, int DPL>
+__device__ __forceinline__ void pack_elements(const float* v, float bias, float inv, uint32_t* packed) {
+  constexpr int EPD = 32 / BITS;
+  constexpr int kQMax = (1 << BITS) - 1;
+#pragma unroll
+  for (int d = 0; d < DPL; ++d) packed[d] = 0;
+#pragma unroll
+  for (int e = 0; e < DPL * EPD; ++e) {
+    const float t = (v[e] - bias) * inv;
+    float q = __builtin_rintf(t);
+    q = q < 0.0f ? 0.0f : q;
+    q = q > (float)kQMax ? (float)kQMax : q;
+    packed[e / EPD] |= (uint32_t)(int)q << ((e % EPD) * BITS);
+  }
+}
+
 template <int BITS>
 __global__ __launch_bounds__(256) void quantize_rows_kernel(const float* in, int64_t rows,
                                                             int32_t dim, uint8_t* out,
@@ -454,18 +495,8 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const float* in, int
   }
   constexpr int kQMax = (1 << BITS) - 1;
   constexpr int kEpb = 8 / BITS;
-  const __half bias_h = __float2half_rn(mn);
-  const float bias = __half2float(bias_h);
-  const float range = mx - bias;
-  float scale = range == 0.0f ? 1.0f : range / (float)kQMax;
-  scale = __half2float(__float2half_rn(scale));
-  if (scale == 0.0f) scale = 1.0f;
-  float inv = 1.0f / scale;
-  if (__builtin_isinf(inv)) {
-    scale = 1.0f;
-    inv = 1.0f;
-  }
-  const __half scale_h = __float2half_rn(scale);
+  float bias, inv;
+  const uint32_t header = row_header<BITS>(mn, mx, bias, inv);
   const int payload = dim / kEpb;
   uint8_t* o = out + r * row_bytes;
   uint8_t* pay = header_first ? o + 4 : o;
@@ -483,11 +514,8 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const float* in, int
     pay[byte] = (uint8_t)packed;
   }
   if (lane == 0) {
-    const uint16_t s = __half_as_ushort(scale_h), b = __half_as_ushort(bias_h);
-    hdr[0] = (uint8_t)(s & 0xff);
-    hdr[1] = (uint8_t)(s >> 8);
-    hdr[2] = (uint8_t)(b & 0xff);
-    hdr[3] = (uint8_t)(b >> 8);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) hdr[i] = (uint8_t)(header >> (8 * i));
   }
 }
 
@@ -503,10 +531,9 @@ template <int BITS, int DPL = 1>
 __global__ __launch_bounds__(256) void quantize_rows_vec_kernel(const float* __restrict__ in, int64_t rows,
                                                                 int32_t dim, uint8_t* __restrict__ out,
                                                                 int64_t row_bytes, int header_first,
-                                                                int lpr) {
+                                                                int lpr, int pad_dwords) {
   constexpr int EPD = 32 / BITS;    // elements per output dword
   constexpr int EPL = DPL * EPD;    // elements per lane and step
-  constexpr int kQMax = (1 << BITS) - 1;
   const int lane = threadIdx.x & (kWaveSize - 1);
   const int g = lane / lpr, c = lane - g * lpr;
   const int rows_per_wave = kWaveSize / lpr;
@@ -538,18 +565,8 @@ __global__ __launch_bounds__(256) void quantize_rows_vec_kernel(const float* __r
     mn = a < mn ? a : mn;
     mx = b > mx ? b : mx;
   }
-  const __half bias_h = __float2half_rn(mn);
-  const float bias = __half2float(bias_h);
-  const float range = mx - bias;
-  float scale = range == 0.0f ? 1.0f : range / (float)kQMax;
-  scale = __half2float(__float2half_rn(scale));
-  if (scale == 0.0f) scale = 1.0f;
-  float inv = 1.0f / scale;
-  if (__builtin_isinf(inv)) {
-    scale = 1.0f;
-    inv = 1.0f;
-  }
-  const __half scale_h = __float2half_rn(scale);
+  float bias, inv;
+  const uint32_t header = row_header<BITS>(mn, mx, bias, inv);
   if (!active) return;
   uint8_t* o = out + r * row_bytes;
   uint32_t* pay = reinterpret_cast<uint32_t*>(header_first ? o + 4 : o);
@@ -567,20 +584,84 @@ __global__ __launch_bounds__(256) void quantize_rows_vec_kernel(const float* __r
       }
     }
     uint32_t packed[DPL];
-#pragma unroll
-    for (int d = 0; d < DPL; ++d) packed[d] = 0;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      const float t = (v[e] - bias) * inv;
-      float q = __builtin_rintf(t);
-      q = q < 0.0f ? 0.0f : q;
-      q = q > (float)kQMax ? (float)kQMax : q;
-      packed[e / EPD] |= (uint32_t)(int)q << ((e % EPD) * BITS);
-    }
+    pack_elements<BITS, DPL>(v, bias, inv, packed);
     // one store of DPL dwords (the payload is 4-byte aligned, not more)
     __builtin_memcpy(__builtin_assume_aligned(pay + ch * DPL, 4), packed, sizeof(packed));
   }
-  if (c == 0) *hdr = (uint32_t)__half_as_ushort(scale_h) | ((uint32_t)__half_as_ushort(bias_h) << 16);
+  if (c == 0) *hdr = header;
+  for (int w = c; w < pad_dwords; w += lpr) pay[chunks * DPL + w] = 0;  // (header_first rows only)
+}
+
+// The same for the padded rows of a lookup operator's store: header, payload,
+// zeros up to the row stride, and `tail_dwords` zeros behind the last row, so
+// that the store needs no clearing first and nothing is copied into it
+// afterwards.  A wave builds its rows in LDS and writes them out as one
+// contiguous run of 16-byte vectors: with a 4-byte store per lane a 68-byte
+// row leaves in pieces (int4 rows of dim 128 at a 128-byte stride, 1 M rows:
+// 122 us written directly, 111 us built in LDS; 8-bit rows are even, 2-bit
+// rows 4 % slower, so those take the kernel above).  Rows of at most 64 lanes.
+template <int BITS, int DPL>
+__global__ __launch_bounds__(256) void quantize_rows_padded_kernel(const float* __restrict__ in, int64_t rows,
+                                                                   int32_t dim, uint32_t* __restrict__ out,
+                                                                   int32_t stride_dwords, int lpr, int tail_dwords) {
+  extern __shared__ __align__(16) uint32_t qrow_smem[];
+  constexpr int EPD = 32 / BITS;
+  constexpr int EPL = DPL * EPD;
+  const int lane = threadIdx.x & (kWaveSize - 1);
+  const int wave = threadIdx.x / kWaveSize;
+  const int g = lane / lpr, c = lane - g * lpr;
+  const int rows_per_wave = kWaveSize / lpr;
+  if (blockIdx.x == 0)
+    for (int w = threadIdx.x; w < tail_dwords; w += blockDim.x) out[rows * stride_dwords + w] = 0;
+  const int64_t base = ((int64_t)blockIdx.x * (blockDim.x / kWaveSize) + wave) * rows_per_wave;
+  if (base >= rows) return;
+  const int64_t r = base + g < rows ? base + g : rows - 1;  // every lane takes part in the reductions
+  const int chunks = dim / EPL;
+  const float* x = in + r * dim + (c < chunks ? c : 0) * EPL;
+  float v[EPL];
+#pragma unroll
+  for (int k = 0; k < EPL / 4; ++k) {
+    const f32x4_t q = *reinterpret_cast<const f32x4_t*>(x + 4 * k);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[4 * k + i] = q[i];
+  }
+  float mn = __shfl(v[0], lane - c, 64), mx = mn;  // (the row's first element, as in the kernels above)
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) {
+    mn = v[e] < mn ? v[e] : mn;
+    mx = v[e] > mx ? v[e] : mx;
+  }
+  for (int off = lpr >> 1; off > 0; off >>= 1) {
+    const float a = __shfl_xor(mn, off, 64), b = __shfl_xor(mx, off, 64);
+    mn = a < mn ? a : mn;
+    mx = b > mx ? b : mx;
+  }
+  float bias, inv;
+  const uint32_t header = row_header<BITS>(mn, mx, bias, inv);
+  uint32_t* row = qrow_smem + (size_t)(wave * rows_per_wave + g) * stride_dwords;
+  if (c < chunks) {
+    uint32_t packed[DPL];
+    pack_elements<BITS, DPL>(v, bias, inv, packed);
+#pragma unroll
+    for (int d = 0; d < DPL; ++d) row[1 + c * DPL + d] = packed[d];
+  }
+  if (c == 0) row[0] = header;
+  for (int w = 1 + chunks * DPL + c; w < stride_dwords; w += lpr) row[w] = 0;
+  wave_lds_sync();
+  // the wave's rows are neighbours in LDS and in the store
+  const uint32_t* src = qrow_smem + (size_t)wave * rows_per_wave * stride_dwords;
+  const int n = (int)(rows - base < rows_per_wave ? rows - base : rows_per_wave) * stride_dwords;
+  uint32_t* dst = out + base * stride_dwords;
+  if (stride_dwords % 4 == 0 && (uintptr_t)out % 16 == 0) {
+    for (int i = lane * 4; i < n; i += 4 * kWaveSize)
+      __builtin_nontemporal_store(*reinterpret_cast<const u32x4_t*>(src + i), reinterpret_cast<u32x4_t*>(dst + i));
+  } else {
+    for (int i = lane; i < n; i += kWaveSize) dst[i] = src[i];
+  }
+}
+
+__global__ __launch_bounds__(256) void zero_dwords_kernel(uint32_t* out, int n) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) out[i] = 0;
 }
 
 // ---- positions inside bags ---------------------------------------------------
@@ -718,10 +799,6 @@ struct RegroupBlocks {
   int32_t first[kRegroupBlocks];       // first vector column of the block
 };
 
-// (native vectors: an array of HIP's uint4 objects is kept in scratch memory, which doubled this kernel's time)
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-
 // blockIdx.x: tile of rp * R rows; blockIdx.y: tile of `cw` vector columns.
 // Thread t of the workgroup holds column t % cw and rows t / cw + k * rp.
 template <typename V, int R>
@@ -854,8 +931,10 @@ static int regroup_impl(F&& block, int32_t num_blocks, int64_t rows, int32_t ele
   return TRA_OK;
 }
 
-static int quantize_impl(const float* in, int64_t rows, int32_t dim, int32_t bits, uint8_t* out,
-                         int64_t row_bytes, int header_first, hipStream_t s) {
+// pad: the bytes between a row's payload and the next row, and tail_bytes behind the last row, are zeroed
+// (header-first rows only).
+static int quantize_impl(const float* in, int64_t rows, int32_t dim, int32_t bits, uint8_t* out, int64_t row_bytes,
+                         int header_first, hipStream_t s, bool pad = false, int64_t tail_bytes = 0) {
   if (bits != 8 && bits != 4 && bits != 2) {
     set_error("quantize: bits must be 8, 4 or 2 (got %d)", bits);
     return TRA_ERR_INVALID_ARGUMENT;
@@ -870,7 +949,12 @@ static int quantize_impl(const float* in, int64_t rows, int32_t dim, int32_t bit
     return TRA_ERR_INVALID_ARGUMENT;
   }
   int epl = 32 / bits;
-  if (dim % epl == 0 && row_bytes % 4 == 0 && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 4 == 0) {
+  const bool vec = dim % epl == 0 && row_bytes % 4 == 0 && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 4 == 0;
+  if (pad && (!vec || tail_bytes < 0 || tail_bytes % 4 != 0 || tail_bytes > (1 << 20))) {
+    set_error("quantize: padded rows need whole dwords, a 16-byte aligned input and a tail of at most 1 MiB");
+    return TRA_ERR_INVALID_ARGUMENT;
+  }
+  if (vec) {
     // 8-bit rows: two output dwords (8 elements, two 16-byte loads) per lane and step where the
     // dim allows.  Measured on 1 M rows x 128: 204 us with one dword per lane, 158 us with two,
     // 170 us with four; 4-bit rows are fastest with one (127 us against 133 us with two).
@@ -886,14 +970,35 @@ static int quantize_impl(const float* in, int64_t rows, int32_t dim, int32_t bit
       return TRA_ERR_TOO_LARGE;
     }
     dim3 vg((unsigned)vblocks), vb(256);
+    const int64_t lds = rows_per_block * row_bytes;
+    if (pad && bits != 2 && chunks <= kWaveSize && lds <= 32 * 1024) {
+      const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, vg, vb, (size_t)lds, s, in, rows, dim, (uint32_t*)out, (int32_t)(row_bytes / 4), lpr,
+                           (int)(tail_bytes / 4));
+      };
+      if (wide)
+        go(quantize_rows_padded_kernel<8, 2>);
+      else if (bits == 8)
+        go(quantize_rows_padded_kernel<8, 1>);
+      else
+        go(quantize_rows_padded_kernel<4, 1>);
+      return check_launch("quantize_rows");
+    }
+    const int pad_dwords = pad ? (int)((row_bytes - 4 - (int64_t)dim * bits / 8) / 4) : 0;
+    const auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, vg, vb, 0, s, in, rows, dim, out, row_bytes, header_first, lpr, pad_dwords);
+    };
     if (wide)
-      hipLaunchKernelGGL((quantize_rows_vec_kernel<8, 2>), vg, vb, 0, s, in, rows, dim, out, row_bytes, header_first, lpr);
+      go(quantize_rows_vec_kernel<8, 2>);
     else if (bits == 8)
-      hipLaunchKernelGGL(quantize_rows_vec_kernel<8>, vg, vb, 0, s, in, rows, dim, out, row_bytes, header_first, lpr);
+      go(quantize_rows_vec_kernel<8>);
     else if (bits == 4)
-      hipLaunchKernelGGL(quantize_rows_vec_kernel<4>, vg, vb, 0, s, in, rows, dim, out, row_bytes, header_first, lpr);
+      go(quantize_rows_vec_kernel<4>);
     else
-      hipLaunchKernelGGL(quantize_rows_vec_kernel<2>, vg, vb, 0, s, in, rows, dim, out, row_bytes, header_first, lpr);
+      go(quantize_rows_vec_kernel<2>);
+    if (pad && tail_bytes > 0)
+      hipLaunchKernelGGL(zero_dwords_kernel, dim3(1), dim3(256), 0, s, (uint32_t*)(out + rows * row_bytes),
+                         (int)(tail_bytes / 4));
     return check_launch("quantize_rows");
   }
   const int64_t blocks = (rows + 3) / 4;
@@ -1150,6 +1255,11 @@ int tra_bucketize_scatter(const void* offsets, const void* indices, int32_t is_i
 int tra_quantize_rows(const float* in, int64_t rows, int32_t dim, int32_t bits, uint8_t* out,
                       int32_t row_bytes, void* stream) {
   return quantize_impl(in, rows, dim, bits, out, row_bytes, 1, (hipStream_t)stream);
+}
+
+int tra_quantize_rows_padded(const float* in, int64_t rows, int32_t dim, int32_t bits, uint8_t* out,
+                             int32_t row_stride, int64_t tail_bytes, void* stream) {
+  return quantize_impl(in, rows, dim, bits, out, row_stride, 1, (hipStream_t)stream, true, tail_bytes);
 }
 
 int tra_quantize_rows_sbhalf(const float* in, int64_t rows, int32_t dim, int32_t bits,

@@ -229,6 +229,40 @@ def quantize_state_dict(
     return device
 
 
+class _FloatTables(Dict[str, Tensor]):
+    """Float weights by table name, in place of ``(payload, scale_bias)`` pairs: the lookup operator
+    quantizes them straight into its rows."""
+
+
+def _quantized_or_float_tables(
+    module: nn.Module,
+    table_name_to_data_type: Dict[str, DataType],
+    table_name_to_num_embeddings_post_pruning: Optional[Dict[str, int]] = None,
+) -> Tuple[torch.device, Dict[str, Any]]:
+    """The weights of a float collection for the constructor of its quantized form: the float tensors
+    themselves where all of them are on one GPU, else what ``quantize_state_dict`` makes of them."""
+    post_pruning = table_name_to_num_embeddings_post_pruning or {}
+    floats = _FloatTables()
+    for key, tensor in module.state_dict().items():
+        table_name = key.split(".")[-2] if "." in key else key
+        ty = table_name_to_data_type.get(table_name)
+        if (
+            not key.endswith(".weight") or not tensor.is_cuda or tensor.dtype not in (torch.float, torch.float16)
+            or (ty not in _INT_TYPES and ty not in (DataType.FP16, DataType.FP32))
+        ):
+            floats.clear()
+            break
+        floats[table_name] = tensor[: post_pruning.get(table_name, tensor.shape[0]), :]
+    devices = {t.device for t in floats.values()}
+    if len(devices) == 1:
+        return devices.pop(), floats
+    quantized: Dict[str, Tuple[Tensor, Tensor]] = {}
+    device = quantize_state_dict(
+        module, quantized, table_name_to_data_type, table_name_to_num_embeddings_post_pruning
+    )
+    return device, quantized
+
+
 def _get_device(module: nn.Module) -> torch.device:
     for _, tensor in module.state_dict().items():
         return tensor.device
@@ -264,8 +298,9 @@ def _build_tbe(
 ) -> IntNBitTableBatchedEmbeddingBagsCodegen:
     location = EmbeddingLocation.HOST if device.type == "cpu" else EmbeddingLocation.DEVICE
     embedding_specs = []
+    floats = table_name_to_quantized_weights if isinstance(table_name_to_quantized_weights, _FloatTables) else None
     weight_lists: Optional[List[Tuple[Tensor, Optional[Tensor]]]] = (
-        [] if table_name_to_quantized_weights else None
+        [] if table_name_to_quantized_weights and floats is None else None
     )
     feature_table_map: List[int] = []
     for idx, table in enumerate(emb_configs):
@@ -287,7 +322,9 @@ def _build_tbe(
         row_alignment=row_alignment,
         feature_table_map=feature_table_map,
     )
-    if weight_lists is None:
+    if floats is not None:
+        emb_module.assign_float_weights([floats[table.name] for table in emb_configs])
+    elif weight_lists is None:
         emb_module.initialize_weights()
     return emb_module
 
@@ -555,12 +592,8 @@ class EmbeddingBagCollection(EmbeddingBagCollectionInterface, ModuleNoCopyMixin,
         )
         embedding_bag_configs = copy.deepcopy(module.embedding_bag_configs())
         _update_embedding_configs(embedding_bag_configs, module.qconfig, pruning_dict)
-        table_name_to_quantized_weights: Dict[str, Tuple[Tensor, Tensor]] = {}
-        device = quantize_state_dict(
-            module,
-            table_name_to_quantized_weights,
-            {table.name: table.data_type for table in embedding_bag_configs},
-            pruning_dict,
+        device, table_name_to_quantized_weights = _quantized_or_float_tables(
+            module, {table.name: table.data_type for table in embedding_bag_configs}, pruning_dict
         )
         return cls(
             embedding_bag_configs,
@@ -660,12 +693,8 @@ class FeatureProcessedEmbeddingBagCollection(EmbeddingBagCollection):
         )
         embedding_bag_configs = copy.deepcopy(ebc.embedding_bag_configs())
         _update_embedding_configs(embedding_bag_configs, qconfig, pruning_dict)
-        table_name_to_quantized_weights: Dict[str, Tuple[Tensor, Tensor]] = {}
-        device = quantize_state_dict(
-            ebc,
-            table_name_to_quantized_weights,
-            {table.name: table.data_type for table in embedding_bag_configs},
-            pruning_dict,
+        device, table_name_to_quantized_weights = _quantized_or_float_tables(
+            ebc, {table.name: table.data_type for table in embedding_bag_configs}, pruning_dict
         )
         feature_processor, _ = module.split()  # a per-feature dict is wrapped into a collection
         return cls(
@@ -748,6 +777,13 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
             for table in emb_configs:
                 self._feature_names.extend(table.feature_names)
             self._feature_splits.append(sum(table.num_features() for table in emb_configs))
+
+        if isinstance(table_name_to_quantized_weights, _FloatTables):
+            self._table_name_to_quantized_weights = {
+                name: pair
+                for op in self._emb_modules
+                for name, pair in zip(op.embedding_names, op.split_embedding_weights())
+            }
 
         self.embeddings: nn.ModuleDict = nn.ModuleDict()
         for (_key, group_tables), emb_module in zip(self._key_to_tables.items(), self._emb_modules):
@@ -864,11 +900,8 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
         assert hasattr(module, "qconfig"), "EmbeddingCollection input float module must have qconfig defined"
         embedding_configs = copy.deepcopy(module.embedding_configs())
         _update_embedding_configs(embedding_configs, module.qconfig)
-        table_name_to_quantized_weights: Dict[str, Tuple[Tensor, Tensor]] = {}
-        device = quantize_state_dict(
-            module,
-            table_name_to_quantized_weights,
-            {table.name: table.data_type for table in embedding_configs},
+        device, table_name_to_quantized_weights = _quantized_or_float_tables(
+            module, {table.name: table.data_type for table in embedding_configs}
         )
         return cls(
             embedding_configs,
@@ -978,9 +1011,8 @@ class QuantManagedCollisionEmbeddingCollection(EmbeddingCollection):
         )
         device = _get_device(ec)
         if table_name_to_quantized_weights is None and device.type != "meta":
-            table_name_to_quantized_weights = {}
-            quantize_state_dict(
-                ec, table_name_to_quantized_weights, {t.name: t.data_type for t in embedding_configs}
+            _, table_name_to_quantized_weights = _quantized_or_float_tables(
+                ec, {t.name: t.data_type for t in embedding_configs}
             )
         return cls(
             embedding_configs,

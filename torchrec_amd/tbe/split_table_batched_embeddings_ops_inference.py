@@ -310,6 +310,48 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
                 ss = ss.view(torch.uint8) if ss.dtype != torch.uint8 else ss
                 ds.copy_(ss.reshape(ds.shape))
 
+    def assign_float_weights(self, tables: List[Tensor]) -> None:
+        """Quantizes one fp32 / fp16 ``[rows, dim]`` tensor per table straight into the packed rows: same
+        bytes as quantizing into a tensor of its own and ``assign_embedding_weights``, but the store is
+        written once, header, payload and padding together (4 tables of 1 M x 128 int4: 1033 us that way,
+        of it 490 us in the quantizer; the rest cleared the store and copied three times)."""
+        dev = self.current_device
+        assert dev.type == "cuda" and len(tables) == len(self.embedding_specs), "one GPU tensor per table"
+        if not self._weights_initialized:
+            self.weights_dev = torch.empty(self.weights_size, dtype=torch.uint8, device=dev)
+            self._weights_initialized = True
+            self.weight_initialized = True
+            self._drop_plan()
+        lib, stream = _lib.lib(), _lib.current_stream(dev)
+        ends = self.weights_physical_offsets[1:] + [self.weights_size]
+        for t, (src, ty, end) in enumerate(zip(tables, self.weight_tys, ends)):
+            rows, dim, stride, begin = self.rows[t], self.dims[t], self.row_stride[t], self.weights_physical_offsets[t]
+            assert src.shape == (rows, dim), f"weight shape {tuple(src.shape)} != table shape {(rows, dim)}"
+            tail = end - begin - rows * stride
+            if ty not in (SparseType.INT8, SparseType.INT4, SparseType.INT2):
+                store = self.weights_dev[begin:end]
+                if tail:
+                    store[rows * stride :].zero_()
+                padded = store[: rows * stride].view(rows, stride)
+                payload = dim * ty.bit_rate() // 8
+                if payload < stride:
+                    padded[:, payload:].zero_()
+                padded[:, :payload].view(torch.float16 if ty == SparseType.FP16 else torch.float32).copy_(src)
+                continue
+            # fp16 sources are widened a piece at a time
+            step = rows if src.dtype == torch.float32 else max(1, (1 << 28) // (4 * dim))
+            for r0 in range(0, rows, step):
+                n = min(step, rows - r0)
+                piece = src[r0 : r0 + n].to(torch.float32).contiguous()
+                if piece.data_ptr() % 16:
+                    piece = piece.clone()
+                _lib.check(
+                    lib.tra_quantize_rows_padded(
+                        piece.data_ptr(), n, dim, ty.bit_rate(), self.weights_dev.data_ptr() + begin + r0 * stride,
+                        stride, tail if r0 + n == rows else 0, stream,
+                    )
+                )
+
     # -- lookup -----------------------------------------------------------------
     def _drop_plan(self) -> None:
         plans = getattr(self, "_plans", None)
