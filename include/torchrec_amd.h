@@ -136,6 +136,17 @@ int tra_tbe_forward(tra_tbe_t tbe, const void* weights, const void* indices,
                     int32_t out_dtype, void* out, int64_t out_stride,
                     void* stream);
 
+/* Sequence lookup (TRA_POOL_NONE) without an offsets array: only where each
+ * key's ids lie matters.  Exactly one of
+ *   key_totals  DEVICE int64[num_keys], ids per key (num_keys <= 256), e.g. from
+ *               tra_key_totals_begin: key k's ids follow those of the keys before it;
+ *   key_starts  HOST int64[num_keys + 1], first id of each key (and the end).
+ * `out` is [num_indices, dim]. */
+int tra_tbe_forward_sequence(tra_tbe_t tbe, const void* weights, const void* indices,
+                             const int64_t* key_totals, const int64_t* key_starts,
+                             int32_t num_keys, int32_t idx_is_i64, int64_t num_indices,
+                             int32_t out_dtype, void* out, void* stream);
+
 /* The same lookup from the KJT's lengths instead of its offsets: what
  * QuantEmbeddingBagCollection.forward does when the KJT was built from
  * lengths, i.e. KeyedJaggedTensor.offsets() -> asynchronous_complete_cumsum
@@ -251,6 +262,20 @@ int tra_cumsum(const void* lengths, int64_t n, int32_t is_i64, void* offsets,
 int tra_length_per_key(const void* lengths, int32_t num_features,
                        int32_t batch_size, int32_t is_i64, int64_t* out,
                        void* stream);
+
+/* Ids per key with the result on the host as soon as it exists: one kernel adds
+ * up each key's lengths (bags_are_offsets: subtracts its offsets), writes
+ * totals[num_keys] on the device (unless null) and, when `ticket` is not null,
+ * into pinned host memory of the library's own.  tra_key_totals_wait(ticket)
+ * then reads them there without waiting for anything queued behind the kernel.
+ * Every ticket is to be waited for, once; at most 64 are open at a time and at
+ * most 1024 keys reach the host (TRA_ERR_TOO_LARGE beyond; TRA_ERR_UNSUPPORTED
+ * on a stream that is being captured).  Replaces
+ * torch.sum(lengths.view(F, B), 1).tolist() (jagged_tensor.py:1201-1212). */
+int tra_key_totals_begin(const void* bags, int32_t bags_are_offsets, int32_t num_keys,
+                         int32_t batch_size, int32_t is_i64, int64_t* totals,
+                         int32_t* ticket, void* stream);
+int tra_key_totals_wait(int32_t ticket, int64_t* totals);
 
 /* Feature permutation of a KJT.  lengths is [T, B]; out_lengths[t', :] =
  * lengths[permute[t'], :]; values (and weights) segments follow in the new

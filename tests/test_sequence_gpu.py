@@ -1,0 +1,113 @@
+"""Sequence lookup from key totals and key starts, and the per-key counts that
+feed it, on the GPU against the CPU oracle."""
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from helpers import bits_equal
+from test_tbe_gpu import build
+from torchrec_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+# One lane per row, lanes that are no power of two, rows of 2 and of 4 output vectors per lane, several column slices.
+@pytest.mark.parametrize("dtype,dim,out", [(O.INT8, 4, O.FP16), (O.INT8, 36, O.FP16), (O.INT8, 128, O.FP16), (O.INT8, 64, O.FP32),
+                                           (O.INT4, 104, O.FP16), (O.INT4, 128, O.FP32), (O.INT2, 64, O.FP16),
+                                           (O.FP16, 40, O.FP32), (O.FP32, 8, O.FP16), (O.INT8, 1028, O.FP16)])
+# Ids per key: fewer than a tile, exactly tiles, uneven and empty keys, more keys than a wave has lanes.
+@pytest.mark.parametrize("totals", [[1], [64, 128, 256, 512], [0, 5000, 0, 3, 129], [7] * 130, [70_000, 1, 2_000]])
+@pytest.mark.parametrize("idt", [np.int32, np.int64])
+def test_sequence_from_totals_and_starts(dtype, dim, out, totals, idt):
+    rng = np.random.default_rng(dim * len(totals))
+    K = len(totals)
+    if dim > 1000 and sum(totals) > 10_000:
+        pytest.skip("wide rows are checked on the short inputs")
+    tables = min(K, 5)
+    specs = [(dtype, 50 + 31 * t, dim) for t in range(tables)]
+    ftm = sorted(f % tables for f in range(K))
+    tbe, store = build(rng, specs, ftm, O.NONE, out, 16)
+    ids = np.concatenate([rng.integers(-1, specs[ftm[f]][1], n) for f, n in enumerate(totals)]).astype(idt)
+    starts = np.concatenate([[0], np.cumsum(totals)])
+    want = O.tbe_forward(store, ftm, 1, ids, starts.astype(idt), None, O.NONE, out)
+    dids = torch.from_numpy(ids).to(DEV)
+    routes = {"totals": {"key_totals": torch.tensor(totals, device=DEV)}, "offsets": {"offsets": torch.from_numpy(starts.astype(idt)).to(DEV)}}
+    if K <= 128:
+        routes["starts"] = {"key_starts": starts.tolist()}
+    for name, kw in routes.items():
+        got = tbe(indices=dids, **{"offsets": None, **kw}).cpu().numpy()
+        assert bits_equal(got, want) == 0, name
+    assert tbe.out_of_range_count() == 0
+
+
+def test_sequence_features_at_other_positions():
+    """Features out of key order, a key no feature sits at, one key that two features share, a padded ids buffer."""
+    rng = np.random.default_rng(2)
+    tbe, store = build(rng, [(O.INT8, 300, 64), (O.INT4, 200, 64)], [0, 0, 1], O.NONE, O.FP16, 16)
+    totals = [300, 0, 170, 40]
+    starts = np.concatenate([[0], np.cumsum(totals)])
+    ids = rng.integers(0, 200, 510).astype(np.int64)
+    padded = torch.from_numpy(np.concatenate([ids, np.full(9, 10**6)])).to(DEV)
+    out = torch.full((519, 64), 7.0, dtype=torch.float16, device=DEV)
+    for positions in ([2, 0, 3], [2, 2, 0]):
+        for kw in ({"key_totals": torch.tensor(totals, device=DEV)}, {"key_starts": starts.tolist()}):
+            out.fill_(7.0)
+            tbe(indices=padded, offsets=None, feature_positions=positions, out=out, **kw)
+            got = out.cpu().numpy()
+            seen = np.zeros(519, bool)
+            for f, p in enumerate(positions):
+                if positions.count(p) > 1:
+                    seen[starts[p]:starts[p + 1]] = True  # two features write here: either may stand
+                    continue
+                part = ids[starts[p]:starts[p + 1]]
+                one = O.tbe_forward(store, [0, 0, 1], 1, np.concatenate([part] * 3),
+                                    np.arange(4) * len(part), None, O.NONE, O.FP16)
+                assert bits_equal(got[starts[p]:starts[p + 1]], one[f * len(part):(f + 1) * len(part)]) == 0
+                seen[starts[p]:starts[p + 1]] = True
+            assert (got[~seen] == 7.0).all()
+    assert tbe.out_of_range_count() == 0
+
+
+@pytest.mark.parametrize("K,B", [(1, 1), (1, 5000), (3, 7), (26, 2048), (256, 3), (257, 3), (1024, 2), (1025, 2)])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("skip", [0, 1])  # 1: the lengths start off a 16-byte boundary
+def test_key_totals(K, B, dtype, skip):
+    lengths = torch.randint(0, 50, (K * B + skip,), dtype=dtype, device=DEV)[skip:]
+    want = lengths.view(K, B).sum(1).tolist()
+    assert ops.length_per_key(lengths, K, B) == want
+    offsets = ops.asynchronous_complete_cumsum(lengths)
+    for bags, are_offsets in ((lengths, False), (offsets, True)):
+        begun = ops.key_totals_begin(bags, are_offsets, K, B, on_device=True)
+        assert (begun is None) == (K > 1024)
+        if begun is not None:
+            totals, finish = begun
+            assert finish() == want and totals.tolist() == want
+
+
+def test_key_totals_threads_and_open_calls():
+    """More calls open than there are slots (the surplus takes the copying route), and threads on streams of their own."""
+    lengths = [torch.full((6,), i, dtype=torch.int32, device=DEV) for i in range(80)]
+    later = [ops.length_per_key_async(t, 2, 3) for t in lengths]
+    assert [f() for f in later] == [[3 * i, 3 * i] for i in range(80)]
+    bad = []
+
+    def work(seed):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for i in range(50):
+                t = torch.full((4 * 33,), seed * 50 + i, dtype=torch.int64, device=DEV)
+                if ops.length_per_key(t, 4, 33) != [33 * (seed * 50 + i)] * 4:
+                    bad.append((seed, i))
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not bad
+
+
+def test_key_totals_reject_other_integer_types():
+    with pytest.raises(TypeError):
+        ops.length_per_key(torch.ones(4, dtype=torch.int16, device=DEV), 2, 2)

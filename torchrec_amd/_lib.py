@@ -30,12 +30,15 @@ EXPORTED_SYMBOLS = [
     "tra_tbe_forward_lengths_static_max_bytes",
     "tra_tbe_forward_lengths_static",
     "tra_tbe_forward_position_weighted",
+    "tra_tbe_forward_sequence",
     "tra_tbe_launch_info",
     "tra_tbe_set_bounds_check_mode",
     "tra_tbe_error_count",
     "tra_cumsum_workspace_bytes",
     "tra_cumsum",
     "tra_length_per_key",
+    "tra_key_totals_begin",
+    "tra_key_totals_wait",
     "tra_permute_2d_lengths",
     "tra_permute_2d_data",
     "tra_bucketize_workspace_bytes",
@@ -54,6 +57,7 @@ EXPORTED_SYMBOLS = [
 ]
 
 TRA_OK = 0
+ERR_UNSUPPORTED, ERR_TOO_LARGE = -2, -5
 FP32, FP16, INT8, INT4, INT2 = 0, 1, 2, 3, 4
 POOL_SUM, POOL_MEAN, POOL_NONE = 0, 1, 2
 
@@ -103,6 +107,7 @@ def lib() -> ctypes.CDLL:
             vp, vp, vp, vp, i32, i32, vp, i64, ctypes.POINTER(i32), ctypes.POINTER(i32), i32, i32, i64, i32, i32,
             vp, i64, vp, vp,
         ]
+        l.tra_tbe_forward_sequence.argtypes = [vp, vp, vp, vp, vp, i32, i32, i64, i32, vp, vp]
         l.tra_tbe_launch_info.argtypes = [vp, i32, i64, i32, i32, ctypes.c_char_p, i32]
         l.tra_tbe_set_bounds_check_mode.argtypes = [vp, i32]
         l.tra_tbe_error_count.argtypes = [vp, vp, ctypes.POINTER(i64)]
@@ -110,6 +115,8 @@ def lib() -> ctypes.CDLL:
         l.tra_cumsum_workspace_bytes.restype = i64
         l.tra_cumsum.argtypes = [vp, i64, i32, vp, vp, vp]
         l.tra_length_per_key.argtypes = [vp, i32, i32, i32, vp, vp]
+        l.tra_key_totals_begin.argtypes = [vp, i32, i32, i32, i32, vp, ctypes.POINTER(i32), vp]
+        l.tra_key_totals_wait.argtypes = [i32, vp]
         l.tra_permute_2d_lengths.argtypes = [vp, i32, i32, i32, vp, i32, vp, vp]
         l.tra_permute_2d_data.argtypes = [vp, i32, i32, vp, vp, i32, vp, i32, vp, vp, vp, vp]
         l.tra_bucketize_workspace_bytes.argtypes = [i32, i32, i32]

@@ -27,6 +27,14 @@ constexpr int kBlockThreads = kWavesPerBlock * kWaveSize;
 constexpr int kMaxSub = 8;
 constexpr int kMaxPos = 128;
 
+// Where a sequence lookup finds the range of ids of the feature at key position p.
+constexpr int kBoundsOffsets = 0;  // offsets[p * B], offsets[(p + 1) * B]
+constexpr int kBoundsTotals = 1;   // a.offsets is int64 totals[num_keys]: ids per key, at most kMaxTotalKeys keys
+constexpr int kBoundsHost = 2;     // in the launch arguments: class feature ci starts at pw_off[ci], pw_len[ci] ids
+constexpr int kMaxTotalKeys = 256;
+// Sequence kernel: rows a lane group has in flight.
+constexpr int kSequenceUnroll = 4;
+
 // Features of one launch that share LPR (i.e. share dim).
 struct SubClass {
   int32_t first;           // index of the first feature in the class feature list
@@ -34,7 +42,7 @@ struct SubClass {
   int32_t lpr;             // lanes per row
   int32_t tiles_per_feat;  // blocks per feature
   int32_t tile_start;      // first block of this sub-class in the grid
-  int32_t window;          // window kernel: bags per block
+  int32_t window;          // window kernel: bags per block; sequence kernel: ids per tile
   int32_t key0;            // key position of the first feature when the sub-class's features sit
                            // at consecutive key positions (feature fi at key0 + fi), else -1
 };
@@ -67,6 +75,9 @@ struct LookupArgs {
   const float* posw;
   int32_t pw_off[kMaxPos];
   int32_t pw_len[kMaxPos];
+  // Sequence lookup: where a feature's ids lie (kBounds*).
+  int32_t bounds_kind;
+  int32_t num_keys;       // kBoundsTotals: input keys
 #ifdef TRA_INSTRUMENT
   unsigned long long* ts;  // [waves][8] wall-clock stamps
 #endif
@@ -1513,56 +1524,6 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
   }
 }
 
-// ---- sequence lookup: one lane group per id, no reduction -----------------
-// Blocks of feature f stride over that feature's ids
-// [offsets[f*B], offsets[(f+1)*B]); output row j is the dequantized row of
-// indices[j] (zeros for a skipped id).
-template <int DTYPE, int CB, typename IdxT>
-__global__ __launch_bounds__(kBlockThreads) void tbe_nobag_kernel(const LookupArgs a) {
-  constexpr int NE = CB * 8 / Traits<DTYPE>::kBits;
-  int f, lpr, tile;
-  if (!locate_tile(a, f, lpr, tile)) return;
-  const FeatureDesc d = a.descs[f];
-  const int lane = threadIdx.x & (kWaveSize - 1);
-  const int wave = threadIdx.x / kWaveSize;
-  const int gpw = kWaveSize / lpr;
-  const int g = lane / lpr;
-  const int c = lane - g * lpr;
-  if (g >= gpw) return;
-  const int64_t first = load_index<IdxT>(a.offsets, (int64_t)d.feature * a.B);
-  const int64_t last = load_index<IdxT>(a.offsets, (int64_t)(d.feature + 1) * a.B);
-  const int rows_per_block = gpw * kWavesPerBlock;
-  // tiles_per_feat of the sub-class = number of blocks striding over one feature
-  int s = 0;
-#pragma unroll
-  for (int i = 1; i < kMaxSub; ++i)
-    if (i < a.n_sub && (int)blockIdx.x >= a.sub[i].tile_start) s = i;
-  const int64_t stride = (int64_t)a.sub[s].tiles_per_feat * rows_per_block;
-
-  RowWalk w;
-  w.chunk_off = Traits<DTYPE>::kHeader + d.payload_off + c * CB;
-  w.lane_base = a.weights + d.table_offset + w.chunk_off;
-  w.set_rows(d.rows, d.row_bytes);
-  w.count_errors = c == 0 && d.payload_off == 0;
-  w.hdr_lane = lane - c;
-  w.sel0 = mfma_byte_selector(lane, 0);
-  w.sel1 = mfma_byte_selector(lane, 1);
-  for (int64_t j = first + (int64_t)tile * rows_per_block + wave * gpw + g; j < last;
-       j += stride) {
-    RowBuf<CB> r;
-    const IdxT id = reinterpret_cast<const IdxT*>(a.indices)[j];
-    const int bad = fetch_row<DTYPE, CB, false, IdxT>(r, id, (IdxT)j, (IdxT)(a.num_indices - 1), a, w);
-    if (bad && w.count_errors) atomicAdd(a.err_count, 1ull);
-    if (bad && a.bad_to_row0 != 0) r.valid = 1;  // the row fetched for it is row 0
-    float acc[NE];
-#pragma unroll
-    for (int i = 0; i < NE; ++i) acc[i] = 0.0f;
-    consume_row<DTYPE, CB, false, /*WHOLE_WAVE=*/false>(acc, r, w);  // lanes leave this loop one by one
-    store_outputs<NE>(a, j * (int64_t)d.dim + d.payload_off * 8 / Traits<DTYPE>::kBits + (int64_t)c * NE,
-                      acc);
-  }
-}
-
 // ---- host side of one launch ----------------------------------------------
 struct LaunchClass {
   int dtype;
@@ -1583,20 +1544,18 @@ struct LaunchParams {
   int unroll;     // rows per pipeline batch: 2, 4 or 8
   bool idx64;
   bool weighted;
-  bool nobag;
   bool from_lengths;  // window kernel reads lengths and derives offsets itself
 };
 
 template <int DTYPE>
 int launch_lookup(const LookupArgs& a, int cb, const LaunchParams& p, hipStream_t stream);
 
+// The sequence lookup of one class (tbe_sequence.hip).
+int launch_sequence(const LookupArgs& a, int dtype, int cb, bool split, bool idx64, int grid, hipStream_t stream);
+
 template <int DTYPE, int CB, typename IdxT>
 void launch_typed(const LookupArgs& a, const LaunchParams& p, hipStream_t stream) {
   dim3 g(p.grid);
-  if (p.nobag) {
-    hipLaunchKernelGGL((tbe_nobag_kernel<DTYPE, CB, IdxT>), g, dim3(kBlockThreads), 0, stream, a);
-    return;
-  }
 // What the window kernel's first fetches need, repeated as its leading parameters.
 #define TRA_CU_LEADING_ARGS                                                                   \
   a.offsets, a.cdescs, a.B, a.xcd_blocks, a.xcd_count, a.n_sub, a.sub[0].window, a.sub[0].count, \

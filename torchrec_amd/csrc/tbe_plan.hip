@@ -588,6 +588,14 @@ struct PositionWeights {
   int32_t num_keys;
 };
 
+// Where the ids of a sequence lookup's keys lie, when not given by offsets: int64 totals[num_keys] on the device,
+// or the keys' first ids on the host (num_keys + 1 of them).
+struct SequenceBounds {
+  const int64_t* totals_dev;
+  const int64_t* starts;
+  int32_t num_keys;
+};
+
 // Grid and windows of every launch class for one call shape.
 static void compute_geometry(const tra_tbe* tbe, const Tuning& tune, bool balanced, bool nobag,
                              int32_t batch_size, int64_t num_indices, Geometry& g) {
@@ -651,12 +659,19 @@ static void compute_geometry(const tra_tbe* tbe, const Tuning& tune, bool balanc
       const int per_block = kWavesPerBlock * gpw;
       sc.tile_start = grid;
       if (nobag) {
-        // Blocks stride over a feature's ids; enough blocks for ~the average
-        // feature, capped so the grid stays modest.
-        int64_t avg = num_indices > 0 ? num_indices / tbe->num_features + 1 : 4096;
-        int64_t t = (avg + per_block - 1) / per_block;
-        sc.tiles_per_feat = (int)std::max<int64_t>(1, std::min<int64_t>(t, 8192));
-        grid += sc.count * sc.tiles_per_feat;
+        // Ids per tile: one step of the kernel's loop (64 to 256 ids, by the row width), at least
+        // 128 ids; less where that leaves fewer than two tiles per compute unit, down to one id
+        // per lane group.  2.1 M int8 rows of 128 columns: 128 ids a tile 187 us, 256 ids 195 us,
+        // 512 ids 197 us, 64 ids 201 us (8-byte lane chunks: 64 and 128 ids 187 us, 256 ids 197 us).
+        // One block per tile: all of the call's ids may belong to this sub-class, and every feature
+        // may leave a partial tile; blocks stride over the tiles if there are more.  No XCD
+        // remap: consecutive tiles on the same die measured 5 % slower.
+        const int64_t step = (int64_t)per_block * kSequenceUnroll;
+        const int64_t busy = 2 * (int64_t)num_cus;
+        const int64_t full = step >= 128 ? step : (128 + step - 1) / step * step;
+        sc.window = (int)(num_indices >= full * busy ? full : num_indices >= step * busy ? step : per_block);
+        sc.tiles_per_feat = (int)std::min<int64_t>(num_indices / sc.window + sc.count, 1 << 20);
+        grid += sc.tiles_per_feat;
       } else if (balanced) {
         const int64_t nb = (int64_t)sc.count * batch_size;
         int64_t window = tune.window > 0 ? tune.window : (work_per_block + bag_cost(i) - 1) / bag_cost(i);
@@ -703,7 +718,8 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
                         const void* offsets, bool from_lengths, int32_t idx_is_i64,
                         const float* per_sample_weights, int32_t batch_size, int64_t num_indices,
                         int32_t pooling_mode, int32_t out_dtype, void* out, int64_t out_stride,
-                        void* stream, const PositionWeights* pw = nullptr, bool one_stream = false) {
+                        void* stream, const PositionWeights* pw = nullptr, bool one_stream = false,
+                        const SequenceBounds* seq = nullptr) {
   if (!tbe) {
     set_error("tra_tbe_forward: null plan");
     return TRA_ERR_INVALID_ARGUMENT;
@@ -727,7 +743,7 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
     set_error("tra_tbe_forward: num_indices is required");
     return TRA_ERR_INVALID_ARGUMENT;
   }
-  if (!weights || !offsets || !out || (!indices && num_indices != 0)) {
+  if (!weights || (!offsets && !seq) || !out || (!indices && num_indices != 0)) {
     set_error("tra_tbe_forward: null buffer");
     return TRA_ERR_INVALID_ARGUMENT;
   }
@@ -845,6 +861,17 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
       a.posw = pw->table;
       a.psw = nullptr;
     }
+    a.bounds_kind = kBoundsOffsets;
+    if (seq != nullptr) {
+      a.num_keys = seq->num_keys;
+      a.offsets = seq->totals_dev;
+      a.bounds_kind = seq->totals_dev ? kBoundsTotals : kBoundsHost;
+      for (size_t i = 0; !seq->totals_dev && i < cls.feats.size(); ++i) {
+        const int key = tbe->slices[cls.feats[i]].feature;
+        a.pw_off[i] = (int32_t)seq->starts[key];
+        a.pw_len[i] = (int32_t)(seq->starts[key + 1] - seq->starts[key]);
+      }
+    }
     a.out = out;
     a.out_stride = out_stride;
     a.bad_to_row0 = tbe->bad_to_row0.load(std::memory_order_relaxed);
@@ -871,9 +898,13 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
     lp.unroll = geo_local.tune.unroll;
     lp.idx64 = idx_is_i64 != 0;
     lp.weighted = a.psw != nullptr || a.posw != nullptr;
-    lp.nobag = nobag;
     lp.from_lengths = from_lengths;
     int rc;
+    if (nobag) {
+      rc = launch_sequence(a, cls.dtype, cls.cb, cls.split, lp.idx64, lp.grid, s);
+      if (rc != TRA_OK) return join(rc);
+      continue;
+    }
     switch (cls.dtype) {
       case TRA_INT8:
         rc = cls.split ? launch_lookup<TRA_INT8 + kSplitHeader>(a, cls.cb, lp, s) : launch_lookup<TRA_INT8>(a, cls.cb, lp, s);
@@ -898,6 +929,38 @@ int tra_tbe_forward(tra_tbe_t tbe, const void* weights, const void* indices,
                     int32_t out_dtype, void* out, int64_t out_stride, void* stream) {
   return forward_impl(tbe, weights, indices, offsets, false, idx_is_i64, per_sample_weights,
                       batch_size, num_indices, pooling_mode, out_dtype, out, out_stride, stream);
+}
+
+int tra_tbe_forward_sequence(tra_tbe_t tbe, const void* weights, const void* indices, const int64_t* key_totals,
+                             const int64_t* key_starts, int32_t num_keys, int32_t idx_is_i64, int64_t num_indices,
+                             int32_t out_dtype, void* out, void* stream) {
+  if (!tbe) {
+    set_error("tra_tbe_forward_sequence: null plan");
+    return TRA_ERR_INVALID_ARGUMENT;
+  }
+  if ((key_totals == nullptr) == (key_starts == nullptr) || num_keys < 1 || tbe->max_key_pos >= num_keys) {
+    set_error("tra_tbe_forward_sequence: one of key_totals and key_starts, for every key a feature sits at");
+    return TRA_ERR_INVALID_ARGUMENT;
+  }
+  if (key_totals != nullptr && (num_keys > kMaxTotalKeys || (uintptr_t)key_totals % 8 != 0)) {
+    set_error("tra_tbe_forward_sequence: %d keys on the device (at most %d, 8-byte aligned)", num_keys, kMaxTotalKeys);
+    return TRA_ERR_UNSUPPORTED;
+  }
+  if (key_starts != nullptr) {
+    if (tbe->max_class_feats > (size_t)kMaxPos || num_indices > 0x7fffffff) {
+      set_error("tra_tbe_forward_sequence: a launch class of %d features (at most %d) or %lld ids",
+                (int)tbe->max_class_feats, kMaxPos, (long long)num_indices);
+      return TRA_ERR_UNSUPPORTED;
+    }
+    for (int k = 0; k < num_keys; ++k)
+      if (key_starts[k] < 0 || key_starts[k + 1] < key_starts[k] || key_starts[k + 1] > num_indices) {
+        set_error("tra_tbe_forward_sequence: key %d lies outside the %lld ids", k, (long long)num_indices);
+        return TRA_ERR_INVALID_ARGUMENT;
+      }
+  }
+  const SequenceBounds seq{key_totals, key_starts, num_keys};
+  return forward_impl(tbe, weights, indices, nullptr, false, idx_is_i64, nullptr, 1, num_indices, TRA_POOL_NONE,
+                      out_dtype, out, 0, stream, nullptr, false, &seq);
 }
 
 int64_t tra_tbe_forward_lengths_workspace_bytes(int32_t num_keys, int32_t batch_size,

@@ -13,6 +13,8 @@ quantization and bucketization have no host form.
 """
 from __future__ import annotations
 
+import ctypes
+from array import array
 from typing import List, Optional, Tuple
 
 import torch
@@ -51,10 +53,45 @@ def asynchronous_complete_cumsum(lengths: torch.Tensor) -> torch.Tensor:
     return out
 
 
+# Keys whose totals a lookup takes from the device, and that reach the host without a copy.
+_MAX_TOTAL_KEYS = 256
+_MAX_HOST_KEYS = 1024
+
+
+def key_totals_begin(bags: torch.Tensor, bags_are_offsets: bool, num_keys: int, stride: int, on_device: bool):
+    """Ids per key of a feature-major KJT on the GPU, from its lengths or its offsets: ``(totals, finish)``.
+    The adding-up is queued now; ``totals`` is the int64 device tensor when ``on_device``, ``finish()`` waits for
+    that kernel alone and returns the list (it has to be called, also when something raises in between).  None
+    when the totals cannot come this way (too many keys or calls at once, stream capture)."""
+    _check_int(bags, "offsets" if bags_are_offsets else "lengths")
+    assert bags.numel() >= num_keys * stride + int(bags_are_offsets), "bag bounds shorter than the keys they must cover"
+    if num_keys > _MAX_HOST_KEYS or stride == 0:
+        return None
+    bags = bags.contiguous()
+    dev = bags.device
+    totals = torch.empty(num_keys, dtype=torch.int64, device=dev) if on_device else None
+    ticket = ctypes.c_int32(-1)
+    l = _lib.lib()
+    rc = l.tra_key_totals_begin(
+        bags.data_ptr(), int(bags_are_offsets), num_keys, stride, int(bags.dtype == torch.int64),
+        _lib.ptr(totals), ctypes.byref(ticket), _lib.current_stream(dev),
+    )
+    if rc in (_lib.ERR_TOO_LARGE, _lib.ERR_UNSUPPORTED):
+        return None
+    _lib.check(rc)
+
+    def finish() -> List[int]:
+        host = array("q", bytes(8 * num_keys))
+        _lib.check(l.tra_key_totals_wait(ticket.value, host.buffer_info()[0]))
+        return host.tolist()
+
+    return totals, finish
+
+
 def length_per_key(lengths: torch.Tensor, num_features: int, stride: int) -> List[int]:
     """Per-feature totals of a feature-major [F * B] lengths tensor as a Python list.
 
-    One reduction kernel and one F-element device-to-host copy (the reference
+    One reduction kernel whose results the host reads from pinned memory (the reference
     does torch.sum(lengths.view(F, B), 1).tolist(), jagged_tensor.py:1201-1212).
     """
     if num_features == 0:
@@ -64,6 +101,16 @@ def length_per_key(lengths: torch.Tensor, num_features: int, stride: int) -> Lis
     _check_int(lengths, "lengths")
     if lengths.device.type != "cuda":
         return torch.sum(lengths.reshape(num_features, stride), dim=1).tolist()
+    return length_per_key_async(lengths, num_features, stride)()
+
+
+def length_per_key_async(lengths: torch.Tensor, num_features: int, stride: int):
+    """``length_per_key`` split in two: the reduction is queued now, the returned function waits for it alone and
+    yields the Python list.  Work queued on the current stream afterwards (a lookup, say) does not hold the host up."""
+    _check_int(lengths, "lengths")
+    begun = key_totals_begin(lengths, False, num_features, stride, on_device=False)
+    if begun is not None:
+        return begun[1]
     lengths = lengths.contiguous()
     out = torch.empty(num_features, dtype=torch.int64, device=lengths.device)
     _lib.check(
@@ -72,54 +119,7 @@ def length_per_key(lengths: torch.Tensor, num_features: int, stride: int) -> Lis
             _lib.ptr(out), _lib.current_stream(lengths.device),
         )
     )
-    return out.tolist()
-
-
-_side_streams: dict = {}  # device index -> a second stream (default priority) for small reads that need not order with the main one
-
-
-def _side_stream(device: torch.device) -> "torch.cuda.Stream":
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    s = _side_streams.get(idx)
-    if s is None:
-        s = _side_streams[idx] = torch.cuda.Stream(device=idx)
-    return s
-
-
-def length_per_key_async(lengths: torch.Tensor, num_features: int, stride: int):
-    """``length_per_key`` split in two: the reduction and its copy to pinned host memory are queued now, on a
-    second stream that waits for what the current stream holds at this moment (whatever produced ``lengths``),
-    and the returned function waits for that copy alone and yields the Python list.  Work queued on the
-    current stream afterwards (a lookup, say) neither waits for the reduction nor holds the host up.
-    ``lengths`` must stay alive until the returned function has been called."""
-    _check_int(lengths, "lengths")
-    lengths = lengths.contiguous()
-    dev = lengths.device
-    side = _side_stream(dev)
-    side.wait_stream(torch.cuda.current_stream(dev))
-    with torch.cuda.stream(side):
-        out = torch.empty(num_features, dtype=torch.int64, device=dev)
-        _lib.check(
-            _lib.lib().tra_length_per_key(
-                _lib.ptr(lengths), num_features, stride, int(lengths.dtype == torch.int64),
-                _lib.ptr(out), _lib.current_stream(dev),
-            )
-        )
-        host = torch.empty(num_features, dtype=torch.int64, pin_memory=True)
-        host.copy_(out, non_blocking=True)
-        arrived = torch.cuda.Event()
-        arrived.record(side)
-
-    # The side stream reads ``lengths`` (possibly a contiguous copy made above, which nobody else
-    # holds): the allocator is told so, and the returned function keeps the tensor until the copy
-    # has arrived, so that its memory is not handed to a later allocation of the current stream.
-    lengths.record_stream(side)
-
-    def finish(_held=lengths) -> List[int]:
-        arrived.synchronize()
-        return host.tolist()
-
-    return finish
+    return out.tolist
 
 
 def permute_2D_sparse_data(
@@ -374,8 +374,6 @@ def mch_remap_keys(
 ) -> torch.Tensor:
     """``mch_remap`` for every key of a KeyedJaggedTensor in one launch: key ``k`` (ids
     ``values[offsets[k*B] : offsets[(k+1)*B]]``) is looked up in ``sorted_ids[k]`` / ``mappings[k]``."""
-    import ctypes
-
     _lib.require_gpu(values, "mch_remap_keys")
     _check_int(values, "values")
     K = len(sorted_ids)

@@ -623,8 +623,8 @@ class EmbeddingBagCollection(EmbeddingBagCollectionInterface, ModuleNoCopyMixin,
         return self._device
 
 
-# The lookup kernel keeps the position-weight layout of a launch in its launch
-# arguments: at most this many features per operator.
+# The lookup kernels keep the position-weight layout (or a sequence lookup's key
+# starts) of a launch in its launch arguments: at most this many features per operator.
 _MAX_FUSED_POSITION_FEATURES = 128
 
 
@@ -817,43 +817,43 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
             order = list(range(len(order)))
         B = features.stride()
         indices = features.values()
-        offsets = features.offsets()
-        lengths = features.lengths()
         L = indices.numel()
-        # Row ranges of the input keys: one small device-to-host copy.  Where the
-        # KJT does not carry the per-key counts, their reduction and copy are
-        # queued in front of the lookup and waited for behind its launch: the
-        # host then waits for work that is already queued and builds the output
-        # views while the lookup runs, and the lookup never waits for the host.
+        K = len(kjt_keys)
+        # The lookups need to know where each key's ids lie, the output's row ranges need it on the
+        # host.  A KJT that carries its per-key counts gives both.  Otherwise one kernel adds them
+        # up, the lookups queued behind it read them on the device, and the host reads them from
+        # pinned memory while the lookups run and builds the output views meanwhile: no offsets are
+        # computed, and neither side waits for the other.
         counts_later = None
-        if (
-            features.length_per_key_or_none() is None
-            and features.offset_per_key_or_none() is None
-            and indices.is_cuda
-            and kjt_keys
-            and L > 0
-            and B > 0
-        ):
-            counts_later = ops.length_per_key_async(features.lengths(), len(kjt_keys), B)
-        else:
+        bounds: Dict[str, Any] = {}
+        on_gpu = indices.is_cuda and K > 0 and L > 0 and B > 0
+        if features.length_per_key_or_none() is not None or features.offset_per_key_or_none() is not None or not on_gpu:
             offset_per_key = features.offset_per_key()
-        lookup = torch.empty((L, self._embedding_dim), dtype=self._output_dtype, device=indices.device)
+            if on_gpu and self._starts_fit(offset_per_key, L):
+                bounds = {"offsets": None, "key_starts": offset_per_key}
+        else:
+            built_from_offsets = features.lengths_or_none() is None
+            begun = ops.key_totals_begin(
+                features.offsets() if built_from_offsets else features.lengths(), built_from_offsets, K, B,
+                on_device=K <= ops._MAX_TOTAL_KEYS,
+            )
+            if begun is None:
+                counts_later = ops.length_per_key_async(features.lengths(), K, B)
+            else:
+                totals, counts_later = begun
+                if totals is not None:
+                    bounds = {"offsets": None, "key_totals": totals}
         try:
-            f0 = 0
-            for emb_module, n_feat in zip(self._emb_modules, self._feature_splits):
+            if not bounds:
+                bounds = {"offsets": features.offsets()}
+            lookup = torch.empty(L, self._embedding_dim, dtype=self._output_dtype, device=indices.device)
+            for emb_module, positions in zip(self._emb_modules, self._group_positions(order)):
                 # (a registered operator is called as a module, torchrec/quant/embedding_modules.py:938-942)
                 call = emb_module if self.register_tbes else emb_module.forward
-                call(
-                    indices=indices,
-                    offsets=offsets,
-                    feature_positions=order[f0 : f0 + n_feat],
-                    batch_size=B,
-                    out=lookup,
-                )
-                f0 += n_feat
+                call(indices=indices, feature_positions=positions, batch_size=B, out=lookup, **bounds)
+            lengths = features.lengths()
         finally:
-            # The reduction queued on the side stream reads the KJT's lengths: it is waited for
-            # also when a lookup raises, before anything of this call is released.
+            # The totals are waited for also when a lookup raises, before anything of this call is released.
             if counts_later is not None:
                 features._length_per_key = counts_later()  # the KJT remembers them, as length_per_key() would
         if counts_later is not None:
@@ -881,17 +881,22 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
             for embedding_name in self._embedding_names_by_batched_tables[key]:
                 pos = order[f]
                 start, end = offset_per_key[pos], offset_per_key[pos + 1]
-                rows = self._rows_for(lookup, f, start, end)
                 feature_embeddings[embedding_name] = JaggedTensor(
-                    values=rows,
+                    values=lookup[start:end],
                     lengths=lengths_rows[pos],
                     weights=indices[start:end] if self._need_indices else None,
                 )
                 f += 1
         return feature_embeddings
 
-    def _rows_for(self, lookup: Tensor, f: int, start: int, end: int) -> Tensor:
-        return lookup[start:end]
+    def _starts_fit(self, offset_per_key: List[int], num_indices: int) -> bool:
+        """Whether the operators can take these key starts as launch arguments."""
+        return (
+            max(self._feature_splits, default=0) <= _MAX_FUSED_POSITION_FEATURES
+            and num_indices < 2**31
+            and all(a <= b for a, b in zip(offset_per_key, offset_per_key[1:]))
+            and offset_per_key[-1] <= num_indices
+        )
 
     @classmethod
     def from_float(

@@ -28,6 +28,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+from array import array
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
@@ -418,6 +419,8 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
         out_col: int = 0,
         lengths: Optional[Tensor] = None,
         position_weights: Optional[Tuple[Tensor, Sequence[int], Sequence[int]]] = None,
+        key_totals: Optional[Tensor] = None,
+        key_starts: Optional[Sequence[int]] = None,
     ) -> Tensor:
         """Pooled: ``[B, total_D]``; ``PoolingMode.NONE``: ``[indices.numel(), D]``.
 
@@ -435,7 +438,11 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
         ``(table, key_start, key_len)`` replaces ``per_sample_weights`` by
         weights looked up inside the kernel: the id at position ``k`` of a bag
         of input key ``p`` gets ``table[key_start[p] + min(k, key_len[p] - 1)]``
-        (1 when ``key_len[p]`` is 0); ``table`` is one fp32 device tensor.
+        (1 when ``key_len[p]`` is 0); ``table`` is one fp32 device tensor.  A
+        sequence lookup (``PoolingMode.NONE``) needs no bag bounds, only where
+        every input key's ids lie: with ``offsets=None`` it takes the ids per key
+        as an int64 device tensor (``key_totals``) or the keys' first ids and the
+        end as integers (``key_starts``).
         """
         dev = self.current_device
         if dev.type != "cuda":
@@ -454,6 +461,8 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
             raise TypeError(f"indices must be int32 or int64, got {idt}")
         if not indices.is_contiguous():
             indices = indices.contiguous()
+        if offsets is None and (key_totals is not None or key_starts is not None):
+            return self._forward_sequence(indices, feature_positions, key_totals, key_starts, out)
         if offsets is None:
             assert lengths is not None and batch_size is not None, "offsets=None needs lengths and batch_size"
             if not lengths.is_cuda:
@@ -549,6 +558,51 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
                     self.output_dtype, out_ptr, out_stride, _lib.current_stream(dev),
                 )
             )
+        if _ENV_BOUNDS_CHECK or self.bounds_check_mode_int == _BOUNDS_FATAL:
+            bad = self.out_of_range_count()
+            if bad:
+                raise IndexError(f"{bad} embedding indices were out of range")
+        return out
+
+    def _forward_sequence(
+        self,
+        indices: Tensor,
+        feature_positions: Optional[Sequence[int]],
+        key_totals: Optional[Tensor],
+        key_starts: Optional[Sequence[int]],
+        out: Optional[Tensor],
+    ) -> Tensor:
+        """``forward`` of a sequence lookup from key totals or key starts (``indices`` checked by the caller)."""
+        assert self.pooling_mode == PoolingMode.NONE, "key_totals / key_starts belong to sequence lookups"
+        dev = self.current_device
+        positions: Optional[Tuple[int, ...]] = None
+        if feature_positions is not None:
+            positions = tuple(feature_positions)
+            if positions == self._identity_positions:
+                positions = None
+        L = indices.numel()
+        out_dtype = torch.float16 if self.output_dtype == _lib.FP16 else torch.float32
+        if out is None:
+            out = torch.empty((L, self.max_D), dtype=out_dtype, device=dev)
+        else:
+            assert out.dtype == out_dtype and out.get_device() == dev.index and out.dim() == 2 and out.is_contiguous()
+            assert out.shape[0] >= L and out.shape[1] == self.max_D
+        totals_ptr, starts_ptr = None, None
+        if key_totals is not None:
+            assert key_totals.dtype == torch.int64 and key_totals.get_device() == dev.index and key_totals.is_contiguous()
+            totals_ptr, num_keys = key_totals.data_ptr(), key_totals.numel()
+        else:
+            starts = array("q", key_starts)
+            starts_ptr, num_keys = starts.buffer_info()[0], len(starts) - 1
+        plan = self._plan_address.get(positions)
+        if plan is None:
+            plan = self._plan_address[positions] = self._get_plan(positions).value
+        rc = _lib.lib().tra_tbe_forward_sequence(
+            plan, self._buffers["weights_dev"].data_ptr(), indices.data_ptr(), totals_ptr, starts_ptr, num_keys,
+            int(indices.dtype is torch.int64), L, self.output_dtype, out.data_ptr(), _lib.current_stream(dev),
+        )
+        if rc != 0:
+            _lib.check(rc)
         if _ENV_BOUNDS_CHECK or self.bounds_check_mode_int == _BOUNDS_FATAL:
             bad = self.out_of_range_count()
             if bad:
