@@ -382,6 +382,21 @@ int tra_mch_remap_keys(const void* values, int64_t n, const void* offsets, int32
                        const int64_t* const* mapping, const int64_t* table_size,
                        const int64_t* miss_id, void* out, void* stream);
 
+/* A KeyedJaggedTensor's keys in another order, in one launch: output key j is
+ * input key permute[j] (HOST array; keys may repeat or be left out).  Its ids
+ * (and weights, and lengths; either output may be null) are copied, or, with
+ * sorted_ids / mapping / table_size / miss_id (HOST arrays over the OUTPUT
+ * keys, null for a plain copy), remapped as above on the way; remapped values
+ * are integers of value_bytes bytes.  key_totals: device, ids per input key
+ * (tra_key_totals_begin).  At most 256 keys on either side. */
+int tra_permute_keys(const int64_t* key_totals, int32_t num_keys, const int32_t* permute,
+                     int32_t num_out_keys, int32_t batch_size, const void* lengths,
+                     int32_t lengths_i64, void* out_lengths, const void* values,
+                     int64_t num_values, int32_t value_bytes, void* out_values,
+                     int64_t num_out_values, const float* weights, float* out_weights,
+                     const int64_t* const* sorted_ids, const int64_t* const* mapping,
+                     const int64_t* table_size, const int64_t* miss_id, void* stream);
+
 /* Column regroup of pooled outputs ------------------------------------------- */
 /* Copies num_blocks column blocks between row-major matrices of `rows` rows:
  * block k is width[k] elements of every row, read at src[k] with row stride

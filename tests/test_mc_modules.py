@@ -164,3 +164,72 @@ def test_collection_remaps_all_keys_in_one_launch(idt):
     assert out.values().cpu().tolist() == want
     assert out.lengths().cpu().tolist() == np.concatenate(
         [lengths[keys.index(k) * B:(keys.index(k) + 1) * B] for k in out.keys()]).tolist()
+
+
+def _remap_numpy(values, sorted_ids, mapping, miss):
+    """First index in [0, size - 1] whose entry is >= the id, searched over the first size - 1 entries."""
+    at = np.searchsorted(sorted_ids[:-1], values)
+    return np.where(sorted_ids[at] == values, mapping[at], miss)
+
+
+@pytest.mark.gpu
+# Around the four entries of a read, the 512 pivots of a block, and segments of many entries.
+@pytest.mark.parametrize("size", [1, 2, 3, 4, 5, 9, 511, 512, 513, 514, 1026, 5000, 70_001])
+@pytest.mark.parametrize("kind", ["even", "clustered", "geometric", "half empty", "repeats"])
+def test_remap_search(size, kind):
+    rng = np.random.default_rng(size)
+    if kind == "clustered":
+        ids = np.concatenate([c + rng.integers(0, 3 * size, size) for c in rng.integers(-2**62, 2**62, 7)])[:size]
+    elif kind == "geometric":
+        ids = np.exp(rng.uniform(0, 43, size)).astype(np.int64)
+    elif kind == "repeats":
+        ids = rng.integers(0, max(1, size // 3), size)
+    else:
+        ids = rng.integers(-2**40, 2**40, size)
+    table = np.sort(ids.astype(np.int64))
+    if kind == "half empty":
+        table[size // 2:] = np.iinfo(np.int64).max
+    table[-1] = np.iinfo(np.int64).max
+    mapping = rng.permutation(size).astype(np.int64)
+    values = np.concatenate([table, table - 1, table + np.where(table == np.iinfo(np.int64).max, 0, 1),
+                             rng.integers(-2**41, 2**41, 1500), [np.iinfo(np.int64).min, np.iinfo(np.int64).max, 0]])
+    dev = torch.device("cuda:0")
+    got = ops.mch_remap(torch.from_numpy(values).to(dev), torch.from_numpy(table).to(dev), torch.from_numpy(mapping).to(dev), 77)
+    assert np.array_equal(got.cpu().numpy(), _remap_numpy(values, table, mapping, 77))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,B", [(1, 1), (3, 5), (70, 9), (256, 2), (257, 2)])
+@pytest.mark.parametrize("shuffled", [False, True])
+@pytest.mark.parametrize("given", ["lengths", "offsets"])
+def test_collection_remap_many_keys(K, B, shuffled, given):
+    """More keys than a launch has tables, more than the one-launch route takes; keys without ids."""
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(K)
+    configs = [EmbeddingConfig(name=f"t{k}", embedding_dim=4, num_embeddings=50 + k, feature_names=[f"f{k}"]) for k in range(K)]
+    modules, tables = {}, {}
+    for c in configs:
+        raw = rng.choice(10_000, 30, replace=False)
+        modules[c.name] = MCHManagedCollisionModule(c.num_embeddings, dev)
+        modules[c.name].set_id_table(torch.from_numpy(raw), torch.arange(30) * 1)
+        tables[c.feature_names[0]] = (modules[c.name]._mch_sorted_raw_ids.cpu().numpy(),
+                                      modules[c.name]._mch_remapped_ids_mapping.cpu().numpy(), c.num_embeddings - 1)
+    mcc = ManagedCollisionCollection(modules, configs).eval()
+    keys = [f"f{k}" for k in (rng.permutation(K) if shuffled else range(K))]
+    lengths = rng.integers(0, 12, (K, B))
+    lengths[rng.random(K) < 0.3] = 0
+    values = [rng.integers(0, 10_000, n) for n in lengths.sum(1)]
+    weights = torch.rand(int(lengths.sum()), device=dev)
+    bags = torch.from_numpy(lengths.reshape(-1)).to(dev)
+    if given == "offsets":
+        bags = ops.asynchronous_complete_cumsum(bags)
+    kjt = KeyedJaggedTensor(keys=keys, values=torch.from_numpy(np.concatenate(values)).to(dev), weights=weights, **{given: bags})
+    out = mcc(kjt)
+    order = [keys.index(f"f{k}") for k in range(K)]
+    assert out.keys() == [f"f{k}" for k in range(K)]
+    want = np.concatenate([_remap_numpy(values[i], *tables[keys[i]]) for i in order])
+    assert np.array_equal(out.values().cpu().numpy(), want)
+    assert np.array_equal(out.lengths().cpu().numpy(), lengths[order].reshape(-1))
+    starts = np.concatenate([[0], np.cumsum(lengths.sum(1))])
+    assert torch.equal(out.weights(), torch.cat([weights[starts[i]:starts[i + 1]] for i in order]))
+    assert out.length_per_key() == lengths.sum(1)[order].tolist()

@@ -325,3 +325,30 @@ def test_quantize_rows_padded_bytes(bits, dim, rows, extra, tail):
     assert np.array_equal(table[:, :4], want[:, payload:]) and np.array_equal(table[:, 4 : 4 + payload], want[:, :payload])
     assert not table[:, 4 + payload :].any() and not got[rows * stride : rows * stride + tail].any()
     assert (got[rows * stride + tail :] == 0xAB).all()
+
+
+@pytest.mark.parametrize("K,B,max_len", [(1, 1, 3), (4, 300, 40), (65, 7, 20), (256, 3, 9), (300, 2, 9), (3, 2, 9000)])
+@pytest.mark.parametrize("pick", ["all", "some", "repeats"])
+@pytest.mark.parametrize("idt,vdt", [(torch.int32, torch.int64), (torch.int64, torch.int32)])
+def test_kjt_permute(K, B, max_len, pick, idt, vdt):
+    """One launch for ids, weights and lengths: every key once, a subset, keys taken more than once, an ids tensor that
+    is longer than the bags, tiles of one and of several steps, more keys than the launch takes."""
+    from torchrec_amd import KeyedJaggedTensor
+
+    rng = np.random.default_rng(K * B)
+    lengths = rng.integers(0, max_len + 1, (K, B))
+    lengths[rng.random(K) < 0.2] = 0
+    n = int(lengths.sum())
+    values = torch.from_numpy(rng.integers(0, 1000, n + 5)).to(DEV, vdt)
+    weights = torch.rand(n + 5, device=DEV)
+    order = rng.permutation(K).tolist()
+    order = order if pick == "all" else order[: (K + 1) // 2] if pick == "some" else order + order[:3]
+    kjt = KeyedJaggedTensor(keys=[f"k{i}" for i in range(K)], values=values, weights=weights,
+                            lengths=torch.from_numpy(lengths.reshape(-1)).to(DEV, idt))
+    got = kjt.permute(order)
+    starts = np.concatenate([[0], np.cumsum(lengths.sum(1))])
+    assert got.keys() == [f"k{i}" for i in order] and got.lengths().dtype == idt
+    assert np.array_equal(got.lengths().cpu().numpy(), lengths[order].reshape(-1))
+    assert torch.equal(got.values(), torch.cat([values[starts[i]:starts[i + 1]] for i in order]))
+    assert torch.equal(got.weights(), torch.cat([weights[starts[i]:starts[i + 1]] for i in order]))
+    assert got.length_per_key() == lengths.sum(1)[order].tolist()

@@ -8,6 +8,7 @@ gfx950 device, every entry point here raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Optional
 
@@ -51,6 +52,7 @@ EXPORTED_SYMBOLS = [
     "tra_position_weights",
     "tra_mch_remap",
     "tra_mch_remap_keys",
+    "tra_permute_keys",
     "tra_regroup_columns",
     "tra_regroup_tensors",
     "tra_copy_bytes",
@@ -115,7 +117,7 @@ def lib() -> ctypes.CDLL:
         l.tra_cumsum_workspace_bytes.restype = i64
         l.tra_cumsum.argtypes = [vp, i64, i32, vp, vp, vp]
         l.tra_length_per_key.argtypes = [vp, i32, i32, i32, vp, vp]
-        l.tra_key_totals_begin.argtypes = [vp, i32, i32, i32, i32, vp, ctypes.POINTER(i32), vp]
+        l.tra_key_totals_begin.argtypes = [vp, i32, i32, i32, i32, vp, vp, vp]
         l.tra_key_totals_wait.argtypes = [i32, vp]
         l.tra_permute_2d_lengths.argtypes = [vp, i32, i32, i32, vp, i32, vp, vp]
         l.tra_permute_2d_data.argtypes = [vp, i32, i32, vp, vp, i32, vp, i32, vp, vp, vp, vp]
@@ -133,13 +135,15 @@ def lib() -> ctypes.CDLL:
             vp, i64, vp, i32, i32, i32, ctypes.POINTER(vp), ctypes.POINTER(vp), ctypes.POINTER(i64),
             ctypes.POINTER(i64), vp, vp,
         ]
+        l.tra_permute_keys.argtypes = [
+            vp, i32, vp, i32, i32, vp, i32, vp, vp, i64, i32, vp, i64, vp, vp, vp, vp, vp, vp, vp,
+        ]
         l.tra_regroup_columns.argtypes = [
             ctypes.POINTER(vp), ctypes.POINTER(i64), ctypes.POINTER(vp), ctypes.POINTER(i64), ctypes.POINTER(i32),
             i32, i64, i32, vp,
         ]
         l.tra_regroup_tensors.argtypes = [
-            ctypes.POINTER(vp), ctypes.POINTER(i64), i32, ctypes.POINTER(vp), ctypes.POINTER(i64), i32,
-            vp, i32, i64, i32, vp,
+            vp, vp, i32, vp, vp, i32, vp, i32, i64, i32, vp,
         ]
         l.tra_copy_bytes.argtypes = [vp, vp, i64, vp]
         _lib = l
@@ -160,28 +164,16 @@ def forward_lengths_entry():
     return _fastcall.forward_lengths
 
 
-def regroup_entry(fast: bool = True):
-    """``tra_regroup_tensors`` as a callable ``(src, src_stride, dst, dst_stride, blocks, num_blocks, rows,
-    elem_bytes, stream)`` of lists of integers and integers: through the extension module when it is
-    there (at most 64 tensors on a side), else (or with ``fast=False``) through ctypes."""
-    l = lib()
+def entry(name: str):
+    """Entry point ``name``, all of whose arguments are integers or pointers, as a callable of integers (addresses
+    as ints, ``None`` for a null pointer) returning its code: through the in-tree extension module when it is
+    there, else the ctypes function; the same symbol of the same library either way."""
+    fn = getattr(lib(), name)
     try:
         from torchrec_amd import _fastcall
     except ImportError:
-        fast = False
-    if not fast:
-        vp, i64 = ctypes.c_void_p, ctypes.c_int64
-
-        def call(src, src_stride, dst, dst_stride, blocks, num_blocks, rows, elem_bytes, stream):
-            ns, nd = len(src), len(dst)
-            return l.tra_regroup_tensors(
-                (vp * ns)(*src), (i64 * ns)(*src_stride), ns, (vp * nd)(*dst), (i64 * nd)(*dst_stride), nd,
-                blocks, num_blocks, rows, elem_bytes, stream,
-            )
-
-        return call
-    _fastcall.bind_regroup(ctypes.cast(l.tra_regroup_tensors, ctypes.c_void_p).value)
-    return _fastcall.regroup_tensors
+        return fn
+    return functools.partial(_fastcall.call, ctypes.cast(fn, ctypes.c_void_p).value)
 
 
 def check(rc: int) -> None:

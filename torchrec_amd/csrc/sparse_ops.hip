@@ -13,6 +13,7 @@ namespace tra {
 // (native vectors: an array of HIP's uint4 objects is kept in scratch memory, which doubled the regroup kernel's time)
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+typedef int64_t i64x2_t __attribute__((ext_vector_type(2), aligned(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kScanThreads = 256;
@@ -31,6 +32,16 @@ __device__ __forceinline__ void st(void* p, int64_t i, int64_t v) {
 __device__ __forceinline__ int64_t wave_sum(int64_t v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+// Inclusive scan over a wave.
+__device__ __forceinline__ int64_t wave_scan(int64_t v, int lane) {
+#pragma unroll
+  for (int off = 1; off < kWaveSize; off <<= 1) {
+    const int64_t o = __shfl_up(v, off, 64);
+    if (lane >= off) v += o;
+  }
   return v;
 }
 
@@ -725,57 +736,226 @@ __global__ __launch_bounds__(kWalkThreads) void position_weights_kernel(
   }
 }
 
-// ---- id remapping through a sorted table --------------------------------------
-// out[j] = mapping[i] when sorted_ids[i] == values[j] with i the first index in
-// [0, size-1] whose entry is >= values[j] (searched over the first size-1
-// entries; the last one is the table's delimiter), else miss_id.
-template <typename T>
-__global__ void mch_remap_kernel(const void* values, int64_t n, const int64_t* sorted_ids,
-                                 const int64_t* mapping, int64_t size, int64_t miss_id, void* out) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += stride) {
-    const int64_t v = ld<T>(values, j);
-    int64_t lo = 0, hi = size - 1;  // lower bound in [0, size - 1)
-    while (lo < hi) {
-      const int64_t mid = lo + ((hi - lo) >> 1);
-      if (sorted_ids[mid] < v) lo = mid + 1; else hi = mid;
-    }
-    st<T>(out, j, sorted_ids[lo] == v ? mapping[lo] : miss_id);
-  }
-}
+// ---- ids moved key by key, with or without a remap -------------------------------
+// Output key j of a launch is input key perm[j]: its ids (and weights, and
+// lengths) are one contiguous run on both sides.  With REMAP every id goes
+// through its key's sorted table on the way:
+//   out = mapping[i] when sorted_ids[i] == id, with i the first index in
+//   [0, size-1] whose entry is >= id (searched over the first size-1 entries;
+//   the last one is the table's delimiter), else miss_id.
+constexpr int kMoveThreads = 512;
+constexpr int kMoveKeys = 256;   // input keys, and output keys, of a call
+constexpr int kRemapKeys = 64;   // keys with a table per launch
+constexpr int kPivots = 512;     // entries of a table that a block keeps in LDS
 
-// The same remap for every key of a KJT in one launch: blockIdx.y is the key,
-// its ids are values[offsets[key*B] .. offsets[(key+1)*B]) and it has its own
-// sorted table.  Tables travel in the launch arguments, kRemapKeys per launch.
-constexpr int kRemapKeys = 64;
+// Where the input keys' ids lie.
+constexpr int kKeysTotals = 0;   // int64 totals[num_in] on the device
+constexpr int kKeysOffsets = 1;  // offsets[k * B]; output positions are the input's
+constexpr int kKeysOne = 2;      // one key, all num_values ids
+
 struct RemapTables {
   const int64_t* sorted_ids[kRemapKeys];
   const int64_t* mapping[kRemapKeys];
   int64_t size[kRemapKeys];
   int64_t miss_id[kRemapKeys];
-  int32_t first_key;  // key of blockIdx.y == 0
+};
+struct MoveArgs {
+  const void* bounds;
+  const void* values;
+  void* out_values;
+  const float* weights;
+  float* out_weights;
+  const void* lengths;
+  void* out_lengths;
+  int64_t num_values;
+  int64_t out_values_end;  // ids the output holds
+  int32_t kind;
+  int32_t bounds_i64;
+  int32_t lengths_i64;
+  int32_t num_in;
+  int32_t num_out;     // output keys of the call
+  int32_t first_key;   // output keys of this launch: first_key .. first_key + launch_keys
+  int32_t launch_keys;
+  int32_t B;
+  int32_t tile;          // ids per tile
+  int32_t tile_blocks;   // blocks that move ids (they stride over the tiles); the ones behind them move lengths
+  int16_t perm[kMoveKeys];
 };
 
-template <typename T>
-__global__ void mch_remap_keys_kernel(const void* values, int64_t n, const void* offsets, int32_t B,
-                                      const RemapTables t, void* out) {
-  const int k = blockIdx.y;
-  const int64_t key = (int64_t)t.first_key + k;
-  int64_t first = ld<T>(offsets, key * B), last = ld<T>(offsets, (key + 1) * B);
-  first = first < 0 ? 0 : first;
-  last = last > n ? n : last;
-  const int64_t* sorted_ids = t.sorted_ids[k];
-  const int64_t* mapping = t.mapping[k];
-  const int64_t size = t.size[k], miss_id = t.miss_id[k];
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t j = first + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < last; j += stride) {
-    const int64_t v = ld<T>(values, j);
-    int64_t lo = 0, hi = size - 1;
-    while (lo < hi) {
-      const int64_t mid = lo + ((hi - lo) >> 1);
-      if (sorted_ids[mid] < v) lo = mid + 1; else hi = mid;
+// First index in [0, n] whose entry is >= v, and that entry; n < 1 or no such
+// index below n: n.  `pivots`: entry min((i + 1) * seg, n) - 1 for i < kPivots.
+//
+// Bound by the reads of the table, one behind the other and each lane in a line
+// of its own: a bisection over half a million entries takes nineteen (8 tables
+// x 500,000, 410 K ids: 37 us).  Here the first nine steps are taken in LDS;
+// inside the segment the place is guessed from the values at its ends (raw ids
+// are usually spread evenly: hashes) and four neighbouring entries are read in
+// two loads, which mostly ends the search in three or four reads; every second
+// later step bisects, so that any distribution ends.  20 us, of it 7 outside
+// the segments; four single loads 29 us, two entries a read 24 us, eight 21 us.
+__device__ __forceinline__ int64_t remap_lower_bound(const int64_t* __restrict__ sorted, int64_t n, int64_t seg,
+                                                     const int64_t* pivots, int64_t v, int64_t& entry) {
+  int p = 0;
+#pragma unroll
+  for (int step = kPivots / 2; step >= 1; step >>= 1)
+    if (pivots[p + step - 1] < v) p += step;
+  if (pivots[p] < v) {  // (only the last pivot: every entry below n is smaller)
+    entry = sorted[n];
+    return n;
+  }
+  int64_t lo = p * seg;
+  int64_t hi = min(lo + seg, n) - 1;
+  int64_t vh = pivots[p];                   // sorted[hi] >= v
+  int64_t vl = p > 0 ? pivots[p - 1] : vh;  // sorted[lo - 1] < v where vl_known
+  bool vl_known = p > 0;
+  for (int it = 0; lo < hi; ++it) {
+    int64_t mid = lo + ((hi - lo) >> 1);
+    if (vl_known && (it < 3 || (it & 1) == 0)) {
+      const float f = (float)((uint64_t)v - (uint64_t)vl) / (float)((uint64_t)vh - (uint64_t)vl);
+      mid = lo + (int64_t)(f * (float)(hi - lo + 1)) - 1;
     }
-    st<T>(out, j, sorted_ids[lo] == v ? mapping[lo] : miss_id);
+    // Entries base .. base + 3: inside [lo, hi] where that holds four, else reaching into what is
+    // known already, but never behind the table (n + 1 entries).
+    int64_t base = max(min(mid - 1, hi - 3), lo);
+    base = max(min(base, n - 3), (int64_t)0);
+    int64_t x[4];
+    if (n >= 3) {
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        const i64x2_t q = *reinterpret_cast<const i64x2_t*>(sorted + base + e);
+        x[e] = q.x;
+        x[e + 1] = q.y;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = sorted[min((int64_t)e, hi)];
+    }
+    int below = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) below += x[e] < v ? 1 : 0;
+    if (below == 4) {
+      lo = base + 4;
+      vl = x[3];
+      vl_known = true;
+    } else {
+      hi = base + below;
+      vh = below == 0 ? x[0] : below == 1 ? x[1] : below == 2 ? x[2] : x[3];
+      if (below != 0) lo = hi;
+    }
+  }
+  entry = vh;
+  return lo;
+}
+
+template <typename T, bool REMAP>
+__global__ __launch_bounds__(kMoveThreads) void move_keys_kernel(const MoveArgs m, const RemapTables t) {
+  __shared__ int64_t s_first[kMoveKeys + 1];
+  __shared__ int64_t s_found[4];
+  __shared__ int64_t s_pivot[REMAP ? kPivots : 1];
+  const int lane = threadIdx.x & (kWaveSize - 1);
+  const int wave = threadIdx.x / kWaveSize;
+  if ((int)blockIdx.x >= m.tile_blocks) {  // lengths: no bounds needed
+    const int64_t stride = (int64_t)(gridDim.x - m.tile_blocks) * kMoveThreads;
+    const int64_t total = (int64_t)m.launch_keys * m.B;
+    for (int64_t i = (int64_t)(blockIdx.x - m.tile_blocks) * kMoveThreads + threadIdx.x; i < total; i += stride) {
+      const int64_t j = i / m.B;
+      const int64_t src = (int64_t)m.perm[m.first_key + j] * m.B + (i - j * m.B), dst = (int64_t)m.first_key * m.B + i;
+      if (m.lengths_i64)
+        st<int64_t>(m.out_lengths, dst, ld<int64_t>(m.lengths, src));
+      else
+        st<int32_t>(m.out_lengths, dst, ld<int32_t>(m.lengths, src));
+    }
+    return;
+  }
+  if (wave == 0) {
+    if (m.kind == kKeysTotals) {
+      int64_t before = 0;
+      for (int k0 = 0; k0 < m.num_in; k0 += kWaveSize) {
+        int64_t incl = k0 + lane < m.num_in ? ld<int64_t>(m.bounds, k0 + lane) : 0;
+        incl = wave_scan(incl, lane);
+        if (k0 + lane < m.num_in) s_first[k0 + lane + 1] = before + incl;
+        before += __shfl(incl, kWaveSize - 1, kWaveSize);
+      }
+      if (lane == 0) s_first[0] = 0;
+    } else {
+      for (int k = lane; k <= m.num_in; k += kWaveSize)
+        s_first[k] = m.kind == kKeysOne ? (k == 0 ? 0 : m.num_values)
+                     : m.bounds_i64     ? ld<int64_t>(m.bounds, (int64_t)k * m.B)
+                                        : ld<int32_t>(m.bounds, (int64_t)k * m.B);
+    }
+  }
+  __syncthreads();
+  for (int64_t tile = blockIdx.x;; tile += m.tile_blocks) {
+    // The tile's output key, and where its ids come from and go to.
+    if (wave == 0) {
+      int64_t to = 0, tiles_before = 0;
+      int key = -1;
+      for (int j0 = 0; key < 0 && j0 < m.num_out; j0 += kWaveSize) {
+        const int j = j0 + lane;
+        int64_t first = 0, n = 0;
+        if (j < m.num_out) {
+          const int k = m.perm[j];
+          first = s_first[k] < 0 ? 0 : s_first[k];
+          n = (s_first[k + 1] > m.num_values ? m.num_values : s_first[k + 1]) - first;
+          n = n < 0 ? 0 : n;
+        }
+        const bool mine = j >= m.first_key && j < m.first_key + m.launch_keys;
+        const int64_t tiles = mine ? (n + m.tile - 1) / m.tile : 0;
+        const int64_t to_incl = wave_scan(n, lane), tiles_incl = wave_scan(tiles, lane);
+        const uint64_t past = __builtin_amdgcn_ballot_w64(tiles_before + tiles_incl > tile);
+        if (past != 0) {
+          const int hit = __builtin_ctzll(past);
+          key = j0 + hit;
+          if (lane == hit) {
+            const int64_t in_key = (tile - (tiles_before + tiles_incl - tiles)) * m.tile;
+            s_found[0] = key;
+            s_found[1] = first + in_key;
+            s_found[2] = (m.kind == kKeysTotals ? to + to_incl - n : first) + in_key;
+            s_found[3] = n - in_key < m.tile ? n - in_key : m.tile;
+          }
+        }
+        to += __shfl(to_incl, kWaveSize - 1, kWaveSize);
+        tiles_before += __shfl(tiles_incl, kWaveSize - 1, kWaveSize);
+      }
+      if (key < 0 && lane == 0) s_found[0] = -1;
+    }
+    __syncthreads();
+    const int key = (int)s_found[0];
+    const int64_t src = s_found[1], dst = s_found[2];
+    int64_t n = s_found[3];
+    if (key < 0) return;
+    n = dst + n > m.out_values_end ? m.out_values_end - dst : n;
+    const T* __restrict__ in = reinterpret_cast<const T*>(m.values) + src;
+    T* __restrict__ out = reinterpret_cast<T*>(m.out_values) + dst;
+    if constexpr (REMAP) {
+      const int tk = key - m.first_key;
+      const int64_t* __restrict__ sorted = t.sorted_ids[tk];
+      const int64_t* __restrict__ mapping = t.mapping[tk];
+      const int64_t last = t.size[tk] - 1, miss = t.miss_id[tk];
+      const int64_t seg = (last + kPivots - 1) / kPivots;
+      if ((int)threadIdx.x < kPivots && last > 0) {
+        const int64_t end = (threadIdx.x + 1) * seg;
+        s_pivot[threadIdx.x] = sorted[(end < last ? end : last) - 1];
+      }
+      __syncthreads();
+      for (int64_t i = threadIdx.x; i < n; i += kMoveThreads) {
+        const int64_t v = (int64_t)in[i];
+        int64_t entry;
+        int64_t at = 0;
+        if (last > 0)
+          at = remap_lower_bound(sorted, last, seg, s_pivot, v, entry);
+        else
+          entry = sorted[0];
+        out[i] = (T)(entry == v ? mapping[at] : miss);
+      }
+    } else {
+#pragma unroll 4
+      for (int64_t i = threadIdx.x; i < n; i += kMoveThreads) out[i] = in[i];
+    }
+    if (m.weights)
+#pragma unroll 4
+      for (int64_t i = threadIdx.x; i < n; i += kMoveThreads) m.out_weights[dst + i] = m.weights[src + i];
+    __syncthreads();  // s_found and s_pivot have been read by everyone
   }
 }
 
@@ -865,6 +1045,61 @@ __global__ __launch_bounds__(256) void tra_copy_kernel(const uint4* __restrict__
 static int check_launch(const char* what) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, what);
+  return TRA_OK;
+}
+
+struct RemapSpec {
+  const int64_t* const* sorted_ids;
+  const int64_t* const* mapping;
+  const int64_t* table_size;
+  const int64_t* miss_id;
+};
+
+// Launches move_keys_kernel over all output keys: in one go, or kRemapKeys keys with a table at a time.
+static int move_keys(MoveArgs& m, int value_bytes, const RemapSpec* spec, hipStream_t s) {
+  const int group = spec ? kRemapKeys : kMoveKeys;
+  for (int k0 = 0; k0 < m.num_out; k0 += group) {
+    m.first_key = k0;
+    m.launch_keys = std::min(group, m.num_out - k0);
+    // Ids per tile: a block's worth, up to eight of them where that leaves one tile per compute
+    // unit (a block with a table reads its pivots once per tile: 410 K ids in tiles of 512 24 us,
+    // of 1024 20 us, of 1536 24 us).
+    const int64_t ids = std::min(m.num_values, m.out_values_end);
+    m.tile = kMoveThreads;
+    while (m.tile < 8 * kMoveThreads && ids / (2 * m.tile) >= 256) m.tile *= 2;
+    // (all ids may belong to this launch's keys, some several times; every key may leave a partial tile)
+    const int64_t tiles = m.out_values_end > 0 ? m.out_values_end / m.tile + m.launch_keys : 0;
+    m.tile_blocks = (int)std::min<int64_t>(tiles, 1 << 20);
+    const int64_t moved = m.out_lengths ? (int64_t)m.launch_keys * m.B : 0;
+    const int64_t blocks = m.tile_blocks + std::min<int64_t>((moved + kMoveThreads - 1) / kMoveThreads, 4096);
+    if (blocks == 0) continue;
+    RemapTables t;
+    if (spec) {
+      for (int k = 0; k < m.launch_keys; ++k) {
+        if (!spec->sorted_ids[k0 + k] || !spec->mapping[k0 + k] || spec->table_size[k0 + k] < 1) {
+          set_error("managed-collision remap: key %d has no table", k0 + k);
+          return TRA_ERR_INVALID_ARGUMENT;
+        }
+        t.sorted_ids[k] = spec->sorted_ids[k0 + k];
+        t.mapping[k] = spec->mapping[k0 + k];
+        t.size[k] = spec->table_size[k0 + k];
+        t.miss_id[k] = spec->miss_id[k0 + k];
+      }
+    }
+    const auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kMoveThreads), 0, s, m, t);
+    };
+    if (spec && value_bytes == 8)
+      go(move_keys_kernel<int64_t, true>);
+    else if (spec)
+      go(move_keys_kernel<int32_t, true>);
+    else if (value_bytes == 8)
+      go(move_keys_kernel<int64_t, false>);
+    else
+      go(move_keys_kernel<int32_t, false>);
+    const int rc = check_launch("move_keys");
+    if (rc != TRA_OK) return rc;
+  }
   return TRA_OK;
 }
 
@@ -1330,14 +1565,15 @@ int tra_mch_remap(const void* values, int64_t n, int32_t is_i64, const int64_t* 
     set_error("tra_mch_remap: null buffer");
     return TRA_ERR_INVALID_ARGUMENT;
   }
-  const unsigned grid = (unsigned)std::min<int64_t>((n + 255) / 256, 256 * 16);
-  if (is_i64)
-    hipLaunchKernelGGL(mch_remap_kernel<int64_t>, dim3(grid), dim3(256), 0, (hipStream_t)stream, values,
-                       n, sorted_ids, mapping, table_size, miss_id, out);
-  else
-    hipLaunchKernelGGL(mch_remap_kernel<int32_t>, dim3(grid), dim3(256), 0, (hipStream_t)stream, values,
-                       n, sorted_ids, mapping, table_size, miss_id, out);
-  return check_launch("tra_mch_remap");
+  MoveArgs m = MoveArgs();
+  m.values = values;
+  m.out_values = out;
+  m.num_values = m.out_values_end = n;
+  m.kind = kKeysOne;
+  m.num_in = m.num_out = 1;
+  m.B = 1;
+  const RemapSpec spec{&sorted_ids, &mapping, &table_size, &miss_id};
+  return move_keys(m, is_i64 ? 8 : 4, &spec, (hipStream_t)stream);
 }
 
 int tra_mch_remap_keys(const void* values, int64_t n, const void* offsets, int32_t is_i64,
@@ -1353,35 +1589,70 @@ int tra_mch_remap_keys(const void* values, int64_t n, const void* offsets, int32
     set_error("tra_mch_remap_keys: null argument");
     return TRA_ERR_INVALID_ARGUMENT;
   }
-  for (int k = 0; k < num_keys; ++k)
-    if (!sorted_ids[k] || !mapping[k] || table_size[k] < 1) {
-      set_error("tra_mch_remap_keys: key %d has no table", k);
-      return TRA_ERR_INVALID_ARGUMENT;
-    }
-  // blocks per key: enough for the average key, at most 1024
-  const int64_t per_key = n / num_keys + 1;
-  const unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>((per_key + 255) / 256, 1024));
-  for (int k0 = 0; k0 < num_keys; k0 += kRemapKeys) {
-    const int nk = std::min(kRemapKeys, num_keys - k0);
-    RemapTables t;
-    std::memset(&t, 0, sizeof(t));
-    for (int k = 0; k < nk; ++k) {
-      t.sorted_ids[k] = sorted_ids[k0 + k];
-      t.mapping[k] = mapping[k0 + k];
-      t.size[k] = table_size[k0 + k];
-      t.miss_id[k] = miss_id[k0 + k];
-    }
-    t.first_key = k0;
-    if (is_i64)
-      hipLaunchKernelGGL(mch_remap_keys_kernel<int64_t>, dim3(gx, nk), dim3(256), 0, (hipStream_t)stream,
-                         values, n, offsets, batch_size, t, out);
-    else
-      hipLaunchKernelGGL(mch_remap_keys_kernel<int32_t>, dim3(gx, nk), dim3(256), 0, (hipStream_t)stream,
-                         values, n, offsets, batch_size, t, out);
-    const int rc = check_launch("tra_mch_remap_keys");
+  // (kMoveKeys keys at a time; a chunk's offsets start at its first key's)
+  for (int k0 = 0; k0 < num_keys; k0 += kMoveKeys) {
+    MoveArgs m = MoveArgs();
+    m.bounds = static_cast<const uint8_t*>(offsets) + (int64_t)k0 * batch_size * (is_i64 ? 8 : 4);
+    m.bounds_i64 = is_i64;
+    m.values = values;
+    m.out_values = out;
+    m.num_values = m.out_values_end = n;
+    m.kind = kKeysOffsets;
+    m.num_in = m.num_out = std::min(kMoveKeys, num_keys - k0);
+    m.B = batch_size;
+    for (int k = 0; k < m.num_in; ++k) m.perm[k] = (int16_t)k;
+    const RemapSpec spec{sorted_ids + k0, mapping + k0, table_size + k0, miss_id + k0};
+    const int rc = move_keys(m, is_i64 ? 8 : 4, &spec, (hipStream_t)stream);
     if (rc != TRA_OK) return rc;
   }
   return TRA_OK;
+}
+
+int tra_permute_keys(const int64_t* key_totals, int32_t num_keys, const int32_t* permute, int32_t num_out_keys,
+                     int32_t batch_size, const void* lengths, int32_t lengths_i64, void* out_lengths,
+                     const void* values, int64_t num_values, int32_t value_bytes, void* out_values,
+                     int64_t num_out_values, const float* weights, float* out_weights,
+                     const int64_t* const* sorted_ids, const int64_t* const* mapping, const int64_t* table_size,
+                     const int64_t* miss_id, void* stream) {
+  if (num_keys < 1 || num_out_keys < 0 || batch_size < 0 || num_values < 0 || num_out_values < 0 ||
+      (value_bytes != 4 && value_bytes != 8) || !key_totals || !permute) {
+    set_error("tra_permute_keys: bad argument (value_bytes must be 4 or 8)");
+    return TRA_ERR_INVALID_ARGUMENT;
+  }
+  if (num_keys > kMoveKeys || num_out_keys > kMoveKeys) {
+    set_error("tra_permute_keys: %d and %d keys, at most %d are supported", num_keys, num_out_keys, kMoveKeys);
+    return TRA_ERR_TOO_LARGE;
+  }
+  if (num_out_keys == 0) return TRA_OK;
+  if ((num_values > 0 && !values) || (num_out_values > 0 && (!out_values || (weights && !out_weights))) ||
+      (out_lengths && !lengths) || (sorted_ids && (!mapping || !table_size || !miss_id))) {
+    set_error("tra_permute_keys: null buffer");
+    return TRA_ERR_INVALID_ARGUMENT;
+  }
+  MoveArgs m = MoveArgs();
+  m.bounds = key_totals;
+  m.values = values;
+  m.out_values = out_values;
+  m.weights = weights;
+  m.out_weights = out_weights;
+  m.lengths = lengths;
+  m.out_lengths = out_lengths;
+  m.lengths_i64 = lengths_i64;
+  m.num_values = num_values;
+  m.out_values_end = num_out_values;
+  m.kind = kKeysTotals;
+  m.num_in = num_keys;
+  m.num_out = num_out_keys;
+  m.B = batch_size;
+  for (int j = 0; j < num_out_keys; ++j) {
+    if (permute[j] < 0 || permute[j] >= num_keys) {
+      set_error("tra_permute_keys: key %d of %d", permute[j], num_keys);
+      return TRA_ERR_INVALID_ARGUMENT;
+    }
+    m.perm[j] = (int16_t)permute[j];
+  }
+  const RemapSpec spec{sorted_ids, mapping, table_size, miss_id};
+  return move_keys(m, value_bytes, sorted_ids ? &spec : nullptr, (hipStream_t)stream);
 }
 
 int tra_regroup_columns(const void* const* src, const int64_t* src_stride, void* const* dst,

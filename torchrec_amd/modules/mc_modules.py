@@ -183,39 +183,53 @@ class ManagedCollisionCollection(nn.Module):
         """Per key of ``features`` (already in table order) the sorted-id table, row
         mapping and miss row of its module, when every module is an inference-mode
         MCH module without an input hash and the ids are on the GPU; else None."""
-        if features.values().device.type != "cuda" or not features.keys():
+        if not features.values().is_cuda or not features.keys():
             return None
+        dev = features.values().get_device()
+        modules = self._managed_collision_modules._modules
         sorted_ids, mappings, miss = [], [], []
         for config in self._embedding_configs:
-            module = self._managed_collision_modules[config.name]
-            if (
-                type(module) is not MCHManagedCollisionModule
-                or module.training
-                or module._input_hash_func is not None
-                or module._mch_sorted_raw_ids.device != features.values().device
-            ):
+            module = modules[config.name]
+            if type(module) is not MCHManagedCollisionModule or module.training or module._input_hash_func is not None:
+                return None
+            buffers = module._buffers
+            ids, rows = buffers["_mch_sorted_raw_ids"], buffers["_mch_remapped_ids_mapping"]
+            if ids.get_device() != dev or rows.get_device() != dev:
                 return None
             for _ in config.feature_names:
-                sorted_ids.append(module._mch_sorted_raw_ids)
-                mappings.append(module._mch_remapped_ids_mapping)
+                sorted_ids.append(ids)
+                mappings.append(rows)
                 miss.append(module._output_global_offset + module._zch_size - 1)
         return sorted_ids, mappings, miss
 
     def forward(self, features: KeyedJaggedTensor) -> KeyedJaggedTensor:
-        order = [features.keys().index(f) for f in self._feature_names]
-        if order != list(range(len(features.keys()))):
-            features = features.permute(order)
+        keys = features.keys()
+        order = None if keys == self._feature_names else [keys.index(f) for f in self._feature_names]
+        if order == list(range(len(keys))):
+            order = None
         tables = self._one_launch_tables(features)
+        if tables is not None and order is not None:
+            # all keys brought into table order and remapped in one launch
+            moved = features._permute_on_gpu(order, remap=tables)
+            if moved is not None:
+                lengths, values, weights, length_per_key = moved
+                return KeyedJaggedTensor(
+                    keys=[keys[i] for i in order], values=values, weights=weights, lengths=lengths,
+                    stride=features.stride(), length_per_key=length_per_key,
+                )
+        if order is not None:
+            features = features.permute(order)
         if tables is not None:
             # all keys in one launch: no split per table, no host read of the
             # per-key id counts, no concatenation
             return KeyedJaggedTensor(
                 keys=features.keys(),
-                values=ops.mch_remap_keys(features.values(), features.offsets(), features.stride(), *tables),
-                lengths=features.lengths(),
-                offsets=features.offsets(),
+                values=ops.mch_remap_kjt(features, tables),
+                lengths=features.lengths_or_none(),
+                offsets=features.offsets_or_none(),
                 weights=features.weights_or_none(),
                 stride=features.stride(),
+                length_per_key=features.length_per_key_or_none(),
             )
         splits = features.split(self._table_feature_splits)
         values: List[torch.Tensor] = []

@@ -53,16 +53,28 @@ def asynchronous_complete_cumsum(lengths: torch.Tensor) -> torch.Tensor:
     return out
 
 
+_entries: dict = {}  # entry points bound by _lib.entry on first use
+
+
+def _entry(name: str):
+    fn = _entries.get(name)
+    if fn is None:
+        fn = _entries[name] = _lib.entry(name)
+    return fn
+
+
 # Keys whose totals a lookup takes from the device, and that reach the host without a copy.
 _MAX_TOTAL_KEYS = 256
 _MAX_HOST_KEYS = 1024
 
 
-def key_totals_begin(bags: torch.Tensor, bags_are_offsets: bool, num_keys: int, stride: int, on_device: bool):
+def key_totals_begin(
+    bags: torch.Tensor, bags_are_offsets: bool, num_keys: int, stride: int, on_device: bool, on_host: bool = True
+):
     """Ids per key of a feature-major KJT on the GPU, from its lengths or its offsets: ``(totals, finish)``.
-    The adding-up is queued now; ``totals`` is the int64 device tensor when ``on_device``, ``finish()`` waits for
-    that kernel alone and returns the list (it has to be called, also when something raises in between).  None
-    when the totals cannot come this way (too many keys or calls at once, stream capture)."""
+    The adding-up is queued now; ``totals`` is the int64 device tensor when ``on_device``, ``finish()`` (when
+    ``on_host``) waits for that kernel alone and returns the list; it has to be called, also when something raises
+    in between.  None when the totals cannot come this way (too many keys or calls at once, stream capture)."""
     _check_int(bags, "offsets" if bags_are_offsets else "lengths")
     assert bags.numel() >= num_keys * stride + int(bags_are_offsets), "bag bounds shorter than the keys they must cover"
     if num_keys > _MAX_HOST_KEYS or stride == 0:
@@ -70,19 +82,24 @@ def key_totals_begin(bags: torch.Tensor, bags_are_offsets: bool, num_keys: int, 
     bags = bags.contiguous()
     dev = bags.device
     totals = torch.empty(num_keys, dtype=torch.int64, device=dev) if on_device else None
-    ticket = ctypes.c_int32(-1)
-    l = _lib.lib()
-    rc = l.tra_key_totals_begin(
-        bags.data_ptr(), int(bags_are_offsets), num_keys, stride, int(bags.dtype == torch.int64),
-        _lib.ptr(totals), ctypes.byref(ticket), _lib.current_stream(dev),
+    ticket = array("i", (-1,))
+    rc = _entry("tra_key_totals_begin")(
+        bags.data_ptr(), bags_are_offsets, num_keys, stride, bags.dtype is torch.int64,
+        None if totals is None else totals.data_ptr(), ticket.buffer_info()[0] if on_host else None,
+        _lib.current_stream(dev),
     )
-    if rc in (_lib.ERR_TOO_LARGE, _lib.ERR_UNSUPPORTED):
-        return None
-    _lib.check(rc)
+    if rc != 0:
+        if rc == _lib.ERR_TOO_LARGE or rc == _lib.ERR_UNSUPPORTED:
+            return None
+        _lib.check(rc)
+    if not on_host:
+        return totals, None
 
     def finish() -> List[int]:
         host = array("q", bytes(8 * num_keys))
-        _lib.check(l.tra_key_totals_wait(ticket.value, host.buffer_info()[0]))
+        rc = _entry("tra_key_totals_wait")(ticket[0], host.buffer_info()[0])
+        if rc != 0:
+            _lib.check(rc)
         return host.tolist()
 
     return totals, finish
@@ -364,6 +381,51 @@ def mch_remap(
     return out
 
 
+def permute_keys(
+    totals: torch.Tensor,
+    order: List[int],
+    stride: int,
+    lengths: torch.Tensor,
+    values: torch.Tensor,
+    num_out: int,
+    weights: Optional[torch.Tensor] = None,
+    remap: Optional[Tuple[List[torch.Tensor], List[torch.Tensor], List[int]]] = None,
+    move_lengths: bool = True,
+) -> Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
+    """Output key j of a feature-major KJT on the GPU is input key ``order[j]``: ``(lengths, values, weights)`` in
+    the new order, in one launch.  ``totals``: ids per input key (``key_totals_begin``); ``num_out``: ids of the
+    output; ``remap``: sorted id table, row mapping and miss row per output key (``mch_remap``)."""
+    dev = values.device
+    K, Kp = totals.numel(), len(order)
+    values = values.contiguous()
+    out_values = torch.empty(num_out, dtype=values.dtype, device=dev)
+    out_lengths = out_weights = None
+    if move_lengths:
+        lengths = lengths.contiguous()
+        out_lengths = torch.empty(Kp * stride, dtype=lengths.dtype, device=dev)
+    if weights is not None:
+        weights = weights.contiguous()
+        out_weights = torch.empty(num_out, dtype=torch.float32, device=dev)
+    tables, at = (), (None, None, None, None)
+    if remap is not None:
+        sorted_ids, mappings, miss = remap
+        tables = (
+            array("q", [t.data_ptr() for t in sorted_ids]), array("q", [t.data_ptr() for t in mappings]),
+            array("q", [t.numel() for t in sorted_ids]), array("q", miss),
+        )
+        at = [a.buffer_info()[0] for a in tables]
+    perm = array("i", order)
+    rc = _entry("tra_permute_keys")(
+        totals.data_ptr(), K, perm.buffer_info()[0], Kp, stride, lengths.data_ptr() if move_lengths else None,
+        lengths.dtype is torch.int64, out_lengths.data_ptr() if move_lengths else None, values.data_ptr(),
+        values.numel(), values.element_size(), out_values.data_ptr(), num_out, _lib.ptr(weights),
+        _lib.ptr(out_weights), *at, _lib.current_stream(dev),
+    )
+    if rc != 0:
+        _lib.check(rc)
+    return (out_lengths if move_lengths else lengths), out_values, out_weights
+
+
 def mch_remap_keys(
     values: torch.Tensor,
     offsets: torch.Tensor,
@@ -397,3 +459,20 @@ def mch_remap_keys(
         )
     )
     return out
+
+
+def mch_remap_kjt(
+    features, tables: Tuple[List[torch.Tensor], List[torch.Tensor], List[int]]
+) -> torch.Tensor:
+    """``mch_remap_keys`` of a KeyedJaggedTensor (its keys in table order): where the ids of each key lie comes from
+    its offsets when it has them, else from its lengths added up per key (no offsets are computed)."""
+    K, B = len(features.keys()), features.stride()
+    offsets = features.offsets_or_none()
+    if offsets is None and 0 < K <= _MAX_TOTAL_KEYS and B > 0:
+        begun = key_totals_begin(features.lengths(), False, K, B, on_device=True, on_host=False)
+        if begun is not None:
+            values = features.values()
+            return permute_keys(
+                begun[0], list(range(K)), B, features.lengths(), values, values.numel(), remap=tables, move_lengths=False
+            )[1]
+    return mch_remap_keys(features.values(), features.offsets(), B, *tables)

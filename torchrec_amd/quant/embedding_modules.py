@@ -356,6 +356,7 @@ class _FeatureOrderMixin:
 
     _feature_names: List[str]
     _features_order: Optional[List[int]]
+    _identity_order: Optional[List[int]] = None  # the order of keys equal to the feature names, once seen
 
     def _resolve_order(self, kjt_keys: List[str]) -> List[int]:
         if getattr(self, MODULE_ATTR_CACHE_FEATURES_ORDER, False):
@@ -363,6 +364,12 @@ class _FeatureOrderMixin:
             if self._features_order is None:
                 self._features_order = [kjt_keys.index(k) for k in self._feature_names]
             return self._features_order
+        if kjt_keys == self._feature_names:
+            identity = self._identity_order
+            if identity is None and len(set(kjt_keys)) == len(kjt_keys):
+                identity = self._identity_order = list(range(len(kjt_keys)))
+            if identity is not None:
+                return identity
         # otherwise resolved per key order, remembered so that a repeated order costs one dict lookup
         cache = self.__dict__.setdefault("_order_by_keys", {})
         ck = tuple(kjt_keys)
@@ -795,6 +802,9 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
             key: list(itertools.chain(*get_embedding_names_by_table(group)))
             for key, group in self._key_to_tables.items()
         }
+        self._flat_embedding_names: List[str] = [
+            name for key in self._key_to_tables for name in self._embedding_names_by_batched_tables[key]
+        ]
         self._embedding_names_by_table: List[List[str]] = get_embedding_names_by_table(
             self._embedding_configs
         )
@@ -809,7 +819,7 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
         """Each feature's JaggedTensor is a row range (view) of one ``[L, D]`` lookup buffer."""
         kjt_keys = _get_kjt_keys(features)
         order = self._resolve_order(kjt_keys)
-        if len(set(order)) != len(order):
+        if order is not self._identity_order and len(set(order)) != len(order):
             # A feature feeding two tables needs two distinct row ranges in the
             # output: materialize the repeated ids once.
             features = features.permute(order)
@@ -861,32 +871,28 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
         # The batching hint sees the flattened lengths by default and the [F, B] lengths when the
         # module is prepared for it (torchrec/quant/embedding_modules.py:943-950); here the lengths
         # are those of the whole KJT, because all operators write one buffer.
-        if getattr(self, MODULE_ATTR_USE_UNFLATTENED_LENGTHS_FOR_BATCHING, False):
+        prepared = self.__dict__
+        if prepared.get(MODULE_ATTR_USE_UNFLATTENED_LENGTHS_FOR_BATCHING, False):
             if kjt_keys:
-                lengths = _get_unflattened_lengths(features.lengths(), len(kjt_keys))
+                lengths = _get_unflattened_lengths(lengths, K)
             lookup = _get_batching_hinted_output(lengths=lengths, output=lookup)
         else:
-            if getattr(self, MODULE_ATTR_USE_BATCHING_HINTED_OUTPUT, True):
-                lookup = _get_batching_hinted_output(lengths=features.lengths(), output=lookup)
+            if prepared.get(MODULE_ATTR_USE_BATCHING_HINTED_OUTPUT, True):
+                lookup = _get_batching_hinted_output(lengths=lengths, output=lookup)
             if kjt_keys:
-                lengths = _get_unflattened_lengths(features.lengths(), len(kjt_keys))
-        if getattr(self, MODULE_ATTR_REMOVE_STBE_PADDING_BOOL, False):
+                lengths = _get_unflattened_lengths(lengths, K)
+        if prepared.get(MODULE_ATTR_REMOVE_STBE_PADDING_BOOL, False):
             # Rows past the last id that belongs to a bag (a padded values tensor) are dropped
             # (construct_jagged_tensors_inference(remove_padding=True), torchrec/modules/utils.py:315-316).
             lookup = lookup[: offset_per_key[-1]]
         lengths_rows = torch.unbind(lengths, dim=0) if kjt_keys else ()
+        need_indices = self._need_indices
         feature_embeddings: Dict[str, JaggedTensor] = {}
-        f = 0
-        for key in self._key_to_tables.keys():
-            for embedding_name in self._embedding_names_by_batched_tables[key]:
-                pos = order[f]
-                start, end = offset_per_key[pos], offset_per_key[pos + 1]
-                feature_embeddings[embedding_name] = JaggedTensor(
-                    values=lookup[start:end],
-                    lengths=lengths_rows[pos],
-                    weights=indices[start:end] if self._need_indices else None,
-                )
-                f += 1
+        for embedding_name, pos in zip(self._flat_embedding_names, order):
+            start, end = offset_per_key[pos], offset_per_key[pos + 1]
+            feature_embeddings[embedding_name] = JaggedTensor._of(
+                lookup[start:end], lengths_rows[pos], indices[start:end] if need_indices else None
+            )
         return feature_embeddings
 
     def _starts_fit(self, offset_per_key: List[int], num_indices: int) -> bool:

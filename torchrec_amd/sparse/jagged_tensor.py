@@ -106,6 +106,16 @@ class JaggedTensor:
         self._lengths: Optional[torch.Tensor] = lengths
         self._offsets: Optional[torch.Tensor] = offsets
 
+    @classmethod
+    def _of(cls, values: torch.Tensor, lengths: torch.Tensor, weights: Optional[torch.Tensor]) -> "JaggedTensor":
+        """``JaggedTensor(values, weights, lengths)`` of parts known to be right (no checks)."""
+        jt = cls.__new__(cls)
+        jt._values = values
+        jt._weights = weights
+        jt._lengths = lengths
+        jt._offsets = None
+        return jt
+
     @staticmethod
     def empty(
         is_weighted: bool = False,
@@ -529,10 +539,17 @@ class KeyedJaggedTensor:
         self, indices: List[int], indices_tensor: Optional[torch.Tensor] = None
     ) -> "KeyedJaggedTensor":
         """New KJT whose feature i is this one's feature indices[i] (repeats allowed)."""
+        permuted_keys = [self._keys[i] for i in indices]
+        moved = self._permute_on_gpu(indices)
+        if moved is not None:
+            lengths, values, weights, permuted_length_per_key = moved
+            return KeyedJaggedTensor(
+                keys=permuted_keys, values=values, weights=weights, lengths=lengths, stride=self._stride,
+                length_per_key=permuted_length_per_key,
+            )
         if indices_tensor is None:
             indices_tensor = torch.tensor(indices, dtype=torch.int, device=self.device())
         length_per_key = self.length_per_key()
-        permuted_keys = [self._keys[i] for i in indices]
         permuted_length_per_key = [length_per_key[i] for i in indices]
         total = sum(permuted_length_per_key)
         permuted_lengths, permuted_values, permuted_weights = ops.permute_2D_sparse_data(
@@ -550,6 +567,47 @@ class KeyedJaggedTensor:
             stride=self._stride,
             length_per_key=permuted_length_per_key if permuted_keys else None,
         )
+
+    def _totals_begin(self):
+        """``ops.key_totals_begin`` of this KJT (device and host), or None."""
+        if self._lengths is None:
+            return ops.key_totals_begin(self._offsets, True, len(self._keys), self.stride(), True)
+        return ops.key_totals_begin(self._lengths, False, len(self._keys), self.stride(), True)
+
+    def _permute_on_gpu(self, indices: List[int], remap=None):
+        """``(lengths, values, weights, length_per_key)`` of the keys in the order ``indices``, moved (and
+        remapped) by one kernel behind the one that adds up the ids per key; None where that does not apply."""
+        values, weights = self._values, self._weights
+        nkeys = len(self._keys)
+        if (
+            not values.is_cuda or values.dim() != 1 or values.element_size() not in (4, 8) or not indices
+            or nkeys > ops._MAX_TOTAL_KEYS or len(indices) > ops._MAX_TOTAL_KEYS or self.stride() == 0
+            or (weights is not None and (weights.dim() != 1 or weights.dtype != torch.float32))
+            or min(indices) < 0
+        ):
+            return None
+        stride = self.stride()
+        begun = self._totals_begin()
+        if begun is None:
+            return None
+        totals, finish = begun
+        moved = None
+        try:
+            lengths = self.lengths()
+            if len(indices) == nkeys and len(set(indices)) == nkeys:
+                # every key once: the output's size is known before the counts are
+                moved = ops.permute_keys(totals, indices, stride, lengths, values, values.numel(), weights, remap)
+        finally:
+            per_key = self._length_per_key = finish()
+        permuted = [per_key[i] for i in indices]
+        total = sum(permuted)
+        if moved is None:
+            moved = ops.permute_keys(totals, indices, stride, lengths, values, total, weights, remap)
+        new_lengths, new_values, new_weights = moved
+        if total != new_values.numel():  # (ids behind the last bag's belong to no key)
+            new_values = new_values[:total]
+            new_weights = None if new_weights is None else new_weights[:total]
+        return new_lengths, new_values, new_weights, permuted
 
     def flatten_lengths(self) -> "KeyedJaggedTensor":
         return KeyedJaggedTensor(
@@ -721,11 +779,11 @@ def regroup_kts(
     if n_blocks and rows:
         global _REGROUP
         if _REGROUP is None:
-            _REGROUP = _lib.regroup_entry()
-        call = _REGROUP if len(src) <= 64 and len(outs) <= 64 else _lib.regroup_entry(fast=False)
-        rc = call(
-            src, src_stride, [o.data_ptr() for o in outs], widths, blocks.buffer_info()[0], n_blocks, rows, esz,
-            _lib.current_stream(dev),
+            _REGROUP = _lib.entry("tra_regroup_tensors")
+        tables = array("q", src), array("q", src_stride), array("q", [o.data_ptr() for o in outs]), array("q", widths)
+        a, b, c, d = [t.buffer_info()[0] for t in tables]
+        rc = _REGROUP(
+            a, b, len(src), c, d, len(outs), blocks.buffer_info()[0], n_blocks, rows, esz, _lib.current_stream(dev)
         )
         if rc != 0:
             _lib.check(rc)

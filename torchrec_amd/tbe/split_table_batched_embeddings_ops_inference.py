@@ -43,6 +43,7 @@ _ENV_BOUNDS_CHECK = os.environ.get("TORCHREC_AMD_BOUNDS_CHECK", "0") == "1"
 _INT_DTYPES = (torch.int32, torch.int64)
 _BOUNDS_FATAL = int(BoundsCheckMode.FATAL)
 _FORWARD_LENGTHS = None  # the library's tra_tbe_forward_lengths, bound on first use
+_FORWARD_SEQUENCE = None  # likewise tra_tbe_forward_sequence
 
 _SUPPORTED_WEIGHTS = (SparseType.FP32, SparseType.FP16, SparseType.INT8, SparseType.INT4, SparseType.INT2)
 _TABLE_ALIGNMENT = 256
@@ -597,9 +598,12 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
         plan = self._plan_address.get(positions)
         if plan is None:
             plan = self._plan_address[positions] = self._get_plan(positions).value
-        rc = _lib.lib().tra_tbe_forward_sequence(
+        global _FORWARD_SEQUENCE
+        if _FORWARD_SEQUENCE is None:
+            _FORWARD_SEQUENCE = _lib.entry("tra_tbe_forward_sequence")
+        rc = _FORWARD_SEQUENCE(
             plan, self._buffers["weights_dev"].data_ptr(), indices.data_ptr(), totals_ptr, starts_ptr, num_keys,
-            int(indices.dtype is torch.int64), L, self.output_dtype, out.data_ptr(), _lib.current_stream(dev),
+            indices.dtype is torch.int64, L, self.output_dtype, out.data_ptr(), _lib.current_stream(dev),
         )
         if rc != 0:
             _lib.check(rc)
