@@ -321,6 +321,23 @@ int tra_bucketize_scatter(const void* offsets, const void* indices,
                           float* new_weights, int64_t* unbucketize_permute,
                           void* stream);
 
+/* Block bucketization from lengths in one call, into at most 64 buckets:
+ * new_lengths [num_buckets * F * B] as above; new_indices / new_weights sized for
+ * num_indices (fewer are written where ids lie beyond the last bucket);
+ * unbucketize_permute and bucket_of (floor(id / block size), type of the ids)
+ * [num_indices] may be null.  workspace: tra_bucketize_ids_workspace_bytes.  The
+ * ids of each bucket reach the host through `ticket`: pass it, with room for
+ * num_buckets numbers, to tra_key_totals_wait.  TRA_ERR_TOO_LARGE beyond 64
+ * buckets or 2^31 ids, and as for tra_key_totals_begin. */
+int64_t tra_bucketize_ids_workspace_bytes(int32_t num_features, int32_t batch_size,
+                                          int32_t num_buckets, int64_t num_indices);
+int tra_bucketize_ids(const void* lengths, const void* indices, int32_t is_i64,
+                      const float* weights, const int64_t* block_sizes, int32_t num_features,
+                      int32_t batch_size, int32_t num_buckets, int64_t num_indices,
+                      int32_t keep_orig_idx, void* workspace, void* new_lengths,
+                      void* new_indices, float* new_weights, int64_t* unbucketize_permute,
+                      void* bucket_of, int32_t* ticket, void* stream);
+
 /* Row-wise quantization --------------------------------------------------- */
 /* fp32 [rows, dim] -> packed TBE rows (header-first, row_bytes stride) written
  * straight into the table buffer at `out`; bits in {8, 4, 2}.  Same bytes as

@@ -352,3 +352,41 @@ def test_kjt_permute(K, B, max_len, pick, idt, vdt):
     assert torch.equal(got.values(), torch.cat([values[starts[i]:starts[i + 1]] for i in order]))
     assert torch.equal(got.weights(), torch.cat([weights[starts[i]:starts[i + 1]] for i in order]))
     assert got.length_per_key() == lengths.sum(1)[order].tolist()
+
+
+@pytest.mark.parametrize("F,B,W,max_len", [(1, 1, 1, 5), (3, 5, 2, 9), (2, 600, 3, 4), (5, 131, 64, 40), (2, 7, 65, 30), (3, 4, 8, 5000),
+                                           (40, 512, 5, 30)])
+@pytest.mark.parametrize("idt", [np.int32, np.int64])
+@pytest.mark.parametrize("weighted,keep", [(True, False), (False, True)])
+def test_bucketize_tiles(F, B, W, max_len, idt, weighted, keep):
+    """Against numpy at the edges of the one-call kernels: one bag, tiles of several features' ends, bags of many steps,
+    64 buckets and one more, ids beyond the last bucket, negative ids, block sizes of one and beyond 32 bits."""
+    rng = np.random.default_rng(F * B + W)
+    lengths = rng.integers(0, max_len + 1, F * B)
+    lengths[rng.random(F * B) < 0.2] = 0
+    bs = rng.integers(1, 1000, F)
+    if idt == np.int64 and F > 1:
+        bs[1] = 2**33 + 5
+    bs[0] = 1 if F > 2 else bs[0]
+    feature = np.repeat(np.arange(F * B) // B, lengths)
+    ids = (rng.random(len(feature)) * (bs[feature] * (W + 1))).astype(np.int64)
+    if len(ids):
+        ids[rng.random(len(ids)) < 0.02] = -3
+    q = np.floor_divide(ids, bs[feature])
+    kept = np.flatnonzero((q >= 0) & (q < W))
+    order = kept[np.argsort(q[kept], kind="stable")]
+    weights = rng.random(len(ids)).astype(np.float32)
+    bag = np.repeat(np.arange(F * B), lengths)
+    want_lengths = np.bincount(q[kept] * F * B + bag[kept], minlength=W * F * B)
+    want_order = np.full(len(ids), -1)
+    want_order[order] = np.arange(len(order))
+    nl, ni, nw, _, unb, buckets = ops._block_bucketize(
+        torch.from_numpy(lengths.astype(idt)).to(DEV), torch.from_numpy(ids.astype(idt)).to(DEV), False, True,
+        torch.from_numpy(bs).to(DEV), W, torch.from_numpy(weights).to(DEV) if weighted else None, keep, want_buckets=True)
+    assert np.array_equal(nl.cpu().numpy(), want_lengths)
+    assert np.array_equal(ni.cpu().numpy(), ids[order] if keep else ids[order] % bs[feature[order]])
+    assert nw is None if not weighted else np.array_equal(nw.cpu().numpy(), weights[order])
+    assert np.array_equal(unb.cpu().numpy(), want_order)
+    assert (buckets is None) == (W > 64 or len(ids) == 0)
+    if buckets is not None:
+        assert np.array_equal(buckets.cpu().numpy(), q)

@@ -45,6 +45,8 @@ EXPORTED_SYMBOLS = [
     "tra_bucketize_workspace_bytes",
     "tra_bucketize_lengths",
     "tra_bucketize_scatter",
+    "tra_bucketize_ids_workspace_bytes",
+    "tra_bucketize_ids",
     "tra_quantize_rows",
     "tra_quantize_rows_padded",
     "tra_quantize_rows_sbhalf",
@@ -125,6 +127,11 @@ def lib() -> ctypes.CDLL:
         l.tra_bucketize_workspace_bytes.restype = i64
         l.tra_bucketize_lengths.argtypes = [vp, vp, i32, vp, i32, i32, i32, vp, vp]
         l.tra_bucketize_scatter.argtypes = [vp, vp, i32, vp, vp, i32, i32, i32, i32, vp, vp, vp, vp, vp, vp]
+        l.tra_bucketize_ids_workspace_bytes.argtypes = [i32, i32, i32, i64]
+        l.tra_bucketize_ids_workspace_bytes.restype = i64
+        l.tra_bucketize_ids.argtypes = [
+            vp, vp, i32, vp, vp, i32, i32, i32, i64, i32, vp, vp, vp, vp, vp, vp, vp, vp,
+        ]
         l.tra_quantize_rows.argtypes = [vp, i64, i32, i32, vp, i32, vp]
         l.tra_quantize_rows_padded.argtypes = [vp, i64, i32, i32, vp, i32, i64, vp]
         l.tra_quantize_rows_sbhalf.argtypes = [vp, i64, i32, i32, vp, vp]

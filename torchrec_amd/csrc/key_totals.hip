@@ -17,12 +17,10 @@ namespace tra {
 constexpr int kTotalsThreads = 256;
 constexpr int kMailSlots = 64;
 constexpr int kMailKeys = 1024;
-// What a slot holds before the kernel has written it (no sum of lengths).
-constexpr int64_t kNotThere = INT64_MIN;
 
-__device__ __forceinline__ void publish_total(int64_t v, int k, int64_t* dev, int64_t* host) {
+__device__ __forceinline__ void store_total(int64_t v, int k, int64_t* dev, int64_t* host) {
   if (dev) dev[k] = v;
-  if (host) __hip_atomic_store(host + k, v == kNotThere ? 0 : v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (host) publish_total(v, host + k);
 }
 
 // One block per key.
@@ -60,7 +58,7 @@ __global__ __launch_bounds__(kTotalsThreads) void key_totals_kernel(const T* __r
     int64_t t = 0;
 #pragma unroll
     for (int w = 0; w < kTotalsThreads / kWaveSize; ++w) t += s_part[w];
-    publish_total(t, blockIdx.x, dev, host);
+    store_total(t, blockIdx.x, dev, host);
   }
 }
 
@@ -68,7 +66,7 @@ template <typename T>
 __global__ __launch_bounds__(kTotalsThreads) void key_totals_of_offsets_kernel(const T* __restrict__ offsets, int32_t K,
                                                                                int32_t B, int64_t* dev, int64_t* host) {
   const int k = blockIdx.x * kTotalsThreads + threadIdx.x;
-  if (k < K) publish_total((int64_t)offsets[(int64_t)(k + 1) * B] - (int64_t)offsets[(int64_t)k * B], k, dev, host);
+  if (k < K) store_total((int64_t)offsets[(int64_t)(k + 1) * B] - (int64_t)offsets[(int64_t)k * B], k, dev, host);
 }
 
 // The host side: kMailSlots slots of kMailKeys totals in one pinned allocation, made on first use and kept until the
@@ -101,9 +99,40 @@ static int take_slot(int32_t* ticket) {
   return TRA_OK;
 }
 
-static void give_slot(int32_t ticket) {
+void mail_cancel(int32_t ticket) {
   std::lock_guard<std::mutex> lock(g_mail_mutex);
   g_mail_used &= ~(1ull << ticket);
+}
+
+int mail_open(hipStream_t s, int n, int32_t* ticket, int64_t** device) {
+  *ticket = -1;
+  if (n > kMailKeys) {
+    set_error("%d totals (at most %d reach the host)", n, kMailKeys);
+    return TRA_ERR_TOO_LARGE;
+  }
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    set_error("the stream is being captured: its kernels do not run now, and the host cannot wait for their totals");
+    return TRA_ERR_UNSUPPORTED;
+  }
+  int32_t slot = 0;
+  const int rc = take_slot(&slot);
+  if (rc != TRA_OK) return rc;
+  int64_t* host = g_mail + (int64_t)slot * kMailKeys;
+  for (int k = 0; k < n; ++k) host[k] = kMailEmpty;
+  std::atomic_thread_fence(std::memory_order_release);
+  void* p = nullptr;
+  const hipError_t e = hipHostGetDevicePointer(&p, host, 0);
+  if (e != hipSuccess) {
+    mail_cancel(slot);
+    return hip_fail(e, "hipHostGetDevicePointer(totals)");
+  }
+  *device = static_cast<int64_t*>(p);
+  g_mail_slot[slot].stream = s;
+  g_mail_slot[slot].num_keys = n;
+  *ticket = slot;
+  return TRA_OK;
 }
 
 }  // namespace tra
@@ -121,33 +150,8 @@ int tra_key_totals_begin(const void* bags, int32_t bags_are_offsets, int32_t num
   hipStream_t s = (hipStream_t)stream;
   int64_t* host_dev = nullptr;
   if (ticket) {
-    *ticket = -1;
-    if (num_keys > kMailKeys) {
-      set_error("tra_key_totals_begin: %d keys (at most %d reach the host)", num_keys, kMailKeys);
-      return TRA_ERR_TOO_LARGE;
-    }
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-      (void)hipGetLastError();
-      set_error("tra_key_totals_begin: the stream is being captured, its kernels do not run now");
-      return TRA_ERR_UNSUPPORTED;
-    }
-    int32_t slot = 0;
-    const int rc = take_slot(&slot);
+    const int rc = mail_open(s, num_keys, ticket, &host_dev);
     if (rc != TRA_OK) return rc;
-    int64_t* host = g_mail + (int64_t)slot * kMailKeys;
-    for (int k = 0; k < num_keys; ++k) host[k] = kNotThere;
-    std::atomic_thread_fence(std::memory_order_release);
-    void* p = nullptr;
-    const hipError_t e = hipHostGetDevicePointer(&p, host, 0);
-    if (e != hipSuccess) {
-      give_slot(slot);
-      return hip_fail(e, "hipHostGetDevicePointer(key totals)");
-    }
-    host_dev = static_cast<int64_t*>(p);
-    g_mail_slot[slot].stream = s;
-    g_mail_slot[slot].num_keys = num_keys;
-    *ticket = slot;
   }
   if (bags_are_offsets) {
     const dim3 g((num_keys + kTotalsThreads - 1) / kTotalsThreads);
@@ -167,7 +171,7 @@ int tra_key_totals_begin(const void* bags, int32_t bags_are_offsets, int32_t num
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     if (ticket) {
-      give_slot(*ticket);
+      mail_cancel(*ticket);
       *ticket = -1;
     }
     return hip_fail(e, "tra_key_totals_begin");
@@ -187,10 +191,10 @@ int tra_key_totals_wait(int32_t ticket, int64_t* totals) {
   // was lost to an earlier fault.
   for (int k = 0; k < slot.num_keys; ++k) {
     int64_t v;
-    for (int spins = 0; (v = __atomic_load_n(host + k, __ATOMIC_RELAXED)) == kNotThere; ++spins) {
+    for (int spins = 0; (v = __atomic_load_n(host + k, __ATOMIC_RELAXED)) == kMailEmpty; ++spins) {
       if ((spins & 0xfff) == 0xfff) {
         const hipError_t e = hipStreamQuery(slot.stream);
-        if (e != hipErrorNotReady && __atomic_load_n(host + k, __ATOMIC_RELAXED) == kNotThere) {
+        if (e != hipErrorNotReady && __atomic_load_n(host + k, __ATOMIC_RELAXED) == kMailEmpty) {
           // (the slot stays taken: nothing says that the kernel will not write to it after all)
           if (e == hipSuccess) {
             set_error("tra_key_totals_wait: the stream is idle and key %d has no total", k);
@@ -204,7 +208,7 @@ int tra_key_totals_wait(int32_t ticket, int64_t* totals) {
     }
     totals[k] = v;
   }
-  give_slot(ticket);
+  mail_cancel(ticket);
   return TRA_OK;
 }
 

@@ -44,6 +44,18 @@ inline int header_bytes(int dtype) {
 void set_error(const char* fmt, ...);
 int hip_fail(hipError_t e, const char* what);
 
+// Totals on their way to the host (key_totals.hip): a slot of `n` int64 in pinned
+// memory.  A kernel queued on `stream` stores every one of them with
+// publish_total; tra_key_totals_wait(ticket) collects them and gives the slot
+// back.  mail_cancel gives it back where nothing was queued.
+int mail_open(hipStream_t stream, int n, int32_t* ticket, int64_t** device);
+void mail_cancel(int32_t ticket);
+constexpr int64_t kMailEmpty = INT64_MIN;  // no sum of lengths
+
+__device__ __forceinline__ void publish_total(int64_t v, int64_t* host) {
+  __hip_atomic_store(host, v == kMailEmpty ? 0 : v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 #define TRA_HIP(call)                                   \
   do {                                                  \
     hipError_t e__ = (call);                            \

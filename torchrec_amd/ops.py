@@ -220,6 +220,24 @@ def block_bucketize_sparse_features(
     new_pos (positions inside the original bag) is not produced: bucketize_pos
     must be False.  ``sequence`` asks for unbucketize_permute.
     """
+    return _block_bucketize(
+        lengths, indices, bucketize_pos, sequence, block_sizes, my_size, weights, keep_orig_idx
+    )[:5]
+
+
+def _block_bucketize(
+    lengths: torch.Tensor,
+    indices: torch.Tensor,
+    bucketize_pos: bool,
+    sequence: bool,
+    block_sizes: torch.Tensor,
+    my_size: int,
+    weights: Optional[torch.Tensor],
+    keep_orig_idx: bool,
+    want_buckets: bool = False,
+):
+    """``block_bucketize_sparse_features`` and, with ``want_buckets``, the bucket ``floor(id / block size)`` of
+    every input id (None where the kernels did not give it)."""
     if bucketize_pos:
         raise NotImplementedError("bucketize_pos is not supported")
     _lib.require_gpu(lengths, "block_bucketize_sparse_features")
@@ -242,6 +260,16 @@ def block_bucketize_sparse_features(
     B = n // F if F else 0
     W = int(my_size)
     bs = block_sizes.to(device=dev, dtype=torch.int64).contiguous()
+    if weights is not None:
+        weights = weights.contiguous().to(torch.float32)
+    one_call = _bucketize_ids(
+        lengths, indices, weights, bs, F, B, W, sequence, keep_orig_idx, want_buckets
+    )
+    if one_call is not None:
+        new_lengths, new_indices, new_weights, unbucketize, buckets = one_call
+        if new_lengths.dtype != lengths_dtype:
+            new_lengths = new_lengths.to(lengths_dtype)
+        return new_lengths, new_indices, new_weights, None, unbucketize, buckets
     offsets = asynchronous_complete_cumsum(lengths)
     new_lengths = torch.empty(W * n, dtype=lengths.dtype, device=dev)
     _lib.check(
@@ -252,10 +280,7 @@ def block_bucketize_sparse_features(
     new_offsets = asynchronous_complete_cumsum(new_lengths)
     total = int(new_offsets[-1].item())
     new_indices = torch.empty(total, dtype=indices.dtype, device=dev)
-    new_weights = None
-    if weights is not None:
-        weights = weights.contiguous().to(torch.float32)
-        new_weights = torch.empty(total, dtype=torch.float32, device=dev)
+    new_weights = torch.empty(total, dtype=torch.float32, device=dev) if weights is not None else None
     unbucketize = (
         torch.empty(indices.numel(), dtype=torch.int64, device=dev) if sequence else None
     )
@@ -272,7 +297,45 @@ def block_bucketize_sparse_features(
     )
     if new_lengths.dtype != lengths_dtype:
         new_lengths = new_lengths.to(lengths_dtype)
-    return new_lengths, new_indices, new_weights, None, unbucketize
+    return new_lengths, new_indices, new_weights, None, unbucketize, None
+
+
+def _bucketize_ids(lengths, indices, weights, block_sizes, F, B, W, sequence, keep_orig_idx, want_buckets):
+    """Bucketization in one call of the library (at most 64 buckets), or None where that does not apply:
+    ``(new_lengths, new_indices, new_weights, unbucketize, buckets)``."""
+    L = indices.numel()
+    if F < 1 or B < 1 or W < 1 or W > 64 or L == 0:
+        return None
+    dev = lengths.device
+    l = _lib.lib()
+    ws_bytes = l.tra_bucketize_ids_workspace_bytes(F, B, W, L)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    new_lengths = torch.empty(W * F * B, dtype=lengths.dtype, device=dev)
+    # Sized for all ids: how many have a bucket is known when the kernels that move them are queued already.
+    new_indices = torch.empty(L, dtype=indices.dtype, device=dev)
+    new_weights = torch.empty(L, dtype=torch.float32, device=dev) if weights is not None else None
+    unbucketize = torch.empty(L, dtype=torch.int64, device=dev) if sequence else None
+    buckets = torch.empty_like(indices) if want_buckets else None
+    ticket = array("i", (-1,))
+    rc = _entry("tra_bucketize_ids")(
+        lengths.data_ptr(), indices.data_ptr(), lengths.dtype is torch.int64, _lib.ptr(weights),
+        block_sizes.data_ptr(), F, B, W, L, bool(keep_orig_idx), ws.data_ptr(), new_lengths.data_ptr(),
+        new_indices.data_ptr(), _lib.ptr(new_weights), _lib.ptr(unbucketize), _lib.ptr(buckets),
+        ticket.buffer_info()[0], _lib.current_stream(dev),
+    )
+    if rc != 0:
+        if rc == _lib.ERR_TOO_LARGE or rc == _lib.ERR_UNSUPPORTED:
+            return None
+        _lib.check(rc)
+    host = array("q", bytes(8 * W))
+    rc = _entry("tra_key_totals_wait")(ticket[0], host.buffer_info()[0])
+    if rc != 0:
+        _lib.check(rc)
+    total = sum(host)
+    if total != L:  # (ids beyond the last bucket)
+        new_indices = new_indices[:total]
+        new_weights = None if new_weights is None else new_weights[:total]
+    return new_lengths, new_indices, new_weights, unbucketize, buckets
 
 
 def FloatOrHalfToFusedNBitRowwiseQuantizedSBHalf(weight: torch.Tensor, bit_rate: int) -> torch.Tensor:

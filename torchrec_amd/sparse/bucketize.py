@@ -24,13 +24,14 @@ def _bucketize(
     bucketize_pos: bool,
     block_bucketize_row_pos: Optional[List[torch.Tensor]],
     keep_original_indices: bool,
+    want_buckets: bool = False,
 ):
     assert block_sizes.numel() == len(kjt.keys()), (
         f"Expecting block sizes for {len(kjt.keys())} features, but {block_sizes.numel()} received."
     )
     if block_bucketize_row_pos is not None:
         raise NotImplementedError("uneven shard sizes (block_bucketize_row_pos) are not supported")
-    return ops.block_bucketize_sparse_features(
+    return ops._block_bucketize(
         kjt.lengths().view(-1),
         kjt.values(),
         bucketize_pos=bucketize_pos,
@@ -39,6 +40,7 @@ def _bucketize(
         my_size=num_buckets,
         weights=kjt.weights_or_none(),
         keep_orig_idx=keep_original_indices,
+        want_buckets=want_buckets,
     )
 
 
@@ -55,7 +57,7 @@ def bucketize_kjt_before_all2all(
     """Returns (bucketized KJT, unbucketize permute when ``output_permute``)."""
     if total_num_blocks is not None:
         raise NotImplementedError("two-level bucketization (total_num_blocks) is not supported")
-    lengths, indices, weights, pos, unbucketize = _bucketize(
+    lengths, indices, weights, pos, unbucketize, _ = _bucketize(
         kjt, num_buckets, block_sizes, output_permute, bucketize_pos, block_bucketize_row_pos, keep_original_indices
     )
     return (
@@ -84,11 +86,11 @@ def bucketize_kjt_inference(
     last two only for sequence features."""
     if total_num_buckets is not None:
         raise NotImplementedError("two-level bucketization (total_num_buckets) is not supported")
-    lengths, indices, weights, pos, unbucketize = _bucketize(
-        kjt, num_buckets, block_sizes, is_sequence, bucketize_pos, block_bucketize_row_pos, keep_original_indices
+    lengths, indices, weights, pos, unbucketize, bucket_mapping = _bucketize(
+        kjt, num_buckets, block_sizes, is_sequence, bucketize_pos, block_bucketize_row_pos, keep_original_indices,
+        want_buckets=is_sequence,
     )
-    bucket_mapping = None
-    if is_sequence:
+    if is_sequence and bucket_mapping is None:
         values = kjt.values()
         per_key = kjt.lengths().view(len(kjt.keys()), -1).sum(dim=1)
         per_id_block = torch.repeat_interleave(
