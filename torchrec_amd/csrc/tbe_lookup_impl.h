@@ -624,80 +624,88 @@ __device__ __forceinline__ int pool_bag(float (&acc)[NE], const LookupArgs& a,
   return bad;
 }
 
-// The same pooling with the ids fetched a whole lane group at a time: lane c of
-// the group loads id number j*lpr + c of the bag (block j), and each row's id
-// is then passed to the group's lanes with a cross-lane read.  One id load per
-// lpr rows instead of one per row.  Needs lpr >= 2*U (a power of two): the
-// block after the current one, requested when the current one is entered, is
-// then at least two batches ahead, like the ids of pool_bag.
-// TWO_BATCHES: lpr == 2 * U, i.e. an id block feeds exactly the two batches of
-// one loop iteration.  The block then changes at a fixed place in the loop and
-// its load is unconditional, so the number of loads in flight is the same on
-// every path and the compiler can wait for the oldest batch alone.  (Behind a
-// conditional load it has to assume the worst and drains all loads, which
-// undoes the double buffering once per iteration.)
-template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, int NE, bool TWO_BATCHES = false>
+// The same pooling with the ids fetched a block at a time: lane c of the group
+// loads id number c of a block, and each row's id is then passed to the group's
+// lanes with a cross-lane read, so there is one id load per block instead of
+// one per row.  The block after the current one, requested when the current one
+// is entered, is at least two batches ahead, like the ids of pool_bag.
+//
+// P == 0: a block is lpr ids (a power of two, 16 or more).
+// P > 0: a block is the 2 * U ids of one loop iteration, in 2 * U / P loads of P
+// ids each (the lane group has at least P lanes; those beyond load ids of the
+// next blocks and nobody reads them).  The block then changes at a fixed
+// place in the loop and its load is unconditional, so the number of loads in
+// flight is the same on every path and the compiler can wait for the oldest
+// batch alone.  (Behind a conditional load it has to assume the worst and
+// drains all loads, which undoes the double buffering once per iteration.)
+template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, int NE, int P>
 __device__ __forceinline__ int pool_bag_bulk(float (&acc)[NE], const LookupArgs& a,
                                               const RowWalk& w, int64_t start64, int len,
                                               int max_len_any_lane, int lpr, int c,
                                               int group_lane0) {
+  constexpr bool TWO_BATCHES = P > 0;
+  constexpr int LOADS = TWO_BATCHES ? 2 * U / P : 1;  // loads (registers) per block
   const int max_len = __builtin_amdgcn_readfirstlane(max_len_any_lane);
-  const int lpr_u = TWO_BATCHES ? 2 * U : __builtin_amdgcn_readfirstlane(lpr);
+  const int block = TWO_BATCHES ? 2 * U : __builtin_amdgcn_readfirstlane(lpr);
   const IdxT start = (IdxT)start64;
   const IdxT last = (IdxT)(a.num_indices - 1);
-  auto load_block = [&](int j) -> IdxT {
-    const int r = j * lpr_u + c;
-    return fetch_id<IdxT>(a, r < len, start + (IdxT)r, last);
-  };
-  // Weights travel the same way: lane c of the group loads the weight of id
-  // number j * lpr + c (per-sample weights: psw at that position; position
-  // weights: the table entry of that place in the bag), one load per lpr rows.
-  auto load_weights = [&](int j) -> float {
-    if constexpr (WEIGHTED == kPerSample) {
-      using UIdxT = typename std::make_unsigned<IdxT>::type;
-      const IdxT p = start + (IdxT)(j * lpr_u + c);
-      return a.psw[(UIdxT)p < (UIdxT)last ? p : last];
-    } else if constexpr (WEIGHTED == kByPosition) {
-      const uint32_t k = (uint32_t)(j * lpr_u + c);
-      const float v = w.pw[k < w.pw_last ? k : w.pw_last];
-      return w.pw_on ? v : 1.0f;
-    } else {
-      return 1.0f;
+  struct IdBlock { IdxT v[LOADS]; };
+  struct WeightBlock { float v[LOADS]; };
+  auto load_block = [&](int j) -> IdBlock {
+    IdBlock x;
+#pragma unroll
+    for (int k = 0; k < LOADS; ++k) {
+      const int r = j * block + k * P + c;
+      x.v[k] = fetch_id<IdxT>(a, r < len, start + (IdxT)r, last);
     }
+    return x;
   };
-  IdxT cur = load_block(0);
-  IdxT nxt = load_block(1);
-  float wcur = load_weights(0);
-  float wnxt = load_weights(1);
+  // Weights travel the same way: the lane that loads an id loads its weight
+  // (per-sample weights: psw at that position; position weights: the table
+  // entry of that place in the bag).
+  auto load_weights = [&](int j) -> WeightBlock {
+    WeightBlock x;
+#pragma unroll
+    for (int k = 0; k < LOADS; ++k) {
+      const int r = j * block + k * P + c;
+      if constexpr (WEIGHTED == kPerSample) {
+        using UIdxT = typename std::make_unsigned<IdxT>::type;
+        const IdxT p = start + (IdxT)r;
+        x.v[k] = a.psw[(UIdxT)p < (UIdxT)last ? p : last];
+      } else if constexpr (WEIGHTED == kByPosition) {
+        const float v = w.pw[(uint32_t)r < w.pw_last ? (uint32_t)r : w.pw_last];
+        x.v[k] = w.pw_on ? v : 1.0f;
+      } else {
+        x.v[k] = 1.0f;
+      }
+    }
+    return x;
+  };
+  IdBlock cur = load_block(0);
+  IdBlock nxt = load_block(1);
+  WeightBlock wcur = load_weights(0);
+  WeightBlock wnxt = load_weights(1);
   int cur_j = 0;
   // Id of row r (wave-uniform), or -1 past the bag's end.  r lies in the
-  // current block: a batch of U rows never straddles two blocks (U divides
-  // lpr) and enter() is called before each batch.  Reading `cur` only matters:
-  // a select between cur and nxt would wait for the load of nxt that enter()
-  // has just issued.
-  auto id_of = [&](int r) -> IdxT {
-    const int src = group_lane0 + (r - cur_j * lpr_u);
-    return (IdxT)__shfl(cur, src, kWaveSize);
+  // current block: a batch of U rows never straddles two blocks and enter() is
+  // called before each batch.  Reading `cur` only matters: a select between
+  // cur and nxt would wait for the load of nxt that enter() has just issued.
+  // `at`: row r's place in its loop iteration (known at compile time).
+  auto id_of = [&](int r, int at) -> IdxT {
+    if constexpr (TWO_BATCHES)
+      return (IdxT)__shfl(cur.v[at / P], group_lane0 + at % P, kWaveSize);
+    else
+      return (IdxT)__shfl(cur.v[0], group_lane0 + (r - cur_j * block), kWaveSize);
   };
-  auto weight_of = [&](int r) -> float {
-    if constexpr (WEIGHTED == 0) return 1.0f;
-    const int src = group_lane0 + (r - cur_j * lpr_u);
-    return __shfl(wcur, src, kWaveSize);
+  auto weight_of = [&](int r, int at) -> float {
+    if constexpr (WEIGHTED == 0)
+      return 1.0f;
+    else if constexpr (TWO_BATCHES)
+      return __shfl(wcur.v[at / P], group_lane0 + at % P, kWaveSize);
+    else
+      return __shfl(wcur.v[0], group_lane0 + (r - cur_j * block), kWaveSize);
   };
-  // Entering the block of row rb: make it the current one and request the next.
-  auto enter = [&](int rb) {
-    const int j = rb / lpr_u;
-    if (j > cur_j) {
-      cur = nxt;
-      nxt = load_block(j + 1);
-      if constexpr (WEIGHTED != 0) {
-        wcur = wnxt;
-        wnxt = load_weights(j + 1);
-      }
-      cur_j = j;
-    }
-  };
-  // The same step where it is known to happen (TWO_BATCHES: at every second batch).
+  // The step to the next block, where it is known to happen (P > 0: at every second batch).
   auto advance = [&]() {
     cur = nxt;
     ++cur_j;
@@ -707,11 +715,15 @@ __device__ __forceinline__ int pool_bag_bulk(float (&acc)[NE], const LookupArgs&
       wnxt = load_weights(cur_j + 1);
     }
   };
+  // Entering the block of row rb: make it the current one and request the next.
+  auto enter = [&](int rb) {
+    if (rb / block > cur_j) advance();
+  };
   RowBuf<CB> bufA[U], bufB[U];
   int bad = 0;
 #pragma unroll
   for (int u = 0; u < U; ++u)
-    bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufA[u], id_of(u), start + u, last, a, w, weight_of(u));
+    bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufA[u], id_of(u, u), start + u, last, a, w, weight_of(u, u));
   int it = 0;
   if constexpr (TWO_BATCHES) {
     // Whole iterations (2 * U rows, all inside the longest bag) run without the
@@ -722,13 +734,13 @@ __device__ __forceinline__ int pool_bag_bulk(float (&acc)[NE], const LookupArgs&
     for (; it + 2 * U <= max_len; it += 2 * U) {
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufB[u], id_of(it + U + u), start + it + U + u, last, a, w, weight_of(it + U + u));
+        bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufB[u], id_of(it + U + u, U + u), start + it + U + u, last, a, w, weight_of(it + U + u, U + u));
 #pragma unroll
       for (int u = 0; u < U; ++u) consume_row<DTYPE, CB, (WEIGHTED != 0)>(acc, bufA[u], w);
       advance();
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufA[u], id_of(it + 2 * U + u), start + it + 2 * U + u, last, a, w, weight_of(it + 2 * U + u));
+        bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufA[u], id_of(it + 2 * U + u, u), start + it + 2 * U + u, last, a, w, weight_of(it + 2 * U + u, u));
 #pragma unroll
       for (int u = 0; u < U; ++u) consume_row<DTYPE, CB, (WEIGHTED != 0)>(acc, bufB[u], w);
     }
@@ -737,7 +749,7 @@ __device__ __forceinline__ int pool_bag_bulk(float (&acc)[NE], const LookupArgs&
     if constexpr (!TWO_BATCHES) enter(it + U);
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufB[u], id_of(it + U + u), start + it + U + u, last, a, w, weight_of(it + U + u));
+      bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufB[u], id_of(it + U + u, U + u), start + it + U + u, last, a, w, weight_of(it + U + u, U + u));
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (it + u < max_len) consume_row<DTYPE, CB, (WEIGHTED != 0)>(acc, bufA[u], w);
@@ -745,7 +757,7 @@ __device__ __forceinline__ int pool_bag_bulk(float (&acc)[NE], const LookupArgs&
     if constexpr (TWO_BATCHES) advance(); else enter(it + 2 * U);
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufA[u], id_of(it + 2 * U + u), start + it + 2 * U + u, last, a, w, weight_of(it + 2 * U + u));
+      bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufA[u], id_of(it + 2 * U + u, u), start + it + 2 * U + u, last, a, w, weight_of(it + 2 * U + u, u));
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (it + U + u < max_len) consume_row<DTYPE, CB, (WEIGHTED != 0)>(acc, bufB[u], w);
@@ -1506,13 +1518,19 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
 #pragma unroll
     for (int k = 0; k < NE; ++k) acc[k] = 0.0f;
     int bad;
-    if (U == 4 && lpr >= 2 * U && (lpr & (lpr - 1)) == 0)
-      if (lpr == 2 * U)
-        bad = pool_bag_bulk<DTYPE, CB, IdxT, WEIGHTED, U, NE, true>(acc, a, w, start, len, max_len, lpr, c, lane - c);
+    // Ids in blocks wherever a lane group has four lanes or more.
+    if constexpr (U == 4) {
+      if (lpr >= 16 && (lpr & (lpr - 1)) == 0)
+        bad = pool_bag_bulk<DTYPE, CB, IdxT, WEIGHTED, U, NE, 0>(acc, a, w, start, len, max_len, lpr, c, lane - c);
+      else if (lpr >= 8)
+        bad = pool_bag_bulk<DTYPE, CB, IdxT, WEIGHTED, U, NE, 8>(acc, a, w, start, len, max_len, lpr, c, lane - c);
+      else if (lpr >= 4)
+        bad = pool_bag_bulk<DTYPE, CB, IdxT, WEIGHTED, U, NE, 4>(acc, a, w, start, len, max_len, lpr, c, lane - c);
       else
-        bad = pool_bag_bulk<DTYPE, CB, IdxT, WEIGHTED, U, NE>(acc, a, w, start, len, max_len, lpr, c, lane - c);
-    else
+        bad = pool_bag<DTYPE, CB, IdxT, WEIGHTED, U, NE>(acc, a, w, start, len, max_len);
+    } else {
       bad = pool_bag<DTYPE, CB, IdxT, WEIGHTED, U, NE>(acc, a, w, start, len, max_len);
+    }
     if (a.bad_to_row0 != 0 && __builtin_amdgcn_ballot_w64(bad != 0) != 0)
       repool_bad_ids_as_row0<DTYPE, CB, IdxT, WEIGHTED, NE>(acc, a, w, start, len, max_len);
     TRA_STAMP(3);
