@@ -175,7 +175,7 @@ def _remap_numpy(values, sorted_ids, mapping, miss):
 @pytest.mark.gpu
 # Around the four entries of a read, the 512 pivots of a block, and segments of many entries.
 @pytest.mark.parametrize("size", [1, 2, 3, 4, 5, 9, 511, 512, 513, 514, 1026, 5000, 70_001])
-@pytest.mark.parametrize("kind", ["even", "clustered", "geometric", "half empty", "repeats"])
+@pytest.mark.parametrize("kind", ["even", "clustered", "geometric", "half empty", "repeats", "delimiter first"])
 def test_remap_search(size, kind):
     rng = np.random.default_rng(size)
     if kind == "clustered":
@@ -190,6 +190,8 @@ def test_remap_search(size, kind):
     if kind == "half empty":
         table[size // 2:] = np.iinfo(np.int64).max
     table[-1] = np.iinfo(np.int64).max
+    if kind == "delimiter first":  # (the last entry is compared, never searched: it may be the smallest)
+        table[-1] = -2**50
     mapping = rng.permutation(size).astype(np.int64)
     values = np.concatenate([table, table - 1, table + np.where(table == np.iinfo(np.int64).max, 0, 1),
                              rng.integers(-2**41, 2**41, 1500), [np.iinfo(np.int64).min, np.iinfo(np.int64).max, 0]])

@@ -832,7 +832,7 @@ __device__ __forceinline__ int64_t remap_lower_bound(const int64_t* __restrict__
     }
     int below = 0;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) below += x[e] < v ? 1 : 0;
+    for (int e = 0; e < 4; ++e) below += x[e] < v && (e < 3 || base + 3 < n) ? 1 : 0;  // (entry n need not be in order)
     if (below == 4) {
       lo = base + 4;
       vl = x[3];
