@@ -641,3 +641,61 @@ def test_qec_prepared_flags_and_registered_operators_give_the_same_rows():
             assert torch.equal(got[k].values().view(torch.int16), want[k].values().view(torch.int16))
             assert torch.equal(got[k].lengths(), want[k].lengths()) and torch.equal(got[k].weights(), want[k].weights())
     assert len(fired) == 2
+
+
+@pytest.mark.parametrize("observer", ["none", "hook", "pre_hook", "global", "replaced", "traced"])
+def test_registered_operator_is_called_where_the_call_can_be_seen(observer):
+    """A registered operator is launched directly only while nothing could see the module call; an observer added
+    after calls that were launched directly sees every later one."""
+    tables = [EmbeddingBagConfig(name="t", embedding_dim=32, num_embeddings=50, feature_names=["a"], data_type=DataType.INT8)]
+    reg = QuantEBC(tables, False, DEV, output_dtype=torch.half, register_tbes=True)
+    op = reg.tbes[0]
+    op.weights_dev.zero_()
+    op._rows_view(0)[:, 0:4] = torch.tensor([0x00, 0x2C, 0x00, 0xAC], dtype=torch.uint8, device=DEV)
+    kjt = KeyedJaggedTensor(keys=["a"], values=torch.arange(7, device=DEV), lengths=torch.tensor([3, 0, 4], device=DEV))
+    want = reg(kjt).values().clone()
+    seen, handle = [], None
+    forward = type(op).forward
+    if observer == "hook":
+        handle = op.register_forward_hook(lambda mod, args, out: seen.append(mod))
+    elif observer == "pre_hook":
+        handle = op.register_forward_pre_hook(lambda mod, args: seen.append(mod))
+    elif observer == "global":
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda mod, args, out: seen.append(mod))
+    elif observer == "replaced":
+        op.forward = lambda *args, **kwargs: (seen.append(op), forward(op, *args, **kwargs))[1]
+    plain = torch.nn.Module.__call__
+    try:
+        if observer == "traced":
+            torch.nn.Module.__call__ = lambda mod, *args, **kwargs: (seen.append(mod), plain(mod, *args, **kwargs))[1]
+        got = reg(kjt).values()
+    finally:
+        torch.nn.Module.__call__ = plain
+        if handle is not None:
+            handle.remove()
+    assert (op in seen) == (observer != "none")
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("first", ["ab", "ba"])
+def test_kept_features_order_with_and_without_the_short_route(first):
+    """``cache_features_order``: the first key order seen holds for every later call, whichever way the operator is
+    launched (a hook keeps the call off the short route)."""
+    tables = [EmbeddingBagConfig(name=f"t{k}", embedding_dim=32, num_embeddings=50, feature_names=[k], data_type=DataType.INT8)
+              for k in "ab"]
+    got = {}
+    for hooked in (False, True):
+        q = QuantEBC(tables, False, DEV, output_dtype=torch.half, register_tbes=True, cache_features_order=True)
+        op = q.tbes[0]
+        g = torch.Generator(device="cuda").manual_seed(5)
+        op.weights_dev.random_(0, 256, generator=g)
+        for t in range(2):
+            op._rows_view(t)[:, 0:4] = torch.tensor([0x00, 0x2C, 0x00, 0xAC], dtype=torch.uint8, device=DEV)
+        if hooked:
+            op.register_forward_hook(lambda mod, args, out: None)
+        lengths = torch.tensor([3, 0, 4, 1, 2, 2], device=DEV)
+        ids = torch.arange(12, device=DEV) * 4
+        got[hooked] = [q(KeyedJaggedTensor(keys=list(keys), values=ids, lengths=lengths)).values().clone()
+                       for keys in (first, "ab", "ba", "ab")]
+    assert all(torch.equal(x, y) for x, y in zip(got[False], got[True]))
+    assert all(torch.equal(x, got[False][0]) for x in got[False])

@@ -362,7 +362,9 @@ class _FeatureOrderMixin:
         if getattr(self, MODULE_ATTR_CACHE_FEATURES_ORDER, False):
             # the reference's contract for this flag: the first key order seen is kept
             if self._features_order is None:
-                self._features_order = [kjt_keys.index(k) for k in self._feature_names]
+                self._features_order = order = [kjt_keys.index(k) for k in self._feature_names]
+                if order == list(range(len(order))):
+                    self._identity_order = order
             return self._features_order
         if kjt_keys == self._feature_names:
             identity = self._identity_order
@@ -393,6 +395,22 @@ class _FeatureOrderMixin:
         if len(cache) < 64:
             cache[id(order)] = (order, groups)
         return groups
+
+
+_module_call = nn.Module.__call__  # (tracers put their own in its place)
+
+
+def _call_is_unobserved(op: nn.Module) -> bool:
+    """Whether calling ``op`` as a module is nothing but its class's forward: no hooks of its own or of all modules,
+    no tracer, not compiled, forward not replaced on the object."""
+    m = torch.nn.modules.module
+    return not (
+        op._forward_hooks or op._forward_pre_hooks or op._backward_hooks or op._backward_pre_hooks
+        or m._global_forward_hooks or m._global_forward_pre_hooks
+        or m._global_backward_hooks or m._global_backward_pre_hooks
+        or op._compiled_call_impl is not None or "forward" in op.__dict__
+        or nn.Module.__call__ is not _module_call or torch._C._get_tracing_state() is not None
+    )
 
 
 # ---------------------------------------------------------------------------
@@ -500,7 +518,8 @@ class EmbeddingBagCollection(EmbeddingBagCollectionInterface, ModuleNoCopyMixin,
             and not self._is_weighted
             and position_weights is None
             and features._offsets is None
-            and not self.register_tbes  # (registered operators are called as modules, below)
+            # (registered operators are called as modules, below, where anything could see the call)
+            and (not self.register_tbes or _call_is_unobserved(ops_[0]))
         ):
             op = ops_[0]
             v, ln, keys = features._values, features._lengths, features._keys
@@ -521,7 +540,11 @@ class EmbeddingBagCollection(EmbeddingBagCollectionInterface, ModuleNoCopyMixin,
                 and ln.is_contiguous()
                 and op._weights_initialized
                 and op._buffers["weights_dev"].get_device() == di
-                and not getattr(self, MODULE_ATTR_CACHE_FEATURES_ORDER, False)
+                # (where the first key order seen is kept for good: that it was the features' own)
+                and (
+                    not getattr(self, MODULE_ATTR_CACHE_FEATURES_ORDER, False)
+                    or (self._features_order is not None and self._features_order is self._identity_order)
+                )
             ):
                 K = len(keys)
                 n_len = ln.numel()
