@@ -31,7 +31,6 @@ class KTRegroupAsDict(torch.nn.Module):
         self._is_inited = False
         self._plan = None
         self._layout = None
-        self._layout = None
 
     def embedding_cast(self, embs: List[torch.Tensor]) -> List[torch.Tensor]:
         if self._emb_dtype is None:
