@@ -8,7 +8,7 @@ import torch
 
 import oracle as O
 from helpers import bucketize_python
-from torchrec_amd import ops
+from torchrec_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
@@ -35,6 +35,24 @@ def test_cumsum_unaligned_view(dtype):
     assert view.data_ptr() % 16 != 0
     got = ops.asynchronous_complete_cumsum(view).cpu().numpy()
     assert np.array_equal(got, O.cumsum(lengths[1:]))
+
+
+@pytest.mark.parametrize("in_shift,out_shift", [(1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("n", [131_073, 139_265, 262_144])
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+def test_cumsum_tiles_unaligned(n, dtype, in_shift, out_shift):
+    """The two-launch scan with input or output off a 16-byte boundary; nothing behind out[n] is written."""
+    rng = np.random.default_rng(n)
+    lengths = rng.integers(0, 50, n + in_shift).astype(dtype)
+    src = torch.from_numpy(lengths).to(DEV)[in_shift:]
+    out = torch.full((n + 8,), -1, dtype=src.dtype, device=DEV)
+    l = _lib.lib()
+    ws = torch.empty(l.tra_cumsum_workspace_bytes(n), dtype=torch.uint8, device=DEV)
+    _lib.check(l.tra_cumsum(src.data_ptr(), n, int(dtype is np.int64), out[out_shift:].data_ptr(), ws.data_ptr(),
+                            _lib.current_stream(DEV)))
+    got = out.cpu().numpy()
+    assert np.array_equal(got[out_shift : out_shift + n + 1], O.cumsum(lengths[in_shift:]))
+    assert (got[:out_shift] == -1).all() and (got[out_shift + n + 1 :] == -1).all()
 
 
 def test_cumsum_int64_beyond_32_bits():

@@ -17,8 +17,6 @@ typedef int64_t i64x2_t __attribute__((ext_vector_type(2), aligned(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kScanThreads = 256;
-constexpr int kScanItems = 16;
-constexpr int kScanTile = kScanThreads * kScanItems;
 
 template <typename T>
 __device__ __forceinline__ int64_t ld(const void* p, int64_t i) {
@@ -58,20 +56,43 @@ __device__ __forceinline__ int64_t block_sum(int64_t v, int64_t* smem) {
 }
 
 // ---- complete cumsum --------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(kScanThreads) void tile_sums_kernel(const void* in, int64_t n,
-                                                                  int64_t* sums) {
-  __shared__ int64_t smem[kScanThreads / kWaveSize];
-  const int64_t base = (int64_t)blockIdx.x * kScanTile;
-  int64_t x[kScanItems];
+// Two launches for inputs beyond the one-launch scan below: sums of tiles of
+// kScanTile lengths, then every tile scanned behind the sum of the sums in front
+// of it.  At 262144 lengths both are bound by the latency of their few dependent
+// steps on 64 blocks, so a thread holds four consecutive lengths that come with
+// one 16-byte load (two for int64), the scan's own loads are under way while the
+// sums are added, and the offsets leave as 16-byte vectors.  One length per load
+// (sixteen consecutive ones per thread in the second kernel) took 10.1 us for
+// 262144 int32 lengths and 20.1 us for 2 M; now 6.6 us, of which two empty
+// launches are about 5, and 10.0 us.
+constexpr int kTileThreads = 1024;
+constexpr int kTileItems = 4;
+constexpr int kScanTile = kTileThreads * kTileItems;
+
+// This thread's lengths of the tile (zeros past the end).  VEC: `in` lies on a 16-byte boundary.
+template <typename T, bool VEC>
+__device__ __forceinline__ void load_tile_items(const T* __restrict__ in, int64_t base, int64_t n,
+                                                int64_t (&x)[kTileItems]) {
+  struct __align__(16) Vec { T v[kTileItems]; };
+  if (VEC && base + kTileItems <= n) {
+    const Vec q = *reinterpret_cast<const Vec*>(in + base);
 #pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    const int64_t i = base + k * kScanThreads + threadIdx.x;
-    x[k] = i < n ? ld<T>(in, i) : 0;
+    for (int i = 0; i < kTileItems; ++i) x[i] = (int64_t)q.v[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < kTileItems; ++i) x[i] = base + i < n ? (int64_t)in[base + i] : 0;
   }
+}
+
+template <typename T, bool VEC>
+__global__ __launch_bounds__(kTileThreads) void tile_sums_kernel(const T* __restrict__ in, int64_t n,
+                                                                 int64_t* __restrict__ sums) {
+  __shared__ int64_t smem[kTileThreads / kWaveSize];
+  int64_t x[kTileItems];
+  load_tile_items<T, VEC>(in, (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kTileItems, n, x);
   int64_t v = 0;
 #pragma unroll
-  for (int k = 0; k < kScanItems; ++k) v += x[k];
+  for (int i = 0; i < kTileItems; ++i) v += x[i];
   v = block_sum(v, smem);
   if (threadIdx.x == 0) sums[blockIdx.x] = v;
 }
@@ -159,46 +180,55 @@ __global__ __launch_bounds__(kSmallThreads) void scan_small_kernel(const T* __re
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kScanThreads) void scan_tiles_kernel(const void* in, int64_t n,
-                                                                   const int64_t* sums, void* out) {
-  __shared__ int64_t smem[kScanThreads / kWaveSize];
-  __shared__ int64_t wave_tot[kScanThreads / kWaveSize];
+// VEC: `in` and `out` lie on 16-byte boundaries.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(kTileThreads) void scan_tiles_kernel(const T* __restrict__ in, int64_t n,
+                                                                  const int64_t* __restrict__ sums,
+                                                                  T* __restrict__ out) {
+  struct __align__(16) Vec { T v[kTileItems]; };
+  __shared__ int64_t smem[kTileThreads / kWaveSize];
+  __shared__ int64_t wave_tot[kTileThreads / kWaveSize];
+  const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kTileItems;
+  int64_t x[kTileItems];
+  load_tile_items<T, VEC>(in, base, n, x);
   // Sum of all earlier tiles.
   int64_t prefix = 0;
-  if (sums) {
-    for (int i = threadIdx.x; i < (int)blockIdx.x; i += kScanThreads) prefix += sums[i];
-    prefix = block_sum(prefix, smem);
-  }
-  // Each thread owns kScanItems consecutive elements.
-  const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
-  int64_t x[kScanItems];
+  for (int i = threadIdx.x; i < (int)blockIdx.x; i += kTileThreads) prefix += sums[i];
+  prefix = block_sum(prefix, smem);
+  // Exclusive scan of the per-thread sums: wave scan, then wave totals.
   int64_t tsum = 0;
 #pragma unroll
-  for (int i = 0; i < kScanItems; ++i) {
-    x[i] = base + i < n ? ld<T>(in, base + i) : 0;
-    tsum += x[i];
-  }
-  // Exclusive scan of the per-thread sums: wave scan, then wave totals.
+  for (int i = 0; i < kTileItems; ++i) tsum += x[i];
   const int lane = threadIdx.x & (kWaveSize - 1);
   const int wave = threadIdx.x / kWaveSize;
-  int64_t inc = tsum;
-#pragma unroll
-  for (int off = 1; off < kWaveSize; off <<= 1) {
-    const int64_t o = __shfl_up(inc, off, 64);
-    if (lane >= off) inc += o;
-  }
+  const int64_t inc = wave_scan(tsum, lane);
   if (lane == kWaveSize - 1) wave_tot[wave] = inc;
   __syncthreads();
-  int64_t wprefix = 0;
-  for (int w = 0; w < wave; ++w) wprefix += wave_tot[w];
-  int64_t run = prefix + wprefix + inc - tsum;
-  if (blockIdx.x == 0 && threadIdx.x == 0) st<T>(out, 0, 0);
+  int64_t run = prefix + inc - tsum;
+  for (int w = 0; w < wave; ++w) run += wave_tot[w];
+  // out[i] is what lies in front of length i: the vectors stay aligned.
+  Vec q;
 #pragma unroll
-  for (int i = 0; i < kScanItems; ++i) {
+  for (int i = 0; i < kTileItems; ++i) {
+    q.v[i] = (T)run;
     run += x[i];
-    if (base + i < n) st<T>(out, base + i + 1, run);
   }
+  if (VEC && base + kTileItems <= n) {
+    *reinterpret_cast<Vec*>(out + base) = q;
+  } else {
+#pragma unroll
+    for (int i = 0; i < kTileItems; ++i)
+      if (base + i < n) out[base + i] = q.v[i];
+  }
+  if (base < n && base + kTileItems >= n) out[n] = (T)run;
+}
+
+template <typename T, bool VEC>
+static void launch_scan_tiles(const void* lengths, int64_t n, int64_t* sums, void* offsets, unsigned tiles,
+                              hipStream_t s) {
+  hipLaunchKernelGGL((tile_sums_kernel<T, VEC>), dim3(tiles), dim3(kTileThreads), 0, s, (const T*)lengths, n, sums);
+  hipLaunchKernelGGL((scan_tiles_kernel<T, VEC>), dim3(tiles), dim3(kTileThreads), 0, s, (const T*)lengths, n, sums,
+                     (T*)offsets);
 }
 
 // ---- per-key totals ---------------------------------------------------------
@@ -1259,12 +1289,11 @@ extern "C" {
 
 // The one-launch scan takes up to 131072 lengths: every block sums what lies in front of its tile
 // itself, so the last block reads the whole input through one compute unit (512 KB of int32 in
-// about 4 us).  At 262144 int32 lengths it measured 18 us against 16 us for the two-kernel scan.
+// about 4 us): 7.8 us for 131072 int32 lengths.
 constexpr int64_t kSmallScanMax = (int64_t)kSmallMaxTiles * kSmallThreads * 2;
 int64_t tra_cumsum_workspace_bytes(int64_t n) {
   if (n <= kSmallScanMax) return 0;
-  const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-  return tiles > 1 ? tiles * (int64_t)sizeof(int64_t) : 0;
+  return (n + kScanTile - 1) / kScanTile * (int64_t)sizeof(int64_t);
 }
 
 int tra_cumsum(const void* lengths, int64_t n, int32_t is_i64, void* offsets, void* workspace,
@@ -1299,28 +1328,19 @@ int tra_cumsum(const void* lengths, int64_t n, int32_t is_i64, void* offsets, vo
     }
     return check_launch("tra_cumsum");
   }
-  const int64_t tiles = n == 0 ? 1 : (n + kScanTile - 1) / kScanTile;
-  int64_t* sums = nullptr;
-  if (tiles > 1) {
-    if (!workspace) {
-      set_error("tra_cumsum: workspace of %lld bytes required",
-                (long long)tra_cumsum_workspace_bytes(n));
-      return TRA_ERR_INVALID_ARGUMENT;
-    }
-    sums = (int64_t*)workspace;
-    if (is_i64)
-      hipLaunchKernelGGL(tile_sums_kernel<int64_t>, dim3((unsigned)tiles), dim3(kScanThreads), 0, s,
-                         lengths, n, sums);
-    else
-      hipLaunchKernelGGL(tile_sums_kernel<int32_t>, dim3((unsigned)tiles), dim3(kScanThreads), 0, s,
-                         lengths, n, sums);
+  const unsigned tiles = (unsigned)((n + kScanTile - 1) / kScanTile);
+  if (!workspace) {
+    set_error("tra_cumsum: workspace of %lld bytes required", (long long)tra_cumsum_workspace_bytes(n));
+    return TRA_ERR_INVALID_ARGUMENT;
   }
+  int64_t* sums = (int64_t*)workspace;
+  const bool vec = (uintptr_t)lengths % 16 == 0 && (uintptr_t)offsets % 16 == 0;
   if (is_i64)
-    hipLaunchKernelGGL(scan_tiles_kernel<int64_t>, dim3((unsigned)tiles), dim3(kScanThreads), 0, s,
-                       lengths, n, sums, offsets);
+    vec ? launch_scan_tiles<int64_t, true>(lengths, n, sums, offsets, tiles, s)
+        : launch_scan_tiles<int64_t, false>(lengths, n, sums, offsets, tiles, s);
   else
-    hipLaunchKernelGGL(scan_tiles_kernel<int32_t>, dim3((unsigned)tiles), dim3(kScanThreads), 0, s,
-                       lengths, n, sums, offsets);
+    vec ? launch_scan_tiles<int32_t, true>(lengths, n, sums, offsets, tiles, s)
+        : launch_scan_tiles<int32_t, false>(lengths, n, sums, offsets, tiles, s);
   return check_launch("tra_cumsum");
 }
 
