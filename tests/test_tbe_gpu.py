@@ -1099,6 +1099,41 @@ def test_bounds_check_warning_and_ignore_pool_row_zero(mode, tuning):
     assert tbe.out_of_range_count() == int((bad == rows + 1).sum())
 
 
+@pytest.mark.parametrize("dt,dim", [(O.INT8, 28), (O.INT8, 112), (O.INT4, 72), (O.INT8, 72), (O.FP16, 80), (O.INT8, 192),
+                                    (O.FP16, 120), (O.INT8, 304)])
+@pytest.mark.parametrize("idt", [np.int32, np.int64])
+def test_bad_ids_are_counted_once_at_every_row_width(dt, dim, idt, tuning):
+    """Row widths whose lane groups (7, 9, 10, 12, 15, 19 lanes) do not divide the wave: the lanes left over behind
+    the last group take no part, so every bad id is counted once, wherever it lies in its bag, and outputs are the
+    oracle's with the bad ids skipped, or pooled as row 0."""
+    from torchrec_amd.tbe.enums import BoundsCheckMode
+    tuning(balanced=1)
+    rng = np.random.default_rng(300 + dim)
+    rows, B = 90, 150
+    specs = [(dt, rows, dim), (dt, rows + 7, dim)]
+    lengths = rng.integers(0, 27, 2 * B)
+    lengths[::3] = 8  # (an id block)
+    offsets = np.zeros(2 * B + 1, dtype=idt)
+    offsets[1:] = np.cumsum(lengths)
+    ids = rng.integers(0, rows, offsets[-1]).astype(idt)
+    for bad in (np.arange(8), np.flatnonzero(rng.random(len(ids)) < 0.3), np.arange(len(ids))):
+        x = ids.copy()
+        x[bad] = rows + 7 + rng.integers(0, 9, len(bad))
+        for mode, instead in ((None, -1), (BoundsCheckMode.WARNING, 0)):
+            tbe, store = build(rng, specs, [0, 1], O.SUM, O.FP32, 16, bounds_check_mode=mode)
+            y = ids.copy()
+            y[bad] = instead
+            want = O.tbe_forward(store, [0, 1], B, y, offsets, None, O.SUM, O.FP32)
+            tx = torch.from_numpy(x).to(DEV)
+            for how in ("offsets", "lengths"):
+                if how == "offsets":
+                    got = tbe(tx, torch.from_numpy(offsets).to(DEV))
+                else:
+                    got = tbe(tx, None, lengths=torch.from_numpy(lengths.astype(idt)).to(DEV), batch_size=B)
+                assert bits_equal(got.cpu().numpy(), want) == 0, (mode, how)
+                assert tbe.out_of_range_count() == len(bad), (mode, how, len(bad))
+
+
 def test_multi_class_call_on_two_streams(tuning):
     """A plan of five or more launch classes runs every other launch on its own second stream,
     forked from and joined to the caller's stream inside the call.  Checked: the same bits as with

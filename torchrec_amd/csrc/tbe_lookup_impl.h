@@ -1505,13 +1505,13 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
     RowWalk w;
     w.chunk_off = Traits<DTYPE>::kHeader + d.payload_off + c * CB;
     w.lane_base = a.weights + d.table_offset + w.chunk_off;
-    w.set_rows(d.rows, d.row_bytes);
-    w.count_errors = c == 0 && d.payload_off == 0;
+    // The lanes behind the last whole group read ids of other groups where pool_bag_bulk's cross-lane
+    // read passes lane 63: for them every id lies outside the table, so none of its rows is fetched.
+    w.set_rows(g < gpw ? d.rows : 0, d.row_bytes);
+    w.count_errors = c == 0 && g < gpw && d.payload_off == 0;
     w.hdr_lane = lane - c;
     w.sel0 = mfma_byte_selector(lane, 0);
     w.sel1 = mfma_byte_selector(lane, 1);
-  w.sel0 = mfma_byte_selector(lane, 0);
-  w.sel1 = mfma_byte_selector(lane, 1);
     w.set_position_weights(a, sc.first + fi, start);
 
     float acc[NE];
@@ -1531,7 +1531,7 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
     } else {
       bad = pool_bag<DTYPE, CB, IdxT, WEIGHTED, U, NE>(acc, a, w, start, len, max_len);
     }
-    if (a.bad_to_row0 != 0 && __builtin_amdgcn_ballot_w64(bad != 0) != 0)
+    if (a.bad_to_row0 != 0 && __builtin_amdgcn_ballot_w64(bad != 0 && g < gpw) != 0)
       repool_bad_ids_as_row0<DTYPE, CB, IdxT, WEIGHTED, NE>(acc, a, w, start, len, max_len);
     TRA_STAMP(3);
 #ifdef TRA_INSTRUMENT
