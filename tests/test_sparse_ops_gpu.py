@@ -408,3 +408,37 @@ def test_bucketize_tiles(F, B, W, max_len, idt, weighted, keep):
     assert (buckets is None) == (W > 64 or len(ids) == 0)
     if buckets is not None:
         assert np.array_equal(buckets.cpu().numpy(), q)
+
+
+@pytest.mark.parametrize("W", [1, 8, 64])
+@pytest.mark.parametrize("idt", [np.int32, np.int64])
+@pytest.mark.parametrize("kind", ["in one tile", "across tiles", "before the ids", "behind the ids"])
+def test_bucketize_malformed_lengths(W, idt, kind):
+    """Lengths that are no partition of the ids: a bag starts at the running sum of the lengths as they stand, a
+    negative one is empty, overlapping bags each have their ids, and nothing lies outside the ids."""
+    rng = np.random.default_rng(W)
+    lengths = {
+        "in one tile": [1000, -990, 1000], "across tiles": [40] * 700 + [-900, 1000] + [3] * 700,
+        "before the ids": [-7, 5, 9, 30], "behind the ids": [20, 50, -60, 25],
+    }[kind]
+    n = len(lengths)
+    offsets = np.cumsum([0] + lengths)
+    L = 45 if kind == "behind the ids" else int(offsets[-1])
+    bs = np.array([37])
+    ids = rng.integers(0, 37 * (W + 1), L)
+    weights = rng.random(L).astype(np.float32)
+    ends = np.clip(offsets, 0, L)
+    at = np.concatenate([np.arange(a, max(a, b)) for a, b in zip(ends[:-1], ends[1:])])
+    bag = np.repeat(np.arange(n), np.maximum(ends[1:] - ends[:-1], 0))
+    q = ids[at] // 37
+    kept = np.flatnonzero(q < W)
+    order = kept[np.argsort(q[kept], kind="stable")]
+    nl, ni, nw, _, unb = ops.block_bucketize_sparse_features(
+        torch.from_numpy(np.asarray(lengths, dtype=idt)).to(DEV), torch.from_numpy(ids.astype(idt)).to(DEV), False, True,
+        torch.from_numpy(bs).to(DEV), W, torch.from_numpy(weights).to(DEV), True)
+    assert np.array_equal(nl.cpu().numpy(), np.bincount(q[kept] * n + bag[kept], minlength=W * n))
+    assert np.array_equal(ni.cpu().numpy(), ids[at[order]])
+    assert np.array_equal(nw.cpu().numpy(), weights[at[order]])
+    unb = unb.cpu().numpy()
+    assert np.all(unb[np.setdiff1d(np.arange(L), at[kept])] == -1)
+    assert np.array_equal(ids[at[order]][unb[unb >= 0]], ids[unb >= 0])

@@ -7,6 +7,9 @@
 //   bucket_counts ids per (bucket, bag) = the new lengths, and per (bucket, tile)
 //   bucket_scan   where each tile's ids of each bucket go; bucket totals to the host
 //   bucket_move   the ids to their place
+// Lengths that are no partition of the ids (a negative one, or more in a tile
+// than there are ids) are found by the first launch; no id is moved then, and
+// every total that reaches the host is -1.
 // Bound by memory: ids are read twice, everything else moves once (7.9 M int64
 // ids with weights in 64 x 4096 bags, 8 buckets: 270 MB).
 #include <algorithm>
@@ -30,11 +33,11 @@ struct BucketArgs {
   const void* indices;
   const float* weights;
   const int64_t* block_sizes;
-  int32_t* tile_total;    // [tiles]
+  int32_t* tile_total;    // [tiles] -1: bad lengths
   int64_t* tile_first;    // [tiles] first id of the tile
-  int32_t* counts;        // [W][tiles] ids of a bucket in a tile
+  int32_t* counts;        // [W][tiles] ids of a bucket in a tile, -1: bad lengths
   int64_t* place;         // [W][tiles] the bucket's ids in front of the tile
-  int64_t* bucket_total;  // [W]
+  int64_t* bucket_total;  // [W] -1: bad lengths somewhere
   int64_t* host_totals;   // [W] pinned
   void* new_lengths;      // [W][n]
   void* new_indices;
@@ -111,9 +114,15 @@ __global__ __launch_bounds__(kBktThreads) void tile_totals_kernel(const BucketAr
   int cnt;
   const int64_t bag = tile_bags(a, tile, cnt);
   int64_t sum = 0;
-  for (int i = lane; i < cnt; i += kWaveSize) sum += (int64_t) reinterpret_cast<const T*>(a.lengths)[bag + i];
+  bool bad = false;
+  for (int i = lane; i < cnt; i += kWaveSize) {
+    const int64_t x = (int64_t) reinterpret_cast<const T*>(a.lengths)[bag + i];
+    bad |= x < 0 || x > a.num_indices;
+    sum += x;
+  }
+  bad = __builtin_amdgcn_ballot_w64(bad) != 0;
   sum = wave_sum64(sum);
-  if (lane == 0) a.tile_total[tile] = (int32_t)sum;
+  if (lane == 0) a.tile_total[tile] = bad || sum > a.num_indices ? -1 : (int32_t)sum;
 }
 
 // One block per tile.  A tile's (bag, bucket) counters are in LDS; a bag's ids are
@@ -170,13 +179,14 @@ __global__ __launch_bounds__(kBktThreads) void bucket_counts_kernel(const Bucket
   if (i0 + 1 < cnt) s_end[i0 + 1] = front + incl;
   if (threadIdx.x == 0) a.tile_first[tile] = before;
   __syncthreads();
-  // (never outside the ids array, whatever the lengths say)
+  // (never outside the ids array, whatever the lengths say; the bags' ends are no places where the lengths are bad)
+  const bool bad = a.tile_total[tile] < 0;
   const int ids = before < 0 ? 0 : (int)max(min((int64_t)total, a.num_indices - before), (int64_t)0);
   const T* in = reinterpret_cast<const T*>(a.indices) + before;
   const Divider div((uint64_t)a.block_sizes[tile / a.per_feature]);
   const int sub = threadIdx.x & (a.lanes - 1);
   constexpr int U = 4;
-  for (int b = threadIdx.x / a.lanes; b < cnt; b += kBktThreads / a.lanes) {
+  for (int b = threadIdx.x / a.lanes; !bad && b < cnt; b += kBktThreads / a.lanes) {
     const int end = min(s_end[b], ids);
     for (int j0 = max(b > 0 ? s_end[b - 1] : 0, 0) + sub; j0 < end; j0 += U * a.lanes) {
       T id[U];
@@ -201,7 +211,7 @@ __global__ __launch_bounds__(kBktThreads) void bucket_counts_kernel(const Bucket
       sum += c;
     }
     sum = (int)wave_sum64(sum);
-    if (lane == 0) a.counts[(int64_t)p * a.tiles + tile] = sum;
+    if (lane == 0) a.counts[(int64_t)p * a.tiles + tile] = bad ? -1 : sum;
   }
 }
 
@@ -214,6 +224,7 @@ __global__ __launch_bounds__(kBktScanThreads) void bucket_scan_kernel(const Buck
   const int32_t* in = a.counts + (int64_t)blockIdx.x * a.tiles;
   int64_t* out = a.place + (int64_t)blockIdx.x * a.tiles;
   int64_t carry = 0;
+  int bad = 0;
   constexpr int U = 4;  // consecutive tiles per thread
   for (int t0 = 0; t0 < a.tiles; t0 += U * kBktScanThreads) {
     const int t = t0 + U * (int)threadIdx.x;
@@ -221,6 +232,7 @@ __global__ __launch_bounds__(kBktScanThreads) void bucket_scan_kernel(const Buck
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       x[u] = t + u < a.tiles ? in[t + u] : 0;
+      bad |= x[u] < 0;
       mine += x[u];
     }
     int64_t incl = mine;
@@ -245,6 +257,7 @@ __global__ __launch_bounds__(kBktScanThreads) void bucket_scan_kernel(const Buck
     carry += all;
     __syncthreads();
   }
+  if (__syncthreads_or(bad)) carry = -1;
   if (threadIdx.x == 0) {
     a.bucket_total[blockIdx.x] = carry;
     publish_total(carry, a.host_totals + blockIdx.x);
@@ -271,6 +284,7 @@ __global__ __launch_bounds__(kBktThreads) void bucket_move_kernel(const BucketAr
   const int lane = threadIdx.x & (kWaveSize - 1);
   const int wave = threadIdx.x / kWaveSize;
   const int tile = blockIdx.x;
+  if (a.bucket_total[0] < 0) return;  // (bad lengths)
   const int64_t first = a.tile_first[tile];
   const int ids = first < 0 ? 0 : (int)max(min((int64_t)a.tile_total[tile], a.num_indices - first), (int64_t)0);
   if (ids == 0) return;

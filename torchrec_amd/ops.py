@@ -266,6 +266,8 @@ def _block_bucketize(
         lengths, indices, weights, bs, F, B, W, sequence, keep_orig_idx, want_buckets
     )
     if one_call is not None:
+        if one_call[0] is None:
+            one_call = _bucketize_bad_lengths(lengths, indices, weights, bs, W, sequence, keep_orig_idx)
         new_lengths, new_indices, new_weights, unbucketize, buckets = one_call
         if new_lengths.dtype != lengths_dtype:
             new_lengths = new_lengths.to(lengths_dtype)
@@ -302,7 +304,8 @@ def _block_bucketize(
 
 def _bucketize_ids(lengths, indices, weights, block_sizes, F, B, W, sequence, keep_orig_idx, want_buckets):
     """Bucketization in one call of the library (at most 64 buckets), or None where that does not apply:
-    ``(new_lengths, new_indices, new_weights, unbucketize, buckets)``."""
+    ``(new_lengths, new_indices, new_weights, unbucketize, buckets)``, all None where the lengths are no partition
+    of the ids."""
     L = indices.numel()
     if F < 1 or B < 1 or W < 1 or W > 64 or L == 0:
         return None
@@ -331,11 +334,33 @@ def _bucketize_ids(lengths, indices, weights, block_sizes, F, B, W, sequence, ke
     rc = _entry("tra_key_totals_wait")(ticket[0], host.buffer_info()[0])
     if rc != 0:
         _lib.check(rc)
+    if host[0] < 0:
+        return None, None, None, None, None
     total = sum(host)
     if total != L:  # (ids beyond the last bucket)
         new_indices = new_indices[:total]
         new_weights = None if new_weights is None else new_weights[:total]
     return new_lengths, new_indices, new_weights, unbucketize, buckets
+
+
+def _bucketize_bad_lengths(lengths, indices, weights, block_sizes, W, sequence, keep_orig_idx):
+    """``_bucketize_ids`` of malformed lengths: bags start at the running sum of the lengths as they stand, a negative
+    one makes its own bag empty and the bags behind it overlap the ones in front; what lies outside the ids belongs
+    to no bag.  The bags' ids are written out one after the other and bucketized as a partition."""
+    L, dev = indices.numel(), lengths.device
+    offsets = torch.cumsum(torch.cat([lengths.new_zeros(1), lengths]), 0, dtype=torch.int64).clamp(0, L)
+    sizes = (offsets[1:] - offsets[:-1]).clamp(min=0)
+    at = torch.repeat_interleave(offsets[:-1] - (torch.cumsum(sizes, 0) - sizes), sizes)
+    at += torch.arange(at.numel(), device=dev)
+    new_lengths, new_indices, new_weights, _, order, _ = _block_bucketize(
+        sizes.to(lengths.dtype), indices[at], False, sequence, block_sizes, W,
+        None if weights is None else weights[at], keep_orig_idx,
+    )
+    unbucketize = None
+    if sequence:
+        unbucketize = torch.full((L,), -1, dtype=torch.int64, device=dev)
+        unbucketize[at] = order  # (an id of several bags: one of its places)
+    return new_lengths, new_indices, new_weights, unbucketize, None
 
 
 def FloatOrHalfToFusedNBitRowwiseQuantizedSBHalf(weight: torch.Tensor, bit_rate: int) -> torch.Tensor:
