@@ -330,7 +330,7 @@ int tra_bucketize_scatter(const void* offsets, const void* indices,
  * num_buckets numbers, to tra_key_totals_wait.  Where the lengths are no
  * partition of the ids (a negative one, or bags of more ids than there are) every
  * one of them is -1 and the outputs hold nothing.  TRA_ERR_TOO_LARGE beyond 64
- * buckets or 2^31 ids, and as for tra_key_totals_begin. */
+ * buckets or (nearly) 2^31 ids, and as for tra_key_totals_begin. */
 int64_t tra_bucketize_ids_workspace_bytes(int32_t num_features, int32_t batch_size,
                                           int32_t num_buckets, int64_t num_indices);
 int tra_bucketize_ids(const void* lengths, const void* indices, int32_t is_i64,

@@ -92,3 +92,14 @@ def test_fastcall_module_binds_the_same_entry_point():
     # a null plan is refused by the entry point itself, with its usual code and message
     rc = fn(None, None, None, None, 0, None, 1, 1, 0, _lib.POOL_SUM, _lib.FP16, None, 0, None, None)
     assert rc < 0 and b"null plan" in lib.tra_last_error()
+
+
+def test_bucketize_ids_refuses_id_counts_its_kernels_cannot_step_over():
+    """The kernels step up to 4096 places behind a tile's last id in 32 bits: a count that near to 2^31 is refused
+    before anything is queued (the general entry points take it)."""
+    l = _lib.lib()
+    word = (ctypes.c_int64 * 8)()
+    at = ctypes.cast(word, ctypes.c_void_p)
+    for n in (2**31 - 1, 2**31 - 4096):
+        rc = l.tra_bucketize_ids(at, at, 1, None, at, 1, 1, 2, n, 0, at, at, at, None, None, None, at, None)
+        assert rc == _lib.ERR_TOO_LARGE and b"ids" in l.tra_last_error()

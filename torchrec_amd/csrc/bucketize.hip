@@ -453,7 +453,8 @@ int tra_bucketize_ids(const void* lengths, const void* indices, int32_t is_i64, 
     return TRA_ERR_INVALID_ARGUMENT;
   }
   const BucketSizes z = bucket_sizes(num_features, batch_size, std::min(num_buckets, (int32_t)kBktMax), num_indices);
-  if (num_buckets > kBktMax || z.tiles > 0x7fffffff || num_indices > 0x7fffffff) {
+  // (the kernels count a tile's ids in 32 bits and look up to a step behind its last one)
+  if (num_buckets > kBktMax || z.tiles > 0x7fffffff || num_indices > 0x7fffffff - 2 * kBktStep) {
     set_error("tra_bucketize_ids: %d buckets (at most %d), %lld ids", num_buckets, kBktMax, (long long)num_indices);
     return TRA_ERR_TOO_LARGE;
   }
