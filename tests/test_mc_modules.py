@@ -235,3 +235,29 @@ def test_collection_remap_many_keys(K, B, shuffled, given):
     starts = np.concatenate([[0], np.cumsum(lengths.sum(1))])
     assert torch.equal(out.weights(), torch.cat([weights[starts[i]:starts[i + 1]] for i in order]))
     assert out.length_per_key() == lengths.sum(1)[order].tolist()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("keys", [["a", "b"], ["b", "a"]])
+@pytest.mark.parametrize("given", ["lengths", "offsets"])
+def test_collection_remap_refuses_what_its_kernels_cannot_read(keys, given):
+    """Values that are no int32 / int64 ids, and tables of another type or size, on every route of the collection."""
+    dev = torch.device("cuda:0")
+    configs = [EmbeddingConfig(name=f"t{f}", embedding_dim=4, num_embeddings=20, feature_names=[f]) for f in "ab"]
+    bags = torch.tensor([1, 2, 0, 1] if given == "lengths" else [0, 1, 3, 3, 4], device=dev)
+
+    def collection():
+        modules = {c.name: MCHManagedCollisionModule(20, dev) for c in configs}
+        return ManagedCollisionCollection(modules, configs).eval()
+
+    for dtype in (torch.float32, torch.float64):
+        with pytest.raises(TypeError, match="int32 or int64"):
+            collection()(KeyedJaggedTensor(keys=keys, values=torch.ones(4, dtype=dtype, device=dev), **{given: bags}))
+    ids = torch.arange(4, device=dev)
+    for name in ("_mch_sorted_raw_ids", "_mch_remapped_ids_mapping"):
+        for bad in (lambda t: t.to(torch.int32), lambda t: t[:-1], lambda t: t.repeat_interleave(2)[::2]):
+            mcc = collection()
+            module = mcc._managed_collision_modules["tb"]
+            setattr(module, name, bad(getattr(module, name)))
+            with pytest.raises(AssertionError):
+                mcc(KeyedJaggedTensor(keys=keys, values=ids, **{given: bags}))

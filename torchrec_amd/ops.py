@@ -469,6 +469,16 @@ def mch_remap(
     return out
 
 
+def _check_remap(values: torch.Tensor, sorted_ids: List[torch.Tensor], mappings: List[torch.Tensor], miss_ids: List[int]):
+    """Ids and tables as the remap kernels read them (one table, row mapping and miss row per key)."""
+    _check_int(values, "values")
+    assert len(mappings) == len(miss_ids) == len(sorted_ids)
+    di = values.get_device()
+    for s_, m_ in zip(sorted_ids, mappings):
+        assert s_.dtype is torch.int64 and m_.dtype is torch.int64 and s_.numel() == m_.numel() > 0
+        assert s_.is_contiguous() and m_.is_contiguous() and s_.get_device() == di and m_.get_device() == di
+
+
 def permute_keys(
     totals: torch.Tensor,
     order: List[int],
@@ -497,6 +507,8 @@ def permute_keys(
     tables, at = (), (None, None, None, None)
     if remap is not None:
         sorted_ids, mappings, miss = remap
+        assert len(sorted_ids) == Kp
+        _check_remap(values, sorted_ids, mappings, miss)
         tables = (
             array("q", [t.data_ptr() for t in sorted_ids]), array("q", [t.data_ptr() for t in mappings]),
             array("q", [t.numel() for t in sorted_ids]), array("q", miss),
@@ -525,13 +537,9 @@ def mch_remap_keys(
     """``mch_remap`` for every key of a KeyedJaggedTensor in one launch: key ``k`` (ids
     ``values[offsets[k*B] : offsets[(k+1)*B]]``) is looked up in ``sorted_ids[k]`` / ``mappings[k]``."""
     _lib.require_gpu(values, "mch_remap_keys")
-    _check_int(values, "values")
     K = len(sorted_ids)
-    assert len(mappings) == K and len(miss_ids) == K
+    _check_remap(values, sorted_ids, mappings, miss_ids)
     assert offsets.numel() == K * batch_size + 1, "offsets must have num_keys * B + 1 entries"
-    for s_, m_ in zip(sorted_ids, mappings):
-        assert s_.dtype == torch.int64 and m_.dtype == torch.int64 and s_.numel() == m_.numel() > 0
-        assert s_.is_contiguous() and m_.is_contiguous() and s_.device == values.device and m_.device == values.device
     values = values.contiguous()
     if offsets.dtype != values.dtype:
         offsets = offsets.to(values.dtype)
