@@ -141,7 +141,11 @@ int tra_tbe_forward(tra_tbe_t tbe, const void* weights, const void* indices,
  *   key_totals  DEVICE int64[num_keys], ids per key (num_keys <= 256), e.g. from
  *               tra_key_totals_begin: key k's ids follow those of the keys before it;
  *   key_starts  HOST int64[num_keys + 1], first id of each key (and the end).
- * `out` is [num_indices, dim]. */
+ * `out` is [num_indices, dim].  tra_tbe_takes_key_starts: 1 where the plan's
+ * launch arguments have room for key_starts (at most 128 column slices in a
+ * launch class; a row wider than 64 lanes is cut into several), else 0, and
+ * key_starts are refused with TRA_ERR_UNSUPPORTED. */
+int tra_tbe_takes_key_starts(tra_tbe_t tbe);
 int tra_tbe_forward_sequence(tra_tbe_t tbe, const void* weights, const void* indices,
                              const int64_t* key_totals, const int64_t* key_starts,
                              int32_t num_keys, int32_t idx_is_i64, int64_t num_indices,

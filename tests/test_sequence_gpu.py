@@ -9,7 +9,9 @@ import torch
 import oracle as O
 from helpers import bits_equal
 from test_tbe_gpu import build
-from torchrec_amd import ops
+from torchrec_amd import KeyedJaggedTensor, ops
+from torchrec_amd.modules.embedding_configs import DataType, EmbeddingConfig
+from torchrec_amd.quant import EmbeddingCollection as QuantEC
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
@@ -111,3 +113,23 @@ def test_key_totals_threads_and_open_calls():
 def test_key_totals_reject_other_integer_types():
     with pytest.raises(TypeError):
         ops.length_per_key(torch.ones(4, dtype=torch.int16, device=DEV), 2, 2)
+
+
+@pytest.mark.parametrize("K,dim", [(64, 1024), (65, 1024), (128, 8), (129, 8)])
+def test_collection_of_more_slices_than_key_starts(K, dim):
+    """One feature more than the launch arguments hold key starts of, in rows of one and of two column slices, from a
+    KJT without its per-key counts and with them (which the first call leaves on it)."""
+    rng = np.random.default_rng(K)
+    rows = torch.randn(9, dim, device=DEV).half()
+    config = EmbeddingConfig(name="t", embedding_dim=dim, num_embeddings=9, feature_names=[f"f{k}" for k in range(K)],
+                             data_type=DataType.FP16)
+    qec = QuantEC([config], DEV, output_dtype=torch.half,
+                  table_name_to_quantized_weights={"t": (rows.view(torch.uint8), None)})
+    assert qec._emb_modules[0].takes_key_starts() == (K * (2 if dim == 1024 else 1) <= 128)
+    lengths = torch.from_numpy(rng.integers(0, 4, 3 * K)).to(DEV)
+    ids = torch.from_numpy(rng.integers(0, 9, int(lengths.sum()))).to(DEV)
+    kjt = KeyedJaggedTensor(keys=[f"f{k}" for k in range(K)], values=ids, lengths=lengths)
+    for _ in range(2):
+        got = qec(kjt)
+        assert torch.equal(torch.cat([got[k].values() for k in kjt.keys()]), rows[ids])
+        assert kjt.length_per_key_or_none() is not None

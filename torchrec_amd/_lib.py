@@ -32,6 +32,7 @@ EXPORTED_SYMBOLS = [
     "tra_tbe_forward_lengths_static",
     "tra_tbe_forward_position_weighted",
     "tra_tbe_forward_sequence",
+    "tra_tbe_takes_key_starts",
     "tra_tbe_launch_info",
     "tra_tbe_set_bounds_check_mode",
     "tra_tbe_error_count",
@@ -112,6 +113,7 @@ def lib() -> ctypes.CDLL:
             vp, i64, vp, vp,
         ]
         l.tra_tbe_forward_sequence.argtypes = [vp, vp, vp, vp, vp, i32, i32, i64, i32, vp, vp]
+        l.tra_tbe_takes_key_starts.argtypes = [vp]
         l.tra_tbe_launch_info.argtypes = [vp, i32, i64, i32, i32, ctypes.c_char_p, i32]
         l.tra_tbe_set_bounds_check_mode.argtypes = [vp, i32]
         l.tra_tbe_error_count.argtypes = [vp, vp, ctypes.POINTER(i64)]

@@ -931,6 +931,10 @@ int tra_tbe_forward(tra_tbe_t tbe, const void* weights, const void* indices,
                       batch_size, num_indices, pooling_mode, out_dtype, out, out_stride, stream);
 }
 
+int tra_tbe_takes_key_starts(tra_tbe_t tbe) {
+  return tbe && tbe->max_class_feats <= (size_t)kMaxPos ? 1 : 0;
+}
+
 int tra_tbe_forward_sequence(tra_tbe_t tbe, const void* weights, const void* indices, const int64_t* key_totals,
                              const int64_t* key_starts, int32_t num_keys, int32_t idx_is_i64, int64_t num_indices,
                              int32_t out_dtype, void* out, void* stream) {
@@ -947,8 +951,8 @@ int tra_tbe_forward_sequence(tra_tbe_t tbe, const void* weights, const void* ind
     return TRA_ERR_UNSUPPORTED;
   }
   if (key_starts != nullptr) {
-    if (tbe->max_class_feats > (size_t)kMaxPos || num_indices > 0x7fffffff) {
-      set_error("tra_tbe_forward_sequence: a launch class of %d features (at most %d) or %lld ids",
+    if (!tra_tbe_takes_key_starts(tbe) || num_indices > 0x7fffffff) {
+      set_error("tra_tbe_forward_sequence: a launch class of %d column slices (at most %d) or %lld ids",
                 (int)tbe->max_class_feats, kMaxPos, (long long)num_indices);
       return TRA_ERR_UNSUPPORTED;
     }

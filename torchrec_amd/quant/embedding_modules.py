@@ -653,8 +653,8 @@ class EmbeddingBagCollection(EmbeddingBagCollectionInterface, ModuleNoCopyMixin,
         return self._device
 
 
-# The lookup kernels keep the position-weight layout (or a sequence lookup's key
-# starts) of a launch in its launch arguments: at most this many features per operator.
+# The lookup kernel keeps the position-weight layout of a launch in its launch
+# arguments: at most this many features per operator.
 _MAX_FUSED_POSITION_FEATURES = 128
 
 
@@ -862,7 +862,7 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
         on_gpu = indices.is_cuda and K > 0 and L > 0 and B > 0
         if features.length_per_key_or_none() is not None or features.offset_per_key_or_none() is not None or not on_gpu:
             offset_per_key = features.offset_per_key()
-            if on_gpu and self._starts_fit(offset_per_key, L):
+            if on_gpu and self._starts_fit(offset_per_key, L, order):
                 bounds = {"offsets": None, "key_starts": offset_per_key}
         else:
             built_from_offsets = features.lengths_or_none() is None
@@ -918,13 +918,13 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
             )
         return feature_embeddings
 
-    def _starts_fit(self, offset_per_key: List[int], num_indices: int) -> bool:
+    def _starts_fit(self, offset_per_key: List[int], num_indices: int, order: List[int]) -> bool:
         """Whether the operators can take these key starts as launch arguments."""
         return (
-            max(self._feature_splits, default=0) <= _MAX_FUSED_POSITION_FEATURES
-            and num_indices < 2**31
+            num_indices < 2**31
             and all(a <= b for a, b in zip(offset_per_key, offset_per_key[1:]))
             and offset_per_key[-1] <= num_indices
+            and all(op.takes_key_starts(p) for op, p in zip(self._emb_modules, self._group_positions(order)))
         )
 
     @classmethod

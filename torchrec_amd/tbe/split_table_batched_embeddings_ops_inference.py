@@ -443,7 +443,7 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
         sequence lookup (``PoolingMode.NONE``) needs no bag bounds, only where
         every input key's ids lie: with ``offsets=None`` it takes the ids per key
         as an int64 device tensor (``key_totals``) or the keys' first ids and the
-        end as integers (``key_starts``).
+        end as integers (``key_starts``, where ``takes_key_starts``).
         """
         dev = self.current_device
         if dev.type != "cuda":
@@ -565,6 +565,22 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
                 raise IndexError(f"{bad} embedding indices were out of range")
         return out
 
+    def _sequence_plan(self, feature_positions: Optional[Sequence[int]]) -> int:
+        positions: Optional[Tuple[int, ...]] = None
+        if feature_positions is not None:
+            positions = tuple(feature_positions)
+            if positions == self._identity_positions:
+                positions = None
+        plan = self._plan_address.get(positions)
+        if plan is None:
+            plan = self._plan_address[positions] = self._get_plan(positions).value
+        return plan
+
+    def takes_key_starts(self, feature_positions: Optional[Sequence[int]] = None) -> bool:
+        """Whether ``forward(offsets=None, key_starts=...)`` can be called: the launch arguments hold the starts of a
+        limited number of column slices (a feature whose rows are wider than a wave has several)."""
+        return _lib.lib().tra_tbe_takes_key_starts(self._sequence_plan(feature_positions)) == 1
+
     def _forward_sequence(
         self,
         indices: Tensor,
@@ -576,11 +592,6 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
         """``forward`` of a sequence lookup from key totals or key starts (``indices`` checked by the caller)."""
         assert self.pooling_mode == PoolingMode.NONE, "key_totals / key_starts belong to sequence lookups"
         dev = self.current_device
-        positions: Optional[Tuple[int, ...]] = None
-        if feature_positions is not None:
-            positions = tuple(feature_positions)
-            if positions == self._identity_positions:
-                positions = None
         L = indices.numel()
         out_dtype = torch.float16 if self.output_dtype == _lib.FP16 else torch.float32
         if out is None:
@@ -595,9 +606,7 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
         else:
             starts = array("q", key_starts)
             starts_ptr, num_keys = starts.buffer_info()[0], len(starts) - 1
-        plan = self._plan_address.get(positions)
-        if plan is None:
-            plan = self._plan_address[positions] = self._get_plan(positions).value
+        plan = self._sequence_plan(feature_positions)
         global _FORWARD_SEQUENCE
         if _FORWARD_SEQUENCE is None:
             _FORWARD_SEQUENCE = _lib.entry("tra_tbe_forward_sequence")
