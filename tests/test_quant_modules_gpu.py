@@ -17,6 +17,7 @@ from torchrec_amd.quant.embedding_modules import (
     EmbeddingBagCollection as QuantEBC,
     EmbeddingCollection as QuantEC,
     quant_prep_enable_quant_state_dict_split_scale_bias,
+    quantize_state_dict,
 )
 
 pytestmark = pytest.mark.gpu
@@ -699,3 +700,25 @@ def test_kept_features_order_with_and_without_the_short_route(first):
                        for keys in (first, "ab", "ba", "ab")]
     assert all(torch.equal(x, y) for x, y in zip(got[False], got[True]))
     assert all(torch.equal(x, got[False][0]) for x in got[False])
+
+
+@pytest.mark.parametrize("weight_dtype", [torch.qint8, torch.quint4x2, torch.quint2x4, torch.half, torch.float])
+@pytest.mark.parametrize("empty", [0, 1, 2])
+def test_from_float_with_a_table_of_no_rows(weight_dtype, empty):
+    """A table without rows among others, in every place: converted like the rest (its lookup is refused, as ever)."""
+    rows = [7, 5, 9]
+    rows[empty] = 0
+    tables = [EmbeddingBagConfig(name=f"t{t}", embedding_dim=32, num_embeddings=n, feature_names=[f"f{t}"],
+                                 weight_init_min=-1.0, weight_init_max=1.0) for t, n in enumerate(rows)]
+    ebc = EmbeddingBagCollection(tables=tables, device=DEV)
+    for dtype in (torch.float, torch.half):
+        ebc = ebc.to(dtype)
+        ebc.qconfig = qconfig(weight_dtype, torch.float)
+        qebc = QuantEBC.from_float(ebc)
+        want = {}
+        quantize_state_dict(ebc, want, {t.name: t.data_type for t in qebc.embedding_bag_configs()})
+        (op,) = qebc._emb_modules
+        for name, n, got in zip(op.embedding_names, op.rows, op.split_embedding_weights()):
+            assert n == rows[int(name[1:])]
+            for g, w in zip(got, want[name]):
+                assert (g is None and w is None) or torch.equal(g, w)

@@ -341,7 +341,7 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
                 padded[:, :payload].view(torch.float16 if ty == SparseType.FP16 else torch.float32).copy_(src)
                 continue
             # fp16 sources are widened a piece at a time
-            step = rows if src.dtype == torch.float32 else max(1, (1 << 28) // (4 * dim))
+            step = max(1, rows if src.dtype == torch.float32 else (1 << 28) // (4 * dim))
             for r0 in range(0, rows, step):
                 n = min(step, rows - r0)
                 piece = src[r0 : r0 + n].to(torch.float32).contiguous()
