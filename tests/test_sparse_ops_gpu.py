@@ -372,6 +372,34 @@ def test_kjt_permute(K, B, max_len, pick, idt, vdt):
     assert got.length_per_key() == lengths.sum(1)[order].tolist()
 
 
+@pytest.mark.parametrize("given", ["lengths", "offsets"])
+@pytest.mark.parametrize("order", [[2, 0, 1], [1, 1], [0]])
+def test_kjt_permute_with_counts_does_not_wait(given, order):
+    """A KJT that carries its per-key counts is permuted without the host waiting for what the stream holds, and the
+    counts stay its own."""
+    from torchrec_amd import KeyedJaggedTensor
+
+    rng = np.random.default_rng(3)
+    lengths = rng.integers(0, 9, (3, 50))
+    values = torch.arange(int(lengths.sum()) + 4, device=DEV)
+    bags = torch.from_numpy(lengths.reshape(-1)).to(DEV)
+    bags = bags if given == "lengths" else ops.asynchronous_complete_cumsum(bags)
+    counts = lengths.sum(1).tolist()
+    starts = np.concatenate([[0], np.cumsum(counts)])
+    for busy in (False, True):  # (the first call loads the kernels and fills the allocator)
+        kjt = KeyedJaggedTensor(keys=["a", "b", "c"], values=values, length_per_key=counts, **{given: bags})
+        torch.cuda.synchronize()
+        if busy:
+            torch.cuda._sleep(20_000_000)
+        slept = torch.cuda.Event()
+        slept.record()
+        got = kjt.permute(order)
+        assert not (busy and slept.query())
+        assert kjt._length_per_key is counts and got.length_per_key() == [counts[i] for i in order]
+        assert torch.equal(got.values(), torch.cat([values[starts[i]:starts[i + 1]] for i in order]))
+        assert np.array_equal(got.lengths().cpu().numpy(), lengths[order].reshape(-1))
+
+
 @pytest.mark.parametrize("F,B,W,max_len", [(1, 1, 1, 5), (3, 5, 2, 9), (2, 600, 3, 4), (5, 131, 64, 40), (2, 7, 65, 30), (3, 4, 8, 5000),
                                            (40, 512, 5, 30)])
 @pytest.mark.parametrize("idt", [np.int32, np.int64])

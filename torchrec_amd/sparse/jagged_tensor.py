@@ -568,15 +568,16 @@ class KeyedJaggedTensor:
             length_per_key=permuted_length_per_key if permuted_keys else None,
         )
 
-    def _totals_begin(self):
-        """``ops.key_totals_begin`` of this KJT (device and host), or None."""
+    def _totals_begin(self, on_host: bool):
+        """``ops.key_totals_begin`` of this KJT (on the device, and on the host as asked), or None."""
         if self._lengths is None:
-            return ops.key_totals_begin(self._offsets, True, len(self._keys), self.stride(), True)
-        return ops.key_totals_begin(self._lengths, False, len(self._keys), self.stride(), True)
+            return ops.key_totals_begin(self._offsets, True, len(self._keys), self.stride(), True, on_host)
+        return ops.key_totals_begin(self._lengths, False, len(self._keys), self.stride(), True, on_host)
 
     def _permute_on_gpu(self, indices: List[int], remap=None):
         """``(lengths, values, weights, length_per_key)`` of the keys in the order ``indices``, moved (and
-        remapped) by one kernel behind the one that adds up the ids per key; None where that does not apply."""
+        remapped) by one kernel behind the one that adds up the ids per key; None where that does not apply.  A KJT
+        that carries its per-key counts does not make the host wait."""
         values, weights = self._values, self._weights
         nkeys = len(self._keys)
         if (
@@ -587,10 +588,14 @@ class KeyedJaggedTensor:
         ):
             return None
         stride = self.stride()
-        begun = self._totals_begin()
+        per_key = self._length_per_key
+        begun = self._totals_begin(on_host=per_key is None)
         if begun is None:
             return None
         totals, finish = begun
+        if per_key is not None:
+            permuted = [per_key[i] for i in indices]
+            return *ops.permute_keys(totals, indices, stride, self.lengths(), values, sum(permuted), weights, remap), permuted
         moved = None
         try:
             lengths = self.lengths()
