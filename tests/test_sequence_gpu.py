@@ -1,5 +1,6 @@
 """Sequence lookup from key totals and key starts, and the per-key counts that
 feed it, on the GPU against the CPU oracle."""
+import ctypes
 import threading
 
 import numpy as np
@@ -9,7 +10,7 @@ import torch
 import oracle as O
 from helpers import bits_equal
 from test_tbe_gpu import build
-from torchrec_amd import KeyedJaggedTensor, ops
+from torchrec_amd import _lib, KeyedJaggedTensor, ops
 from torchrec_amd.modules.embedding_configs import DataType, EmbeddingConfig
 from torchrec_amd.quant import EmbeddingCollection as QuantEC
 
@@ -108,6 +109,24 @@ def test_key_totals_threads_and_open_calls():
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not bad
+
+
+def test_key_totals_after_an_earlier_error():
+    """An error that another HIP call left behind is reported with nothing queued: a kernel under way would store its
+    totals into a slot that was given back, and that the next call may hold."""
+    l, hip = _lib.lib(), ctypes.CDLL(_lib.LIB_PATH)  # (the HIP runtime this library is linked to)
+    lengths, totals = torch.arange(12, device=DEV), torch.full((3,), -7, device=DEV)
+    ticket = ctypes.c_int32(5)
+    args = (lengths.data_ptr(), 0, 3, 4, 1, totals.data_ptr(), ctypes.byref(ticket), _lib.current_stream(DEV))
+    torch.cuda.synchronize()
+    assert hip.hipSetDevice(1 << 20) != 0
+    assert l.tra_key_totals_begin(*args) != 0 and b"earlier" in l.tra_last_error() and ticket.value == -1
+    torch.cuda.synchronize()
+    assert totals.tolist() == [-7] * 3
+    assert l.tra_key_totals_begin(*args) == 0
+    host = (ctypes.c_int64 * 3)()
+    assert l.tra_key_totals_wait(ticket, host) == 0
+    assert list(host) == totals.tolist() == [6, 22, 38]
 
 
 def test_key_totals_reject_other_integer_types():

@@ -149,6 +149,11 @@ int tra_key_totals_begin(const void* bags, int32_t bags_are_offsets, int32_t num
   }
   hipStream_t s = (hipStream_t)stream;
   int64_t* host_dev = nullptr;
+  if (ticket) *ticket = -1;
+  // An error left by an earlier call is reported before anything is queued: what hipGetLastError says after the
+  // launch is then the launch's own, and the slot is given back only where no kernel will store into it.
+  const hipError_t earlier = hipGetLastError();
+  if (earlier != hipSuccess) return hip_fail(earlier, "tra_key_totals_begin: an earlier call");
   if (ticket) {
     const int rc = mail_open(s, num_keys, ticket, &host_dev);
     if (rc != TRA_OK) return rc;
