@@ -1134,6 +1134,33 @@ def test_bad_ids_are_counted_once_at_every_row_width(dt, dim, idt, tuning):
                 assert tbe.out_of_range_count() == len(bad), (mode, how, len(bad))
 
 
+# Launch classes whose slices are mostly of odd lane groups, half of them, fewer; lanes of 16, 32 and 64 accumulators.
+@pytest.mark.parametrize("dt,dims", [(O.INT4, (64, 80, 144, 128)), (O.INT4, (64, 80, 128, 48)), (O.INT4, (80, 128, 16, 256 - 16)),
+                                     (O.INT8, (112, 144, 192, 128)), (O.INT8, (112, 128, 256, 128)), (O.INT8, (304, 464, 128)),
+                                     (O.INT2, (80, 112, 144, 128)), (O.INT2, (128, 160, 224)), (O.INT2, (320, 384, 512)),
+                                     (O.INT4, (320, 288, 256))])
+@pytest.mark.parametrize("idt", [np.int32, np.int64])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_window_kernel_over_the_widths_of_a_class(dt, dims, idt, weighted, tuning):
+    tuning(balanced=1)
+    rng = np.random.default_rng(sum(dims))
+    F, B = len(dims), 120
+    specs = [(dt, 70 + 3 * f, d) for f, d in enumerate(dims)]
+    lengths = rng.integers(0, 35, F * B)
+    lengths[::5] = 8
+    offsets = np.zeros(F * B + 1, dtype=idt)
+    offsets[1:] = np.cumsum(lengths)
+    ids = rng.integers(-1, 70, offsets[-1]).astype(idt)
+    psw = rng.random(len(ids)).astype(np.float32) if weighted else None
+    tbe, store = build(rng, specs, list(range(F)), O.SUM, O.FP32, 16)
+    want = O.tbe_forward(store, list(range(F)), B, ids, offsets, psw, O.SUM, O.FP32)
+    tx, tw = torch.from_numpy(ids).to(DEV), None if psw is None else torch.from_numpy(psw).to(DEV)
+    got = tbe(tx, torch.from_numpy(offsets).to(DEV), per_sample_weights=tw)
+    assert bits_equal(got.cpu().numpy(), want) == 0
+    got = tbe(tx, None, per_sample_weights=tw, lengths=torch.from_numpy(lengths.astype(idt)).to(DEV), batch_size=B)
+    assert bits_equal(got.cpu().numpy(), want) == 0
+
+
 def test_multi_class_call_on_two_streams(tuning):
     """A plan of five or more launch classes runs every other launch on its own second stream,
     forked from and joined to the caller's stream inside the call.  Checked: the same bits as with

@@ -1172,10 +1172,13 @@ __global__ __launch_bounds__(kBlockThreads) void tbe_pooled_kernel(const LookupA
   TRA_STAMP(3);
 }
 
+constexpr int kNarrowLane = 8;  // accumulators per lane up to which one instance serves all widths (see odd_lanes)
+
 // FROM_LENGTHS: a.offsets points at the KJT's lengths instead of its offsets
 // and the block derives its bags' start positions itself: one block-wide sum
 // of everything in front of the window plus a scan of the window in LDS.
-template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, bool FROM_LENGTHS = false>
+// ODD: the instance for launch classes of mostly odd lane groups (kOddInstance).
+template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, bool FROM_LENGTHS = false, bool ODD = false>
 __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
     const void* p_offsets, const FeatureDesc* p_cdescs, int32_t p_B, int32_t p_xcd_blocks,
     int32_t p_xcd_count, int32_t p_n_sub, int32_t p_window0, int32_t p_count0, int32_t p_key0,
@@ -1518,13 +1521,19 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
 #pragma unroll
     for (int k = 0; k < NE; ++k) acc[k] = 0.0f;
     int bad;
-    // Ids in blocks wherever a lane group has four lanes or more.
-    if constexpr (U == 4) {
+    // Which bodies an instance holds: see odd_lanes.
+    constexpr bool kAllWidths = NE <= kNarrowLane || (CB == 4 && NE <= 2 * kNarrowLane);
+    if constexpr (U == 4 && ODD) {
+      if (lpr >= 4)
+        bad = pool_bag_bulk<DTYPE, CB, IdxT, WEIGHTED, U, NE, 4>(acc, a, w, start, len, max_len, lpr, c, lane - c);
+      else
+        bad = pool_bag<DTYPE, CB, IdxT, WEIGHTED, U, NE>(acc, a, w, start, len, max_len);
+    } else if constexpr (U == 4) {
       if (lpr >= 16 && (lpr & (lpr - 1)) == 0)
         bad = pool_bag_bulk<DTYPE, CB, IdxT, WEIGHTED, U, NE, 0>(acc, a, w, start, len, max_len, lpr, c, lane - c);
-      else if (lpr >= 8)
+      else if (kAllWidths ? lpr >= 8 : lpr == 8)
         bad = pool_bag_bulk<DTYPE, CB, IdxT, WEIGHTED, U, NE, 8>(acc, a, w, start, len, max_len, lpr, c, lane - c);
-      else if (lpr >= 4)
+      else if (kAllWidths && lpr >= 4)
         bad = pool_bag_bulk<DTYPE, CB, IdxT, WEIGHTED, U, NE, 4>(acc, a, w, start, len, max_len, lpr, c, lane - c);
       else
         bad = pool_bag<DTYPE, CB, IdxT, WEIGHTED, U, NE>(acc, a, w, start, len, max_len);
@@ -1543,9 +1552,29 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
 }
 
 // ---- host side of one launch ----------------------------------------------
+// Lane groups that fetch their ids in blocks only in some instances of the
+// window kernel: 4 to 7 lanes, and more where they are no power of two.  Every
+// body that an instance holds costs all of its widths registers, and where a
+// lane holds many accumulators they are spilled.  So:
+//   up to 8 accumulators a lane, and 16 in 4-byte chunks (whose lane groups are
+//   odd by themselves): one instance with the bodies for all widths;
+//   16: two instances, and a launch class takes the one for most of its slices;
+//   32 and 64: no blocks for these widths.
+// Measured on 12 tables, bags of 1 - 40 ids, us with the rows in the L2 / in HBM:
+//   int8 dim 72 (9 lanes of 8 accumulators): ids one by one 13.1 / 16.8, in
+//   blocks 10.4 / 16.6; weighted 17.2 / 19.7 and 10.2 / 16.5;
+//   int8 dim 112 (7 lanes of 16): one by one 15.9 / 18.1, in blocks 13.9 / 17.3;
+//   int8 dim 128, int64 ids (8 lanes of 16): 15.4 / 29.3 in an instance that
+//   holds what the powers of two need, 16.4 / 33.0 in one with all bodies;
+//   int2 dim 320 (5 lanes of 64): one by one 36 / 47, in blocks 84 / 104.
+inline bool odd_lanes(int lpr) { return lpr >= 4 && lpr != 8 && !(lpr >= 16 && (lpr & (lpr - 1)) == 0); }
+template <int DTYPE, int CB>
+constexpr bool kOddInstance = DTYPE < kSplitHeader && CB > 4 && CB * 8 / Traits<DTYPE>::kBits == 2 * kNarrowLane;
+
 struct LaunchClass {
   int dtype;
   int cb;
+  bool odd = false;    // more slices of odd_lanes than others
   bool split = false;  // rows cut into several column slices, header loaded on its own (kSplitHeader)
   std::vector<int32_t> feats;  // plan order: sorted by lpr
   std::vector<int32_t> lprs;   // lanes per row of each feature
@@ -1563,6 +1592,7 @@ struct LaunchParams {
   bool idx64;
   bool weighted;
   bool from_lengths;  // window kernel reads lengths and derives offsets itself
+  bool odd;           // window kernel: the instance for odd lane groups, where there is one
 };
 
 template <int DTYPE>
@@ -1580,7 +1610,14 @@ void launch_typed(const LookupArgs& a, const LaunchParams& p, hipStream_t stream
       a.sub[0].key0
 #define TRA_POOLED(W, U)                                                                       \
   do {                                                                                         \
-    if (p.balanced && p.from_lengths)                                                          \
+    constexpr bool O = kOddInstance<DTYPE, CB>;                                                \
+    if (O && p.balanced && p.odd && p.from_lengths)                                            \
+      hipLaunchKernelGGL((tbe_pooled_cu_kernel<DTYPE, CB, IdxT, W, 4, true, O>), g,            \
+                         dim3(kCuThreads), p.lds_bytes, stream, TRA_CU_LEADING_ARGS, a);       \
+    else if (O && U == 4 && p.balanced && p.odd)                                               \
+      hipLaunchKernelGGL((tbe_pooled_cu_kernel<DTYPE, CB, IdxT, W, U, false, O && U == 4>), g, \
+                         dim3(kCuThreads), p.lds_bytes, stream, TRA_CU_LEADING_ARGS, a);       \
+    else if (p.balanced && p.from_lengths)                                                     \
       hipLaunchKernelGGL((tbe_pooled_cu_kernel<DTYPE, CB, IdxT, W, 4, true>), g,               \
                          dim3(kCuThreads), p.lds_bytes, stream, TRA_CU_LEADING_ARGS, a);       \
     else if (p.balanced)                                                                       \

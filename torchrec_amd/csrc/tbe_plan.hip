@@ -438,6 +438,7 @@ int tra_tbe_create(const tra_table_spec* tables, int32_t num_tables,
       cls.cols_aligned_fp32 = cls.cols_aligned_fp32 && (int64_t)plan->slices[id].out_col * 4 % 16 == 0;
     }
     plan->max_class_feats = std::max(plan->max_class_feats, cls.feats.size());
+    cls.odd = 2 * std::count_if(cls.lprs.begin(), cls.lprs.end(), odd_lanes) > (int64_t)cls.lprs.size();
     LookupArgs a;
     memset(&a, 0, sizeof(a));
     a.descs = plan->slices_dev;
@@ -899,6 +900,7 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
     lp.idx64 = idx_is_i64 != 0;
     lp.weighted = a.psw != nullptr || a.posw != nullptr;
     lp.from_lengths = from_lengths;
+    lp.odd = cls.odd;
     int rc;
     if (nobag) {
       rc = launch_sequence(a, cls.dtype, cls.cb, cls.split, lp.idx64, lp.grid, s);
