@@ -124,3 +124,16 @@ def test_kt_regroup_as_dict_module(dev):
         KTRegroupAsDict([["f1"]], ["a"])(dup)
     m.clear_cache()
     assert not m._is_inited
+
+
+@pytest.mark.parametrize("dev", DEVICES)
+def test_regroup_module_saved_without_its_layout(dev):
+    """A module that was saved after its first batch, before it kept the layout of its plan."""
+    from torchrec_amd.modules.regroup import KTRegroupAsDict
+    tensors = [torch.randn(3, 4, device=dev) for _ in range(3)]
+    kt = KeyedTensor.from_tensor_list(["a", "b", "c"], tensors, 1)
+    m = KTRegroupAsDict([["c", "a"], ["b"]], ["x", "y"])
+    m([kt])
+    del m.__dict__["_layout"]
+    got = m([kt])
+    assert torch.equal(got["x"], torch.cat([tensors[2], tensors[0]], 1)) and torch.equal(got["y"], tensors[1])

@@ -152,3 +152,15 @@ def test_collection_of_more_slices_than_key_starts(K, dim):
         got = qec(kjt)
         assert torch.equal(torch.cat([got[k].values() for k in kjt.keys()]), rows[ids])
         assert kjt.length_per_key_or_none() is not None
+
+
+def test_collection_saved_without_its_flat_names():
+    """A collection that was saved before it kept its embedding names in one list."""
+    tables = [EmbeddingConfig(name=f"t{k}", embedding_dim=8, num_embeddings=9, feature_names=[f"f{k}"],
+                              data_type=DataType.INT8 if k else DataType.FP16) for k in range(2)]
+    qec = QuantEC(tables, DEV, output_dtype=torch.half)
+    kjt = KeyedJaggedTensor(keys=["f1", "f0"], values=torch.tensor([1, 2, 3], device=DEV), lengths=torch.tensor([1, 2], device=DEV))
+    want = qec(kjt)
+    qec.__dict__.pop("_flat_embedding_names")
+    got = qec(kjt)
+    assert list(got) == list(want) and all(torch.equal(got[k].values(), want[k].values()) for k in want)

@@ -19,6 +19,8 @@ class KTRegroupAsDict(torch.nn.Module):
     signature parity (nothing here lives on a fixed device).  A key held by two
     of the KeyedTensors is an error, as in the reference."""
 
+    _layout = None  # (saved modules may lack it: made from the plan on each call then)
+
     def __init__(self, groups: List[List[str]], keys: List[str], emb_dtype: Optional[DataType] = None,
                  multi_device: bool = False) -> None:
         super().__init__()

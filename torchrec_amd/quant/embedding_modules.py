@@ -750,6 +750,8 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
     Tables are grouped by ``(data_type, use_virtual_table)``; all share one dim.
     """
 
+    _flat_embedding_names: Optional[List[str]] = None
+
     def __init__(  # noqa C901
         self,
         tables: List[EmbeddingConfig],
@@ -825,9 +827,6 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
             key: list(itertools.chain(*get_embedding_names_by_table(group)))
             for key, group in self._key_to_tables.items()
         }
-        self._flat_embedding_names: List[str] = [
-            name for key in self._key_to_tables for name in self._embedding_names_by_batched_tables[key]
-        ]
         self._embedding_names_by_table: List[List[str]] = get_embedding_names_by_table(
             self._embedding_configs
         )
@@ -911,12 +910,20 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
         lengths_rows = torch.unbind(lengths, dim=0) if kjt_keys else ()
         need_indices = self._need_indices
         feature_embeddings: Dict[str, JaggedTensor] = {}
-        for embedding_name, pos in zip(self._flat_embedding_names, order):
+        for embedding_name, pos in zip(self._flat_names(), order):
             start, end = offset_per_key[pos], offset_per_key[pos + 1]
             feature_embeddings[embedding_name] = JaggedTensor._of(
                 lookup[start:end], lengths_rows[pos], indices[start:end] if need_indices else None
             )
         return feature_embeddings
+
+    def _flat_names(self) -> List[str]:
+        """Embedding names in the operators' feature order (made on first use: saved modules may lack them)."""
+        names = self._flat_embedding_names
+        if names is None:
+            by_key = self._embedding_names_by_batched_tables
+            names = self._flat_embedding_names = [name for key in self._key_to_tables for name in by_key[key]]
+        return names
 
     def _starts_fit(self, offset_per_key: List[int], num_indices: int, order: List[int]) -> bool:
         """Whether the operators can take these key starts as launch arguments."""
