@@ -722,3 +722,37 @@ def test_from_float_with_a_table_of_no_rows(weight_dtype, empty):
             assert n == rows[int(name[1:])]
             for g, w in zip(got, want[name]):
                 assert (g is None and w is None) or torch.equal(g, w)
+
+
+@pytest.mark.parametrize("registered,observer", [(True, "pre_hook"), (True, "replaced"), (False, "replaced"), (True, "class"),
+                                                 (True, "none")])
+@pytest.mark.parametrize("counts", [False, True])
+def test_sequence_lookups_that_can_be_seen_get_offsets(registered, observer, counts):
+    """Whatever looks at, or stands in for, the operators of a sequence collection is called with the ids and the
+    bags' offsets, whether the KJT carries its per-key counts or not."""
+    table = EmbeddingConfig(name="t", embedding_dim=16, num_embeddings=30, feature_names=["f", "g"], data_type=DataType.INT8)
+    qec = QuantEC([table], DEV, output_dtype=torch.half, register_tbes=registered)
+    (op,) = qec._emb_modules
+    seen = []
+    own = type(op).forward
+
+    def stand_in(indices, offsets, feature_positions=None, batch_size=None, out=None):
+        seen.append(offsets)
+        return own(op, indices, offsets, feature_positions=feature_positions, batch_size=batch_size, out=out)
+
+    kjt = random_kjt(np.random.default_rng(5), ["g", "f"], [30, 30], B=9, max_len=4)
+    if counts:
+        kjt.length_per_key()
+    want = qec(kjt)
+    if observer == "pre_hook":
+        op.register_forward_pre_hook(lambda m, args, kw: seen.append(kw["offsets"]), with_kwargs=True)
+    elif observer == "replaced":
+        op.forward = stand_in
+    elif observer == "class":
+        op.__class__ = type("Other", (type(op),), {"forward": lambda self, **kw: stand_in(**kw)})
+    kjt = random_kjt(np.random.default_rng(5), ["g", "f"], [30, 30], B=9, max_len=4)
+    if counts:
+        kjt.length_per_key()
+    got = qec(kjt)
+    assert all(torch.equal(got[k].values(), want[k].values()) for k in "fg")
+    assert len(seen) == (observer != "none") and all(torch.equal(x, kjt.offsets()) for x in seen)

@@ -861,13 +861,13 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
         on_gpu = indices.is_cuda and K > 0 and L > 0 and B > 0
         if features.length_per_key_or_none() is not None or features.offset_per_key_or_none() is not None or not on_gpu:
             offset_per_key = features.offset_per_key()
-            if on_gpu and self._starts_fit(offset_per_key, L, order):
+            if on_gpu and self._lookups_are_own() and self._starts_fit(offset_per_key, L, order):
                 bounds = {"offsets": None, "key_starts": offset_per_key}
         else:
             built_from_offsets = features.lengths_or_none() is None
             begun = ops.key_totals_begin(
                 features.offsets() if built_from_offsets else features.lengths(), built_from_offsets, K, B,
-                on_device=K <= ops._MAX_TOTAL_KEYS,
+                on_device=K <= ops._MAX_TOTAL_KEYS and self._lookups_are_own(),
             )
             if begun is None:
                 counts_later = ops.length_per_key_async(features.lengths(), K, B)
@@ -924,6 +924,15 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
             by_key = self._embedding_names_by_batched_tables
             names = self._flat_embedding_names = [name for key in self._key_to_tables for name in by_key[key]]
         return names
+
+    def _lookups_are_own(self) -> bool:
+        """Whether nothing but the operators' own forward sees the lookups: hooks and replaced operators are given
+        the bags' offsets."""
+        own = IntNBitTableBatchedEmbeddingBagsCodegen.forward
+        return all(
+            type(op).forward is own and (_call_is_unobserved(op) if self.register_tbes else "forward" not in op.__dict__)
+            for op in self._emb_modules
+        )
 
     def _starts_fit(self, offset_per_key: List[int], num_indices: int, order: List[int]) -> bool:
         """Whether the operators can take these key starts as launch arguments."""
