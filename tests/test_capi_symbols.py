@@ -103,3 +103,18 @@ def test_bucketize_ids_refuses_id_counts_its_kernels_cannot_step_over():
     for n in (2**31 - 1, 2**31 - 4096):
         rc = l.tra_bucketize_ids(at, at, 1, None, at, 1, 1, 2, n, 0, at, at, at, None, None, None, at, None)
         assert rc == _lib.ERR_TOO_LARGE and b"ids" in l.tra_last_error()
+
+
+def test_int64_vectors_describe_and_refuse(monkeypatch):
+    """The same description, and the same refusals, with and without the extension module."""
+    import pytest
+    import torch
+
+    a, b = torch.arange(5), torch.arange(0)
+    for vectors in (_lib._vectors, _lib._int64_vectors_python):
+        monkeypatch.setattr(_lib, "_vectors", vectors)
+        assert _lib.int64_vectors([a, b, a]).tolist() == [a.data_ptr(), b.data_ptr(), a.data_ptr(), 5, 0, 5]
+        assert _lib.int64_vectors([]).tolist() == []
+        for bad in (a.int(), torch.arange(8)[::2], torch.rand(3).double()):
+            with pytest.raises(AssertionError):
+                _lib.int64_vectors([a, bad])

@@ -10,7 +10,8 @@ from __future__ import annotations
 import ctypes
 import functools
 import os
-from typing import Optional
+from array import array
+from typing import List, Optional
 
 import torch
 
@@ -141,8 +142,7 @@ def lib() -> ctypes.CDLL:
         l.tra_position_weights.argtypes = [vp, i32, i32, i32, vp, vp, vp, vp, vp]
         l.tra_mch_remap.argtypes = [vp, i64, i32, vp, vp, i64, i64, vp, vp]
         l.tra_mch_remap_keys.argtypes = [
-            vp, i64, vp, i32, i32, i32, ctypes.POINTER(vp), ctypes.POINTER(vp), ctypes.POINTER(i64),
-            ctypes.POINTER(i64), vp, vp,
+            vp, i64, vp, i32, i32, i32, vp, vp, vp, vp, vp, vp,
         ]
         l.tra_permute_keys.argtypes = [
             vp, i32, vp, i32, i32, vp, i32, vp, vp, i64, i32, vp, i64, vp, vp, vp, vp, vp, vp, vp,
@@ -183,6 +183,22 @@ def entry(name: str):
     except ImportError:
         return fn
     return functools.partial(_fastcall.call, ctypes.cast(fn, ctypes.c_void_p).value)
+
+
+def _int64_vectors_python(tensors: List[torch.Tensor], dtype: torch.dtype) -> bytes:
+    assert all(t.dtype is dtype and t.is_contiguous() for t in tensors)
+    return array("q", [t.data_ptr() for t in tensors] + [t.numel() for t in tensors]).tobytes()
+
+
+try:  # (the in-tree extension module when it is there)
+    from torchrec_amd._fastcall import vectors as _vectors
+except ImportError:
+    _vectors = _int64_vectors_python
+
+
+def int64_vectors(tensors: List[torch.Tensor]) -> array:
+    """Addresses, then element counts, of contiguous int64 tensors (AssertionError for any other), as int64."""
+    return array("q", _vectors(tensors, torch.int64))
 
 
 def check(rc: int) -> None:

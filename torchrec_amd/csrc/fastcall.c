@@ -10,10 +10,13 @@
  * whose arguments are all integers or pointers goes through call().  That one relies on the
  * x86-64 System V calling convention: every such argument, of whatever width, takes one
  * register or one 8-byte stack slot, and the caller removes them.
+ *
+ * vectors() checks and describes many tensors for such a call.
  */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <stdint.h>
+#include <string.h>
 
 typedef int (*forward_lengths_fn)(void* tbe, const void* weights, const void* indices, const void* lengths,
                                   int32_t idx_is_i64, const float* per_sample_weights, int32_t batch_size,
@@ -94,12 +97,69 @@ static PyObject* call(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
   return PyLong_FromLong(rc);
 }
 
+/* One tensor's address and element count; -1 with an exception set where it is not contiguous or of another type. */
+static int vector(PyObject* t, PyObject* dtype, int64_t* address, int64_t* numel) {
+  static PyObject *s_dtype, *s_contiguous, *s_numel, *s_data_ptr; /* interned on first use, under the interpreter lock */
+  PyObject *d, *c, *n, *p;
+  if (s_data_ptr == NULL) {
+    s_dtype = PyUnicode_InternFromString("dtype");
+    s_contiguous = PyUnicode_InternFromString("is_contiguous");
+    s_numel = PyUnicode_InternFromString("numel");
+    s_data_ptr = PyUnicode_InternFromString("data_ptr");
+    if (s_dtype == NULL || s_contiguous == NULL || s_numel == NULL || s_data_ptr == NULL) return -1;
+  }
+  if ((d = PyObject_GetAttr(t, s_dtype)) == NULL) return -1;
+  Py_DECREF(d);
+  if (d != dtype) {
+    PyErr_SetString(PyExc_AssertionError, "a table of another element type");
+    return -1;
+  }
+  if ((c = PyObject_CallMethodNoArgs(t, s_contiguous)) == NULL) return -1;
+  Py_DECREF(c);
+  if (c != Py_True) {
+    PyErr_SetString(PyExc_AssertionError, "a table that is not contiguous");
+    return -1;
+  }
+  if ((n = PyObject_CallMethodNoArgs(t, s_numel)) == NULL) return -1;
+  *numel = PyLong_AsLongLong(n);
+  Py_DECREF(n);
+  if ((p = PyObject_CallMethodNoArgs(t, s_data_ptr)) == NULL) return -1;
+  *address = (int64_t)PyLong_AsUnsignedLongLongMask(p);
+  Py_DECREF(p);
+  return PyErr_Occurred() ? -1 : 0;
+}
+
+/* vectors(list of n tensors, dtype) -> bytes: n addresses, then n element counts (int64). */
+static PyObject* vectors(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  (void)self;
+  if (nargs != 2 || !PyList_Check(args[0])) {
+    PyErr_SetString(PyExc_TypeError, "vectors takes a list of tensors and a dtype");
+    return NULL;
+  }
+  const Py_ssize_t n = PyList_GET_SIZE(args[0]);
+  PyObject* out = PyBytes_FromStringAndSize(NULL, 16 * n);
+  if (out == NULL) return NULL;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    int64_t address = 0, numel = 0;
+    if (i >= PyList_GET_SIZE(args[0]) || vector(PyList_GET_ITEM(args[0], i), args[1], &address, &numel) != 0) {
+      if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "vectors: the list changed");
+      Py_DECREF(out);
+      return NULL;
+    }
+    memcpy(PyBytes_AS_STRING(out) + 8 * i, &address, 8);
+    memcpy(PyBytes_AS_STRING(out) + 8 * (n + i), &numel, 8);
+  }
+  return out;
+}
+
 static PyMethodDef methods[] = {
     {"bind", bind, METH_O, "bind(address of tra_tbe_forward_lengths)"},
     {"forward_lengths", (PyCFunction)(void (*)(void))forward_lengths, METH_FASTCALL,
      "tra_tbe_forward_lengths(...) with integer arguments; returns its return code"},
     {"call", (PyCFunction)(void (*)(void))call, METH_FASTCALL,
      "call(address of an entry point, integer arguments ...); returns its return code"},
+    {"vectors", (PyCFunction)(void (*)(void))vectors, METH_FASTCALL,
+     "vectors(list of tensors, dtype): their addresses, then their element counts, as int64"},
     {NULL, NULL, 0, NULL}};
 
 static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fastcall", NULL, -1, methods, NULL, NULL, NULL, NULL};

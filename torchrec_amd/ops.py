@@ -13,7 +13,6 @@ quantization and bucketization have no host form.
 """
 from __future__ import annotations
 
-import ctypes
 from array import array
 from typing import List, Optional, Tuple
 
@@ -469,14 +468,20 @@ def mch_remap(
     return out
 
 
-def _check_remap(values: torch.Tensor, sorted_ids: List[torch.Tensor], mappings: List[torch.Tensor], miss_ids: List[int]):
-    """Ids and tables as the remap kernels read them (one table, row mapping and miss row per key)."""
+def _remap_tables(
+    values: torch.Tensor, sorted_ids: List[torch.Tensor], mappings: List[torch.Tensor], miss_ids: List[int]
+) -> Tuple[array, array, List[int]]:
+    """``tra_permute_keys``' description of the tables (one table, row mapping and miss row per key), once they and the
+    ids are what the remap kernels read (that they lie on the ids' device is the caller's to know): addresses of the
+    tables, of the mappings and the tables' sizes in one array, the miss rows, and where each of the four begins."""
     _check_int(values, "values")
-    assert len(mappings) == len(miss_ids) == len(sorted_ids)
-    di = values.get_device()
-    for s_, m_ in zip(sorted_ids, mappings):
-        assert s_.dtype is torch.int64 and m_.dtype is torch.int64 and s_.numel() == m_.numel() > 0
-        assert s_.is_contiguous() and m_.is_contiguous() and s_.get_device() == di and m_.get_device() == di
+    K = len(sorted_ids)
+    assert len(mappings) == K and len(miss_ids) == K
+    tables, miss = _lib.int64_vectors([*sorted_ids, *mappings]), array("q", miss_ids)
+    sizes = tables[2 * K : 3 * K]
+    assert sizes == tables[3 * K :] and 0 not in sizes, "a table and its row mapping differ in size, or are empty"
+    first = tables.buffer_info()[0]
+    return tables, miss, [first, first + 8 * K, first + 16 * K, miss.buffer_info()[0]]
 
 
 def permute_keys(
@@ -496,24 +501,18 @@ def permute_keys(
     dev = values.device
     K, Kp = totals.numel(), len(order)
     values = values.contiguous()
-    out_values = torch.empty(num_out, dtype=values.dtype, device=dev)
+    out_values = values.new_empty(num_out)
     out_lengths = out_weights = None
     if move_lengths:
         lengths = lengths.contiguous()
-        out_lengths = torch.empty(Kp * stride, dtype=lengths.dtype, device=dev)
+        out_lengths = lengths.new_empty(Kp * stride)
     if weights is not None:
         weights = weights.contiguous()
-        out_weights = torch.empty(num_out, dtype=torch.float32, device=dev)
-    tables, at = (), (None, None, None, None)
+        out_weights = weights.new_empty(num_out)
+    at = (None, None, None, None)
     if remap is not None:
-        sorted_ids, mappings, miss = remap
-        assert len(sorted_ids) == Kp
-        _check_remap(values, sorted_ids, mappings, miss)
-        tables = (
-            array("q", [t.data_ptr() for t in sorted_ids]), array("q", [t.data_ptr() for t in mappings]),
-            array("q", [t.numel() for t in sorted_ids]), array("q", miss),
-        )
-        at = [a.buffer_info()[0] for a in tables]
+        assert len(remap[0]) == Kp
+        tables, miss, at = _remap_tables(values, *remap)
     perm = array("i", order)
     rc = _entry("tra_permute_keys")(
         totals.data_ptr(), K, perm.buffer_info()[0], Kp, stride, lengths.data_ptr() if move_lengths else None,
@@ -538,19 +537,17 @@ def mch_remap_keys(
     ``values[offsets[k*B] : offsets[(k+1)*B]]``) is looked up in ``sorted_ids[k]`` / ``mappings[k]``."""
     _lib.require_gpu(values, "mch_remap_keys")
     K = len(sorted_ids)
-    _check_remap(values, sorted_ids, mappings, miss_ids)
+    tables, miss, at = _remap_tables(values, sorted_ids, mappings, miss_ids)
+    assert all(t.device == values.device for t in [*sorted_ids, *mappings])
     assert offsets.numel() == K * batch_size + 1, "offsets must have num_keys * B + 1 entries"
     values = values.contiguous()
     if offsets.dtype != values.dtype:
         offsets = offsets.to(values.dtype)
     offsets = offsets.contiguous()
     out = torch.empty_like(values)
-    vp, i64 = ctypes.c_void_p, ctypes.c_int64
     _lib.check(
-        _lib.lib().tra_mch_remap_keys(
-            _lib.ptr(values), values.numel(), _lib.ptr(offsets), int(values.dtype == torch.int64), K, int(batch_size),
-            (vp * max(K, 1))(*[t.data_ptr() for t in sorted_ids]), (vp * max(K, 1))(*[t.data_ptr() for t in mappings]),
-            (i64 * max(K, 1))(*[t.numel() for t in sorted_ids]), (i64 * max(K, 1))(*[int(m) for m in miss_ids]),
+        _entry("tra_mch_remap_keys")(
+            _lib.ptr(values), values.numel(), _lib.ptr(offsets), values.dtype is torch.int64, K, int(batch_size), *at,
             _lib.ptr(out), _lib.current_stream(values.device),
         )
     )

@@ -929,19 +929,21 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
         """Whether nothing but the operators' own forward sees the lookups: hooks and replaced operators are given
         the bags' offsets."""
         own = IntNBitTableBatchedEmbeddingBagsCodegen.forward
-        return all(
-            type(op).forward is own and (_call_is_unobserved(op) if self.register_tbes else "forward" not in op.__dict__)
-            for op in self._emb_modules
-        )
+        for op in self._emb_modules:
+            if type(op).forward is not own or "forward" in op.__dict__:
+                return False
+            if self.register_tbes and not _call_is_unobserved(op):
+                return False
+        return True
 
     def _starts_fit(self, offset_per_key: List[int], num_indices: int, order: List[int]) -> bool:
         """Whether the operators can take these key starts as launch arguments."""
-        return (
-            num_indices < 2**31
-            and all(a <= b for a, b in zip(offset_per_key, offset_per_key[1:]))
-            and offset_per_key[-1] <= num_indices
-            and all(op.takes_key_starts(p) for op, p in zip(self._emb_modules, self._group_positions(order)))
-        )
+        if num_indices >= 2**31 or offset_per_key[-1] > num_indices or sorted(offset_per_key) != offset_per_key:
+            return False
+        for op, positions in zip(self._emb_modules, self._group_positions(order)):
+            if not op.takes_key_starts(positions):
+                return False
+        return True
 
     @classmethod
     def from_float(

@@ -44,6 +44,7 @@ _INT_DTYPES = (torch.int32, torch.int64)
 _BOUNDS_FATAL = int(BoundsCheckMode.FATAL)
 _FORWARD_LENGTHS = None  # the library's tra_tbe_forward_lengths, bound on first use
 _FORWARD_SEQUENCE = None  # likewise tra_tbe_forward_sequence
+_KEY_START_SLICES = 128  # column slices whose key starts surely fit the launch arguments
 
 _SUPPORTED_WEIGHTS = (SparseType.FP32, SparseType.FP16, SparseType.INT8, SparseType.INT4, SparseType.INT2)
 _TABLE_ALIGNMENT = 256
@@ -579,6 +580,9 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
     def takes_key_starts(self, feature_positions: Optional[Sequence[int]] = None) -> bool:
         """Whether ``forward(offsets=None, key_starts=...)`` can be called: the launch arguments hold the starts of a
         limited number of column slices (a feature whose rows are wider than a wave has several)."""
+        # (a slice is at least 64 lanes of 4 bytes: short rows need not ask the plan)
+        if len(self.feature_table_map) * (max(self.row_bytes, default=0) + 255 >> 8) <= _KEY_START_SLICES:
+            return True
         return _lib.lib().tra_tbe_takes_key_starts(self._sequence_plan(feature_positions)) == 1
 
     def _forward_sequence(
