@@ -137,3 +137,29 @@ def test_regroup_module_saved_without_its_layout(dev):
     del m.__dict__["_layout"]
     got = m([kt])
     assert torch.equal(got["x"], torch.cat([tensors[2], tensors[0]], 1)) and torch.equal(got["y"], tensors[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("elem,widths", [(2, [3, 8, 1]), (4, [5, 4, 64]), (4, [0, 7]), (2, [256] * 100)])
+def test_regroup_columns_entry(elem, widths):
+    """``tra_regroup_columns`` (blocks given by address): blocks in reverse order, in a wider row; bad blocks refused."""
+    import ctypes
+
+    from torchrec_amd import _lib
+    dev, rows, total = torch.device("cuda:0"), 37, sum(widths)
+    dtype = {2: torch.int16, 4: torch.int32}[elem]
+    src = torch.randint(-30000, 30000, (rows, total + 3), device=dev).to(dtype)
+    dst = torch.zeros(rows, total + 5, dtype=dtype, device=dev)
+    n, at = len(widths), np.concatenate([[0], np.cumsum(widths)])
+    to = total - at[1:]  # (the blocks from the right)
+    vp, i64, i32 = ctypes.c_void_p * n, ctypes.c_int64 * n, ctypes.c_int32 * n
+    args = [vp(*[src.data_ptr() + int(a) * elem for a in at[:-1]]), i64(*[total + 3] * n),
+            vp(*[dst.data_ptr() + int(a) * elem for a in to]), i64(*[total + 5] * n), i32(*widths), n, rows, elem,
+            _lib.current_stream(dev)]
+    assert _lib.lib().tra_regroup_columns(*args) == 0
+    want = torch.zeros_like(dst)
+    for a, b, w in zip(at, to, widths):
+        want[:, int(b):int(b) + w] = src[:, int(a):int(a) + w]
+    assert torch.equal(dst, want)
+    args[1] = i64(*[max(widths) - 1] * n)
+    assert _lib.lib().tra_regroup_columns(*args) == -1

@@ -397,8 +397,10 @@ __global__ __launch_bounds__(kBktThreads) void bucket_move_kernel(const BucketAr
 }
 
 // Bags per tile: an average of 4096 ids (two steps of bucket_move) where that
-// leaves six tiles per compute unit (7.9 M ids in 64 x 4096 bags, the whole
-// call: 4096 ids a tile 64 us, 2048 74 us, 1024 99 us, 8192 71 us), down to 256
+// leaves 1536 tiles, six for each of an MI355X's 256 compute units (7.9 M ids in
+// 64 x 4096 bags, the four kernels together, best passes: 4096 ids a tile 64 us,
+// 2048 74 us, 1024 99 us, 8192 71 us; a fixed figure, so that the workspace
+// does not depend on the device that asks for its size), down to 256
 // ids; more where that makes over 8192 tiles (every block of bucket_counts adds
 // up the totals of the tiles in front of its own); no more than the counters hold.
 static int bags_per_tile(int64_t n, int64_t num_indices, int32_t B, int32_t W) {

@@ -638,8 +638,9 @@ __global__ __launch_bounds__(256) void quantize_rows_vec_kernel(const float* __r
 // that the store needs no clearing first and nothing is copied into it
 // afterwards.  A wave builds its rows in LDS and writes them out as one
 // contiguous run of 16-byte vectors: with a 4-byte store per lane a 68-byte
-// row leaves in pieces (int4 rows of dim 128 at a 128-byte stride, 1 M rows:
-// 122 us written directly, 111 us built in LDS; 8-bit rows are even, 2-bit
+// row leaves in pieces (int4 rows of dim 128 at a 128-byte stride, 1 M rows,
+// steady state of one table quantized again and again: 122 us written directly,
+// 111 us built in LDS; four tables in turn take 133 us each; 8-bit rows are even, 2-bit
 // rows 4 % slower, so those take the kernel above).  Rows of at most 64 lanes.
 template <int BITS, int DPL>
 __global__ __launch_bounds__(256) void quantize_rows_padded_kernel(const float* __restrict__ in, int64_t rows,
@@ -821,8 +822,9 @@ struct MoveArgs {
 // inside the segment the place is guessed from the values at its ends (raw ids
 // are usually spread evenly: hashes) and four neighbouring entries are read in
 // two loads, which mostly ends the search in three or four reads; every second
-// later step bisects, so that any distribution ends.  20 us, of it 7 outside
-// the segments; four single loads 29 us, two entries a read 24 us, eight 21 us.
+// later step bisects, so that any distribution ends.  20 us on warm tables, of
+// it 7 outside the segments; four single loads 29 us, two entries a read 24 us,
+// eight 21 us (24 us behind other work, which takes the tables out of the caches).
 __device__ __forceinline__ int64_t remap_lower_bound(const int64_t* __restrict__ sorted, int64_t n, int64_t seg,
                                                      const int64_t* pivots, int64_t v, int64_t& entry) {
   int p = 0;
@@ -845,20 +847,15 @@ __device__ __forceinline__ int64_t remap_lower_bound(const int64_t* __restrict__
       mid = lo + (int64_t)(f * (float)(hi - lo + 1)) - 1;
     }
     // Entries base .. base + 3: inside [lo, hi] where that holds four, else reaching into what is
-    // known already, but never behind the table (n + 1 entries).
+    // known already, but never behind the table (n + 1 entries; a segment of two means n > 512).
     int64_t base = max(min(mid - 1, hi - 3), lo);
     base = max(min(base, n - 3), (int64_t)0);
     int64_t x[4];
-    if (n >= 3) {
 #pragma unroll
-      for (int e = 0; e < 4; e += 2) {
-        const i64x2_t q = *reinterpret_cast<const i64x2_t*>(sorted + base + e);
-        x[e] = q.x;
-        x[e + 1] = q.y;
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = sorted[min((int64_t)e, hi)];
+    for (int e = 0; e < 4; e += 2) {
+      const i64x2_t q = *reinterpret_cast<const i64x2_t*>(sorted + base + e);
+      x[e] = q.x;
+      x[e + 1] = q.y;
     }
     int below = 0;
 #pragma unroll
@@ -1048,8 +1045,9 @@ static void launch_regroup(const RegroupBlocks& b, int n_blocks, int columns, in
   const int cw = (columns + tiles - 1) / tiles;
   const int rp = (int)std::max<int64_t>(1, std::min<int64_t>(256 / cw, rows));
   const unsigned threads = (unsigned)((cw * rp + kWaveSize - 1) / kWaveSize * kWaveSize);
-  // Rows per thread: as many as leave two workgroups per compute unit (16 loads in flight: 12.9 us
-  // for 4096 rows of 4480 fp16 columns in 60 blocks, 8: 13.9 us, 4: 14.1 us; the copy rate is 14.5 us.
+  // Rows per thread: as many as leave 512 workgroups, two for each of an MI355X's 256 compute units
+  // (best passes: 16 loads in flight 12.9 us for 4096 rows of 4480 fp16 columns in 60 blocks, 8 13.9 us,
+  // 4 14.1 us; 13.4 us on average; the copy rate is 14.5 us.
   // One thread per element and a grid row per block took 42 us).
   const auto row_tiles = [&](int r) { return (rows + (int64_t)rp * r - 1) / ((int64_t)rp * r); };
   const auto go = [&](auto kernel, int r) {
@@ -1091,9 +1089,9 @@ static int move_keys(MoveArgs& m, int value_bytes, const RemapSpec* spec, hipStr
   for (int k0 = 0; k0 < m.num_out; k0 += group) {
     m.first_key = k0;
     m.launch_keys = std::min(group, m.num_out - k0);
-    // Ids per tile: a block's worth, up to eight of them where that leaves one tile per compute
-    // unit (a block with a table reads its pivots once per tile: 410 K ids in tiles of 512 24 us,
-    // of 1024 20 us, of 1536 24 us).
+    // Ids per tile: a block's worth, up to eight of them where that leaves 256 tiles, one for each
+    // of an MI355X's compute units (a block with a table reads its pivots once per tile: 410 K ids in
+    // tiles of 512 24 us, of 1024 20 us, of 1536 24 us, warm tables).
     const int64_t ids = std::min(m.num_values, m.out_values_end);
     m.tile = kMoveThreads;
     while (m.tile < 8 * kMoveThreads && ids / (2 * m.tile) >= 256) m.tile *= 2;

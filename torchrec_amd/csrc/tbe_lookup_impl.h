@@ -447,11 +447,10 @@ __device__ __forceinline__ int fetch_row(RowBuf<CB>& r, IdxT id, IdxT j, IdxT la
 // starts at +0 and a round-to-nearest sum is -0 only if both addends are), and
 // q is a finite integer.  For fp16 / fp32 rows the payload of an invalid row is
 // zeroed as well, so a stored inf / nan in row 0 cannot leak in.
-// WHOLE_WAVE: every lane of the wave is executing (the pooling loops: their
-// trip counts are wave-uniform and skipped rows are masked, never branched
-// around).  The matrix instruction reads its operands from all 64 lanes
-// whatever the execution mask, so it is used only there.
-template <int DTYPE, int CB, bool WEIGHTED, bool WHOLE_WAVE = true>
+// Every lane of the wave calls this (trip counts are wave-uniform, skipped rows
+// and rows past an end are masked, never branched around): the matrix
+// instruction reads its operands from all 64 lanes whatever the execution mask.
+template <int DTYPE, int CB, bool WEIGHTED>
 __device__ __forceinline__ void consume_row(float* acc, const RowBuf<CB>& r0, const RowWalk& w) {
   constexpr int EPD = 32 / Traits<DTYPE>::kBits;  // elements per dword
   RowBuf<CB> r = r0;
@@ -473,8 +472,7 @@ __device__ __forceinline__ void consume_row(float* acc, const RowBuf<CB>& r0, co
     }
     // int4 fields go through the matrix core where a lane holds at most 16
     // accumulators (8-byte chunks), int2 fields always.
-    constexpr bool kMatrix =
-        WHOLE_WAVE && (Traits<DTYPE>::kBits == 2 || (Traits<DTYPE>::kBits == 4 && CB <= 8));
+    constexpr bool kMatrix = Traits<DTYPE>::kBits == 2 || (Traits<DTYPE>::kBits == 4 && CB <= 8);
     if constexpr (kMatrix)
       asm volatile("" : "+v"(s));  // the converted scale stays in a register: no fp16 operand in the fused multiply-adds
 #pragma unroll

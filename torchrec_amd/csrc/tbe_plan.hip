@@ -660,7 +660,7 @@ static void compute_geometry(const tra_tbe* tbe, const Tuning& tune, bool balanc
       const int per_block = kWavesPerBlock * gpw;
       sc.tile_start = grid;
       if (nobag) {
-        // Ids per tile: one step of the kernel's loop (64 to 256 ids, by the row width), at least
+        // Ids per tile: one step of the kernel's loop (16 to 1024 ids, by the row width), at least
         // 128 ids; less where that leaves fewer than two tiles per compute unit, down to one id
         // per lane group.  2.1 M int8 rows of 128 columns: 128 ids a tile 187 us, 256 ids 195 us,
         // 512 ids 197 us, 64 ids 201 us (8-byte lane chunks: 64 and 128 ids 187 us, 256 ids 197 us).

@@ -105,7 +105,7 @@ __global__ __launch_bounds__(kBlockThreads) void tbe_nobag_kernel(const LookupAr
       const int pos = sc.key0 >= 0 ? sc.key0 + i : a.cdescs[ci].feature;
       int64_t f1, n1;
       sequence_bounds<IdxT>(a, ci, pos, s_starts, f1, n1);
-      // (32-bit arithmetic: fewer than 2^31 tiles of at least 16 ids)
+      // (32-bit arithmetic: tiles of under 128 ids are taken only for calls of a few thousand tiles)
       const int tiles = i0 + lane < sc.count ? (int)((n1 + tile_ids - 1) / tile_ids) : 0;
       const int incl = wave_scan_incl((int32_t)tiles);
       const uint64_t past = __builtin_amdgcn_ballot_w64(before + incl > t);

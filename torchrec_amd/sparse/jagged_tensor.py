@@ -15,7 +15,6 @@ permutation run in the HIP kernels behind ``torchrec_amd.ops``.
 """
 from __future__ import annotations
 
-import ctypes
 from array import array
 from typing import Dict, List, Optional, Tuple, Union
 
