@@ -1,0 +1,114 @@
+"""The sixteen-lane pooled kernel (calls too small for the window kernel) at the sizes where its lane groups, blocks of
+sixteen ids and column slices begin and end, against the CPU oracle, bit for bit."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from helpers import bits_equal, make_table
+from test_tbe_gpu import DEV, build, _from_lengths
+from torchrec_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+# one lane's columns change at 16, 32, 64, 128 and 256; 100, 300 and 520 (int8), 200 (int4) are several slices
+DIMS = {O.INT8: [4, 16, 20, 32, 64, 72, 100, 128, 256, 300, 520], O.INT4: [8, 16, 40, 64, 104, 128, 200, 256, 264],
+        O.INT2: [16, 32, 64, 80, 256, 272], O.FP16: [2, 16, 18, 64, 66, 128, 130, 256], O.FP32: [1, 16, 17, 33, 64, 65, 128]}
+
+
+def _lengths(rng, n):
+    return rng.choice([0, 0, 1, 2, 7, 8, 9, 15, 16, 17, 31, 33, 70], n)
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("dtype", [O.INT8, O.INT4, O.INT2, O.FP16, O.FP32])
+def test_group_widths(tuning, dtype, weighted):
+    tuning(balanced=0)
+    rng = np.random.default_rng(70 + dtype * 2 + weighted)
+    specs = [(dtype, 200 + 3 * i, dim) for i, dim in enumerate(DIMS[dtype])]
+    ftm = list(range(len(specs)))
+    idt, pooling, out = (np.int64, O.MEAN, O.FP32) if weighted else (np.int32, O.SUM, O.FP16)
+    tbe, store = build(rng, specs, ftm, pooling, out, 4)
+    for B in (1, 17, 65):
+        lengths = _lengths(rng, len(specs) * B).astype(idt)
+        offsets = np.zeros(len(lengths) + 1, dtype=idt)
+        offsets[1:] = np.cumsum(lengths)
+        per = lengths.reshape(len(specs), B).sum(1)
+        ids = np.concatenate([rng.integers(-1, s[1], n) for s, n in zip(specs, per)]).astype(idt)
+        psw = rng.uniform(-1, 1, len(ids)).astype(np.float32) if weighted else None
+        want = O.tbe_forward(store, ftm, B, ids, offsets, psw, pooling, out)
+        got = _from_lengths(tbe, ids, lengths, psw, B)
+        assert bits_equal(got, want) == 0, B
+        got = tbe(torch.from_numpy(ids).to(DEV), torch.from_numpy(offsets).to(DEV),
+                  None if psw is None else torch.from_numpy(psw).to(DEV)).cpu().numpy()
+        assert bits_equal(got, want) == 0, B
+
+
+@pytest.mark.parametrize("bags", [40_000, 300_000])  # 3 and 16 bags per group
+def test_several_bags_per_group(tuning, bags):
+    tuning(balanced=0)
+    rng = np.random.default_rng(bags)
+    specs, B = [(O.INT8, 300, 16), (O.INT4, 200, 40)], bags // 2
+    tbe, store = build(rng, specs, [0, 1], O.MEAN, O.FP32, 16)
+    lengths = rng.choice([0, 1, 2, 17], 2 * B, p=[0.4, 0.3, 0.28, 0.02]).astype(np.int32)
+    offsets = np.zeros(2 * B + 1, dtype=np.int32)
+    offsets[1:] = np.cumsum(lengths)
+    ids = rng.integers(0, 200, int(offsets[-1])).astype(np.int32)
+    want = O.tbe_forward(store, [0, 1], B, ids, offsets, None, O.MEAN, O.FP32)
+    assert bits_equal(_from_lengths(tbe, ids, lengths, None, B), want) == 0
+
+
+def test_position_weights_of_many_slices():
+    """150 features of two weight types: more than the launch arguments describe at once, no class above the limit."""
+    rng = np.random.default_rng(5)
+    T, B = 150, 5
+    specs = [((O.INT8, O.INT4)[t % 2], 50, 16) for t in range(T)]
+    tbe, store = build(rng, specs, list(range(T)), O.SUM, O.FP32, 16)
+    lengths = rng.integers(0, 6, T * B).astype(np.int32)
+    offsets = np.zeros(T * B + 1, dtype=np.int32)
+    offsets[1:] = np.cumsum(lengths)
+    ids = rng.integers(0, 50, int(offsets[-1])).astype(np.int32)
+    table = rng.uniform(-1, 1, 4 * T).astype(np.float32)
+    start, n = [4 * t for t in range(T)], [4 if t % 3 else 0 for t in range(T)]
+    place = np.arange(len(ids)) - np.repeat(offsets[:-1], lengths)
+    key = np.repeat(np.arange(T * B) // B, lengths)
+    psw = np.where(np.take(n, key) > 0, table[np.take(start, key) + np.minimum(place, 3)], 1.0).astype(np.float32)
+    want = O.tbe_forward(store, list(range(T)), B, ids, offsets, psw, O.SUM, O.FP32)
+    got = tbe(torch.from_numpy(ids).to(DEV), torch.from_numpy(offsets).to(DEV),
+              position_weights=(torch.from_numpy(table).to(DEV), start, n)).cpu().numpy()
+    assert bits_equal(got, want) == 0
+
+
+@pytest.mark.parametrize("dtype,dim", [(O.INT8, 64), (O.INT4, 128), (O.INT2, 256), (O.FP16, 64), (O.INT8, 300)])
+def test_table_beyond_four_gib(tuning, dtype, dim):
+    """Rows 4 MiB apart, 1100 of them: offsets beyond 32 bits.  The same rows close together give the same bits."""
+    tuning(balanced=0)
+    rng = np.random.default_rng(dim)
+    rows, B = 1100, 33
+    data = make_table(rng, dtype, rows, dim)
+    if dtype not in (O.FP16, O.FP32):
+        data = np.concatenate([data[:, -4:], data[:, :-4]], 1)  # (the operator's rows have the header in front)
+    data = torch.from_numpy(np.ascontiguousarray(data).view(np.uint8).reshape(rows, -1)).to(DEV)
+    lengths = _lengths(rng, B)
+    offsets = torch.zeros(B + 1, dtype=torch.int32, device=DEV)
+    offsets[1:] = torch.from_numpy(np.cumsum(lengths)).to(DEV)
+    ids = torch.from_numpy(rng.integers(0, rows, int(lengths.sum())).astype(np.int32)).to(DEV)
+    outs = []
+    for stride in (data.shape[1], 4 << 20):
+        store = torch.empty(rows * stride, dtype=torch.uint8, device=DEV)
+        store.view(rows, stride)[:, : data.shape[1]].copy_(data)
+        spec = (_lib.TableSpec * 1)()
+        spec[0].offset, spec[0].rows, spec[0].dim, spec[0].row_bytes = 0, rows, dim, stride
+        spec[0].dtype = {O.INT8: _lib.INT8, O.INT4: _lib.INT4, O.INT2: _lib.INT2, O.FP16: _lib.FP16}[dtype]
+        plan = ctypes.c_void_p()
+        l = _lib.lib()
+        _lib.check(l.tra_tbe_create(spec, 1, (ctypes.c_int32 * 1)(0), None, 1, ctypes.byref(plan)))
+        out = torch.empty(B, dim, device=DEV)
+        _lib.check(l.tra_tbe_forward(plan, _lib.ptr(store), _lib.ptr(ids), _lib.ptr(offsets), 0, None, B, ids.numel(),
+                                     _lib.POOL_SUM, _lib.FP32, _lib.ptr(out), dim, _lib.current_stream(DEV)))
+        torch.cuda.synchronize()
+        _lib.check(l.tra_tbe_destroy(plan))
+        outs.append(out)
+    assert outs[0].abs().max() > 0 and torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))

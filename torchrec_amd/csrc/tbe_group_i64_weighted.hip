@@ -1,0 +1,6 @@
+// Instantiates the sixteen-lane lookup kernels for int64_t ids, kPerSample (see tbe_group_impl.h).
+#include "tbe_group_impl.h"
+
+namespace tra {
+TRA_DEFINE_GROUP(int64_t, kPerSample)
+}  // namespace tra

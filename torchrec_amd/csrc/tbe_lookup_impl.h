@@ -60,7 +60,7 @@ struct LookupArgs {
   unsigned long long* err_count;
   int64_t num_indices;
   int32_t B;
-  int32_t n_sub;
+  int32_t n_sub;  // window and sequence kernels
   int32_t mean;
   int32_t vec_store;  // 1: every lane's output slice is 16-byte aligned
   int32_t out_fp16;
@@ -486,14 +486,15 @@ __device__ __forceinline__ void consume_row(float* acc, const RowBuf<CB>& r0, co
   }
 }
 
-// Store NE consecutive outputs starting at element `pos`.
+// Store NE consecutive outputs starting at element `pos`.  `vec`: every lane's
+// output slice is 16-byte aligned.
 template <int NE>
 __device__ __forceinline__ void store_outputs(const LookupArgs& a, int64_t pos,
-                                              const float* acc) {
+                                              const float* acc, bool vec) {
   if (a.out_fp16) {
     __half* o = reinterpret_cast<__half*>(a.out) + pos;
     if constexpr (NE >= 8) {
-      if (a.vec_store) {
+      if (vec) {
 #pragma unroll
         for (int i = 0; i < NE; i += 8) {
           uint4 v;
@@ -514,7 +515,7 @@ __device__ __forceinline__ void store_outputs(const LookupArgs& a, int64_t pos,
   } else {
     float* o = reinterpret_cast<float*>(a.out) + pos;
     if constexpr (NE >= 4) {
-      if (a.vec_store) {
+      if (vec) {
 #pragma unroll
         for (int i = 0; i < NE; i += 4)
           *reinterpret_cast<float4*>(o + i) =
@@ -534,25 +535,6 @@ __device__ __forceinline__ int wave_max(int v) {
     v = o > v ? o : v;
   }
   return v;
-}
-
-// Locate this block's (sub-class, feature, tile).  Uniform across the block.
-__device__ __forceinline__ bool locate_tile(const LookupArgs& a, int& f, int& lpr,
-                                            int& tile, int* class_index = nullptr) {
-  const int blk = blockIdx.x;
-  int s = 0;
-#pragma unroll
-  for (int i = 1; i < kMaxSub; ++i)
-    if (i < a.n_sub && blk >= a.sub[i].tile_start) s = i;
-  const SubClass sc = a.sub[s];
-  const int local = blk - sc.tile_start;
-  const int fi = local / sc.tiles_per_feat;
-  if (fi >= sc.count) return false;
-  tile = local - fi * sc.tiles_per_feat;
-  f = a.feats[sc.first + fi];
-  if (class_index) *class_index = sc.first + fi;
-  lpr = sc.lpr;
-  return true;
 }
 
 // Built with -DTRA_INSTRUMENT (never in the shipped library), every wave
@@ -804,14 +786,14 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 template <int NE>
 __device__ __forceinline__ void finish_bag(float (&acc)[NE], const LookupArgs& a, int len,
-                                           int64_t row_pos, int c, int lpr, int lane, bool active) {
+                                           int64_t row_pos, int c, int lpr, int lane, bool active, bool vec) {
   if (a.mean && len > 0) {
     const float inv = 1.0f / (float)len;
 #pragma unroll
     for (int i = 0; i < NE; ++i) acc[i] *= inv;
   }
   if constexpr (NE == 16 || NE == 8) {
-    const bool two_vectors = a.vec_store && lpr >= 2 && (lpr & (lpr - 1)) == 0 &&
+    const bool two_vectors = vec && lpr >= 2 && (lpr & (lpr - 1)) == 0 &&
                              (a.out_fp16 ? NE == 16 : NE == 8);  // wave-uniform
     if (two_vectors) {
       uint32_t v[2][4];
@@ -851,7 +833,7 @@ __device__ __forceinline__ void finish_bag(float (&acc)[NE], const LookupArgs& a
       return;
     }
   }
-  if (active) store_outputs<NE>(a, row_pos + (int64_t)c * NE, acc);
+  if (active) store_outputs<NE>(a, row_pos + (int64_t)c * NE, acc, vec);
 }
 
 // Balanced mapping.  One 1024-thread block per compute unit owns a window of
@@ -1067,107 +1049,6 @@ __device__ __forceinline__ int feat_key_pos(const LookupArgs& a, const SubClass&
   if (sc.key0 >= 0) return sc.key0 + fi;  // no load: the bag bounds can be requested at once
   return sc.first + fi < kMaxPos ? (int)a.feat_pos[sc.first + fi]
                                  : a.descs[a.feats[sc.first + fi]].feature;
-}
-
-// Static mapping: lane group g of wave w of tile t owns bag (t*waves + w)*gpw + g.
-// Used for small problems, where there are not enough bags to balance.
-// FROM_LENGTHS: a.offsets points at the KJT's lengths; the block sums what
-// lies in front of its first bag (every block reads that prefix again: this
-// form is for calls with few bags, where a scan kernel of its own would cost
-// more than the lookup) and scans its own bags, which are consecutive.
-template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, bool FROM_LENGTHS = false>
-__global__ __launch_bounds__(kBlockThreads) void tbe_pooled_kernel(const LookupArgs a) {
-  constexpr int NE = CB * 8 / Traits<DTYPE>::kBits;  // columns per lane
-  TRA_STAMP(0);
-  int f, lpr, tile, ci;
-  if (!locate_tile(a, f, lpr, tile, &ci)) return;
-  const FeatureDesc d = a.descs[f];
-  const int lane = threadIdx.x & (kWaveSize - 1);
-  const int wave = threadIdx.x / kWaveSize;
-  const int gpw = kWaveSize / lpr;  // lane groups (bags) per wave
-  const int g = lane / lpr;
-  const int c = lane - g * lpr;
-  const int bag_in_feat = (tile * kWavesPerBlock + wave) * gpw + g;
-  const bool active = g < gpw && bag_in_feat < a.B;
-
-  int64_t start = 0;
-  int len = 0;
-  if (FROM_LENGTHS) {
-    using Sum = typename SumOf<IdxT>::type;
-    constexpr int V = 16 / (int)sizeof(IdxT);
-    struct __align__(16) Vec { IdxT v[V]; };
-    __shared__ Sum s_front[kWavesPerBlock];
-    __shared__ Sum s_wave_tot[kWavesPerBlock];
-    const IdxT* lengths = reinterpret_cast<const IdxT*>(a.offsets);
-    // this lane group's own length first: its load shares the latency of the prefix loads
-    const int64_t bag = (int64_t)d.feature * a.B + min(bag_in_feat, a.B - 1);
-    const Sum raw = active ? (Sum)lengths[bag] : (Sum)0;
-    // sum(lengths[0 .. p)), p = position of the block's first bag (16-byte steps, then the rest)
-    const int64_t p = (int64_t)d.feature * a.B + (int64_t)tile * kWavesPerBlock * gpw;
-    const int nvec = (int)(p / V);
-    Sum part = 0;
-    for (int v0 = 0; v0 < nvec; v0 += 4 * kBlockThreads) {
-      Vec x[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) x[k] = reinterpret_cast<const Vec*>(lengths)[min(v0 + k * kBlockThreads + (int)threadIdx.x, nvec - 1)];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        Sum sum = 0;
-#pragma unroll
-        for (int i = 0; i < V; ++i) sum += (Sum)x[k].v[i];
-        part += v0 + k * kBlockThreads + (int)threadIdx.x < nvec ? sum : (Sum)0;
-      }
-    }
-    {
-      const int64_t ti = (int64_t)nvec * V + threadIdx.x;
-      if (ti < p) part += (Sum)lengths[ti];
-    }
-    // bag starts inside the block: scan over the lane groups (the group's first
-    // lane carries its length), then over the block's waves
-    const Sum incl = wave_scan_incl(c == 0 && g < gpw ? raw : (Sum)0);
-    const Sum front_w = wave_last(wave_scan_incl(part));
-    if (lane == kWaveSize - 1) s_wave_tot[wave] = incl;
-    if (lane == 0) s_front[wave] = front_w;
-    __syncthreads();
-    Sum before = 0, front = 0;
-#pragma unroll
-    for (int w = 0; w < kWavesPerBlock; ++w) {
-      front += s_front[w];
-      if (w < wave) before += s_wave_tot[w];
-    }
-    start = (int64_t)(front + before + incl - raw);
-    len = raw > 0 ? (int)raw : 0;
-  } else if (active) {
-    const int64_t bag = (int64_t)d.feature * a.B + bag_in_feat;
-    start = load_index<IdxT>(a.offsets, bag);
-    len = (int)(load_index<IdxT>(a.offsets, bag + 1) - start);
-  }
-  const int max_len = wave_max(len);
-  TRA_STAMP(1);
-
-  RowWalk w;
-  w.chunk_off = Traits<DTYPE>::kHeader + d.payload_off + c * CB;
-  w.lane_base = a.weights + d.table_offset + w.chunk_off;
-  w.set_rows(d.rows, d.row_bytes);
-  w.count_errors = c == 0 && d.payload_off == 0;
-  w.hdr_lane = lane - c;
-  w.sel0 = mfma_byte_selector(lane, 0);
-  w.sel1 = mfma_byte_selector(lane, 1);
-  w.set_position_weights(a, ci, start);
-
-  float acc[NE];
-#pragma unroll
-  for (int i = 0; i < NE; ++i) acc[i] = 0.0f;
-  const int bad = pool_bag<DTYPE, CB, IdxT, WEIGHTED, U, NE>(acc, a, w, start, len, max_len);
-  if (a.bad_to_row0 != 0 && __builtin_amdgcn_ballot_w64(bad != 0) != 0)
-    repool_bad_ids_as_row0<DTYPE, CB, IdxT, WEIGHTED, NE>(acc, a, w, start, len, max_len);
-  TRA_STAMP(2);
-#ifdef TRA_INSTRUMENT
-  if ((threadIdx.x & 63) == 0)
-    a.ts[((size_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64) * 8 + 4] = max_len;
-#endif
-  finish_bag<NE>(acc, a, len, (int64_t)bag_in_feat * a.out_stride + d.out_col, c, lpr, lane, active);
-  TRA_STAMP(3);
 }
 
 constexpr int kNarrowLane = 8;  // accumulators per lane up to which one instance serves all widths (see odd_lanes)
@@ -1544,7 +1425,7 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
 #ifdef TRA_INSTRUMENT
     if (lane == 0) a.ts[((size_t)blockIdx.x * (blockDim.x / 64) + wave) * 8 + 5] = (unsigned long long)max_len;
 #endif
-    finish_bag<NE>(acc, a, len, (int64_t)b * a.out_stride + d.out_col, c, lpr, lane, active);
+    finish_bag<NE>(acc, a, len, (int64_t)b * a.out_stride + d.out_col, c, lpr, lane, active, a.vec_store != 0);
     TRA_STAMP(4);
   }
 }
@@ -1584,8 +1465,7 @@ struct LaunchClass {
 
 struct LaunchParams {
   int grid;
-  int balanced;   // 1: one 1024-thread block per window of bags (tbe_pooled_cu_kernel)
-  int lds_bytes;  // dynamic LDS of the balanced kernel (sized so one block fits per CU)
+  int lds_bytes;  // dynamic LDS (sized so one block fits per CU)
   int unroll;     // rows per pipeline batch: 2, 4 or 8
   bool idx64;
   bool weighted;
@@ -1595,6 +1475,50 @@ struct LaunchParams {
 
 template <int DTYPE>
 int launch_lookup(const LookupArgs& a, int cb, const LaunchParams& p, hipStream_t stream);
+
+// Consecutive columns of one feature, as the sixteen-lane kernel takes them.
+struct GroupSlice {
+  int64_t table_offset;
+  int64_t rows;
+  uint32_t rows32;      // min(rows, 2^31)
+  int32_t row_bytes;    // stride
+  int32_t cols;
+  int32_t out_col;
+  int32_t payload;      // byte offset of the slice's columns inside a row
+  int32_t kind;         // group_kind(weight type, columns per lane, mode)
+  int32_t key;          // key position
+  uint8_t even;         // the first output column is
+  uint8_t first_slice;  // holds column 0 of its feature
+  uint16_t unused;
+};
+// How the sixteen-lane kernel addresses a slice's rows.
+constexpr int kNear = 0;   // 32-bit offsets, header in front of the columns (or none)
+constexpr int kFar = 1;    // a table beyond 4 GiB
+constexpr int kSplit = 2;  // one of several slices of a row with a header
+constexpr int group_kind(int dtype, int ne, int mode) { return (dtype * 4 + mode) * 32 + ne; }
+struct GroupArgs {
+  LookupArgs common;  // (descriptors, sub, n_sub, pw_off, pw_len and the sequence lookup's fields are not read;
+                      //  vec_store: two fp16 results of an even column make an aligned dword)
+  const GroupSlice* slices;
+};
+// Position weights of the launch's slices, as in LookupArgs (a parameter of its own: indexed at run time, it has to
+// stay apart from what the kernel's functions take by reference).
+struct GroupPositions {
+  int32_t off[kMaxPos];
+  int32_t len[kMaxPos];
+};
+static_assert(sizeof(GroupArgs) + sizeof(GroupPositions) + 48 <= 4096, "launch arguments");
+struct GroupLaunch {
+  int grid;
+  int per_group;  // bags per lane group (at most 16)
+  int tiles;      // blocks per slice
+  int key0;       // slice i sits at key key0 + i; -1: each slice says where
+};
+
+// Pooled lookup, all weight types in one launch (tbe_group_impl.h).
+template <typename IdxT, int WEIGHTED>
+void launch_group(const GroupArgs& a, const GroupPositions& p, const GroupLaunch& l, bool from_lengths,
+                  hipStream_t stream);
 
 // The sequence lookup of one class (tbe_sequence.hip).
 int launch_sequence(const LookupArgs& a, int dtype, int cb, bool split, bool idx64, int grid, hipStream_t stream);
@@ -1609,24 +1533,18 @@ void launch_typed(const LookupArgs& a, const LaunchParams& p, hipStream_t stream
 #define TRA_POOLED(W, U)                                                                       \
   do {                                                                                         \
     constexpr bool O = kOddInstance<DTYPE, CB>;                                                \
-    if (O && p.balanced && p.odd && p.from_lengths)                                            \
+    if (O && p.odd && p.from_lengths)                                                          \
       hipLaunchKernelGGL((tbe_pooled_cu_kernel<DTYPE, CB, IdxT, W, 4, true, O>), g,            \
                          dim3(kCuThreads), p.lds_bytes, stream, TRA_CU_LEADING_ARGS, a);       \
-    else if (O && U == 4 && p.balanced && p.odd)                                               \
+    else if (O && U == 4 && p.odd)                                                             \
       hipLaunchKernelGGL((tbe_pooled_cu_kernel<DTYPE, CB, IdxT, W, U, false, O && U == 4>), g, \
                          dim3(kCuThreads), p.lds_bytes, stream, TRA_CU_LEADING_ARGS, a);       \
-    else if (p.balanced && p.from_lengths)                                                     \
+    else if (p.from_lengths)                                                                   \
       hipLaunchKernelGGL((tbe_pooled_cu_kernel<DTYPE, CB, IdxT, W, 4, true>), g,               \
                          dim3(kCuThreads), p.lds_bytes, stream, TRA_CU_LEADING_ARGS, a);       \
-    else if (p.balanced)                                                                       \
+    else                                                                                       \
       hipLaunchKernelGGL((tbe_pooled_cu_kernel<DTYPE, CB, IdxT, W, U>), g, dim3(kCuThreads),   \
                          p.lds_bytes, stream, TRA_CU_LEADING_ARGS, a);                         \
-    else if (p.from_lengths)                                                                   \
-      hipLaunchKernelGGL((tbe_pooled_kernel<DTYPE, CB, IdxT, W, 4, true>), g,                  \
-                         dim3(kBlockThreads), 0, stream, a);                                   \
-    else                                                                                       \
-      hipLaunchKernelGGL((tbe_pooled_kernel<DTYPE, CB, IdxT, W, U>), g, dim3(kBlockThreads), 0, \
-                         stream, a);                                                           \
   } while (0)
   if constexpr (DTYPE >= kSplitHeader) {  // (one unroll depth for the rare split rows)
     if (a.posw != nullptr) TRA_POOLED(kByPosition, 4); else if (p.weighted) TRA_POOLED(kPerSample, 4); else TRA_POOLED(kUnweighted, 4);

@@ -46,6 +46,19 @@ template <>
 int launch_lookup<TRA_FP16>(const LookupArgs&, int, const LaunchParams&, hipStream_t);
 template <>
 int launch_lookup<TRA_FP32>(const LookupArgs&, int, const LaunchParams&, hipStream_t);
+// ... and in tbe_group_<id type>_<weight mode>.hip.
+template <>
+void launch_group<int32_t, kUnweighted>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
+template <>
+void launch_group<int32_t, kPerSample>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
+template <>
+void launch_group<int32_t, kByPosition>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
+template <>
+void launch_group<int64_t, kUnweighted>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
+template <>
+void launch_group<int64_t, kPerSample>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
+template <>
+void launch_group<int64_t, kByPosition>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
 
 // Launch shape of the pooled kernels.  Defaults are chosen from the problem
 // size when a plan first sees a (batch size, route) pair and are remembered in
@@ -56,7 +69,7 @@ int launch_lookup<TRA_FP32>(const LookupArgs&, int, const LaunchParams&, hipStre
 struct Tuning {
   int balanced;  // 1: tbe_pooled_cu_kernel, one block per CU-sized window of bags
   int window;    // bags per block (0: derive from the problem size)
-  int unroll;
+  int unroll;    // window kernel
   int lds_bytes;
 };
 
@@ -95,11 +108,17 @@ static Overrides g_ovr = overrides_from_env();
 // Bumped by tra_set_tuning: launch geometry remembered under an older value is recomputed.
 static std::atomic<int> g_ovr_gen{0};
 
-static Tuning choose_tuning(int num_cus, int64_t bags, int64_t num_indices) {
+static Tuning choose_tuning(int num_cus, size_t classes, int64_t bags, int64_t num_indices) {
   Tuning t;
-  // Ranking bags by length pays once every CU gets a few dozen bags (measured
-  // crossover on 26 int4 tables: between 6.6k bags / 130k ids and 13k / 260k).
-  t.balanced = bags >= 40 * (int64_t)num_cus && num_indices >= 640 * (int64_t)num_cus;
+  // Ranking bags by length pays once every CU gets a few dozen bags; below that the sixteen-lane kernel is
+  // faster, and with several launch classes it stays so for longer, being one launch for all of them.  Graph
+  // replays of the whole call, us (sixteen-lane / window), ids a bag 3 and 20:
+  //   one class (int8 dim 64): 8192 bags 5.3 / 5.3 and 9.0 / 9.1; 13 K bags of 2 ids 6.2 / 5.6; 33 K bags 13.8 / 6.9
+  //   and 22.8 / 11.7
+  //   two classes (int8 dims 32 - 256): 33 K bags 16.7 / 17.2 and 34 / 30
+  //   seven classes: 33 K bags 16.5 / 32 and 34 / 58; 131 K bags 34 / 68 and 86 / 120 (such calls are not told apart
+  //   from hot ones with more ids, where the window kernel's two streams win; they keep the general rule)
+  t.balanced = bags >= 40 * (int64_t)num_cus && (classes <= 1 || num_indices >= 640 * (int64_t)num_cus);
   t.window = 0;
   t.unroll = 4;
   t.lds_bytes = 48 * 1024;  // with the static arrays > half of a CU's LDS: one block per CU
@@ -169,6 +188,7 @@ struct Geometry {
   int gen = -1;
   Tuning tune{};
   std::vector<ClassGeometry> cls;
+  GroupLaunch group{};  // pooled calls that are not balanced: windows (the grid is per launch)
 };
 
 constexpr int kGeometrySlots = 8;
@@ -206,6 +226,10 @@ struct tra_tbe {
   std::vector<uint8_t> on_side;      // per class index: 1 = launched on `side`
   std::vector<LaunchClass> classes;
   std::vector<LookupArgs> base_args;  // per class: everything a call does not change
+  // Column slices for the sixteen-lane kernel, in feature order.
+  std::vector<GroupSlice> group_slices;
+  GroupSlice* group_slices_dev = nullptr;
+  LookupArgs group_base;  // everything a call does not change
   std::mutex geo_mutex;
   std::shared_ptr<const Geometry> geo[kGeometrySlots];
   int geo_next = 0;
@@ -339,6 +363,41 @@ int tra_tbe_create(const tra_table_spec* tables, int32_t num_tables,
       plan->slices.push_back(d);
       slice_lpr.push_back(bytes / cb);
     }
+    // The sixteen-lane kernel's slices: the row as one where sixteen lanes can hold it (16 columns of an
+    // integer row each, 16 bytes of others), else as wide ones as there are.
+    const bool header = header_bytes(s.dtype) != 0;
+    const int most = s.dtype == TRA_FP32 ? 4 : s.dtype == TRA_FP16 ? 8 : 16;
+    const auto fits = [](int ne, int cols) { return ne * 16 >= cols && cols % ne == 0; };
+    bool one_slice = false;
+    for (int ne = 1; ne <= most; ne *= 2) one_slice = one_slice || fits(ne, s.dim);
+    for (int off = 0; off < s.dim;) {
+      const int left = s.dim - off;
+      int ne = 1;
+      if (one_slice) {
+        while (!fits(ne, left)) ne *= 2;
+      } else if (header) {
+        ne = left >= 256 || left % 16 == 0 ? 16 : 32 / bits;  // (the kernel's split kinds: 16, or a dword's columns)
+      } else {
+        ne = most;
+        while (ne > 1 && ne * 16 > left && left % ne != 0) ne /= 2;
+      }
+      GroupSlice w;
+      w.table_offset = s.offset;
+      w.rows = s.rows;
+      w.rows32 = (uint32_t)std::min<int64_t>(s.rows, int64_t(1) << 31);
+      w.row_bytes = s.row_bytes;
+      w.cols = std::min(left, ne * 16);
+      w.out_col = col + off;
+      w.payload = header_bytes(s.dtype) + off * bits / 8;
+      w.key = feature_positions ? feature_positions[f] : f;
+      w.even = w.out_col % 2 == 0 ? 1 : 0;
+      w.first_slice = off == 0 ? 1 : 0;
+      w.unused = 0;
+      // (near: row offset and place in the row are added in 32 bits)
+      w.kind = group_kind(s.dtype, ne, header && !one_slice ? kSplit : s.rows * s.row_bytes > 0xffffffffll ? kFar : kNear);
+      plan->group_slices.push_back(w);
+      off += w.cols;
+    }
     col += s.dim;
   }
   // Classes: slices sorted by lanes-per-row; at most kMaxSub distinct values each.
@@ -425,6 +484,12 @@ int tra_tbe_create(const tra_table_spec* tables, int32_t num_tables,
       e = hipMemcpy(plan->cdescs_dev, ordered.data(), total * sizeof(FeatureDesc), hipMemcpyHostToDevice);
     }
   }
+  if (e == hipSuccess && !plan->group_slices.empty()) {
+    e = hipMalloc((void**)&plan->group_slices_dev, plan->group_slices.size() * sizeof(GroupSlice));
+    if (e == hipSuccess)
+      e = hipMemcpy(plan->group_slices_dev, plan->group_slices.data(), plan->group_slices.size() * sizeof(GroupSlice),
+                    hipMemcpyHostToDevice);
+  }
   if (e == hipSuccess) e = hipMalloc((void**)&plan->err_dev, sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMemset(plan->err_dev, 0, sizeof(unsigned long long));
   if (e != hipSuccess) {
@@ -449,6 +514,8 @@ int tra_tbe_create(const tra_table_spec* tables, int32_t num_tables,
       a.feat_pos[i] = (int16_t)plan->slices[cls.feats[i]].feature;
     plan->base_args.push_back(a);
   }
+  memset(&plan->group_base, 0, sizeof(plan->group_base));
+  plan->group_base.err_count = plan->err_dev;
   // Launch order and streams.  The launches of a call write disjoint output columns, so they may
   // overlap.  A launch leaves compute units idle before its first rows arrive and while its last
   // blocks finish; with consecutive launches on alternating streams the next launch's blocks fill
@@ -490,6 +557,7 @@ int tra_tbe_destroy(tra_tbe_t tbe) {
   if (tbe->slices_dev) (void)hipFree(tbe->slices_dev);
   if (tbe->feats_dev) (void)hipFree(tbe->feats_dev);
   if (tbe->cdescs_dev) (void)hipFree(tbe->cdescs_dev);
+  if (tbe->group_slices_dev) (void)hipFree(tbe->group_slices_dev);
   if (tbe->err_dev) (void)hipFree(tbe->err_dev);
   if (tbe->side) (void)hipStreamDestroy(tbe->side);
   if (tbe->ev_join) (void)hipEventDestroy(tbe->ev_join);
@@ -516,7 +584,7 @@ static bool fused_scan_possible(const tra_tbe* tbe, int32_t batch_size, int32_t 
                                 int64_t num_indices, int32_t pooling_mode, const void* lengths) {
   if (pooling_mode == TRA_POOL_NONE || batch_size <= 0 || tbe->num_features == 0) return false;
   if ((uintptr_t)lengths % 16 != 0) return false;
-  const Tuning tune = choose_tuning(tbe->num_cus, (int64_t)tbe->num_features * batch_size, num_indices);
+  const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
   if (!use_window_kernel(tbe, tune, false, batch_size)) return false;
   const int fused = g_ovr.fused_scan;
   if (fused >= 0) return fused != 0;
@@ -530,15 +598,15 @@ static bool fused_scan_possible(const tra_tbe* tbe, int32_t batch_size, int32_t 
 }
 
 // A pooled call too small for the window kernel whose lengths are few enough
-// that every block of the static kernel can sum the ones in front of its bags
-// itself: one launch instead of a scan and a lookup.
+// that every block of the sixteen-lane kernel can sum the ones in front of its
+// bags itself: one launch instead of a scan and a lookup.
 constexpr int64_t kSmallFusedMaxLengths = 16384;
 
 static bool small_fused_scan_possible(const tra_tbe* tbe, int32_t batch_size, int32_t num_keys,
                                       int64_t num_indices, int32_t pooling_mode, const void* lengths) {
   if (pooling_mode == TRA_POOL_NONE || batch_size <= 0 || tbe->num_features == 0) return false;
   if ((uintptr_t)lengths % 16 != 0 || g_ovr.fused_scan == 0) return false;
-  const Tuning tune = choose_tuning(tbe->num_cus, (int64_t)tbe->num_features * batch_size, num_indices);
+  const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
   if (use_window_kernel(tbe, tune, false, batch_size)) return false;
   return (int64_t)num_keys * batch_size <= kSmallFusedMaxLengths;
 }
@@ -551,7 +619,7 @@ int tra_tbe_launch_info(tra_tbe_t tbe, int32_t batch_size, int64_t num_indices,
     return TRA_ERR_INVALID_ARGUMENT;
   }
   const bool nobag = pooling_mode == TRA_POOL_NONE;
-  const Tuning tune = choose_tuning(tbe->num_cus, (int64_t)tbe->num_features * batch_size, num_indices);
+  const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
   const bool balanced = use_window_kernel(tbe, tune, nobag, batch_size);
   // lengths entry point: same decision as tra_tbe_forward_lengths (aligned lengths assumed)
   const bool fused = lengths_num_keys > 0 &&
@@ -561,14 +629,20 @@ int tra_tbe_launch_info(tra_tbe_t tbe, int32_t batch_size, int64_t num_indices,
                                                 (const void*)16));
   static const char* const kDtypeName[] = {"fp32", "fp16", "int8", "int4", "int2"};
   std::string text;
+  if (!nobag && !balanced) {
+    char line[120];
+    snprintf(line, sizeof(line), "tbe_pooled_kernel slices=%d%s", (int)tbe->group_slices.size(), fused ? " from_lengths" : "");
+    text = line;
+  }
   // In launch order; a plan with a second stream alternates between the two.
   const bool two_streams = tbe->side != nullptr && balanced && g_ovr.fork != 0;
   for (const int ci : tbe->launch_order) {
+    if (!nobag && !balanced) break;
     const LaunchClass& cls = tbe->classes[ci];
     char line[200];
     snprintf(line, sizeof(line), "%s%s dtype=%s lane_bytes=%d slices=%d%s%s",
              text.empty() ? "" : "; ",
-             nobag ? "tbe_nobag_kernel" : (balanced ? "tbe_pooled_cu_kernel" : "tbe_pooled_kernel"),
+             nobag ? "tbe_nobag_kernel" : "tbe_pooled_cu_kernel",
              kDtypeName[cls.dtype], cls.cb, (int)cls.feats.size(),
              two_streams ? (tbe->on_side[ci] ? " on the plan's second stream" : " on the caller's stream") : "",
              fused ? " from_lengths" : "");
@@ -597,6 +671,20 @@ struct SequenceBounds {
   int32_t num_keys;
 };
 
+// Windows of the sixteen-lane kernel: one bag per lane group until every compute unit has four blocks, then more (33 K
+// bags of 3 and 20 ids, us: one bag per group 16.7 / 25.0, two 13.9 / 22.8, three 13.8 / 24.1, eight 15.5 / 30.3; 8 K
+// bags: one 5.3 / 9.0, two 5.7 / 10.2).
+static GroupLaunch group_windows(const tra_tbe* tbe, int32_t batch_size) {
+  GroupLaunch l{};
+  constexpr int groups = kBlockThreads / 16;
+  const int64_t bags = (int64_t)tbe->group_slices.size() * batch_size;
+  const int64_t at_once = 4 * (int64_t)tbe->num_cus * groups;
+  const int64_t per_group = std::min<int64_t>((bags + at_once - 1) / at_once, 16);
+  l.per_group = (int)std::min<int64_t>(per_group, (batch_size + groups - 1) / groups);
+  l.tiles = (batch_size + l.per_group * groups - 1) / (l.per_group * groups);
+  return l;
+}
+
 // Grid and windows of every launch class for one call shape.
 static void compute_geometry(const tra_tbe* tbe, const Tuning& tune, bool balanced, bool nobag,
                              int32_t batch_size, int64_t num_indices, Geometry& g) {
@@ -606,6 +694,10 @@ static void compute_geometry(const tra_tbe* tbe, const Tuning& tune, bool balanc
   g.balanced = balanced ? 1 : 0;
   g.nobag = nobag ? 1 : 0;
   g.tune = tune;
+  if (!balanced && !nobag) {
+    g.group = group_windows(tbe, batch_size);
+    return;
+  }
   g.cls.assign(tbe->classes.size(), ClassGeometry());
   for (size_t ci = 0; ci < tbe->classes.size(); ++ci) {
     const LaunchClass& cls = tbe->classes[ci];
@@ -673,16 +765,13 @@ static void compute_geometry(const tra_tbe* tbe, const Tuning& tune, bool balanc
         sc.window = (int)(num_indices >= full * busy ? full : num_indices >= step * busy ? step : per_block);
         sc.tiles_per_feat = (int)std::min<int64_t>(num_indices / sc.window + sc.count, 1 << 20);
         grid += sc.tiles_per_feat;
-      } else if (balanced) {
+      } else {
         const int64_t nb = (int64_t)sc.count * batch_size;
         int64_t window = tune.window > 0 ? tune.window : (work_per_block + bag_cost(i) - 1) / bag_cost(i);
         window = std::max<int64_t>(64, std::min<int64_t>(window, kMaxWindow));
         sc.tiles_per_feat = 0;
         sc.window = (int)window;
         grid += (int)((nb + window - 1) / window);
-      } else {
-        sc.tiles_per_feat = (batch_size + per_block - 1) / per_block;
-        grid += sc.count * sc.tiles_per_feat;
       }
       i = j;
     }
@@ -778,7 +867,7 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
   {
     std::lock_guard<std::mutex> lock(tbe->geo_mutex);
     const int gen = g_ovr_gen.load(std::memory_order_relaxed);
-    const Tuning tune = choose_tuning(tbe->num_cus, (int64_t)tbe->num_features * batch_size, num_indices);
+    const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
     const int balanced = use_window_kernel(tbe, tune, nobag, batch_size) ? 1 : 0;
     const int64_t geo_indices = nobag ? quantized_id_count(num_indices) : num_indices;
     for (const auto& g : tbe->geo)
@@ -801,7 +890,7 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
   // A call of several launch classes runs them on two streams: the caller's stream forks into the
   // plan's second stream before the first launch and joins it after the last.  One call at a time
   // per plan enqueues such a sequence (the events are the plan's).  Not while the caller's stream
-  // is being captured, not for the small-batch kernel, not from the entry point that must not
+  // is being captured, not for the sixteen-lane kernel, not from the entry point that must not
   // allocate (an event's first record may), and `fork` = 0 (tuning) switches it off.
   bool forked = false;
   std::unique_lock<std::mutex> fork_lock(tbe->fork_mutex, std::defer_lock);
@@ -825,11 +914,8 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
     }
     return rc;
   };
-  for (const int ci : tbe->launch_order) {
-    s = forked && tbe->on_side[ci] ? tbe->side : caller_stream;
-    const LaunchClass& cls = tbe->classes[ci];
-    const ClassGeometry& cg = geo_local.cls[ci];
-    LookupArgs a = tbe->base_args[ci];
+  // What a call adds to the arguments of a launch of n features; key_of(i): the i-th one's key position.
+  auto fill = [&](LookupArgs& a, size_t n_features, auto&& key_of) -> int {
     a.weights = (const uint8_t*)weights;
     // Lanes past the end of their bag still issue (clamped) id loads, so the
     // kernels need one readable element even when there are no ids at all.
@@ -838,23 +924,23 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
     // (no ids: nothing to weigh, and the weights pointer may not be readable)
     a.psw = nobag || num_indices == 0 ? nullptr : per_sample_weights;
     if (pw != nullptr && !nobag && num_indices > 0) {
-      if (cls.feats.size() > (size_t)kMaxPos) {
+      if (tbe->max_class_feats > (size_t)kMaxPos) {
         set_error("position-weighted lookup: a launch class has %d features, at most %d are supported",
-                  (int)cls.feats.size(), kMaxPos);
-        return join(TRA_ERR_TOO_LARGE);
+                  (int)tbe->max_class_feats, kMaxPos);
+        return TRA_ERR_TOO_LARGE;
       }
-      for (size_t i = 0; i < cls.feats.size(); ++i) {
-        const int key = tbe->slices[cls.feats[i]].feature;
+      for (size_t i = 0; i < n_features; ++i) {
+        const int key = key_of(i);
         if (key < 0 || key >= pw->num_keys) {
           set_error("position-weighted lookup: feature at key position %d, but %d keys were described", key,
                     pw->num_keys);
-          return join(TRA_ERR_INVALID_ARGUMENT);
+          return TRA_ERR_INVALID_ARGUMENT;
         }
         const int64_t st = pw->key_start[key], n = pw->key_len[key];
         if (n < 0 || st < 0 || (n > 0 && st + n > pw->table_len)) {
           set_error("position-weighted lookup: key %d has weights [%lld, %lld) outside the table of %lld", key,
                     (long long)st, (long long)(st + n), (long long)pw->table_len);
-          return join(TRA_ERR_INVALID_ARGUMENT);
+          return TRA_ERR_INVALID_ARGUMENT;
         }
         a.pw_off[i] = (int32_t)st;
         a.pw_len[i] = (int32_t)n;
@@ -862,6 +948,66 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
       a.posw = pw->table;
       a.psw = nullptr;
     }
+    a.out = out;
+    a.out_stride = out_stride;
+    a.bad_to_row0 = tbe->bad_to_row0.load(std::memory_order_relaxed);
+    a.num_indices = num_indices > 0 ? num_indices : 1;
+    a.B = batch_size;
+    a.mean = pooling_mode == TRA_POOL_MEAN;
+    a.out_fp16 = out_dtype == TRA_FP16;
+    return TRA_OK;
+  };
+  auto vec_store = [&](const LaunchClass& cls) -> bool {
+    const int ne = cls.cb * 8 / bits_of(cls.dtype);
+    if ((uintptr_t)out % 16 != 0 || (int64_t)ne * esz % 16 != 0) return false;
+    if (nobag) return (int64_t)tbe->dim0 * esz % 16 == 0;
+    return out_stride * esz % 16 == 0 && (esz == 2 ? cls.cols_aligned_fp16 : cls.cols_aligned_fp32);
+  };
+  if (!balanced && !nobag) {
+    // (position weights: the launch arguments hold the layout of kMaxPos slices)
+    const size_t step = pw != nullptr && num_indices > 0 ? kMaxPos : tbe->group_slices.size();
+    for (size_t s0 = 0; s0 < tbe->group_slices.size(); s0 += step) {
+      const size_t n = std::min(step, tbe->group_slices.size() - s0);
+      const GroupSlice* slices = tbe->group_slices.data() + s0;
+      GroupArgs a;
+      a.common = tbe->group_base;
+      a.slices = tbe->group_slices_dev + s0;
+      const int rc = fill(a.common, n, [&](size_t i) { return slices[i].key; });
+      if (rc != TRA_OK) return rc;
+      GroupPositions p;
+      memcpy(p.off, a.common.pw_off, sizeof(p.off));
+      memcpy(p.len, a.common.pw_len, sizeof(p.len));
+      a.common.vec_store = (uintptr_t)out % 4 == 0 && out_stride % 2 == 0;
+      GroupLaunch l = geo_local.group;
+      l.grid = (int)n * l.tiles;
+      l.key0 = slices[0].key;
+      for (size_t i = 1; i < n; ++i)
+        if (slices[i].key != l.key0 + (int)i) {
+          l.key0 = -1;
+          break;
+        }
+      const auto go = [&](auto ids) {
+        using IdxT = decltype(ids);
+        if (a.common.posw != nullptr)
+          launch_group<IdxT, kByPosition>(a, p, l, from_lengths, s);
+        else if (a.common.psw != nullptr)
+          launch_group<IdxT, kPerSample>(a, p, l, from_lengths, s);
+        else
+          launch_group<IdxT, kUnweighted>(a, p, l, from_lengths, s);
+      };
+      if (idx_is_i64) go(int64_t()); else go(int32_t());
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return hip_fail(e, "tbe lookup launch");
+    }
+    return TRA_OK;
+  }
+  for (const int ci : tbe->launch_order) {
+    s = forked && tbe->on_side[ci] ? tbe->side : caller_stream;
+    const LaunchClass& cls = tbe->classes[ci];
+    const ClassGeometry& cg = geo_local.cls[ci];
+    LookupArgs a = tbe->base_args[ci];
+    const int filled = fill(a, cls.feats.size(), [&](size_t i) { return tbe->slices[cls.feats[i]].feature; });
+    if (filled != TRA_OK) return join(filled);
     a.bounds_kind = kBoundsOffsets;
     if (seq != nullptr) {
       a.num_keys = seq->num_keys;
@@ -873,27 +1019,12 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
         a.pw_len[i] = (int32_t)(seq->starts[key + 1] - seq->starts[key]);
       }
     }
-    a.out = out;
-    a.out_stride = out_stride;
-    a.bad_to_row0 = tbe->bad_to_row0.load(std::memory_order_relaxed);
-    a.num_indices = num_indices > 0 ? num_indices : 1;
-    a.B = batch_size;
-    a.mean = pooling_mode == TRA_POOL_MEAN;
-    a.out_fp16 = out_dtype == TRA_FP16;
-    const int ne = cls.cb * 8 / bits_of(cls.dtype);
-    bool vec = ((uintptr_t)out % 16 == 0) && ((int64_t)ne * esz % 16 == 0);
-    if (nobag) {
-      vec = vec && ((int64_t)tbe->dim0 * esz % 16 == 0);
-    } else {
-      vec = vec && (out_stride * esz % 16 == 0) && (esz == 2 ? cls.cols_aligned_fp16 : cls.cols_aligned_fp32);
-    }
-    a.vec_store = vec;
+    a.vec_store = vec_store(cls) ? 1 : 0;
     memcpy(a.sub, cg.sub, sizeof(a.sub));
     a.n_sub = cg.n_sub;
     a.xcd_blocks = cg.xcd_blocks;
     a.xcd_count = cg.xcd_count;
     LaunchParams lp;
-    lp.balanced = balanced ? 1 : 0;
     lp.lds_bytes = geo_local.tune.lds_bytes;
     lp.grid = cg.grid;
     lp.unroll = geo_local.tune.unroll;

@@ -43,7 +43,7 @@ __device__ __forceinline__ void store_row(float (&acc)[NE], const LookupArgs& a,
       return;
     }
   }
-  finish_bag<NE>(acc, a, 0, pos, c, lpr, lane, active);
+  finish_bag<NE>(acc, a, 0, pos, c, lpr, lane, active, a.vec_store != 0);
 }
 
 // A feature's ids are cut into tiles of sc.window consecutive ids; the tiles of
