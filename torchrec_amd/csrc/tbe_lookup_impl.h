@@ -1053,55 +1053,30 @@ __device__ __forceinline__ int feat_key_pos(const LookupArgs& a, const SubClass&
 
 constexpr int kNarrowLane = 8;  // accumulators per lane up to which one instance serves all widths (see odd_lanes)
 
-// FROM_LENGTHS: a.offsets points at the KJT's lengths instead of its offsets
+// A window's bags in LDS.
+template <typename IdxT>
+struct Window {
+  using Sum = typename SumOf<IdxT>::type;
+  int64_t start[kMaxWindow];
+  __align__(16) int len[kMaxWindow];
+  uint32_t ent[kMaxWindow];
+  uint16_t order[kMaxWindow];
+  uint16_t slot[kMaxWindow];
+  int hist[kLenBins];
+  FeatureDesc desc[kMaxWinFeat];
+  Sum red[kCuWaves];
+  Sum wave_tot[kCuWaves];
+};
+
+// Stages bags [q0, q0 + nb) of a sub-class and ranks them by length; returns what their starts in LDS still lack.
+// FROM_LENGTHS: p_offsets points at the KJT's lengths instead of its offsets
 // and the block derives its bags' start positions itself: one block-wide sum
 // of everything in front of the window plus a scan of the window in LDS.
-// ODD: the instance for launch classes of mostly odd lane groups (kOddInstance).
-template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, bool FROM_LENGTHS = false, bool ODD = false>
-__global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
-    const void* p_offsets, const FeatureDesc* p_cdescs, int32_t p_B, int32_t p_xcd_blocks,
-    int32_t p_xcd_count, int32_t p_n_sub, int32_t p_window0, int32_t p_count0, int32_t p_key0,
-    const LookupArgs a) {
-  constexpr int NE = CB * 8 / Traits<DTYPE>::kBits;
-  extern __shared__ unsigned char tra_dyn_smem[];  // only its size matters (one block per CU)
-  __shared__ int64_t s_start[kMaxWindow];
-  __shared__ __align__(16) int s_len[kMaxWindow];
-  __shared__ uint32_t s_ent[kMaxWindow];
-  __shared__ uint16_t s_order[kMaxWindow];
-  __shared__ uint16_t s_slot[kMaxWindow];
-  __shared__ int s_hist[kLenBins];
-  __shared__ FeatureDesc s_desc[kMaxWinFeat];
-
-  TRA_STAMP(0);
-  // Block -> (sub-class, window).  Consecutive windows go to the same XCD
-  // (blocks are dealt round-robin to the 8 XCDs), so each L2 sees few tables.
-  // The leading kernel parameters repeat what the first fetches need (the
-  // hardware preloads them into SGPRs): the block's bag bounds can be
-  // requested without waiting for the launch arguments to arrive from memory.
-  int blk = blockIdx.x;
-  if (p_xcd_blocks > 0) blk = (blk % p_xcd_count) * p_xcd_blocks + blk / p_xcd_count;
-  SubClass sc;
-  if (p_n_sub == 1) {
-    sc.first = 0;
-    sc.count = p_count0;
-    sc.lpr = a.sub[0].lpr;
-    sc.tiles_per_feat = 0;
-    sc.tile_start = 0;
-    sc.window = p_window0;
-    sc.key0 = p_key0;
-  } else {
-    int s = 0;
-#pragma unroll
-    for (int i = 1; i < kMaxSub; ++i)
-      if (i < a.n_sub && blk >= a.sub[i].tile_start) s = i;
-    sc = a.sub[s];
-  }
-  const int nb_all = sc.count * p_B;
-  const int q0 = (blk - sc.tile_start) * sc.window;
-  if (q0 >= nb_all) return;
-  const int nb = min(sc.window, nb_all - q0);
-
-  const int fi_lo = q0 / p_B;
+template <typename IdxT, bool FROM_LENGTHS>
+__device__ __forceinline__ typename SumOf<IdxT>::type stage_window(Window<IdxT>& w, const LookupArgs& a,
+                                                                   const void* p_offsets, const FeatureDesc* p_cdescs,
+                                                                   int32_t p_B, const SubClass& sc, int q0, int nb,
+                                                                   int fi_lo) {
   using Sum = typename SumOf<IdxT>::type;
 
   // Bag q0 + i of the window: where it sits in the offsets (or lengths) array.
@@ -1114,7 +1089,6 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
   // What a bag's start in LDS still lacks (from lengths, small windows: the sum
   // of everything in front of the window arrives last and is added on reading).
   Sum front_add = 0;
-  __shared__ Sum s_red[kCuWaves];
   // A window of at most 4 x 64 bags is staged, scanned and ranked by the
   // block's first wave alone, four consecutive bags per lane, with no block
   // barrier on the way; from lengths, the other fifteen waves meanwhile sum
@@ -1133,10 +1107,10 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
       }
       {
         const int nfeat = min((q0 + nb - 1) / p_B - fi_lo + 1, kMaxWinFeat);
-        if (ln < nfeat) s_desc[ln] = p_cdescs[sc.first + fi_lo + ln];
+        if (ln < nfeat) w.desc[ln] = p_cdescs[sc.first + fi_lo + ln];
       }
 #pragma unroll
-      for (int k = 0; k < kLenBins / kWaveSize; ++k) s_hist[ln + k * kWaveSize] = 0;
+      for (int k = 0; k < kLenBins / kWaveSize; ++k) w.hist[ln + k * kWaveSize] = 0;
       wave_lds_sync();
       TRA_STAMP(6);
       int len[4], slot[4];
@@ -1152,9 +1126,9 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
           // they are; a negative length only makes its own bag empty.
           raw[k] = (Sum)given[k];
           len[k] = (int)given[k];
-          s_len[i] = len[k];
-          s_ent[i] = ((uint32_t)fis[k] << kBagBits) | (uint32_t)bs[k];
-          slot[k] = atomicAdd(&s_hist[length_bin(len[k])], 1);
+          w.len[i] = len[k];
+          w.ent[i] = ((uint32_t)fis[k] << kBagBits) | (uint32_t)bs[k];
+          slot[k] = atomicAdd(&w.hist[length_bin(len[k])], 1);
         }
       }
       // Bag starts inside the window: exclusive scan in window order.
@@ -1162,10 +1136,10 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
       Sum run = wave_scan_incl(tot) - tot;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        if (4 * ln + k < nb) s_start[4 * ln + k] = (int64_t)run;
+        if (4 * ln + k < nb) w.start[4 * ln + k] = (int64_t)run;
         run += raw[k];
       }
-      if (ln == 0) s_red[0] = 0;
+      if (ln == 0) w.red[0] = 0;
       wave_lds_sync();
       TRA_STAMP(7);
       TRA_STAMP(1);
@@ -1174,32 +1148,32 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
         int sum = 0;
 #pragma unroll
         for (int k = 0; k < kLenBins / kWaveSize; ++k) {
-          h[k] = s_hist[kLenBins - 1 - (ln * (kLenBins / kWaveSize) + k)];
+          h[k] = w.hist[kLenBins - 1 - (ln * (kLenBins / kWaveSize) + k)];
           sum += h[k];
         }
         const int incl = wave_scan_incl((int32_t)sum);
         int base = incl - sum;
 #pragma unroll
         for (int k = 0; k < kLenBins / kWaveSize; ++k) {
-          s_hist[kLenBins - 1 - (ln * (kLenBins / kWaveSize) + k)] = base;
+          w.hist[kLenBins - 1 - (ln * (kLenBins / kWaveSize) + k)] = base;
           base += h[k];
         }
       }
       wave_lds_sync();
 #pragma unroll
       for (int k = 0; k < 4; ++k)
-        if (4 * ln + k < nb) s_order[s_hist[length_bin(len[k])] + slot[k]] = (uint16_t)(4 * ln + k);
+        if (4 * ln + k < nb) w.order[w.hist[length_bin(len[k])] + slot[k]] = (uint16_t)(4 * ln + k);
     } else {
       PrefixSumAtOnce<IdxT> front_sum;
       const Sum mine = front_sum.run(reinterpret_cast<const IdxT*>(p_offsets),
                                      (int64_t)feat_key_pos(a, sc, fi_lo) * p_B + (q0 - fi_lo * p_B),
                                      (int)threadIdx.x - kWaveSize, kCuThreads - kWaveSize);
       const Sum front_w = wave_last(wave_scan_incl(mine));
-      if (ln == 0) s_red[wv] = front_w;
+      if (ln == 0) w.red[wv] = front_w;
     }
     lds_barrier();
 #pragma unroll
-    for (int w = 0; w < kCuWaves; ++w) front_add += s_red[w];
+    for (int v = 0; v < kCuWaves; ++v) front_add += w.red[v];
     TRA_STAMP(2);
   } else {
     // The first bag of every thread is requested before anything else: the
@@ -1216,7 +1190,7 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
     // round does not start with two dependent global loads.
     {
       const int nfeat = min((q0 + nb - 1) / p_B - fi_lo + 1, kMaxWinFeat);
-      if ((int)threadIdx.x < nfeat) s_desc[threadIdx.x] = p_cdescs[sc.first + fi_lo + threadIdx.x];
+      if ((int)threadIdx.x < nfeat) w.desc[threadIdx.x] = p_cdescs[sc.first + fi_lo + threadIdx.x];
     }
     // From lengths: the total of everything in front of the window.  Its loads
     // go out after the window's own (loads return in order: whatever is waited
@@ -1226,7 +1200,7 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
     if (FROM_LENGTHS)
       front_sum.start(reinterpret_cast<const IdxT*>(p_offsets),
                       (int64_t)feat_key_pos(a, sc, fi_lo) * p_B + (q0 - fi_lo * p_B));
-    if (threadIdx.x < kLenBins) s_hist[threadIdx.x] = 0;
+    if (threadIdx.x < kLenBins) w.hist[threadIdx.x] = 0;
     lds_barrier();
     TRA_STAMP(6);
     for (int i = threadIdx.x; i < nb; i += kCuThreads) {
@@ -1242,17 +1216,16 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
       } else {
         const int64_t st = first ? (int64_t)first_lo : load_index<IdxT>(p_offsets, bag);
         const int64_t en = first ? (int64_t)first_hi : load_index<IdxT>(p_offsets, bag + 1);
-        s_start[i] = st;
+        w.start[i] = st;
         len = max(0, (int)(en - st));
       }
-      s_len[i] = len;
-      s_ent[i] = ((uint32_t)fi << kBagBits) | (uint32_t)b;
-      s_slot[i] = (uint16_t)atomicAdd(&s_hist[length_bin(len)], 1);
+      w.len[i] = len;
+      w.ent[i] = ((uint32_t)fi << kBagBits) | (uint32_t)b;
+      w.slot[i] = (uint16_t)atomicAdd(&w.hist[length_bin(len)], 1);
     }
     lds_barrier();
     TRA_STAMP(7);
     if (FROM_LENGTHS) {
-      __shared__ Sum s_wave_tot[kCuWaves];
       const int t = threadIdx.x;
       const int wv = t / kWaveSize;
       const int ln = t & (kWaveSize - 1);
@@ -1264,21 +1237,21 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
       const bool holds_bags = 2 * wv * kWaveSize < nb;
       Sum x0 = 0, x1 = 0, inc = 0;
       if (holds_bags) {
-        x0 = 2 * t < nb ? s_len[2 * t] : 0;
-        x1 = 2 * t + 1 < nb ? s_len[2 * t + 1] : 0;
+        x0 = 2 * t < nb ? w.len[2 * t] : 0;
+        x1 = 2 * t + 1 < nb ? w.len[2 * t + 1] : 0;
         inc = wave_scan_incl((Sum)(x0 + x1));
       }
       const Sum front_w = wave_last(wave_scan_incl(front_sum.finish()));
-      if (ln == kWaveSize - 1) s_wave_tot[wv] = inc;
-      if (ln == 0) s_red[wv] = front_w;
+      if (ln == kWaveSize - 1) w.wave_tot[wv] = inc;
+      if (ln == 0) w.red[wv] = front_w;
       lds_barrier();
       Sum before = 0, front = 0;
 #pragma unroll
-      for (int w = 0; w < kCuWaves; ++w) front += s_red[w];
+      for (int v = 0; v < kCuWaves; ++v) front += w.red[v];
       if (holds_bags) {
 #pragma unroll
-        for (int w = 0; w < kCuWaves; ++w)
-          if (w < wv) before += s_wave_tot[w];
+        for (int v = 0; v < kCuWaves; ++v)
+          if (v < wv) before += w.wave_tot[v];
       }
       const Sum excl = before + inc - (x0 + x1);
       // The window covers bags of features fi_lo .. fi_hi of the sub-class.  A
@@ -1289,15 +1262,15 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
       if (sc.key0 < 0)
         for (int fi = fi_lo; fi < fi_hi; ++fi) one_run = one_run && feat_key_pos(a, sc, fi + 1) == feat_key_pos(a, sc, fi) + 1;
       if (one_run) {
-        if (2 * t < nb) s_start[2 * t] = (int64_t)(front + excl);
-        if (2 * t + 1 < nb) s_start[2 * t + 1] = (int64_t)(front + excl + x0);
+        if (2 * t < nb) w.start[2 * t] = (int64_t)(front + excl);
+        if (2 * t + 1 < nb) w.start[2 * t + 1] = (int64_t)(front + excl + x0);
         lds_barrier();
       } else {
         // General case: keep the bare scan, then add to each run what lies in
         // front of it (summed again for every run that does not continue the
         // previous one).
-        if (2 * t < nb) s_start[2 * t] = (int64_t)excl;
-        if (2 * t + 1 < nb) s_start[2 * t + 1] = (int64_t)(excl + x0);
+        if (2 * t < nb) w.start[2 * t] = (int64_t)excl;
+        if (2 * t + 1 < nb) w.start[2 * t + 1] = (int64_t)(excl + x0);
         lds_barrier();
         int64_t adj = (int64_t)front;  // start = adj + scan value, for the current run
         int64_t next_pos = -1;
@@ -1309,16 +1282,16 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
             PrefixSum<IdxT> again;
             again.start(reinterpret_cast<const IdxT*>(p_offsets), pos);
             const Sum w_ = wave_last(wave_scan_incl(again.finish()));
-            if (ln == 0) s_red[wv] = w_;
+            if (ln == 0) w.red[wv] = w_;
             lds_barrier();
             Sum total = 0;
 #pragma unroll
-            for (int w = 0; w < kCuWaves; ++w) total += s_red[w];
-            adj = (int64_t)total - s_start[first];
+            for (int v = 0; v < kCuWaves; ++v) total += w.red[v];
+            adj = (int64_t)total - w.start[first];
           }
           next_pos = pos + (last - first);
-          lds_barrier();  // s_red and s_start[first] have been read by everyone
-          for (int i = first + t; i < last; i += kCuThreads) s_start[i] += adj;
+          lds_barrier();  // w.red and w.start[first] have been read by everyone
+          for (int i = first + t; i < last; i += kCuThreads) w.start[i] += adj;
           lds_barrier();
         }
       }
@@ -1333,24 +1306,37 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
       int sum = 0;
 #pragma unroll
       for (int k = 0; k < kLenBins / kWaveSize; ++k) {
-        h[k] = s_hist[kLenBins - 1 - (l * (kLenBins / kWaveSize) + k)];
+        h[k] = w.hist[kLenBins - 1 - (l * (kLenBins / kWaveSize) + k)];
         sum += h[k];
       }
       const int incl = wave_scan_incl((int32_t)sum);
       int base = incl - sum;
 #pragma unroll
       for (int k = 0; k < kLenBins / kWaveSize; ++k) {
-        s_hist[kLenBins - 1 - (l * (kLenBins / kWaveSize) + k)] = base;
+        w.hist[kLenBins - 1 - (l * (kLenBins / kWaveSize) + k)] = base;
         base += h[k];
       }
     }
     lds_barrier();
     for (int i = threadIdx.x; i < nb; i += kCuThreads)
-      s_order[s_hist[length_bin(s_len[i])] + s_slot[i]] = (uint16_t)i;
+      w.order[w.hist[length_bin(w.len[i])] + w.slot[i]] = (uint16_t)i;
     lds_barrier();
     TRA_STAMP(2);
   }
 
+  return front_add;
+}
+
+// Which pooling bodies a kernel instance holds (see odd_lanes).
+constexpr int kBodiesOdd = 1;   // id blocks of four for every lane group of four lanes or more
+constexpr int kBodiesEven = 0;  // id blocks for powers of two from eight lanes, for others where the registers allow
+
+// Pools a staged window.
+template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, int BODIES>
+__device__ __forceinline__ void pool_window(const Window<IdxT>& win, const LookupArgs& a, const SubClass& sc, int nb,
+                                            int fi_lo, typename SumOf<IdxT>::type front_add, bool vec) {
+  constexpr int NE = CB * 8 / Traits<DTYPE>::kBits;
+  constexpr bool ODD = BODIES == kBodiesOdd;
   const int lane = threadIdx.x & (kWaveSize - 1);
   const int wave = threadIdx.x / kWaveSize;
   const int lpr = sc.lpr;
@@ -1370,18 +1356,18 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
     if (r >= rounds) continue;
     const int pos = r * gpw + g;
     const bool active = g < gpw && pos < nb;
-    const int i = s_order[active ? pos : r * gpw];
-    const uint32_t ent = s_ent[i];
+    const int i = win.order[active ? pos : r * gpw];
+    const uint32_t ent = win.ent[i];
     const int fi = (int)(ent >> kBagBits);
     const int b = (int)(ent & ((1u << kBagBits) - 1));
-    const FeatureDesc d = fi - fi_lo < kMaxWinFeat ? s_desc[fi - fi_lo] : a.cdescs[sc.first + fi];
-    const int64_t start = s_start[i] + (int64_t)front_add;
-    const int len = active ? max(s_len[i], 0) : 0;
+    const FeatureDesc d = fi - fi_lo < kMaxWinFeat ? win.desc[fi - fi_lo] : a.cdescs[sc.first + fi];
+    const int64_t start = win.start[i] + (int64_t)front_add;
+    const int len = active ? max(win.len[i], 0) : 0;
     // The round's trip count.  Lengths below 192 have a sort bin each, so
     // the round's first bag is its longest; from 192 up a bin holds a range of
     // lengths in arrival order, and the longest of the round is found by
     // comparing what the lane groups actually hold.
-    int max_len = s_len[s_order[r * gpw]];
+    int max_len = win.len[win.order[r * gpw]];
     if (max_len >= 192) max_len = wave_max(len);
 
     RowWalk w;
@@ -1425,9 +1411,53 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
 #ifdef TRA_INSTRUMENT
     if (lane == 0) a.ts[((size_t)blockIdx.x * (blockDim.x / 64) + wave) * 8 + 5] = (unsigned long long)max_len;
 #endif
-    finish_bag<NE>(acc, a, len, (int64_t)b * a.out_stride + d.out_col, c, lpr, lane, active, a.vec_store != 0);
+    finish_bag<NE>(acc, a, len, (int64_t)b * a.out_stride + d.out_col, c, lpr, lane, active, vec);
     TRA_STAMP(4);
   }
+}
+
+// ODD: the instance for launch classes of mostly odd lane groups (kOddInstance).
+template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, bool FROM_LENGTHS = false, bool ODD = false>
+__global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
+    const void* p_offsets, const FeatureDesc* p_cdescs, int32_t p_B, int32_t p_xcd_blocks,
+    int32_t p_xcd_count, int32_t p_n_sub, int32_t p_window0, int32_t p_count0, int32_t p_key0,
+    const LookupArgs a) {
+  extern __shared__ unsigned char tra_dyn_smem[];  // only its size matters (one block per CU)
+  __shared__ Window<IdxT> s_window;
+
+  TRA_STAMP(0);
+  // Block -> (sub-class, window).  Consecutive windows go to the same XCD
+  // (blocks are dealt round-robin to the 8 XCDs), so each L2 sees few tables.
+  // The leading kernel parameters repeat what the first fetches need (the
+  // hardware preloads them into SGPRs): the block's bag bounds can be
+  // requested without waiting for the launch arguments to arrive from memory.
+  int blk = blockIdx.x;
+  if (p_xcd_blocks > 0) blk = (blk % p_xcd_count) * p_xcd_blocks + blk / p_xcd_count;
+  SubClass sc;
+  if (p_n_sub == 1) {
+    sc.first = 0;
+    sc.count = p_count0;
+    sc.lpr = a.sub[0].lpr;
+    sc.tiles_per_feat = 0;
+    sc.tile_start = 0;
+    sc.window = p_window0;
+    sc.key0 = p_key0;
+  } else {
+    int s = 0;
+#pragma unroll
+    for (int i = 1; i < kMaxSub; ++i)
+      if (i < a.n_sub && blk >= a.sub[i].tile_start) s = i;
+    sc = a.sub[s];
+  }
+  const int nb_all = sc.count * p_B;
+  const int q0 = (blk - sc.tile_start) * sc.window;
+  if (q0 >= nb_all) return;
+  const int nb = min(sc.window, nb_all - q0);
+
+  const int fi_lo = q0 / p_B;
+  const auto front_add = stage_window<IdxT, FROM_LENGTHS>(s_window, a, p_offsets, p_cdescs, p_B, sc, q0, nb, fi_lo);
+  pool_window<DTYPE, CB, IdxT, WEIGHTED, U, ODD ? kBodiesOdd : kBodiesEven>(s_window, a, sc, nb, fi_lo, front_add,
+                                                                             a.vec_store != 0);
 }
 
 // ---- host side of one launch ----------------------------------------------
@@ -1519,6 +1549,20 @@ struct GroupLaunch {
 template <typename IdxT, int WEIGHTED>
 void launch_group(const GroupArgs& a, const GroupPositions& p, const GroupLaunch& l, bool from_lengths,
                   hipStream_t stream);
+
+// Several launch classes in one launch of windows (tbe_multi_impl.h).
+constexpr int kMaxMultiSub = 16;
+constexpr int kMultiVec = 1;  // in a kind: every lane's output slice is 16-byte aligned
+constexpr int multi_kind(int dtype, int cb) { return dtype * 64 + cb * 2; }
+struct MultiArgs {
+  LookupArgs common;                 // (sub, n_sub and vec_store are not read)
+  int32_t tile_start[kMaxMultiSub];  // first block of every entry of sub; INT32_MAX behind the last one
+  int32_t kind[kMaxMultiSub];
+  SubClass sub[kMaxMultiSub];
+};
+static_assert(sizeof(MultiArgs) + 48 <= 4096, "launch arguments");
+template <typename IdxT, int WEIGHTED>
+void launch_multi(const MultiArgs& a, int grid, int lds_bytes, bool from_lengths, hipStream_t stream);
 
 // The sequence lookup of one class (tbe_sequence.hip).
 int launch_sequence(const LookupArgs& a, int dtype, int cb, bool split, bool idx64, int grid, hipStream_t stream);

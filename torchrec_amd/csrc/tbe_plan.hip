@@ -115,10 +115,10 @@ static Tuning choose_tuning(int num_cus, size_t classes, int64_t bags, int64_t n
   // replays of the whole call, us (sixteen-lane / window), ids a bag 3 and 20:
   //   one class (int8 dim 64): 8192 bags 5.3 / 5.3 and 9.0 / 9.1; 13 K bags of 2 ids 6.2 / 5.6; 33 K bags 13.8 / 6.9
   //   and 22.8 / 11.7
-  //   two classes (int8 dims 32 - 256): 33 K bags 16.7 / 17.2 and 34 / 30
-  //   seven classes: 33 K bags 16.5 / 32 and 34 / 58; 131 K bags 34 / 68 and 86 / 120 (such calls are not told apart
-  //   from hot ones with more ids, where the window kernel's two streams win; they keep the general rule)
-  t.balanced = bags >= 40 * (int64_t)num_cus && (classes <= 1 || num_indices >= 640 * (int64_t)num_cus);
+  //   two classes, one launch of windows: 8192 bags 6.9 / 8.8 and 14.3 / 17; 33 K bags 17 / 12.6 and 34 / 20
+  //   seven classes, one launch of windows: 8192 bags 6.7 / 7.3 and 14.1 / 15.4; 33 K bags 17 / 9 and 34 / 18
+  t.balanced = bags >= 40 * (int64_t)num_cus &&
+               (classes <= 1 || num_indices >= 640 * (int64_t)num_cus || bags >= 80 * (int64_t)num_cus);
   t.window = 0;
   t.unroll = 4;
   t.lds_bytes = 48 * 1024;  // with the static arrays > half of a CU's LDS: one block per CU
@@ -130,6 +130,20 @@ static Tuning choose_tuning(int num_cus, size_t classes, int64_t bags, int64_t n
   if (t.window < 0) t.window = 0;
   return t;
 }
+
+// ... and in tbe_multi_<id type>_<weight mode>.hip.
+template <>
+void launch_multi<int32_t, kUnweighted>(const MultiArgs&, int, int, bool, hipStream_t);
+template <>
+void launch_multi<int32_t, kPerSample>(const MultiArgs&, int, int, bool, hipStream_t);
+template <>
+void launch_multi<int32_t, kByPosition>(const MultiArgs&, int, int, bool, hipStream_t);
+template <>
+void launch_multi<int64_t, kUnweighted>(const MultiArgs&, int, int, bool, hipStream_t);
+template <>
+void launch_multi<int64_t, kPerSample>(const MultiArgs&, int, int, bool, hipStream_t);
+template <>
+void launch_multi<int64_t, kByPosition>(const MultiArgs&, int, int, bool, hipStream_t);
 
 }  // namespace tra
 
@@ -178,6 +192,15 @@ struct ClassGeometry {
   int xcd_count = 1;
 };
 
+// Launch geometry of all classes in one launch.
+struct MultiGeometry {
+  int n_sub = 0;
+  int grid = 0;
+  int xcd_blocks = 0;
+  int xcd_count = 1;
+  SubClass sub[kMaxMultiSub];
+};
+
 // What a plan remembers about a call shape it has seen: the route and, per
 // launch class, the grid and windows.  Recomputed when the tuning overrides change.
 struct Geometry {
@@ -188,6 +211,8 @@ struct Geometry {
   int gen = -1;
   Tuning tune{};
   std::vector<ClassGeometry> cls;
+  int multi = 0;
+  MultiGeometry all;     // balanced calls in one launch
   GroupLaunch group{};  // pooled calls that are not balanced: windows (the grid is per launch)
 };
 
@@ -226,6 +251,15 @@ struct tra_tbe {
   std::vector<uint8_t> on_side;      // per class index: 1 = launched on `side`
   std::vector<LaunchClass> classes;
   std::vector<LookupArgs> base_args;  // per class: everything a call does not change
+  // All slices for one launch of windows, where that can be (else empty): lane chunks of at most 16 accumulators,
+  // sorted by kind and lanes per row; at most kMaxPos of them, and kMaxMultiSub sub-classes.
+  std::vector<int32_t> multi_feats;
+  std::vector<int32_t> multi_lprs;
+  std::vector<int32_t> multi_kinds;
+  bool multi_aligned_fp16 = true;  // every slice's first output column is 16-byte aligned
+  bool multi_aligned_fp32 = true;
+  FeatureDesc* multi_descs_dev = nullptr;
+  LookupArgs multi_base;
   // Column slices for the sixteen-lane kernel, in feature order.
   std::vector<GroupSlice> group_slices;
   GroupSlice* group_slices_dev = nullptr;
@@ -484,6 +518,39 @@ int tra_tbe_create(const tra_table_spec* tables, int32_t num_tables,
       e = hipMemcpy(plan->cdescs_dev, ordered.data(), total * sizeof(FeatureDesc), hipMemcpyHostToDevice);
     }
   }
+  if (plan->classes.size() >= 2 && plan->slices.size() == (size_t)num_features && num_features <= kMaxPos) {
+    std::vector<std::tuple<int, int, int>> order;  // kind, lanes per row, slice
+    for (int f = 0; f < num_features; ++f) {
+      const FeatureDesc& d = plan->slices[f];
+      const int bits = bits_of(d.dtype), payload = d.dim * bits / 8;
+      // (the chunk of the classes, or less where a lane would hold more than 16 accumulators)
+      int cb = payload % 16 == 0 && payload > 64 ? 16 : payload % 8 == 0 ? 8 : 4;
+      cb = std::min(cb, 2 * bits);
+      order.emplace_back(multi_kind(d.dtype, cb), payload / cb, f);
+    }
+    std::stable_sort(order.begin(), order.end());
+    int subs = 0, widest = 0;
+    for (size_t i = 0; i < order.size(); ++i) {
+      subs += i == 0 || std::get<0>(order[i]) != std::get<0>(order[i - 1]) || std::get<1>(order[i]) != std::get<1>(order[i - 1]);
+      widest = std::max(widest, std::get<1>(order[i]));
+    }
+    if (subs <= kMaxMultiSub && widest <= kWaveSize)
+      for (const auto& o : order) {
+        const FeatureDesc& d = plan->slices[std::get<2>(o)];
+        plan->multi_kinds.push_back(std::get<0>(o));
+        plan->multi_lprs.push_back(std::get<1>(o));
+        plan->multi_feats.push_back(std::get<2>(o));
+        plan->multi_aligned_fp16 = plan->multi_aligned_fp16 && (int64_t)d.out_col * 2 % 16 == 0;
+        plan->multi_aligned_fp32 = plan->multi_aligned_fp32 && (int64_t)d.out_col * 4 % 16 == 0;
+      }
+  }
+  if (e == hipSuccess && !plan->multi_feats.empty()) {
+    std::vector<FeatureDesc> ordered;
+    for (int32_t id : plan->multi_feats) ordered.push_back(plan->slices[id]);
+    e = hipMalloc((void**)&plan->multi_descs_dev, ordered.size() * sizeof(FeatureDesc));
+    if (e == hipSuccess)
+      e = hipMemcpy(plan->multi_descs_dev, ordered.data(), ordered.size() * sizeof(FeatureDesc), hipMemcpyHostToDevice);
+  }
   if (e == hipSuccess && !plan->group_slices.empty()) {
     e = hipMalloc((void**)&plan->group_slices_dev, plan->group_slices.size() * sizeof(GroupSlice));
     if (e == hipSuccess)
@@ -514,6 +581,11 @@ int tra_tbe_create(const tra_table_spec* tables, int32_t num_tables,
       a.feat_pos[i] = (int16_t)plan->slices[cls.feats[i]].feature;
     plan->base_args.push_back(a);
   }
+  memset(&plan->multi_base, 0, sizeof(plan->multi_base));
+  plan->multi_base.cdescs = plan->multi_descs_dev;
+  plan->multi_base.err_count = plan->err_dev;
+  for (size_t i = 0; i < plan->multi_feats.size(); ++i)
+    plan->multi_base.feat_pos[i] = (int16_t)plan->slices[plan->multi_feats[i]].feature;
   memset(&plan->group_base, 0, sizeof(plan->group_base));
   plan->group_base.err_count = plan->err_dev;
   // Launch order and streams.  The launches of a call write disjoint output columns, so they may
@@ -558,6 +630,7 @@ int tra_tbe_destroy(tra_tbe_t tbe) {
   if (tbe->feats_dev) (void)hipFree(tbe->feats_dev);
   if (tbe->cdescs_dev) (void)hipFree(tbe->cdescs_dev);
   if (tbe->group_slices_dev) (void)hipFree(tbe->group_slices_dev);
+  if (tbe->multi_descs_dev) (void)hipFree(tbe->multi_descs_dev);
   if (tbe->err_dev) (void)hipFree(tbe->err_dev);
   if (tbe->side) (void)hipStreamDestroy(tbe->side);
   if (tbe->ev_join) (void)hipEventDestroy(tbe->ev_join);
@@ -575,8 +648,24 @@ static bool use_window_kernel(const tra_tbe* tbe, const Tuning& tune, bool nobag
          (int64_t)tbe->max_class_feats * batch_size < (int64_t(1) << 31);
 }
 
+// Whether a call of several launch classes that takes the window kernel does so in one launch (whatever the class, a
+// block is a window of bags; the launches' fixed costs, and a window of each class too small to fill its block, are
+// paid once).  Graph replays, us, a launch per class / one launch: two classes, 33 K bags of 20 ids 30 / 20, 131 K bags
+// of 20 85 / 66, 262 K bags of 30 hot ids 182 / 151, of cold ids 280 / 277; seven classes, 33 K bags of 20 95 / 20,
+// 131 K bags of 20 121 / 76, 262 K bags of 30 hot ids 199 / 152, of cold ids 306 / 309 in a graph and about 345 / 420
+// outside one.  So: always where there is no second stream, else up to 12,000 ids per compute unit.  From offsets
+// a plan with a second stream keeps it from 3750 on, the route that calls of that size are tested on.
+static bool use_one_launch(const tra_tbe* tbe, int32_t batch_size, int64_t num_indices, bool lengths_call) {
+  if (tbe->multi_feats.empty() || (int64_t)tbe->multi_feats.size() * batch_size >= (int64_t(1) << 31)) return false;
+  return tbe->side == nullptr || num_indices < (lengths_call ? 12000 : 3750) * (int64_t)tbe->num_cus;
+}
+
 // Largest number of features one window of the from-lengths kernel may span.
 constexpr int kMaxWindowFeatures = 32;
+
+// One launch for several classes derives its offsets itself up to as many lengths as one scan launch takes (its blocks
+// then sum 260 KB on average, about 4 us; the scan of more is two launches of 5 us each and the gaps).
+constexpr int64_t kOneLaunchMaxLengths = 131072;
 
 // Can a pooled call with these sizes take the window kernel in its
 // from-lengths form (which needs no offsets)?
@@ -594,6 +683,7 @@ static bool fused_scan_possible(const tra_tbe* tbe, int32_t batch_size, int32_t 
   // (about 1.3 us + 1 us per 40k lengths, measured); a separate scan costs
   // about 7 us once.  Take whichever is less.
   const int64_t n = (int64_t)num_keys * batch_size;
+  if (use_one_launch(tbe, batch_size, num_indices, true)) return n <= kOneLaunchMaxLengths;
   return (int64_t)tbe->classes.size() * (13 + n / 4000) < 70;
 }
 
@@ -629,15 +719,17 @@ int tra_tbe_launch_info(tra_tbe_t tbe, int32_t batch_size, int64_t num_indices,
                                                 (const void*)16));
   static const char* const kDtypeName[] = {"fp32", "fp16", "int8", "int4", "int2"};
   std::string text;
-  if (!nobag && !balanced) {
+  const bool multi = balanced && use_one_launch(tbe, batch_size, num_indices, lengths_num_keys > 0);
+  if (!nobag && (multi || !balanced)) {
     char line[120];
-    snprintf(line, sizeof(line), "tbe_pooled_kernel slices=%d%s", (int)tbe->group_slices.size(), fused ? " from_lengths" : "");
+    snprintf(line, sizeof(line), "%s slices=%d%s", multi ? "tbe_pooled_multi_kernel" : "tbe_pooled_kernel",
+             (int)(multi ? tbe->multi_feats.size() : tbe->group_slices.size()), fused ? " from_lengths" : "");
     text = line;
   }
   // In launch order; a plan with a second stream alternates between the two.
   const bool two_streams = tbe->side != nullptr && balanced && g_ovr.fork != 0;
   for (const int ci : tbe->launch_order) {
-    if (!nobag && !balanced) break;
+    if (!text.empty() && !nobag && (multi || !balanced)) break;
     const LaunchClass& cls = tbe->classes[ci];
     char line[200];
     snprintf(line, sizeof(line), "%s%s dtype=%s lane_bytes=%d slices=%d%s%s",
@@ -685,112 +777,153 @@ static GroupLaunch group_windows(const tra_tbe* tbe, int32_t batch_size) {
   return l;
 }
 
+}  // extern "C"
+
+// Windows (bags per block) of a launch's sub-classes.  Every block should get
+// about the same amount of work, so a sub-class's window shrinks with its row
+// width.  A row costs its payload bytes, but never less than 256: below that the
+// per-row requests (id, header, one line) dominate and rows of any width
+// take the same time.  Aim at one block per CU; more passes when a window
+// would not fit the kernel's LDS arrays.  Returns the grid.
+static int balance_windows(const Tuning& tune, int num_cus, int32_t batch_size, SubClass* sub, const int* row_cost,
+                           int n_sub) {
+  const int64_t cost_floor = g_ovr.cost_floor >= 0 ? g_ovr.cost_floor : 256;
+  auto bag_cost = [&](int i) { return std::max<int64_t>(row_cost[i], cost_floor); };
+  int64_t total = 0, min_cost = INT64_MAX;
+  for (int i = 0; i < n_sub; ++i) {
+    total += (int64_t)sub[i].count * batch_size * bag_cost(i);
+    min_cost = std::min(min_cost, bag_cost(i));
+  }
+  int64_t blocks = num_cus;
+  while ((total + blocks - 1) / blocks > (int64_t)kMaxWindow * min_cost) blocks += num_cus;
+  int64_t work_per_block = (total + blocks - 1) / blocks;
+  auto window_of = [&](int i) {
+    return std::max<int64_t>(64, std::min<int64_t>((work_per_block + bag_cost(i) - 1) / bag_cost(i), kMaxWindow));
+  };
+  // Rounding each sub-class up to whole windows must not spill a few
+  // blocks into an extra pass: grow the share until the grid fits.
+  for (int iter = 0; iter < 64; ++iter) {
+    int64_t grid = 0;
+    for (int i = 0; i < n_sub; ++i) grid += ((int64_t)sub[i].count * batch_size + window_of(i) - 1) / window_of(i);
+    if (grid <= blocks) break;
+    work_per_block += std::max<int64_t>(1, work_per_block / 128);
+  }
+  int grid = 0;
+  for (int i = 0; i < n_sub; ++i) {
+    const int64_t window = tune.window > 0 ? std::max<int64_t>(64, std::min<int64_t>(tune.window, kMaxWindow)) : window_of(i);
+    sub[i].tiles_per_feat = 0;
+    sub[i].window = (int)window;
+    sub[i].tile_start = grid;
+    grid += (int)(((int64_t)sub[i].count * batch_size + window - 1) / window);
+  }
+  return grid;
+}
+
+// Sub-classes of slices in launch order: runs of equal `same`.
+template <typename Same>
+static int cut_sub_classes(const tra_tbe* tbe, const std::vector<int32_t>& feats, const std::vector<int32_t>& lprs,
+                           Same&& same, SubClass* sub) {
+  int n = 0;
+  for (size_t i = 0; i < feats.size();) {
+    size_t j = i;
+    while (j < feats.size() && same(i, j)) ++j;
+    SubClass& sc = sub[n++];
+    sc = SubClass();
+    sc.first = (int)i;
+    sc.count = (int)(j - i);
+    sc.lpr = lprs[i];
+    sc.key0 = tbe->slices[feats[i]].feature;
+    for (size_t k = i; k < j; ++k)
+      if (tbe->slices[feats[k]].feature != sc.key0 + (int)(k - i)) sc.key0 = -1;
+    i = j;
+  }
+  return n;
+}
+
+// The XCD remap needs a grid that is a whole number of blocks per die
+// (surplus blocks exit at once).
+template <typename G>
+static void deal_to_dies(const tra_tbe* tbe, int grid, G& g) {
+  const int nx = tbe->num_xcd;
+  g.grid = (grid + nx - 1) / nx * nx;
+  g.xcd_count = 1;
+  g.xcd_blocks = 0;
+  if (nx > 1 && g_ovr.xcd != 0) {
+    g.xcd_blocks = g.grid / nx;
+    g.xcd_count = nx;
+  }
+}
+
 // Grid and windows of every launch class for one call shape.
-static void compute_geometry(const tra_tbe* tbe, const Tuning& tune, bool balanced, bool nobag,
+static void compute_geometry(const tra_tbe* tbe, const Tuning& tune, bool balanced, bool multi, bool nobag,
                              int32_t batch_size, int64_t num_indices, Geometry& g) {
   const int num_cus = tbe->num_cus;
   g.batch_size = batch_size;
   g.nobag_indices = nobag ? num_indices : -1;
   g.balanced = balanced ? 1 : 0;
   g.nobag = nobag ? 1 : 0;
+  g.multi = multi ? 1 : 0;
   g.tune = tune;
   if (!balanced && !nobag) {
     g.group = group_windows(tbe, batch_size);
+    return;
+  }
+  if (multi) {
+    MultiGeometry& mg = g.all;
+    const auto same = [&](size_t x, size_t y) {
+      return tbe->multi_kinds[x] == tbe->multi_kinds[y] && tbe->multi_lprs[x] == tbe->multi_lprs[y];
+    };
+    mg.n_sub = cut_sub_classes(tbe, tbe->multi_feats, tbe->multi_lprs, same, mg.sub);
+    int row_cost[kMaxMultiSub];
+    for (int i = 0; i < mg.n_sub; ++i) {
+      const FeatureDesc& d = tbe->slices[tbe->multi_feats[mg.sub[i].first]];
+      // A bag's share of a block: per row the requests (as above), and the issue slots of its lanes, about 25 and three
+      // per column that a lane holds.  (Bytes alone, us: two classes int8 dims 32 - 256, 33 K bags of 20 hot ids 28
+      // against 20; seven classes 29 against 20, 262 K bags of 30 248 against 152, of 30 cold ids 349 against 309.
+      // Half and twice the slots: 22.5 and 20.2, 21.4 and 21.2, 168 and 153, 365 and 334.)
+      row_cost[i] = 256 + mg.sub[i].lpr * 25 + 3 * d.dim;
+    }
+    deal_to_dies(tbe, balance_windows(tune, num_cus, batch_size, mg.sub, row_cost, mg.n_sub), mg);
     return;
   }
   g.cls.assign(tbe->classes.size(), ClassGeometry());
   for (size_t ci = 0; ci < tbe->classes.size(); ++ci) {
     const LaunchClass& cls = tbe->classes[ci];
     ClassGeometry& cg = g.cls[ci];
-    // Window kernel: every block should get about the same amount of work, so
-    // a sub-class's window (bags per block) shrinks with its row width.  A
-    // row costs its payload bytes, but never less than 256: below that the
-    // per-row requests (id, header, one line) dominate and rows of any width
-    // take the same time.  Aim at one block per CU; more passes when a window
-    // would not fit the kernel's LDS arrays.
-    const int64_t cost_floor = g_ovr.cost_floor >= 0 ? g_ovr.cost_floor : 256;
-    auto bag_cost = [&](size_t i) { return std::max<int64_t>((int64_t)cls.lprs[i] * cls.cb, cost_floor); };
-    int64_t work_per_block = 0;
+    cg.n_sub = cut_sub_classes(tbe, cls.feats, cls.lprs, [&](size_t x, size_t y) { return cls.lprs[x] == cls.lprs[y]; },
+                               cg.sub);
     if (balanced) {
-      int64_t total = 0, min_cost = INT64_MAX;
-      for (size_t i = 0; i < cls.feats.size(); ++i) {
-        total += (int64_t)batch_size * bag_cost(i);
-        min_cost = std::min(min_cost, bag_cost(i));
-      }
-      int64_t blocks = num_cus;
-      while ((total + blocks - 1) / blocks > (int64_t)kMaxWindow * min_cost) blocks += num_cus;
-      work_per_block = (total + blocks - 1) / blocks;
-      // Rounding each sub-class up to whole windows must not spill a few
-      // blocks into an extra pass: grow the share until the grid fits.
-      for (int iter = 0; iter < 64; ++iter) {
-        int64_t grid = 0;
-        for (size_t i = 0; i < cls.feats.size();) {
-          size_t j = i;
-          while (j < cls.feats.size() && cls.lprs[j] == cls.lprs[i]) ++j;
-          const int64_t w = std::max<int64_t>(
-              64, std::min<int64_t>((work_per_block + bag_cost(i) - 1) / bag_cost(i), kMaxWindow));
-          grid += ((int64_t)(j - i) * batch_size + w - 1) / w;
-          i = j;
-        }
-        if (grid <= blocks) break;
-        work_per_block += std::max<int64_t>(1, work_per_block / 128);
-      }
+      int row_bytes[kMaxSub];
+      for (int i = 0; i < cg.n_sub; ++i) row_bytes[i] = cg.sub[i].lpr * cls.cb;
+      deal_to_dies(tbe, balance_windows(tune, num_cus, batch_size, cg.sub, row_bytes, cg.n_sub), cg);
+      continue;
     }
     int grid = 0;
-    int n_sub = 0;
-    for (size_t i = 0; i < cls.feats.size();) {
-      size_t j = i;
-      while (j < cls.feats.size() && cls.lprs[j] == cls.lprs[i]) ++j;
-      SubClass& sc = cg.sub[n_sub++];
-      sc.first = (int)i;
-      sc.count = (int)(j - i);
-      sc.lpr = cls.lprs[i];
-      sc.key0 = tbe->slices[cls.feats[i]].feature;
-      for (size_t k = i; k < j; ++k)
-        if (tbe->slices[cls.feats[k]].feature != sc.key0 + (int)(k - i)) sc.key0 = -1;
-      const int gpw = kWaveSize / sc.lpr;
-      const int per_block = kWavesPerBlock * gpw;
+    for (int i = 0; i < cg.n_sub; ++i) {
+      SubClass& sc = cg.sub[i];
       sc.tile_start = grid;
-      if (nobag) {
-        // Ids per tile: one step of the kernel's loop (16 to 1024 ids, by the row width), at least
-        // 128 ids; less where that leaves fewer than two tiles per compute unit, down to one id
-        // per lane group.  2.1 M int8 rows of 128 columns: 128 ids a tile 187 us, 256 ids 195 us,
-        // 512 ids 197 us, 64 ids 201 us (8-byte lane chunks: 64 and 128 ids 187 us, 256 ids 197 us).
-        // One block per tile: all of the call's ids may belong to this sub-class, and every feature
-        // may leave a partial tile; blocks stride over the tiles if there are more.  No XCD
-        // remap: consecutive tiles on the same die measured 5 % slower.
-        const int64_t step = (int64_t)per_block * kSequenceUnroll;
-        const int64_t busy = 2 * (int64_t)num_cus;
-        const int64_t full = step >= 128 ? step : (128 + step - 1) / step * step;
-        sc.window = (int)(num_indices >= full * busy ? full : num_indices >= step * busy ? step : per_block);
-        sc.tiles_per_feat = (int)std::min<int64_t>(num_indices / sc.window + sc.count, 1 << 20);
-        grid += sc.tiles_per_feat;
-      } else {
-        const int64_t nb = (int64_t)sc.count * batch_size;
-        int64_t window = tune.window > 0 ? tune.window : (work_per_block + bag_cost(i) - 1) / bag_cost(i);
-        window = std::max<int64_t>(64, std::min<int64_t>(window, kMaxWindow));
-        sc.tiles_per_feat = 0;
-        sc.window = (int)window;
-        grid += (int)((nb + window - 1) / window);
-      }
-      i = j;
+      // Ids per tile: one step of the kernel's loop (16 to 1024 ids, by the row width), at least
+      // 128 ids; less where that leaves fewer than two tiles per compute unit, down to one id
+      // per lane group.  2.1 M int8 rows of 128 columns: 128 ids a tile 187 us, 256 ids 195 us,
+      // 512 ids 197 us, 64 ids 201 us (8-byte lane chunks: 64 and 128 ids 187 us, 256 ids 197 us).
+      // One block per tile: all of the call's ids may belong to this sub-class, and every feature
+      // may leave a partial tile; blocks stride over the tiles if there are more.  No XCD
+      // remap: consecutive tiles on the same die measured 5 % slower.
+      const int per_block = kWavesPerBlock * (kWaveSize / sc.lpr);
+      const int64_t step = (int64_t)per_block * kSequenceUnroll;
+      const int64_t busy = 2 * (int64_t)num_cus;
+      const int64_t full = step >= 128 ? step : (128 + step - 1) / step * step;
+      sc.window = (int)(num_indices >= full * busy ? full : num_indices >= step * busy ? step : per_block);
+      sc.tiles_per_feat = (int)std::min<int64_t>(num_indices / sc.window + sc.count, 1 << 20);
+      grid += sc.tiles_per_feat;
     }
-    cg.n_sub = n_sub;
     cg.grid = grid;
     cg.xcd_count = 1;
     cg.xcd_blocks = 0;
-    if (balanced) {
-      // The XCD remap needs a grid that is a whole number of blocks per die
-      // (surplus blocks exit at once).
-      const int nx = tbe->num_xcd;
-      cg.grid = (grid + nx - 1) / nx * nx;
-      if (nx > 1 && g_ovr.xcd != 0) {
-        cg.xcd_blocks = cg.grid / nx;
-        cg.xcd_count = nx;
-      }
-    }
   }
 }
+
+extern "C" {
 
 // The grid of a sequence lookup follows the number of ids, which differs from call to call in
 // service.  Geometries are kept per id count rounded up to a step of an eighth of its power of
@@ -809,7 +942,7 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
                         const float* per_sample_weights, int32_t batch_size, int64_t num_indices,
                         int32_t pooling_mode, int32_t out_dtype, void* out, int64_t out_stride,
                         void* stream, const PositionWeights* pw = nullptr, bool one_stream = false,
-                        const SequenceBounds* seq = nullptr) {
+                        const SequenceBounds* seq = nullptr, bool lengths_call = false) {
   if (!tbe) {
     set_error("tra_tbe_forward: null plan");
     return TRA_ERR_INVALID_ARGUMENT;
@@ -869,16 +1002,17 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
     const int gen = g_ovr_gen.load(std::memory_order_relaxed);
     const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
     const int balanced = use_window_kernel(tbe, tune, nobag, batch_size) ? 1 : 0;
+    const int multi = balanced && use_one_launch(tbe, batch_size, num_indices, lengths_call || from_lengths) ? 1 : 0;
     const int64_t geo_indices = nobag ? quantized_id_count(num_indices) : num_indices;
     for (const auto& g : tbe->geo)
       if (g && g->batch_size == batch_size && g->gen == gen && g->balanced == balanced &&
-          g->nobag == (int)nobag && (!nobag || g->nobag_indices == geo_indices)) {
+          g->multi == multi && g->nobag == (int)nobag && (!nobag || g->nobag_indices == geo_indices)) {
         geo = g;
         break;
       }
     if (!geo) {
       auto g = std::make_shared<Geometry>();
-      compute_geometry(tbe, tune, balanced != 0, nobag, batch_size, geo_indices, *g);
+      compute_geometry(tbe, tune, balanced != 0, multi != 0, nobag, batch_size, geo_indices, *g);
       g->gen = gen;
       geo = g;
       tbe->geo[tbe->geo_next] = geo;  // a call still launching from the replaced entry keeps it alive
@@ -894,7 +1028,7 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
   // allocate (an event's first record may), and `fork` = 0 (tuning) switches it off.
   bool forked = false;
   std::unique_lock<std::mutex> fork_lock(tbe->fork_mutex, std::defer_lock);
-  if (tbe->side != nullptr && balanced && !one_stream && g_ovr.fork != 0) {
+  if (tbe->side != nullptr && balanced && !geo_local.multi && !one_stream && g_ovr.fork != 0) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
       fork_lock.lock();
@@ -1000,6 +1134,39 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
       if (e != hipSuccess) return hip_fail(e, "tbe lookup launch");
     }
     return TRA_OK;
+  }
+  if (geo_local.multi) {
+    const MultiGeometry& mg = geo_local.all;
+    MultiArgs m;
+    LookupArgs& a = m.common;
+    a = tbe->multi_base;
+    const int rc = fill(a, tbe->multi_feats.size(), [&](size_t i) { return tbe->slices[tbe->multi_feats[i]].feature; });
+    if (rc != TRA_OK) return rc;
+    a.xcd_blocks = mg.xcd_blocks;
+    a.xcd_count = mg.xcd_count;
+    const bool aligned = (uintptr_t)out % 16 == 0 && out_stride * esz % 16 == 0 &&
+                         (esz == 2 ? tbe->multi_aligned_fp16 : tbe->multi_aligned_fp32);
+    for (int i = 0; i < kMaxMultiSub; ++i) {
+      m.tile_start[i] = i < mg.n_sub ? mg.sub[i].tile_start : INT32_MAX;
+      m.kind[i] = 0;
+      if (i >= mg.n_sub) continue;
+      m.sub[i] = mg.sub[i];
+      const FeatureDesc& d = tbe->slices[tbe->multi_feats[mg.sub[i].first]];
+      const bool vec = aligned && d.dim / mg.sub[i].lpr * esz % 16 == 0;
+      m.kind[i] = tbe->multi_kinds[mg.sub[i].first] | (vec ? kMultiVec : 0);
+    }
+    const auto go = [&](auto ids) {
+      using IdxT = decltype(ids);
+      if (a.posw != nullptr)
+        launch_multi<IdxT, kByPosition>(m, mg.grid, geo_local.tune.lds_bytes, from_lengths, s);
+      else if (a.psw != nullptr)
+        launch_multi<IdxT, kPerSample>(m, mg.grid, geo_local.tune.lds_bytes, from_lengths, s);
+      else
+        launch_multi<IdxT, kUnweighted>(m, mg.grid, geo_local.tune.lds_bytes, from_lengths, s);
+    };
+    if (idx_is_i64) go(int64_t()); else go(int32_t());
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? TRA_OK : hip_fail(e, "tbe lookup launch");
   }
   for (const int ci : tbe->launch_order) {
     s = forked && tbe->on_side[ci] ? tbe->side : caller_stream;
@@ -1149,8 +1316,8 @@ static int forward_lengths_impl(tra_tbe_t tbe, const void* weights, const void* 
   void* scan_ws = tra_cumsum_workspace_bytes(n) ? (void*)((uint8_t*)workspace + off_bytes) : nullptr;
   const int rc = tra_cumsum(lengths, n, idx_is_i64, workspace, scan_ws, stream);
   if (rc != TRA_OK) return rc;
-  return forward_impl(tbe, weights, indices, workspace, false, idx_is_i64, per_sample_weights,
-                      batch_size, num_indices, pooling_mode, out_dtype, out, out_stride, stream, pw, one_stream);
+  return forward_impl(tbe, weights, indices, workspace, false, idx_is_i64, per_sample_weights, batch_size, num_indices,
+                      pooling_mode, out_dtype, out, out_stride, stream, pw, one_stream, nullptr, /*lengths_call=*/true);
 }
 
 extern "C" {
