@@ -438,6 +438,22 @@ def test_bucketize_tiles(F, B, W, max_len, idt, weighted, keep):
         assert np.array_equal(buckets.cpu().numpy(), q)
 
 
+@pytest.mark.parametrize("F,B,W,max_len", [(16, 1000, 8, 40), (2, 10_000, 3, 2), (3, 50, 4, 9)])
+@pytest.mark.parametrize("idt", [np.int32, np.int64])
+def test_bucketize_launches(F, B, W, max_len, idt):
+    """Few lengths and many tiles (three launches), many lengths and few tiles (three), both few (two; four launches
+    from lengths that are not 16-byte aligned): against numpy, and the same from aligned and unaligned lengths."""
+    test_bucketize_tiles(F, B, W, max_len, idt, True, False)
+    rng = np.random.default_rng(B)
+    lengths = torch.from_numpy(rng.integers(0, max_len + 1, F * B + 1).astype(idt)).to(DEV)
+    shifted, whole = lengths[1:], lengths[1:].clone()
+    assert shifted.data_ptr() % 16 != 0 and whole.data_ptr() % 16 == 0
+    ids = torch.from_numpy(rng.integers(0, 4000, int(whole.sum())).astype(idt)).to(DEV)
+    bs = torch.full((F,), 1000, dtype=torch.int64, device=DEV)
+    for a, b in zip(*(ops.block_bucketize_sparse_features(x, ids, False, True, bs, W) for x in (shifted, whole))):
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+
+
 @pytest.mark.parametrize("W", [1, 8, 64])
 @pytest.mark.parametrize("idt", [np.int32, np.int64])
 @pytest.mark.parametrize("kind", ["in one tile", "across tiles", "before the ids", "behind the ids"])

@@ -7,6 +7,10 @@
 //   bucket_counts ids per (bucket, bag) = the new lengths, and per (bucket, tile)
 //   bucket_scan   where each tile's ids of each bucket go; bucket totals to the host
 //   bucket_move   the ids to their place
+// Calls of few lengths leave the first out (every block of bucket_counts adds up
+// the lengths in front of its tile), calls of few tiles the third (every block
+// of bucket_move adds up the counts): two launches where the launches themselves
+// are most of the call.
 // Lengths that are no partition of the ids (a negative one, or more in a tile
 // than there are ids) are found by the first launch; no id is moved then, and
 // every total that reaches the host is -1.
@@ -54,7 +58,11 @@ struct BucketArgs {
   int32_t bits;           // W <= 1 << bits
   int32_t lanes;          // bucket_counts: lanes per bag (a power of two)
   int32_t keep;
+  int32_t own_prefix;     // bucket_counts: no tile totals yet, from the lengths
+  int32_t own_scan;       // bucket_move: no places yet, from the counts
 };
+constexpr int kBktOwnLengths = 16384;  // lengths up to which bucket_counts sums them itself
+constexpr int kBktOwnCounts = 4096;    // tiles * buckets up to which bucket_move adds the counts itself
 
 // q = id / bs, r = id % bs of unsigned ids for one block size.  Below 2^32:
 // id * floor(2^32 / bs) / 2^32 is the quotient or one less.
@@ -135,8 +143,8 @@ __global__ __launch_bounds__(kBktThreads) void bucket_counts_kernel(const Bucket
   extern __shared__ int bkt_smem[];
   int* s_end = bkt_smem;           // [bags] ids up to and including the bag
   int* s_cnt = bkt_smem + a.bags;  // [W][bags]
-  __shared__ int64_t s_sum[kBktWaves];
-  __shared__ int s_wave[kBktWaves];
+  __shared__ int64_t s_sum[kBktWaves], s_own[kBktWaves];
+  __shared__ int s_wave[kBktWaves], s_bad[kBktWaves];
   const int lane = threadIdx.x & (kWaveSize - 1);
   const int wave = threadIdx.x / kWaveSize;
   const int tile = blockIdx.x;
@@ -145,10 +153,29 @@ __global__ __launch_bounds__(kBktThreads) void bucket_counts_kernel(const Bucket
   // the bags' ends: two bags per thread
   const T* lengths = reinterpret_cast<const T*>(a.lengths) + bag;
   const int i0 = 2 * threadIdx.x;
-  const int l0 = i0 < cnt ? (int)lengths[i0] : 0, l1 = i0 + 1 < cnt ? (int)lengths[i0 + 1] : 0;
+  const int64_t g0 = i0 < cnt ? (int64_t)lengths[i0] : 0, g1 = i0 + 1 < cnt ? (int64_t)lengths[i0 + 1] : 0;
+  const int l0 = (int)g0, l1 = (int)g1;
   // ids in front of the tile: 16 bytes per load, four loads in flight
   int64_t before = 0;
-  {
+  if (a.own_prefix) {
+    constexpr int V = 16 / (int)sizeof(T);
+    struct __align__(16) Vec { T v[V]; };
+    const Vec* v = reinterpret_cast<const Vec*>(a.lengths);
+    const int nv = (int)(bag / V);
+    for (int u0 = threadIdx.x; u0 < nv; u0 += 4 * kBktThreads) {
+      Vec x[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x[k] = v[min(u0 + k * kBktThreads, nv - 1)];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        int64_t sum = 0;
+#pragma unroll
+        for (int i = 0; i < V; ++i) sum += (int64_t)x[k].v[i];
+        before += u0 + k * kBktThreads < nv ? sum : 0;
+      }
+    }
+    if (V * nv + (int64_t)threadIdx.x < bag) before += (int64_t) reinterpret_cast<const T*>(a.lengths)[V * nv + threadIdx.x];
+  } else {
     const i32x4_t* v = reinterpret_cast<const i32x4_t*>(a.tile_total);
     const int nv = tile / 4;
     for (int u0 = threadIdx.x; u0 < nv; u0 += 4 * kBktThreads) {
@@ -164,23 +191,42 @@ __global__ __launch_bounds__(kBktThreads) void bucket_counts_kernel(const Bucket
   for (int x = threadIdx.x; x < a.bags * a.W; x += kBktThreads) s_cnt[x] = 0;
   const int incl = wave_scan32(l0 + l1, lane);
   before = wave_sum64(before);
+  if (a.own_prefix) {
+    const bool odd = g0 < 0 || g0 > a.num_indices || g1 < 0 || g1 > a.num_indices;
+    const int64_t own = wave_sum64(g0 + g1);
+    const bool any = __builtin_amdgcn_ballot_w64(odd) != 0;
+    if (lane == 0) {
+      s_own[wave] = own;
+      s_bad[wave] = any;
+    }
+  }
   if (lane == kWaveSize - 1) s_wave[wave] = incl;
   if (lane == 0) s_sum[wave] = before;
   __syncthreads();
   int front = 0, total = 0;
+  int64_t own = 0;
+  bool odd = false;
   before = 0;
 #pragma unroll
   for (int w = 0; w < kBktWaves; ++w) {
     front += w < wave ? s_wave[w] : 0;
     total += s_wave[w];
     before += s_sum[w];
+    if (a.own_prefix) {
+      own += s_own[w];
+      odd = odd || s_bad[w] != 0;
+    }
   }
+  const int tile_total = !a.own_prefix ? a.tile_total[tile] : odd || own > a.num_indices ? -1 : (int)own;
   if (i0 < cnt) s_end[i0] = front + incl - l1;
   if (i0 + 1 < cnt) s_end[i0 + 1] = front + incl;
-  if (threadIdx.x == 0) a.tile_first[tile] = before;
+  if (threadIdx.x == 0) {
+    a.tile_first[tile] = before;
+    if (a.own_prefix) a.tile_total[tile] = tile_total;
+  }
   __syncthreads();
   // (never outside the ids array, whatever the lengths say; the bags' ends are no places where the lengths are bad)
-  const bool bad = a.tile_total[tile] < 0;
+  const bool bad = tile_total < 0;
   const int ids = before < 0 ? 0 : (int)max(min((int64_t)total, a.num_indices - before), (int64_t)0);
   const T* in = reinterpret_cast<const T*>(a.indices) + before;
   const Divider div((uint64_t)a.block_sizes[tile / a.per_feature]);
@@ -281,24 +327,48 @@ __global__ __launch_bounds__(kBktThreads) void bucket_move_kernel(const BucketAr
   __shared__ int s_from[kBktWaves][kBktMax];  // place in the step of the wave's first id of a bucket
   __shared__ int s_start[kBktMax];            // place in the step of a bucket's first id
   __shared__ int64_t s_to[kBktMax];           // output position of the bucket's next id
+  __shared__ int64_t s_all[kBktMax];
   const int lane = threadIdx.x & (kWaveSize - 1);
   const int wave = threadIdx.x / kWaveSize;
   const int tile = blockIdx.x;
-  if (a.bucket_total[0] < 0) return;  // (bad lengths)
+  if (a.own_scan) {
+    // The buckets' totals, and their ids in the tiles in front of this one: a wave takes every fourth bucket.
+    int bad = 0;
+    for (int p = wave; p < a.W; p += kBktWaves) {
+      int64_t in_front = 0, all = 0;
+      for (int t = lane; t < a.tiles; t += kWaveSize) {
+        const int c = a.counts[(int64_t)p * a.tiles + t];
+        bad |= c < 0;
+        all += c;
+        in_front += t < tile ? c : 0;
+      }
+      all = wave_sum64(all);
+      in_front = wave_sum64(in_front);
+      if (lane == 0) {
+        s_all[p] = all;
+        s_to[p] = in_front;
+      }
+    }
+    bad = __syncthreads_or(bad);
+    if (tile == 0 && (int)threadIdx.x < a.W) publish_total(bad ? -1 : s_all[threadIdx.x], a.host_totals + threadIdx.x);
+    if (bad) return;  // (bad lengths)
+  } else if (a.bucket_total[0] < 0) {
+    return;
+  }
   const int64_t first = a.tile_first[tile];
   const int ids = first < 0 ? 0 : (int)max(min((int64_t)a.tile_total[tile], a.num_indices - first), (int64_t)0);
   if (ids == 0) return;
   const Divider div((uint64_t)a.block_sizes[tile / a.per_feature]);
   if (wave == 0) {
     // buckets in front of this one, and its ids in the tiles in front
-    const int64_t total = lane < a.W ? a.bucket_total[lane] : 0;
+    const int64_t total = lane >= a.W ? 0 : a.own_scan ? s_all[lane] : a.bucket_total[lane];
     int64_t incl = total;
 #pragma unroll
     for (int off = 1; off < kWaveSize; off <<= 1) {
       const int64_t o = __shfl_up(incl, off, 64);
       if (lane >= off) incl += o;
     }
-    if (lane < a.W) s_to[lane] = incl - total + a.place[(int64_t)lane * a.tiles + tile];
+    if (lane < a.W) s_to[lane] = incl - total + (a.own_scan ? s_to[lane] : a.place[(int64_t)lane * a.tiles + tile]);
   }
   const T* in = reinterpret_cast<const T*>(a.indices) + first;
   const float* win = a.weights + first;
@@ -488,6 +558,9 @@ int tra_bucketize_ids(const void* lengths, const void* indices, int32_t is_i64, 
   while ((1 << a.bits) < num_buckets) ++a.bits;
   a.lanes = 1;
   while (a.lanes < kWaveSize && 8 * a.lanes * a.n < num_indices) a.lanes *= 2;  // an average bag in two steps of four
+  // (calls, us, four launches / two: 5 keys x 133 bags, 1.3 K ids, 2 buckets 46 / 38; 52 x 29, 44 K ids, 3 buckets 61 / 52)
+  a.own_prefix = a.n <= kBktOwnLengths && (uintptr_t)lengths % 16 == 0;
+  a.own_scan = num_indices > 0 && z.tiles * num_buckets <= kBktOwnCounts;
   const int rc = mail_open(s, num_buckets, ticket, &a.host_totals);
   if (rc != TRA_OK) return rc;
   const dim3 block(kBktThreads), tiles((unsigned)z.tiles), waves((unsigned)((z.tiles + kBktWaves - 1) / kBktWaves));
@@ -496,13 +569,13 @@ int tra_bucketize_ids(const void* lengths, const void* indices, int32_t is_i64, 
   };
   const size_t counters = (size_t)z.bags * (num_buckets + 1) * sizeof(int);
   if (is_i64) {
-    go(tile_totals_kernel<int64_t>, waves, block);
+    if (!a.own_prefix) go(tile_totals_kernel<int64_t>, waves, block);
     go(bucket_counts_kernel<int64_t>, tiles, block, counters);
   } else {
-    go(tile_totals_kernel<int32_t>, waves, block);
+    if (!a.own_prefix) go(tile_totals_kernel<int32_t>, waves, block);
     go(bucket_counts_kernel<int32_t>, tiles, block, counters);
   }
-  go(bucket_scan_kernel, dim3(num_buckets), dim3(kBktScanThreads));
+  if (!a.own_scan) go(bucket_scan_kernel, dim3(num_buckets), dim3(kBktScanThreads));
   if (num_indices > 0) {
     if (is_i64 && weights)
       go(bucket_move_kernel<int64_t, true>, tiles, block);
