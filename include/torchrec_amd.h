@@ -69,7 +69,7 @@ const char* tra_last_error(void);
 int tra_device_arch(char* buf, int buf_len);
 
 /* Tuning override for experiments and tests: name is one of "balanced" (1:
- * window kernel, 0: static kernel), "window" (bags per block), "unroll", "lds",
+ * window kernel, 0: sixteen-lane kernel), "window" (bags per block), "unroll", "lds",
  * "xcd" (0: no remap of blocks to dies), "cost_floor", "fused_scan" (from-lengths
  * prologue inside the lookup kernel: 1 always, 0 never), "cb" (lane chunk bytes,
  * acts on plans created afterwards), "fork" (0: the launches of a call of five
@@ -125,10 +125,11 @@ int tra_tbe_destroy(tra_tbe_t tbe);
  * tra_tbe_set_bounds_check_mode asked for that.  Every buffer sits at a multiple
  * of its element size (weights: 4 bytes), else TRA_ERR_INVALID_ARGUMENT.
  * Ordering: everything the call launches runs after what `stream` holds at the
- * call and before what is put on `stream` afterwards.  A plan of five or more
- * launch classes (weight type x lane chunk) runs every other launch on a second
- * stream of its own, forked from and joined to `stream` with events inside the
- * call; not while `stream` is being captured into a graph. */
+ * call and before what is put on `stream` afterwards.  Where a call of five or
+ * more launch classes (weight type x lane chunk) is too large for one launch
+ * (tra_tbe_launch_info), it runs every other launch on a second stream of the
+ * plan's own, forked from and joined to `stream` with events inside the call;
+ * not while `stream` is being captured into a graph. */
 int tra_tbe_forward(tra_tbe_t tbe, const void* weights, const void* indices,
                     const void* offsets, int32_t idx_is_i64,
                     const float* per_sample_weights, int32_t batch_size,

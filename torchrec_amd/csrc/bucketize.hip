@@ -58,8 +58,6 @@ struct BucketArgs {
   int32_t bits;           // W <= 1 << bits
   int32_t lanes;          // bucket_counts: lanes per bag (a power of two)
   int32_t keep;
-  int32_t own_prefix;     // bucket_counts: no tile totals yet, from the lengths
-  int32_t own_scan;       // bucket_move: no places yet, from the counts
 };
 constexpr int kBktOwnLengths = 16384;  // lengths up to which bucket_counts sums them itself
 constexpr int kBktOwnCounts = 4096;    // tiles * buckets up to which bucket_move adds the counts itself
@@ -137,14 +135,14 @@ __global__ __launch_bounds__(kBktThreads) void tile_totals_kernel(const BucketAr
 // walked by a.lanes lanes, four ids per lane in flight.  (Walking the tile's ids
 // in order and looking each id's bag up in LDS took 48 us where this takes
 // 19 us: 7.9 M ids in 64 x 4096 bags.)
-template <typename T>
+template <typename T, bool OWN_PREFIX>
 __global__ __launch_bounds__(kBktThreads) void bucket_counts_kernel(const BucketArgs a) {
   // (sized by the launch: with room for the largest tile only four blocks fit a compute unit)
   extern __shared__ int bkt_smem[];
   int* s_end = bkt_smem;           // [bags] ids up to and including the bag
   int* s_cnt = bkt_smem + a.bags;  // [W][bags]
-  __shared__ int64_t s_sum[kBktWaves], s_own[kBktWaves];
-  __shared__ int s_wave[kBktWaves], s_bad[kBktWaves];
+  __shared__ int64_t s_sum[kBktWaves], s_own[OWN_PREFIX ? kBktWaves : 1];
+  __shared__ int s_wave[kBktWaves], s_bad[OWN_PREFIX ? kBktWaves : 1];
   const int lane = threadIdx.x & (kWaveSize - 1);
   const int wave = threadIdx.x / kWaveSize;
   const int tile = blockIdx.x;
@@ -153,11 +151,11 @@ __global__ __launch_bounds__(kBktThreads) void bucket_counts_kernel(const Bucket
   // the bags' ends: two bags per thread
   const T* lengths = reinterpret_cast<const T*>(a.lengths) + bag;
   const int i0 = 2 * threadIdx.x;
-  const int64_t g0 = i0 < cnt ? (int64_t)lengths[i0] : 0, g1 = i0 + 1 < cnt ? (int64_t)lengths[i0 + 1] : 0;
+  const T g0 = i0 < cnt ? lengths[i0] : (T)0, g1 = i0 + 1 < cnt ? lengths[i0 + 1] : (T)0;
   const int l0 = (int)g0, l1 = (int)g1;
   // ids in front of the tile: 16 bytes per load, four loads in flight
   int64_t before = 0;
-  if (a.own_prefix) {
+  if constexpr (OWN_PREFIX) {
     constexpr int V = 16 / (int)sizeof(T);
     struct __align__(16) Vec { T v[V]; };
     const Vec* v = reinterpret_cast<const Vec*>(a.lengths);
@@ -191,9 +189,9 @@ __global__ __launch_bounds__(kBktThreads) void bucket_counts_kernel(const Bucket
   for (int x = threadIdx.x; x < a.bags * a.W; x += kBktThreads) s_cnt[x] = 0;
   const int incl = wave_scan32(l0 + l1, lane);
   before = wave_sum64(before);
-  if (a.own_prefix) {
-    const bool odd = g0 < 0 || g0 > a.num_indices || g1 < 0 || g1 > a.num_indices;
-    const int64_t own = wave_sum64(g0 + g1);
+  if constexpr (OWN_PREFIX) {
+    const bool odd = g0 < 0 || (int64_t)g0 > a.num_indices || g1 < 0 || (int64_t)g1 > a.num_indices;
+    const int64_t own = wave_sum64((int64_t)g0 + (int64_t)g1);
     const bool any = __builtin_amdgcn_ballot_w64(odd) != 0;
     if (lane == 0) {
       s_own[wave] = own;
@@ -212,21 +210,21 @@ __global__ __launch_bounds__(kBktThreads) void bucket_counts_kernel(const Bucket
     front += w < wave ? s_wave[w] : 0;
     total += s_wave[w];
     before += s_sum[w];
-    if (a.own_prefix) {
+    if constexpr (OWN_PREFIX) {
       own += s_own[w];
       odd = odd || s_bad[w] != 0;
     }
   }
-  const int tile_total = !a.own_prefix ? a.tile_total[tile] : odd || own > a.num_indices ? -1 : (int)own;
+  const int tile_total = OWN_PREFIX && (odd || own > a.num_indices) ? -1 : (int)own;
   if (i0 < cnt) s_end[i0] = front + incl - l1;
   if (i0 + 1 < cnt) s_end[i0 + 1] = front + incl;
   if (threadIdx.x == 0) {
     a.tile_first[tile] = before;
-    if (a.own_prefix) a.tile_total[tile] = tile_total;
+    if constexpr (OWN_PREFIX) a.tile_total[tile] = tile_total;
   }
   __syncthreads();
   // (never outside the ids array, whatever the lengths say; the bags' ends are no places where the lengths are bad)
-  const bool bad = tile_total < 0;
+  const bool bad = (OWN_PREFIX ? tile_total : a.tile_total[tile]) < 0;
   const int ids = before < 0 ? 0 : (int)max(min((int64_t)total, a.num_indices - before), (int64_t)0);
   const T* in = reinterpret_cast<const T*>(a.indices) + before;
   const Divider div((uint64_t)a.block_sizes[tile / a.per_feature]);
@@ -318,7 +316,7 @@ __global__ __launch_bounds__(kBktScanThreads) void bucket_scan_kernel(const Buck
 // leave in runs of a bucket instead of one by one: 38 us for the ids and weights
 // above, 188 MB at the rate of a copy (84 us when every wave stored its ids one
 // by one behind cursors per bucket and bag).
-template <typename T, bool WEIGHTED>
+template <typename T, bool WEIGHTED, bool OWN_SCAN>
 __global__ __launch_bounds__(kBktThreads) void bucket_move_kernel(const BucketArgs a) {
   __shared__ T s_val[kBktStep];
   __shared__ float s_w[WEIGHTED ? kBktStep : 1];
@@ -327,11 +325,11 @@ __global__ __launch_bounds__(kBktThreads) void bucket_move_kernel(const BucketAr
   __shared__ int s_from[kBktWaves][kBktMax];  // place in the step of the wave's first id of a bucket
   __shared__ int s_start[kBktMax];            // place in the step of a bucket's first id
   __shared__ int64_t s_to[kBktMax];           // output position of the bucket's next id
-  __shared__ int64_t s_all[kBktMax];
+  __shared__ int64_t s_all[OWN_SCAN ? kBktMax : 1];
   const int lane = threadIdx.x & (kWaveSize - 1);
   const int wave = threadIdx.x / kWaveSize;
   const int tile = blockIdx.x;
-  if (a.own_scan) {
+  if constexpr (OWN_SCAN) {
     // The buckets' totals, and their ids in the tiles in front of this one: a wave takes every fourth bucket.
     int bad = 0;
     for (int p = wave; p < a.W; p += kBktWaves) {
@@ -352,8 +350,8 @@ __global__ __launch_bounds__(kBktThreads) void bucket_move_kernel(const BucketAr
     bad = __syncthreads_or(bad);
     if (tile == 0 && (int)threadIdx.x < a.W) publish_total(bad ? -1 : s_all[threadIdx.x], a.host_totals + threadIdx.x);
     if (bad) return;  // (bad lengths)
-  } else if (a.bucket_total[0] < 0) {
-    return;
+  } else {
+    if (a.bucket_total[0] < 0) return;  // (bad lengths)
   }
   const int64_t first = a.tile_first[tile];
   const int ids = first < 0 ? 0 : (int)max(min((int64_t)a.tile_total[tile], a.num_indices - first), (int64_t)0);
@@ -361,14 +359,14 @@ __global__ __launch_bounds__(kBktThreads) void bucket_move_kernel(const BucketAr
   const Divider div((uint64_t)a.block_sizes[tile / a.per_feature]);
   if (wave == 0) {
     // buckets in front of this one, and its ids in the tiles in front
-    const int64_t total = lane >= a.W ? 0 : a.own_scan ? s_all[lane] : a.bucket_total[lane];
+    const int64_t total = lane >= a.W ? 0 : OWN_SCAN ? s_all[lane] : a.bucket_total[lane];
     int64_t incl = total;
 #pragma unroll
     for (int off = 1; off < kWaveSize; off <<= 1) {
       const int64_t o = __shfl_up(incl, off, 64);
       if (lane >= off) incl += o;
     }
-    if (lane < a.W) s_to[lane] = incl - total + (a.own_scan ? s_to[lane] : a.place[(int64_t)lane * a.tiles + tile]);
+    if (lane < a.W) s_to[lane] = incl - total + (OWN_SCAN ? s_to[lane] : a.place[(int64_t)lane * a.tiles + tile]);
   }
   const T* in = reinterpret_cast<const T*>(a.indices) + first;
   const float* win = a.weights + first;
@@ -559,8 +557,9 @@ int tra_bucketize_ids(const void* lengths, const void* indices, int32_t is_i64, 
   a.lanes = 1;
   while (a.lanes < kWaveSize && 8 * a.lanes * a.n < num_indices) a.lanes *= 2;  // an average bag in two steps of four
   // (calls, us, four launches / two: 5 keys x 133 bags, 1.3 K ids, 2 buckets 46 / 38; 52 x 29, 44 K ids, 3 buckets 61 / 52)
-  a.own_prefix = a.n <= kBktOwnLengths && (uintptr_t)lengths % 16 == 0;
-  a.own_scan = num_indices > 0 && z.tiles * num_buckets <= kBktOwnCounts;
+  // (instances of their own: the branches alone cost the large calls 3 %)
+  const bool own_prefix = a.n <= kBktOwnLengths && (uintptr_t)lengths % 16 == 0;
+  const bool own_scan = num_indices > 0 && z.tiles * num_buckets <= kBktOwnCounts;
   const int rc = mail_open(s, num_buckets, ticket, &a.host_totals);
   if (rc != TRA_OK) return rc;
   const dim3 block(kBktThreads), tiles((unsigned)z.tiles), waves((unsigned)((z.tiles + kBktWaves - 1) / kBktWaves));
@@ -568,24 +567,26 @@ int tra_bucketize_ids(const void* lengths, const void* indices, int32_t is_i64, 
     hipLaunchKernelGGL(kernel, grid, threads, lds, s, a);
   };
   const size_t counters = (size_t)z.bags * (num_buckets + 1) * sizeof(int);
-  if (is_i64) {
-    if (!a.own_prefix) go(tile_totals_kernel<int64_t>, waves, block);
-    go(bucket_counts_kernel<int64_t>, tiles, block, counters);
-  } else {
-    if (!a.own_prefix) go(tile_totals_kernel<int32_t>, waves, block);
-    go(bucket_counts_kernel<int32_t>, tiles, block, counters);
-  }
-  if (!a.own_scan) go(bucket_scan_kernel, dim3(num_buckets), dim3(kBktScanThreads));
-  if (num_indices > 0) {
-    if (is_i64 && weights)
-      go(bucket_move_kernel<int64_t, true>, tiles, block);
-    else if (is_i64)
-      go(bucket_move_kernel<int64_t, false>, tiles, block);
+  const auto launch = [&](auto id) {
+    using T = decltype(id);
+    if (own_prefix) {
+      go(bucket_counts_kernel<T, true>, tiles, block, counters);
+    } else {
+      go(tile_totals_kernel<T>, waves, block);
+      go(bucket_counts_kernel<T, false>, tiles, block, counters);
+    }
+    if (!own_scan) go(bucket_scan_kernel, dim3(num_buckets), dim3(kBktScanThreads));
+    if (num_indices == 0) return;
+    if (weights && own_scan)
+      go(bucket_move_kernel<T, true, true>, tiles, block);
     else if (weights)
-      go(bucket_move_kernel<int32_t, true>, tiles, block);
+      go(bucket_move_kernel<T, true, false>, tiles, block);
+    else if (own_scan)
+      go(bucket_move_kernel<T, false, true>, tiles, block);
     else
-      go(bucket_move_kernel<int32_t, false>, tiles, block);
-  }
+      go(bucket_move_kernel<T, false, false>, tiles, block);
+  };
+  if (is_i64) launch(int64_t()); else launch(int32_t());
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     // (the scan may have been queued: its slot is not given back)

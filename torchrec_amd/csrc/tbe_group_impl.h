@@ -112,7 +112,7 @@ __device__ __forceinline__ void for_each_row(std::integer_sequence<int, I...>, F
 // MODE: kNear, kFar (the table's rows lie beyond the reach of 32-bit offsets) or kSplit (the slice is not its row's
 // only one: the header does not lie in front of it).
 template <int DTYPE, int NE, typename IdxT, int WEIGHTED, int MODE>
-__device__ __forceinline__ void pool_group_bags(const LookupArgs& a, const GroupSlice& d, const float* pw,
+__device__ __forceinline__ void pool_group_bags(const GroupArgs& a, const GroupSlice& d, const float* pw,
                                                 int pw_len, const int64_t* s_start, const int* s_len, int bag0,
                                                 int first, int count, int lane) {
   using Cols = Columns<DTYPE, NE>;
@@ -142,7 +142,7 @@ __device__ __forceinline__ void pool_group_bags(const LookupArgs& a, const Group
   const int64_t out_row = a.out_stride * elem;
   uint8_t* const out =
       reinterpret_cast<uint8_t*>(a.out) + (int64_t)(bag0 + first) * out_row + (int64_t)(d.out_col + c * NE) * elem;
-  const bool pairs = d.even != 0 && a.vec_store != 0;
+  const bool pairs = d.even != 0 && a.pairs != 0;
   auto store = [&](int b, const float (&acc)[NE]) {
     if (!has_cols) return;
     uint8_t* o = out + b * out_row;
@@ -358,8 +358,7 @@ __device__ __forceinline__ void pool_group_bags(const LookupArgs& a, const Group
 template <typename IdxT, int WEIGHTED, bool FROM_LENGTHS>
 __global__ __launch_bounds__(kBlockThreads, 4) void tbe_pooled_kernel(
     const void* p_bags, const GroupSlice* p_slices, int32_t p_B, int32_t p_per_group, int32_t p_tiles, int32_t p_key0,
-    const GroupArgs args, const GroupPositions positions) {
-  const LookupArgs& a = args.common;
+    const GroupArgs a, const std::conditional_t<WEIGHTED == kByPosition, GroupPositions, NoPositions> positions) {
   constexpr int kGroups = kBlockThreads / kGroup;
   __shared__ int64_t s_start[kBlockThreads];
   __shared__ int s_len[kBlockThreads];
@@ -437,16 +436,21 @@ __global__ __launch_bounds__(kBlockThreads, 4) void tbe_pooled_kernel(
 #undef TRA_GROUP
 }
 
+template <int WEIGHTED>
+auto positions_of(const GroupPositions* p) {
+  if constexpr (WEIGHTED == kByPosition) return *p; else return NoPositions();
+}
+
 #define TRA_DEFINE_GROUP(T, W)                                                                                \
   template <>                                                                                                 \
-  void launch_group<T, W>(const GroupArgs& a, const GroupPositions& p, const GroupLaunch& l, bool from_lengths, \
+  void launch_group<T, W>(const GroupArgs& a, const GroupPositions* p, const GroupLaunch& l, bool from_lengths, \
                           hipStream_t stream) {                                                               \
-    if (from_lengths)                                                                                         \
-      hipLaunchKernelGGL((tbe_pooled_kernel<T, W, true>), dim3(l.grid), dim3(kBlockThreads), 0, stream,       \
-                         a.common.offsets, a.slices, a.common.B, l.per_group, l.tiles, l.key0, a, p);           \
-    else                                                                                                      \
-      hipLaunchKernelGGL((tbe_pooled_kernel<T, W, false>), dim3(l.grid), dim3(kBlockThreads), 0, stream,      \
-                         a.common.offsets, a.slices, a.common.B, l.per_group, l.tiles, l.key0, a, p);           \
+    const auto positions = positions_of<W>(p);                                                                \
+    const auto go = [&](auto kernel) {                                                                        \
+      hipLaunchKernelGGL(kernel, dim3(l.grid), dim3(kBlockThreads), 0, stream, a.offsets, a.slices, a.B,      \
+                         l.per_group, l.tiles, l.key0, a, positions);                                         \
+    };                                                                                                        \
+    if (from_lengths) go(tbe_pooled_kernel<T, W, true>); else go(tbe_pooled_kernel<T, W, false>);             \
   }
 
 }  // namespace tra

@@ -1053,27 +1053,38 @@ __device__ __forceinline__ int feat_key_pos(const LookupArgs& a, const SubClass&
 
 constexpr int kNarrowLane = 8;  // accumulators per lane up to which one instance serves all widths (see odd_lanes)
 
-// A window's bags in LDS.
+// A window's bags in LDS, in arrays of their own (so that the compiler can tell
+// accesses to one from accesses to another).
 template <typename IdxT>
 struct Window {
   using Sum = typename SumOf<IdxT>::type;
-  int64_t start[kMaxWindow];
-  __align__(16) int len[kMaxWindow];
-  uint32_t ent[kMaxWindow];
-  uint16_t order[kMaxWindow];
-  uint16_t slot[kMaxWindow];
-  int hist[kLenBins];
-  FeatureDesc desc[kMaxWinFeat];
-  Sum red[kCuWaves];
-  Sum wave_tot[kCuWaves];
+  int64_t* start;
+  int* len;
+  uint32_t* ent;
+  uint16_t* order;
+  uint16_t* slot;
+  int* hist;
+  FeatureDesc* desc;
+  Sum* red;
+  Sum* wave_tot;
 };
+#define TRA_WINDOW(IdxT, name)                                                                       \
+  __shared__ int64_t s_start[kMaxWindow];                                                            \
+  __shared__ __align__(16) int s_len[kMaxWindow];                                                    \
+  __shared__ uint32_t s_ent[kMaxWindow];                                                             \
+  __shared__ uint16_t s_order[kMaxWindow];                                                           \
+  __shared__ uint16_t s_slot[kMaxWindow];                                                            \
+  __shared__ int s_hist[kLenBins];                                                                   \
+  __shared__ FeatureDesc s_desc[kMaxWinFeat];                                                        \
+  __shared__ typename SumOf<IdxT>::type s_red[kCuWaves], s_wave_tot[kCuWaves];                       \
+  const Window<IdxT> name{s_start, s_len, s_ent, s_order, s_slot, s_hist, s_desc, s_red, s_wave_tot}
 
 // Stages bags [q0, q0 + nb) of a sub-class and ranks them by length; returns what their starts in LDS still lack.
 // FROM_LENGTHS: p_offsets points at the KJT's lengths instead of its offsets
 // and the block derives its bags' start positions itself: one block-wide sum
 // of everything in front of the window plus a scan of the window in LDS.
 template <typename IdxT, bool FROM_LENGTHS>
-__device__ __forceinline__ typename SumOf<IdxT>::type stage_window(Window<IdxT>& w, const LookupArgs& a,
+__device__ __forceinline__ typename SumOf<IdxT>::type stage_window(const Window<IdxT> w, const LookupArgs& a,
                                                                    const void* p_offsets, const FeatureDesc* p_cdescs,
                                                                    int32_t p_B, const SubClass& sc, int q0, int nb,
                                                                    int fi_lo) {
@@ -1333,7 +1344,7 @@ constexpr int kBodiesEven = 0;  // id blocks for powers of two from eight lanes,
 
 // Pools a staged window.
 template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, int BODIES>
-__device__ __forceinline__ void pool_window(const Window<IdxT>& win, const LookupArgs& a, const SubClass& sc, int nb,
+__device__ __forceinline__ void pool_window(const Window<IdxT> win, const LookupArgs& a, const SubClass& sc, int nb,
                                             int fi_lo, typename SumOf<IdxT>::type front_add, bool vec) {
   constexpr int NE = CB * 8 / Traits<DTYPE>::kBits;
   constexpr bool ODD = BODIES == kBodiesOdd;
@@ -1423,7 +1434,7 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
     int32_t p_xcd_count, int32_t p_n_sub, int32_t p_window0, int32_t p_count0, int32_t p_key0,
     const LookupArgs a) {
   extern __shared__ unsigned char tra_dyn_smem[];  // only its size matters (one block per CU)
-  __shared__ Window<IdxT> s_window;
+  TRA_WINDOW(IdxT, s_window);
 
   TRA_STAMP(0);
   // Block -> (sub-class, window).  Consecutive windows go to the same XCD
@@ -1526,18 +1537,32 @@ constexpr int kNear = 0;   // 32-bit offsets, header in front of the columns (or
 constexpr int kFar = 1;    // a table beyond 4 GiB
 constexpr int kSplit = 2;  // one of several slices of a row with a header
 constexpr int group_kind(int dtype, int ne, int mode) { return (dtype * 4 + mode) * 32 + ne; }
+// What a launch needs and no more: the launch arguments are written over the bus for every call, and a small call's
+// time is its launch (with the window kernel's arguments, 3.0 KB, the entry point takes 4.2 us of the host's time, with
+// these 3.5; two boxes, evened out by the time of torch.empty).
 struct GroupArgs {
-  LookupArgs common;  // (descriptors, sub, n_sub, pw_off, pw_len and the sequence lookup's fields are not read;
-                      //  vec_store: two fp16 results of an even column make an aligned dword)
+  const uint8_t* weights;
   const GroupSlice* slices;
+  const void* indices;
+  const void* offsets;
+  const float* psw;
+  const float* posw;
+  void* out;
+  int64_t out_stride;  // elements
+  unsigned long long* err_count;
+  int64_t num_indices;
+  int32_t B;
+  uint8_t mean;
+  uint8_t out_fp16;
+  uint8_t pairs;        // two fp16 results of an even column make an aligned dword
+  uint8_t bad_to_row0;  // as in LookupArgs
 };
-// Position weights of the launch's slices, as in LookupArgs (a parameter of its own: indexed at run time, it has to
-// stay apart from what the kernel's functions take by reference).
+// Position weights of the launch's slices, as in LookupArgs.
 struct GroupPositions {
   int32_t off[kMaxPos];
   int32_t len[kMaxPos];
 };
-static_assert(sizeof(GroupArgs) + sizeof(GroupPositions) + 48 <= 4096, "launch arguments");
+struct NoPositions {};
 struct GroupLaunch {
   int grid;
   int per_group;  // bags per lane group (at most 16)
@@ -1547,7 +1572,7 @@ struct GroupLaunch {
 
 // Pooled lookup, all weight types in one launch (tbe_group_impl.h).
 template <typename IdxT, int WEIGHTED>
-void launch_group(const GroupArgs& a, const GroupPositions& p, const GroupLaunch& l, bool from_lengths,
+void launch_group(const GroupArgs& a, const GroupPositions* p, const GroupLaunch& l, bool from_lengths,
                   hipStream_t stream);
 
 // Several launch classes in one launch of windows (tbe_multi_impl.h).

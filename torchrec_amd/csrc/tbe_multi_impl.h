@@ -14,7 +14,7 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_multi_kernel(const void
                                                                       int32_t p_B, int32_t p_xcd_blocks,
                                                                       int32_t p_xcd_count, const MultiArgs m) {
   extern __shared__ unsigned char tra_dyn_smem[];  // only its size matters (one block per CU)
-  __shared__ Window<IdxT> s_window;
+  TRA_WINDOW(IdxT, s_window);
   const LookupArgs& a = m.common;
   int blk = blockIdx.x;
   if (p_xcd_blocks > 0) blk = (blk % p_xcd_count) * p_xcd_blocks + blk / p_xcd_count;

@@ -48,17 +48,17 @@ template <>
 int launch_lookup<TRA_FP32>(const LookupArgs&, int, const LaunchParams&, hipStream_t);
 // ... and in tbe_group_<id type>_<weight mode>.hip.
 template <>
-void launch_group<int32_t, kUnweighted>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
+void launch_group<int32_t, kUnweighted>(const GroupArgs&, const GroupPositions*, const GroupLaunch&, bool, hipStream_t);
 template <>
-void launch_group<int32_t, kPerSample>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
+void launch_group<int32_t, kPerSample>(const GroupArgs&, const GroupPositions*, const GroupLaunch&, bool, hipStream_t);
 template <>
-void launch_group<int32_t, kByPosition>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
+void launch_group<int32_t, kByPosition>(const GroupArgs&, const GroupPositions*, const GroupLaunch&, bool, hipStream_t);
 template <>
-void launch_group<int64_t, kUnweighted>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
+void launch_group<int64_t, kUnweighted>(const GroupArgs&, const GroupPositions*, const GroupLaunch&, bool, hipStream_t);
 template <>
-void launch_group<int64_t, kPerSample>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
+void launch_group<int64_t, kPerSample>(const GroupArgs&, const GroupPositions*, const GroupLaunch&, bool, hipStream_t);
 template <>
-void launch_group<int64_t, kByPosition>(const GroupArgs&, const GroupPositions&, const GroupLaunch&, bool, hipStream_t);
+void launch_group<int64_t, kByPosition>(const GroupArgs&, const GroupPositions*, const GroupLaunch&, bool, hipStream_t);
 
 // Launch shape of the pooled kernels.  Defaults are chosen from the problem
 // size when a plan first sees a (batch size, route) pair and are remembered in
@@ -263,7 +263,6 @@ struct tra_tbe {
   // Column slices for the sixteen-lane kernel, in feature order.
   std::vector<GroupSlice> group_slices;
   GroupSlice* group_slices_dev = nullptr;
-  LookupArgs group_base;  // everything a call does not change
   std::mutex geo_mutex;
   std::shared_ptr<const Geometry> geo[kGeometrySlots];
   int geo_next = 0;
@@ -586,8 +585,6 @@ int tra_tbe_create(const tra_table_spec* tables, int32_t num_tables,
   plan->multi_base.err_count = plan->err_dev;
   for (size_t i = 0; i < plan->multi_feats.size(); ++i)
     plan->multi_base.feat_pos[i] = (int16_t)plan->slices[plan->multi_feats[i]].feature;
-  memset(&plan->group_base, 0, sizeof(plan->group_base));
-  plan->group_base.err_count = plan->err_dev;
   // Launch order and streams.  The launches of a call write disjoint output columns, so they may
   // overlap.  A launch leaves compute units idle before its first rows arrive and while its last
   // blocks finish; with consecutive launches on alternating streams the next launch's blocks fill
@@ -1048,39 +1045,46 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
     }
     return rc;
   };
-  // What a call adds to the arguments of a launch of n features; key_of(i): the i-th one's key position.
+  const bool positions = pw != nullptr && !nobag && num_indices > 0;
+  // Where the position weights of a launch's n features lie; key_of(i): the i-th one's key position.
+  auto fill_positions = [&](int32_t* off, int32_t* len, size_t n_features, auto&& key_of) -> int {
+    if (tbe->max_class_feats > (size_t)kMaxPos) {
+      set_error("position-weighted lookup: a launch class has %d features, at most %d are supported",
+                (int)tbe->max_class_feats, kMaxPos);
+      return TRA_ERR_TOO_LARGE;
+    }
+    for (size_t i = 0; i < n_features; ++i) {
+      const int key = key_of(i);
+      if (key < 0 || key >= pw->num_keys) {
+        set_error("position-weighted lookup: feature at key position %d, but %d keys were described", key, pw->num_keys);
+        return TRA_ERR_INVALID_ARGUMENT;
+      }
+      const int64_t st = pw->key_start[key], n = pw->key_len[key];
+      if (n < 0 || st < 0 || (n > 0 && st + n > pw->table_len)) {
+        set_error("position-weighted lookup: key %d has weights [%lld, %lld) outside the table of %lld", key,
+                  (long long)st, (long long)(st + n), (long long)pw->table_len);
+        return TRA_ERR_INVALID_ARGUMENT;
+      }
+      off[i] = (int32_t)st;
+      len[i] = (int32_t)n;
+    }
+    return TRA_OK;
+  };
+  // Lanes past the end of their bag still issue (clamped) id loads, so the
+  // kernels need one readable element even when there are no ids at all.
+  const void* const readable_ids = num_indices > 0 ? indices : (const void*)tbe->err_dev;
+  // (no ids: nothing to weigh, and the weights pointer may not be readable)
+  const float* const psw = nobag || num_indices == 0 || positions ? nullptr : per_sample_weights;
+  // What a call adds to the arguments of a window or sequence launch of n features.
   auto fill = [&](LookupArgs& a, size_t n_features, auto&& key_of) -> int {
     a.weights = (const uint8_t*)weights;
-    // Lanes past the end of their bag still issue (clamped) id loads, so the
-    // kernels need one readable element even when there are no ids at all.
-    a.indices = num_indices > 0 ? indices : (const void*)tbe->err_dev;
+    a.indices = readable_ids;
     a.offsets = offsets;
-    // (no ids: nothing to weigh, and the weights pointer may not be readable)
-    a.psw = nobag || num_indices == 0 ? nullptr : per_sample_weights;
-    if (pw != nullptr && !nobag && num_indices > 0) {
-      if (tbe->max_class_feats > (size_t)kMaxPos) {
-        set_error("position-weighted lookup: a launch class has %d features, at most %d are supported",
-                  (int)tbe->max_class_feats, kMaxPos);
-        return TRA_ERR_TOO_LARGE;
-      }
-      for (size_t i = 0; i < n_features; ++i) {
-        const int key = key_of(i);
-        if (key < 0 || key >= pw->num_keys) {
-          set_error("position-weighted lookup: feature at key position %d, but %d keys were described", key,
-                    pw->num_keys);
-          return TRA_ERR_INVALID_ARGUMENT;
-        }
-        const int64_t st = pw->key_start[key], n = pw->key_len[key];
-        if (n < 0 || st < 0 || (n > 0 && st + n > pw->table_len)) {
-          set_error("position-weighted lookup: key %d has weights [%lld, %lld) outside the table of %lld", key,
-                    (long long)st, (long long)(st + n), (long long)pw->table_len);
-          return TRA_ERR_INVALID_ARGUMENT;
-        }
-        a.pw_off[i] = (int32_t)st;
-        a.pw_len[i] = (int32_t)n;
-      }
+    a.psw = psw;
+    if (positions) {
+      const int rc = fill_positions(a.pw_off, a.pw_len, n_features, key_of);
+      if (rc != TRA_OK) return rc;
       a.posw = pw->table;
-      a.psw = nullptr;
     }
     a.out = out;
     a.out_stride = out_stride;
@@ -1098,20 +1102,32 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
     return out_stride * esz % 16 == 0 && (esz == 2 ? cls.cols_aligned_fp16 : cls.cols_aligned_fp32);
   };
   if (!balanced && !nobag) {
+    GroupArgs a;
+    a.weights = (const uint8_t*)weights;
+    a.indices = readable_ids;
+    a.offsets = offsets;
+    a.psw = psw;
+    a.posw = positions ? pw->table : nullptr;
+    a.out = out;
+    a.out_stride = out_stride;
+    a.err_count = tbe->err_dev;
+    a.num_indices = num_indices > 0 ? num_indices : 1;
+    a.B = batch_size;
+    a.mean = pooling_mode == TRA_POOL_MEAN;
+    a.out_fp16 = out_dtype == TRA_FP16;
+    a.pairs = (uintptr_t)out % 4 == 0 && out_stride % 2 == 0;
+    a.bad_to_row0 = tbe->bad_to_row0.load(std::memory_order_relaxed) != 0;
     // (position weights: the launch arguments hold the layout of kMaxPos slices)
-    const size_t step = pw != nullptr && num_indices > 0 ? kMaxPos : tbe->group_slices.size();
+    const size_t step = positions ? kMaxPos : tbe->group_slices.size();
     for (size_t s0 = 0; s0 < tbe->group_slices.size(); s0 += step) {
       const size_t n = std::min(step, tbe->group_slices.size() - s0);
       const GroupSlice* slices = tbe->group_slices.data() + s0;
-      GroupArgs a;
-      a.common = tbe->group_base;
       a.slices = tbe->group_slices_dev + s0;
-      const int rc = fill(a.common, n, [&](size_t i) { return slices[i].key; });
-      if (rc != TRA_OK) return rc;
       GroupPositions p;
-      memcpy(p.off, a.common.pw_off, sizeof(p.off));
-      memcpy(p.len, a.common.pw_len, sizeof(p.len));
-      a.common.vec_store = (uintptr_t)out % 4 == 0 && out_stride % 2 == 0;
+      if (positions) {
+        const int rc = fill_positions(p.off, p.len, n, [&](size_t i) { return slices[i].key; });
+        if (rc != TRA_OK) return rc;
+      }
       GroupLaunch l = geo_local.group;
       l.grid = (int)n * l.tiles;
       l.key0 = slices[0].key;
@@ -1122,12 +1138,12 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
         }
       const auto go = [&](auto ids) {
         using IdxT = decltype(ids);
-        if (a.common.posw != nullptr)
-          launch_group<IdxT, kByPosition>(a, p, l, from_lengths, s);
-        else if (a.common.psw != nullptr)
-          launch_group<IdxT, kPerSample>(a, p, l, from_lengths, s);
+        if (positions)
+          launch_group<IdxT, kByPosition>(a, &p, l, from_lengths, s);
+        else if (psw != nullptr)
+          launch_group<IdxT, kPerSample>(a, nullptr, l, from_lengths, s);
         else
-          launch_group<IdxT, kUnweighted>(a, p, l, from_lengths, s);
+          launch_group<IdxT, kUnweighted>(a, nullptr, l, from_lengths, s);
       };
       if (idx_is_i64) go(int64_t()); else go(int32_t());
       const hipError_t e = hipGetLastError();
