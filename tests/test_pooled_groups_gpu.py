@@ -60,6 +60,37 @@ def test_several_bags_per_group(tuning, bags):
     assert bits_equal(_from_lengths(tbe, ids, lengths, None, B), want) == 0
 
 
+@pytest.mark.parametrize("route", ["lengths", "scan", "offsets"])
+@pytest.mark.parametrize("T,B,dim", [(1, 1000, 16), (1, 16_000, 100), (2, 40_000, 16)])  # 1, 2 and 5 bags per group
+def test_counts_beyond_32_bits(tuning, T, B, dim, route):
+    """Malformed 64-bit lengths and the offsets that they sum to: a count is cut to 32 bits, its bag is empty if that
+    is negative, positions outside the ids read the last one; every other bag is pooled from its own bounds."""
+    tuning(balanced=0)
+    if route == "scan":
+        tuning(fused_scan=0)
+    rng = np.random.default_rng(T)
+    tbe, store = build(rng, [(O.INT8, 300 + t, dim) for t in range(T)], list(range(T)), O.SUM, O.FP32, 16)
+    lengths = rng.integers(0, 4, T * B).astype(np.int64)
+    odd = rng.choice(T * B - 40, 200, replace=False)
+    for k, x in enumerate((2**32 + 3, -(2**32) + 2, 2**40, -(2**40), 2**31 + 9, -(2**32) - 6, -5, 2**33 + 1)):
+        lengths[odd[k::8]] = x
+    lengths[0] = 3
+    offsets = np.concatenate([[0], np.cumsum(lengths)])
+    ids = rng.integers(0, 300, int(lengths[(lengths > 0) & (lengths < 4)].sum())).astype(np.int64)
+    cut = lengths.astype(np.int32).clip(min=0).astype(np.int64)
+    assert cut.max() < 4
+    place = np.arange(int(cut.sum())) - np.repeat(np.cumsum(cut) - cut, cut)
+    at = np.repeat(offsets[:-1], cut) + place
+    at = np.where((at >= 0) & (at < len(ids)), at, len(ids) - 1)
+    want = O.tbe_forward(store, list(range(T)), B, ids[at], np.concatenate([[0], np.cumsum(cut)]), None, O.SUM, O.FP32)
+    ti = torch.from_numpy(ids).to(DEV)
+    if route == "offsets":
+        got = tbe(ti, torch.from_numpy(offsets).to(DEV), batch_size=B)
+    else:
+        got = tbe(ti, None, lengths=torch.from_numpy(lengths).to(DEV), batch_size=B)
+    assert bits_equal(got.cpu().numpy(), want) == 0
+
+
 def test_position_weights_of_many_slices():
     """150 features of two weight types: more than the launch arguments describe at once, no class above the limit."""
     rng = np.random.default_rng(5)

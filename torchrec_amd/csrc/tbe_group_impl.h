@@ -2,6 +2,7 @@
 // Included by one .hip file per (id type, weight mode).
 #pragma once
 
+#include "tbe_group_run.h"
 #include "tbe_lookup_impl.h"
 
 namespace tra {
@@ -88,7 +89,7 @@ __device__ __forceinline__ void for_each_row(std::integer_sequence<int, I...>, F
 }
 
 // The bags [first, first + count) of a window, at most 16, by one group of lanes.  s_start, s_len: where the window's bags' ids
-// start and how many there are (as given); bag0: the sample of the window's first bag.
+// start and how many there are (none: zero); bag0: the sample of the window's first bag.
 //
 // A lane owns NE columns (NE = 1, 2, 4, 8 or 16: up to 16, 32, 64, 128, 256
 // columns of a row) and the group walks the rows one after the other, so a bag's
@@ -170,11 +171,15 @@ __device__ __forceinline__ void pool_group_bags(const GroupArgs& a, const GroupS
   // The group's lane j holds bag j.
   const int n_bags = max(count, 0);
   const int64_t bag_start = c < n_bags ? s_start[first + c] : 0;
-  const int given = c < n_bags ? s_len[first + c] : 0;
-  // A negative length (only a malformed input holds one) makes its own bag empty and moves the starts of the
-  // ones behind it: the bags are then no run and are walked one by one.
-  const bool one_run = __builtin_amdgcn_ballot_w64(given < 0) == 0;
-  const int bag_len = max(given, 0);
+  const int bag_len = c < n_bags ? s_len[first + c] : 0;
+  bool one_run = true;  // (unless the input is malformed)
+  if (__builtin_amdgcn_ballot_w64(n_bags > 1) != 0) {
+    // the next lane's start, by a row shift
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)bag_start, 0x101, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(bag_start >> 32), 0x101, 0xf, 0xf, true);
+    const bool joins = bags_join(bag_start, bag_len, (int64_t)(((uint64_t)hi << 32) | lo));
+    one_run = __builtin_amdgcn_ballot_w64(c + 1 < n_bags && !joins) == 0;
+  }
   const float inv = a.mean && bag_len > 0 ? 1.0f / (float)bag_len : 1.0f;
   const int most = one_run ? 1 : kGroup;  // runs
   for (int seg = 0; seg < most; ++seg) {
@@ -392,13 +397,13 @@ __global__ __launch_bounds__(kBlockThreads, 4) void tbe_pooled_kernel(
     for (int w = 0; w < kWavesPerBlock; ++w) at += s_front[w] + (w < wave ? s_tot[w] : (Sum)0);
     if ((int)threadIdx.x < nb) {
       s_start[threadIdx.x] = (int64_t)(at + incl - raw);
-      s_len[threadIdx.x] = (int)raw;
+      s_len[threadIdx.x] = bag_ids((int64_t)raw);
     }
   } else {
     const int64_t start = (int64_t)bags[t], end = (int64_t)bags[t + 1];
     if ((int)threadIdx.x < nb) {
       s_start[threadIdx.x] = start;
-      s_len[threadIdx.x] = (int)(end - start);
+      s_len[threadIdx.x] = bag_ids((int64_t)((uint64_t)end - (uint64_t)start));
     }
   }
   __syncthreads();
