@@ -1079,6 +1079,15 @@ struct Window {
   __shared__ typename SumOf<IdxT>::type s_red[kCuWaves], s_wave_tot[kCuWaves];                       \
   const Window<IdxT> name{s_start, s_len, s_ent, s_order, s_slot, s_hist, s_desc, s_red, s_wave_tot}
 
+// The launch arguments that pooling reads, asked for together while the window is staged: fetched one behind the
+// other after the staging's barrier, as the compiler places them, they cost every wave a trip to memory each with
+// nothing else in flight (graph replays, us, without / with this: 26 int4 tables of 128 columns, 2048 samples
+// 19.1 / 18.7; 16 int2 tables of 256 columns, 2048 samples 20.8 / 20.5; 8 fp16 tables, 8192 samples 18.0 / 17.85).
+__device__ __forceinline__ void hold_pool_args(const LookupArgs& a) {
+  asm volatile("" ::"s"(a.weights), "s"(a.cdescs), "s"(a.indices), "s"(a.out), "s"(a.out_stride), "s"(a.num_indices),
+               "s"(a.mean), "s"(a.vec_store), "s"(a.out_fp16), "s"(a.bad_to_row0));
+}
+
 // Stages bags [q0, q0 + nb) of a sub-class and ranks them by length; returns what their starts in LDS still lack.
 // FROM_LENGTHS: p_offsets points at the KJT's lengths instead of its offsets
 // and the block derives its bags' start positions itself: one block-wide sum
@@ -1152,6 +1161,7 @@ __device__ __forceinline__ typename SumOf<IdxT>::type stage_window(const Window<
       }
       if (ln == 0) w.red[0] = 0;
       wave_lds_sync();
+      hold_pool_args(a);
       TRA_STAMP(7);
       TRA_STAMP(1);
       {  // counting sort, longest first (as in the general route below)
@@ -1179,6 +1189,7 @@ __device__ __forceinline__ typename SumOf<IdxT>::type stage_window(const Window<
       const Sum mine = front_sum.run(reinterpret_cast<const IdxT*>(p_offsets),
                                      (int64_t)feat_key_pos(a, sc, fi_lo) * p_B + (q0 - fi_lo * p_B),
                                      (int)threadIdx.x - kWaveSize, kCuThreads - kWaveSize);
+      hold_pool_args(a);
       const Sum front_w = wave_last(wave_scan_incl(mine));
       if (ln == 0) w.red[wv] = front_w;
     }
@@ -1342,10 +1353,10 @@ __device__ __forceinline__ typename SumOf<IdxT>::type stage_window(const Window<
 constexpr int kBodiesOdd = 1;   // id blocks of four for every lane group of four lanes or more
 constexpr int kBodiesEven = 0;  // id blocks for powers of two from eight lanes, for others where the registers allow
 
-// Pools a staged window.
-template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, int BODIES>
+// Pools a staged window.  vec(): whether every lane's output slice is 16-byte aligned (asked where a bag is stored).
+template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, int BODIES, typename Vec>
 __device__ __forceinline__ void pool_window(const Window<IdxT> win, const LookupArgs& a, const SubClass& sc, int nb,
-                                            int fi_lo, typename SumOf<IdxT>::type front_add, bool vec) {
+                                            int fi_lo, typename SumOf<IdxT>::type front_add, Vec&& vec) {
   constexpr int NE = CB * 8 / Traits<DTYPE>::kBits;
   constexpr bool ODD = BODIES == kBodiesOdd;
   const int lane = threadIdx.x & (kWaveSize - 1);
@@ -1422,7 +1433,7 @@ __device__ __forceinline__ void pool_window(const Window<IdxT> win, const Lookup
 #ifdef TRA_INSTRUMENT
     if (lane == 0) a.ts[((size_t)blockIdx.x * (blockDim.x / 64) + wave) * 8 + 5] = (unsigned long long)max_len;
 #endif
-    finish_bag<NE>(acc, a, len, (int64_t)b * a.out_stride + d.out_col, c, lpr, lane, active, vec);
+    finish_bag<NE>(acc, a, len, (int64_t)b * a.out_stride + d.out_col, c, lpr, lane, active, vec());
     TRA_STAMP(4);
   }
 }
@@ -1468,7 +1479,7 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
   const int fi_lo = q0 / p_B;
   const auto front_add = stage_window<IdxT, FROM_LENGTHS>(s_window, a, p_offsets, p_cdescs, p_B, sc, q0, nb, fi_lo);
   pool_window<DTYPE, CB, IdxT, WEIGHTED, U, ODD ? kBodiesOdd : kBodiesEven>(s_window, a, sc, nb, fi_lo, front_add,
-                                                                             a.vec_store != 0);
+                                                                             [&] { return a.vec_store != 0; });
 }
 
 // ---- host side of one launch ----------------------------------------------

@@ -33,7 +33,7 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_multi_kernel(const void
   const bool vec = (kind & kMultiVec) != 0;
 #define TRA_MULTI(D, CB)                                                                                       \
   case multi_kind(D, CB):                                                                                      \
-    pool_window<D, CB, IdxT, WEIGHTED, 4, kBodiesOdd>(s_window, a, sc, nb, fi_lo, front_add, vec);             \
+    pool_window<D, CB, IdxT, WEIGHTED, 4, kBodiesOdd>(s_window, a, sc, nb, fi_lo, front_add, [&] { return vec; }); \
     break;
   switch (kind & ~kMultiVec) {
     TRA_MULTI(TRA_INT8, 16)
