@@ -46,6 +46,46 @@ def test_group_widths(tuning, dtype, weighted):
         assert bits_equal(got, want) == 0, B
 
 
+# 32 and 64 lanes a bag, and what 64 cannot hold
+WIDE = {O.INT8: [100, 260, 264, 300, 504, 512, 1020, 1024, 1040], O.INT4: [264, 512, 520, 1024, 1032],
+        O.INT2: [272, 512, 1024, 1040], O.FP16: [130, 136, 256, 258, 512, 522], O.FP32: [65, 68, 128, 130, 256, 259, 516]}
+
+
+@pytest.mark.parametrize("weights", ["none", "sample", "position"])
+@pytest.mark.parametrize("dtype", list(WIDE))
+def test_rows_of_more_than_sixteen_lanes(tuning, dtype, weights):
+    tuning(balanced=0)
+    rng = np.random.default_rng(dtype * 3 + len(weights))
+    rows, T = 120, len(WIDE[dtype])
+    idt, pooling, out = {"none": (np.int32, O.SUM, O.FP16), "sample": (np.int64, O.MEAN, O.FP32),
+                         "position": (np.int32, O.SUM, O.FP32)}[weights]
+    tbe, store = build(rng, [(dtype, rows, dim) for dim in WIDE[dtype]], list(range(T)), pooling, out, 4)
+    bad = 0
+    for B in (1, 9, 2000 if weights == "none" else 40):  # (2000: several bags per lane group)
+        lengths = (rng.integers(0, 4, T * B) if B == 2000 else _lengths(rng, T * B)).astype(idt)
+        offsets = np.zeros(T * B + 1, dtype=idt)
+        offsets[1:] = np.cumsum(lengths)
+        ids = rng.integers(-2, rows + 1, int(offsets[-1])).astype(idt)
+        outside = (ids < -1) | (ids >= rows)
+        psw, kw = None, {}
+        if weights == "sample":
+            psw = rng.uniform(-1, 1, len(ids)).astype(np.float32)
+        elif weights == "position":
+            table = rng.uniform(-1, 1, 6 * T).astype(np.float32)
+            place, key = np.arange(len(ids)) - np.repeat(offsets[:-1], lengths), np.repeat(np.arange(T * B) // B, lengths)
+            w = table[6 * key + np.minimum(place, 5)]
+            kw = {"position_weights": (torch.from_numpy(table).to(DEV), [6 * t for t in range(T)], [6] * T)}
+        want = O.tbe_forward(store, list(range(T)), B, np.where(outside, -1, ids).astype(idt), offsets,
+                             w if weights == "position" else psw, pooling, out)
+        got = _from_lengths(tbe, ids, lengths, psw, B, **kw)
+        assert bits_equal(got, want) == 0, B
+        got = tbe(torch.from_numpy(ids).to(DEV), torch.from_numpy(offsets).to(DEV),
+                  None if psw is None else torch.from_numpy(psw).to(DEV), **kw).cpu().numpy()
+        assert bits_equal(got, want) == 0, B
+        bad += 2 * int(outside.sum())
+    assert tbe.out_of_range_count() == bad
+
+
 @pytest.mark.parametrize("bags", [40_000, 300_000])  # 3 and 16 bags per group
 def test_several_bags_per_group(tuning, bags):
     tuning(balanced=0)

@@ -92,7 +92,8 @@ __device__ __forceinline__ void for_each_row(std::integer_sequence<int, I...>, F
 // start and how many there are (none: zero); bag0: the sample of the window's first bag.
 //
 // A lane owns NE columns (NE = 1, 2, 4, 8 or 16: up to 16, 32, 64, 128, 256
-// columns of a row) and the group walks the rows one after the other, so a bag's
+// columns of a row; of wider rows two or four groups walk the same bags, each
+// for its columns) and the group walks the rows one after the other, so a bag's
 // sum is evaluated in id order as everywhere.  The bags' ids follow one another
 // in memory and are walked as one run, sixteen at a time, one per lane; that
 // lane also works out the row's offset, and a row step takes it (and the weight,
@@ -110,8 +111,8 @@ __device__ __forceinline__ void for_each_row(std::integer_sequence<int, I...>, F
 // one load instruction per row: 50 us where this takes 33 on 1 M ids); ids dealt evenly to the groups instead of bags
 // (+0.8 us for a barrier more, nothing gained); headers gathered with the ids (every row's line then comes twice
 // through the L1).
-// MODE: kNear, kFar (the table's rows lie beyond the reach of 32-bit offsets) or kSplit (the slice is not its row's
-// only one: the header does not lie in front of it).
+// MODE: kNear, kFar (the table's rows lie beyond the reach of 32-bit offsets) or kSplit (not every group's columns
+// begin behind the row's header).
 template <int DTYPE, int NE, typename IdxT, int WEIGHTED, int MODE>
 __device__ __forceinline__ void pool_group_bags(const GroupArgs& a, const GroupSlice& d, const float* pw,
                                                 int pw_len, const int64_t* s_start, const int* s_len, int bag0,
@@ -122,8 +123,9 @@ __device__ __forceinline__ void pool_group_bags(const GroupArgs& a, const GroupS
   constexpr bool kHasHeader = Traits<DTYPE>::kHeader != 0;
   const int c = lane & (kGroup - 1);
   const int lane0 = lane - c;  // the group's first lane
-  const bool has_cols = c * NE < d.cols;
-  const int bit0 = has_cols ? c * NE * Cols::kBits : 0;
+  const int cl = lane & ((1 << d.lanes_log2) - 1);  // the lane's place among those of its bag
+  const bool has_cols = cl * NE < d.cols;
+  const int bit0 = has_cols ? cl * NE * Cols::kBits : 0;
   // where what the lane loads of a row starts
   const uint32_t lane_off = (uint32_t)(d.payload + (kHasHeader ? bit0 / 32 * 4 - 4 : bit0 / 8));
   const uint32_t shift = bit0 % 32;
@@ -142,7 +144,7 @@ __device__ __forceinline__ void pool_group_bags(const GroupArgs& a, const GroupS
   const int elem = a.out_fp16 ? 2 : 4;
   const int64_t out_row = a.out_stride * elem;
   uint8_t* const out =
-      reinterpret_cast<uint8_t*>(a.out) + (int64_t)(bag0 + first) * out_row + (int64_t)(d.out_col + c * NE) * elem;
+      reinterpret_cast<uint8_t*>(a.out) + (int64_t)(bag0 + first) * out_row + (int64_t)(d.out_col + cl * NE) * elem;
   const bool pairs = d.even != 0 && a.pairs != 0;
   auto store = [&](int b, const float (&acc)[NE]) {
     if (!has_cols) return;
@@ -352,8 +354,8 @@ __device__ __forceinline__ void pool_group_bags(const GroupArgs& a, const GroupS
       cur = nxt;
     }
   }
-  // Bad ids are counted by the slice that holds column 0.
-  if (d.first_slice != 0 && bad != 0) atomicAdd(a.err_count, (unsigned long long)bad);
+  // Bad ids are counted by the lanes that hold column 0 and their fifteen neighbours.
+  if (d.first_slice != 0 && cl < kGroup && bad != 0) atomicAdd(a.err_count, (unsigned long long)bad);
 }
 
 // A block owns a window of consecutive bags of one feature (column slice), each
@@ -407,7 +409,7 @@ __global__ __launch_bounds__(kBlockThreads, 4) void tbe_pooled_kernel(
     }
   }
   __syncthreads();
-  const int first = (int)(threadIdx.x / kGroup) * p_per_group;
+  const int first = (((int)threadIdx.x >> d.lanes_log2) + d.part * (kBlockThreads >> d.lanes_log2)) * p_per_group;
   const int count = min(p_per_group, nb - first);  // (negative: none)
   if (__builtin_amdgcn_ballot_w64(count > 0) == 0) return;
   const float* pw = nullptr;
@@ -432,7 +434,7 @@ __global__ __launch_bounds__(kBlockThreads, 4) void tbe_pooled_kernel(
   switch (d.kind) {
     TRA_GROUP_TYPES(kNear)
     TRA_GROUP_TYPES(kFar)
-    TRA_GROUP(TRA_INT8, 4, kSplit) TRA_GROUP(TRA_INT8, 16, kSplit)
+    TRA_GROUP(TRA_INT8, 4, kSplit) TRA_GROUP(TRA_INT8, 8, kSplit) TRA_GROUP(TRA_INT8, 16, kSplit)
     TRA_GROUP(TRA_INT4, 8, kSplit) TRA_GROUP(TRA_INT4, 16, kSplit)
     TRA_GROUP(TRA_INT2, 16, kSplit)
   }

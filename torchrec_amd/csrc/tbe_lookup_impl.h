@@ -1541,12 +1541,13 @@ struct GroupSlice {
   int32_t key;          // key position
   uint8_t even;         // the first output column is
   uint8_t first_slice;  // holds column 0 of its feature
-  uint16_t unused;
+  uint8_t lanes_log2;   // lanes per bag: 16, 32 or 64
+  uint8_t part;         // which of the lanes / 16 descriptors of the slice: a block takes that share of its window's bags
 };
 // How the sixteen-lane kernel addresses a slice's rows.
 constexpr int kNear = 0;   // 32-bit offsets, header in front of the columns (or none)
 constexpr int kFar = 1;    // a table beyond 4 GiB
-constexpr int kSplit = 2;  // one of several slices of a row with a header
+constexpr int kSplit = 2;  // a row with a header, in several slices or by more than sixteen lanes
 constexpr int group_kind(int dtype, int ne, int mode) { return (dtype * 4 + mode) * 32 + ne; }
 // What a launch needs and no more: the launch arguments are written over the bus for every call, and a small call's
 // time is its launch (with the window kernel's arguments, 3.0 KB, the entry point takes 4.2 us of the host's time, with

@@ -108,6 +108,37 @@ static Overrides g_ovr = overrides_from_env();
 // Bumped by tra_set_tuning: launch geometry remembered under an older value is recomputed.
 static std::atomic<int> g_ovr_gen{0};
 
+// How the sixteen-lane kernel takes the columns of a row from `off` on: the first slice of them.
+struct GroupShape {
+  int ne;  // columns per lane
+  int lanes_log2;
+  int cols;
+};
+
+// A row is one slice where sixteen lanes can hold it (16 columns of an integer row each, 16 bytes of others), else
+// where 32 or 64 can; only what 64 cannot hold is cut.  The walk over the ids and its trip count belong to a wave,
+// so two or one bags in it are better for wide rows than four bags of each of several slices.  Graph replays of 8
+// tables, ~20 ids a bag, us, slices of sixteen lanes / this: int8 100 columns, 6400 bags 13.3 / 11.9; int8 512, 512 bags
+// 10.9 / 10.2, 6400 bags 28.4 / 24.0; int8 300, 512 bags 10.5 / 8.3; int4 512, 6400 bags of 45 45.2 / 38.7; fp16 512
+// 55.6 / 50.3; fp32 256 53.3 / 48.8.  What is cut starts with a slice of half the most columns a lane can hold (int8 300:
+// 64 lanes of 4 columns 7.5 and 45.3 us at 512 bags of 20 and 6400 of 45, 32 of 8 8.3 and 43.1, 16 of 16 10.5 and 39.5).
+static GroupShape group_shape(int dtype, int dim, int off) {
+  const int bits = bits_of(dtype), left = dim - off;
+  const int most = dtype == TRA_FP32 ? 4 : dtype == TRA_FP16 ? 8 : 16;
+  for (int log2 = 4; log2 <= 6; ++log2) {
+    // (more than sixteen lanes, or a part of the row: with a header, the kernel's split kinds, whole dwords a lane)
+    const int least = header_bytes(dtype) != 0 && (log2 > 4 || off > 0) ? 32 / bits : 1;
+    for (int ne = least; ne <= most; ne *= 2)
+      if (left % ne == 0 && ne << log2 >= left) return {ne, log2, left};
+  }
+  int cols = most << 6;
+  while (cols > left) cols /= 2;
+  int ne = most / 2, log2 = 4;
+  while (ne << 6 < cols) ne *= 2;
+  while (ne << log2 < cols) ++log2;
+  return {ne, log2, cols};
+}
+
 static Tuning choose_tuning(int num_cus, size_t classes, int64_t bags, int64_t num_indices) {
   Tuning t;
   // Ranking bags by length pays once every CU gets a few dozen bags; below that the sixteen-lane kernel is
@@ -396,40 +427,29 @@ int tra_tbe_create(const tra_table_spec* tables, int32_t num_tables,
       plan->slices.push_back(d);
       slice_lpr.push_back(bytes / cb);
     }
-    // The sixteen-lane kernel's slices: the row as one where sixteen lanes can hold it (16 columns of an
-    // integer row each, 16 bytes of others), else as wide ones as there are.
-    const bool header = header_bytes(s.dtype) != 0;
-    const int most = s.dtype == TRA_FP32 ? 4 : s.dtype == TRA_FP16 ? 8 : 16;
-    const auto fits = [](int ne, int cols) { return ne * 16 >= cols && cols % ne == 0; };
-    bool one_slice = false;
-    for (int ne = 1; ne <= most; ne *= 2) one_slice = one_slice || fits(ne, s.dim);
+    // The sixteen-lane kernel's slices.
     for (int off = 0; off < s.dim;) {
-      const int left = s.dim - off;
-      int ne = 1;
-      if (one_slice) {
-        while (!fits(ne, left)) ne *= 2;
-      } else if (header) {
-        ne = left >= 256 || left % 16 == 0 ? 16 : 32 / bits;  // (the kernel's split kinds: 16, or a dword's columns)
-      } else {
-        ne = most;
-        while (ne > 1 && ne * 16 > left && left % ne != 0) ne /= 2;
-      }
+      const GroupShape shape = group_shape(s.dtype, s.dim, off);
       GroupSlice w;
       w.table_offset = s.offset;
       w.rows = s.rows;
       w.rows32 = (uint32_t)std::min<int64_t>(s.rows, int64_t(1) << 31);
       w.row_bytes = s.row_bytes;
-      w.cols = std::min(left, ne * 16);
+      w.cols = shape.cols;
       w.out_col = col + off;
       w.payload = header_bytes(s.dtype) + off * bits / 8;
       w.key = feature_positions ? feature_positions[f] : f;
       w.even = w.out_col % 2 == 0 ? 1 : 0;
       w.first_slice = off == 0 ? 1 : 0;
-      w.unused = 0;
+      w.lanes_log2 = (uint8_t)shape.lanes_log2;
       // (near: row offset and place in the row are added in 32 bits)
-      w.kind = group_kind(s.dtype, ne, header && !one_slice ? kSplit : s.rows * s.row_bytes > 0xffffffffll ? kFar : kNear);
-      plan->group_slices.push_back(w);
-      off += w.cols;
+      const bool split = header_bytes(s.dtype) != 0 && (shape.cols < s.dim || shape.lanes_log2 > 4);
+      w.kind = group_kind(s.dtype, shape.ne, split ? kSplit : s.rows * s.row_bytes > 0xffffffffll ? kFar : kNear);
+      for (int part = 0; part < (1 << shape.lanes_log2) / 16; ++part) {
+        w.part = (uint8_t)part;
+        plan->group_slices.push_back(w);
+      }
+      off += shape.cols;
     }
     col += s.dim;
   }
