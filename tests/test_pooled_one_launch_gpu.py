@@ -61,3 +61,17 @@ def test_one_launch_of_several_classes(tuning, name, weights):
         assert bits_equal(got, want) == 0, order
     assert "tbe_pooled_multi_kernel" in _launch_text(tbe, B, len(ids), T)
     assert tbe.out_of_range_count() == 0
+
+
+def test_route_is_the_same_from_lengths_and_from_offsets():
+    """Seven launch classes: one launch below 12,000 ids per compute unit, whatever the bags' bounds come from; a launch
+    per class from there on.  Few classes own no second stream and take one launch at any size."""
+    rng = np.random.default_rng(21)
+    dts, dims = (O.INT8, O.INT4, O.INT2, O.FP16), (32, 64, 128, 256)
+    seven, _ = build(rng, [(dts[t % 4], 50, dims[t // 4]) for t in range(16)], list(range(16)), O.SUM, O.FP32, 16)
+    two, _ = build(rng, [(dts[t % 2], 50, 64) for t in range(16)], list(range(16)), O.SUM, O.FP32, 16)
+    line = 12_000 * torch.cuda.get_device_properties(0).multi_processor_count
+    for n_keys in (0, 16):
+        assert "tbe_pooled_multi_kernel" in _launch_text(seven, 4096, line - 1, n_keys)
+        assert _launch_text(seven, 4096, line, n_keys).count("tbe_pooled_cu_kernel") == 7
+        assert "tbe_pooled_multi_kernel" in _launch_text(two, 4096, 2 * line, n_keys)

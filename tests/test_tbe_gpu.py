@@ -1177,7 +1177,8 @@ def test_multi_class_call_on_two_streams(tuning):
     specs = [(dts[t % 4], rows, dims[(t // 4) % 4]) for t in range(T)]
     ftm = list(range(T))
     tbe, store = build(rng, specs, ftm, O.SUM, O.FP32, 16)
-    lengths = rng.poisson(30, T * B).astype(np.int32)
+    # more than 12,000 ids per compute unit: below that such a call is one launch
+    lengths = rng.poisson(104, T * B).astype(np.int32)
     offsets = np.zeros(T * B + 1, dtype=np.int32)
     offsets[1:] = np.cumsum(lengths)
     n = int(offsets[-1])

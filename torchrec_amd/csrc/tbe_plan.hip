@@ -665,16 +665,34 @@ static bool use_window_kernel(const tra_tbe* tbe, const Tuning& tune, bool nobag
          (int64_t)tbe->max_class_feats * batch_size < (int64_t(1) << 31);
 }
 
+// Whether launches on a stream are being captured into a graph (or the runtime cannot say).
+static bool captured(hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// Where a call's launches go.
+struct CallStream {
+  hipStream_t stream;
+  bool one_stream;  // never on the plan's second stream
+  bool described;   // a call that is only described, and taken as not captured
+};
+
 // Whether a call of several launch classes that takes the window kernel does so in one launch (whatever the class, a
 // block is a window of bags; the launches' fixed costs, and a window of each class too small to fill its block, are
-// paid once).  Graph replays, us, a launch per class / one launch: two classes, 33 K bags of 20 ids 30 / 20, 131 K bags
-// of 20 85 / 66, 262 K bags of 30 hot ids 182 / 151, of cold ids 280 / 277; seven classes, 33 K bags of 20 95 / 20,
-// 131 K bags of 20 121 / 76, 262 K bags of 30 hot ids 199 / 152, of cold ids 306 / 309 in a graph and about 345 / 420
-// outside one.  So: always where there is no second stream, else up to 12,000 ids per compute unit.  From offsets
-// a plan with a second stream keeps it from 3750 on, the route that calls of that size are tested on.
-static bool use_one_launch(const tra_tbe* tbe, int32_t batch_size, int64_t num_indices, bool lengths_call) {
+// paid once).  Two classes, graph replays, us, a launch per class / one launch: 33 K bags of 20 ids 30 / 20, 131 K bags
+// of 20 85 / 66, 262 K bags of 30 hot ids 182 / 151, of cold ids 280 / 277.  So: always where there is no second stream.
+// Seven classes, thousands of ids per compute unit, rows in the caches and in memory:
+//   on two streams, from offsets (from lengths: 6 - 10 / 0 - 4 more)
+//     3.8: 77 / 26, 99 / 46   7.7: 92 / 45, 121 / 96   11.5: 117 / 63, 159 / 139   15.4: 110 / 84, 180 / 192   31: 171 / 156, 307 / 361
+//   captured or from the entry that must not allocate, on one stream
+//     11.5: 138 / 63, 193 / 139   15.4: 126 / 84, 205 / 192   23: 163 / 120, 267 / 277   31: 201 / 156, 330 / 361
+static bool use_one_launch(const tra_tbe* tbe, int32_t batch_size, int64_t num_indices, const CallStream& c) {
   if (tbe->multi_feats.empty() || (int64_t)tbe->multi_feats.size() * batch_size >= (int64_t(1) << 31)) return false;
-  return tbe->side == nullptr || num_indices < (lengths_call ? 12000 : 3750) * (int64_t)tbe->num_cus;
+  if (tbe->side == nullptr || num_indices < 12000 * (int64_t)tbe->num_cus) return true;
+  return num_indices < 18000 * (int64_t)tbe->num_cus && (c.one_stream || (!c.described && captured(c.stream)));
 }
 
 // Largest number of features one window of the from-lengths kernel may span.
@@ -687,7 +705,7 @@ constexpr int64_t kOneLaunchMaxLengths = 131072;
 // Can a pooled call with these sizes take the window kernel in its
 // from-lengths form (which needs no offsets)?
 static bool fused_scan_possible(const tra_tbe* tbe, int32_t batch_size, int32_t num_keys,
-                                int64_t num_indices, int32_t pooling_mode, const void* lengths) {
+                                int64_t num_indices, int32_t pooling_mode, const void* lengths, const CallStream& c) {
   if (pooling_mode == TRA_POOL_NONE || batch_size <= 0 || tbe->num_features == 0) return false;
   if ((uintptr_t)lengths % 16 != 0) return false;
   const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
@@ -700,7 +718,7 @@ static bool fused_scan_possible(const tra_tbe* tbe, int32_t batch_size, int32_t 
   // (about 1.3 us + 1 us per 40k lengths, measured); a separate scan costs
   // about 7 us once.  Take whichever is less.
   const int64_t n = (int64_t)num_keys * batch_size;
-  if (use_one_launch(tbe, batch_size, num_indices, true)) return n <= kOneLaunchMaxLengths;
+  if (use_one_launch(tbe, batch_size, num_indices, c)) return n <= kOneLaunchMaxLengths;
   return (int64_t)tbe->classes.size() * (13 + n / 4000) < 70;
 }
 
@@ -728,15 +746,16 @@ int tra_tbe_launch_info(tra_tbe_t tbe, int32_t batch_size, int64_t num_indices,
   const bool nobag = pooling_mode == TRA_POOL_NONE;
   const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
   const bool balanced = use_window_kernel(tbe, tune, nobag, batch_size);
-  // lengths entry point: same decision as tra_tbe_forward_lengths (aligned lengths assumed)
+  const CallStream c{nullptr, false, true};
+  // lengths entry point: same decision as tra_tbe_forward_lengths (aligned lengths and no capture assumed)
   const bool fused = lengths_num_keys > 0 &&
                      (fused_scan_possible(tbe, batch_size, lengths_num_keys, num_indices, pooling_mode,
-                                          (const void*)16) ||
+                                          (const void*)16, c) ||
                       small_fused_scan_possible(tbe, batch_size, lengths_num_keys, num_indices, pooling_mode,
                                                 (const void*)16));
   static const char* const kDtypeName[] = {"fp32", "fp16", "int8", "int4", "int2"};
   std::string text;
-  const bool multi = balanced && use_one_launch(tbe, batch_size, num_indices, lengths_num_keys > 0);
+  const bool multi = balanced && use_one_launch(tbe, batch_size, num_indices, c);
   if (!nobag && (multi || !balanced)) {
     char line[120];
     snprintf(line, sizeof(line), "%s slices=%d%s", multi ? "tbe_pooled_multi_kernel" : "tbe_pooled_kernel",
@@ -959,7 +978,7 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
                         const float* per_sample_weights, int32_t batch_size, int64_t num_indices,
                         int32_t pooling_mode, int32_t out_dtype, void* out, int64_t out_stride,
                         void* stream, const PositionWeights* pw = nullptr, bool one_stream = false,
-                        const SequenceBounds* seq = nullptr, bool lengths_call = false) {
+                        const SequenceBounds* seq = nullptr) {
   if (!tbe) {
     set_error("tra_tbe_forward: null plan");
     return TRA_ERR_INVALID_ARGUMENT;
@@ -1019,7 +1038,8 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
     const int gen = g_ovr_gen.load(std::memory_order_relaxed);
     const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
     const int balanced = use_window_kernel(tbe, tune, nobag, batch_size) ? 1 : 0;
-    const int multi = balanced && use_one_launch(tbe, batch_size, num_indices, lengths_call || from_lengths) ? 1 : 0;
+    const CallStream where{(hipStream_t)stream, one_stream, false};
+    const int multi = balanced && use_one_launch(tbe, batch_size, num_indices, where) ? 1 : 0;
     const int64_t geo_indices = nobag ? quantized_id_count(num_indices) : num_indices;
     for (const auto& g : tbe->geo)
       if (g && g->batch_size == batch_size && g->gen == gen && g->balanced == balanced &&
@@ -1045,16 +1065,11 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
   // allocate (an event's first record may), and `fork` = 0 (tuning) switches it off.
   bool forked = false;
   std::unique_lock<std::mutex> fork_lock(tbe->fork_mutex, std::defer_lock);
-  if (tbe->side != nullptr && balanced && !geo_local.multi && !one_stream && g_ovr.fork != 0) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
-      fork_lock.lock();
-      TRA_HIP(hipEventRecord(tbe->ev_fork, s));
-      TRA_HIP(hipStreamWaitEvent(tbe->side, tbe->ev_fork, 0));
-      forked = true;
-    } else {
-      (void)hipGetLastError();
-    }
+  if (tbe->side != nullptr && balanced && !geo_local.multi && !one_stream && g_ovr.fork != 0 && !captured(s)) {
+    fork_lock.lock();
+    TRA_HIP(hipEventRecord(tbe->ev_fork, s));
+    TRA_HIP(hipStreamWaitEvent(tbe->side, tbe->ev_fork, 0));
+    forked = true;
   }
   hipStream_t const caller_stream = s;
   // (an error on the way still joins the side streams before it is returned)
@@ -1337,7 +1352,8 @@ static int forward_lengths_impl(tra_tbe_t tbe, const void* weights, const void* 
     set_error("tra_tbe_forward_lengths: null lengths");
     return TRA_ERR_INVALID_ARGUMENT;
   }
-  if (fused_scan_possible(tbe, batch_size, num_keys, num_indices, pooling_mode, lengths) ||
+  const CallStream where{(hipStream_t)stream, one_stream, false};
+  if (fused_scan_possible(tbe, batch_size, num_keys, num_indices, pooling_mode, lengths, where) ||
       small_fused_scan_possible(tbe, batch_size, num_keys, num_indices, pooling_mode, lengths))
     return forward_impl(tbe, weights, indices, lengths, true, idx_is_i64, per_sample_weights,
                         batch_size, num_indices, pooling_mode, out_dtype, out, out_stride, stream, pw, one_stream);
@@ -1353,7 +1369,7 @@ static int forward_lengths_impl(tra_tbe_t tbe, const void* weights, const void* 
   const int rc = tra_cumsum(lengths, n, idx_is_i64, workspace, scan_ws, stream);
   if (rc != TRA_OK) return rc;
   return forward_impl(tbe, weights, indices, workspace, false, idx_is_i64, per_sample_weights, batch_size, num_indices,
-                      pooling_mode, out_dtype, out, out_stride, stream, pw, one_stream, nullptr, /*lengths_call=*/true);
+                      pooling_mode, out_dtype, out, out_stride, stream, pw, one_stream);
 }
 
 extern "C" {
