@@ -75,3 +75,29 @@ def test_route_is_the_same_from_lengths_and_from_offsets():
         assert "tbe_pooled_multi_kernel" in _launch_text(seven, 4096, line - 1, n_keys)
         assert _launch_text(seven, 4096, line, n_keys).count("tbe_pooled_cu_kernel") == 7
         assert "tbe_pooled_multi_kernel" in _launch_text(two, 4096, 2 * line, n_keys)
+
+
+@pytest.mark.parametrize("name", ["features", "cut row"])
+def test_no_one_launch_of_windows(name):
+    """Plans of several classes that windows cannot serve in one launch: the sixteen-lane kernel, one launch for all
+    classes, up to 2500 ids per compute unit, whatever the number of bags; windows, a launch per class, from there on.
+    Few ids in many bags against the oracle."""
+    rng = np.random.default_rng(len(name))
+    specs = {"features": [((O.INT8, O.FP16)[t % 2], 50 + t, 16) for t in range(130)],
+             "cut row": [(O.INT8, 60, 16)] * 15 + [(O.FP32, 40, 1028)]}[name]
+    T = len(specs)
+    tbe, store = build(rng, specs, list(range(T)), O.SUM, O.FP16, 16)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    B = 80 * cus // T + 1
+    lengths = rng.choice([0, 0, 1, 2, 9], T * B).astype(np.int32)
+    offsets = np.zeros(T * B + 1, dtype=np.int32)
+    offsets[1:] = np.cumsum(lengths)
+    ids = rng.integers(0, 40, int(offsets[-1])).astype(np.int32)
+    assert len(ids) < 2500 * cus and "tbe_pooled_kernel" in _launch_text(tbe, B, len(ids), T)
+    for n_keys in (0, T):
+        assert "tbe_pooled_kernel" in _launch_text(tbe, B, 2500 * cus - 1, n_keys)
+        assert "tbe_pooled_cu_kernel" in _launch_text(tbe, B, 2500 * cus, n_keys)
+    want = O.tbe_forward(store, list(range(T)), B, ids, offsets, None, O.SUM, O.FP16)
+    assert bits_equal(_from_lengths(tbe, ids, lengths, None, B), want) == 0
+    got = tbe(torch.from_numpy(ids).to(DEV), torch.from_numpy(offsets).to(DEV)).cpu().numpy()
+    assert bits_equal(got, want) == 0

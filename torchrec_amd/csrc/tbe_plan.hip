@@ -139,17 +139,10 @@ static GroupShape group_shape(int dtype, int dim, int off) {
   return {ne, log2, cols};
 }
 
-static Tuning choose_tuning(int num_cus, size_t classes, int64_t bags, int64_t num_indices) {
+// balanced: what the call's size says (the overrides come first).
+static Tuning choose_tuning(bool balanced) {
   Tuning t;
-  // Ranking bags by length pays once every CU gets a few dozen bags; below that the sixteen-lane kernel is
-  // faster, and with several launch classes it stays so for longer, being one launch for all of them.  Graph
-  // replays of the whole call, us (sixteen-lane / window), ids a bag 3 and 20:
-  //   one class (int8 dim 64): 8192 bags 5.3 / 5.3 and 9.0 / 9.1; 13 K bags of 2 ids 6.2 / 5.6; 33 K bags 13.8 / 6.9
-  //   and 22.8 / 11.7
-  //   two classes, one launch of windows: 8192 bags 6.9 / 8.8 and 14.3 / 17; 33 K bags 17 / 12.6 and 34 / 20
-  //   seven classes, one launch of windows: 8192 bags 6.7 / 7.3 and 14.1 / 15.4; 33 K bags 17 / 9 and 34 / 18
-  t.balanced = bags >= 40 * (int64_t)num_cus &&
-               (classes <= 1 || num_indices >= 640 * (int64_t)num_cus || bags >= 80 * (int64_t)num_cus);
+  t.balanced = balanced ? 1 : 0;
   t.window = 0;
   t.unroll = 4;
   t.lds_bytes = 48 * 1024;  // with the static arrays > half of a CU's LDS: one block per CU
@@ -656,6 +649,25 @@ int tra_tbe_destroy(tra_tbe_t tbe) {
   return TRA_OK;
 }
 
+// Ranking bags by length pays once every CU gets a few dozen bags; below that the sixteen-lane kernel is
+// faster, and with several launch classes it stays so for longer, being one launch for all of them.  Graph
+// replays of the whole call, us (sixteen-lane / window), ids a bag 3 and 20:
+//   one class (int8 dim 64): 8192 bags 5.3 / 5.3 and 9.0 / 9.1; 13 K bags of 2 ids 6.2 / 5.6; 33 K bags 13.8 / 6.9
+//   and 22.8 / 11.7
+//   two classes, one launch of windows: 8192 bags 6.9 / 8.8 and 14.3 / 17; 33 K bags 17 / 12.6 and 34 / 20
+//   seven classes, one launch of windows: 8192 bags 6.7 / 7.3 and 14.1 / 15.4; 33 K bags 17 / 9 and 34 / 18
+// Where a plan has no such launch (over 128 features, cut rows), the window kernel is a launch per class and
+// pays with the ids, not with the bags:
+//   150 features, two classes: 12 K bags of 20 ids 11.0 / 24.4, 33 K of 4 15.2 / 20.6, 33 K of 20 25.7 / 25.6 (rows in
+//   memory 27.3 / 29.1), 60 K of 20 44.3 / 43.2; with a cut fp32 row 33 K of 4 25.9 / 28.9, of 20 72.9 / 70.3
+//   136 features, seven classes: 60 K bags of 2.5 ids 24 / 59, 33 K of 20 40 / 93, rows in memory 43 / 105
+static Tuning tuning_of(const tra_tbe* tbe, int32_t batch_size, int64_t num_indices) {
+  const int64_t cus = tbe->num_cus, bags = (int64_t)tbe->num_features * batch_size;
+  if (tbe->classes.size() <= 1) return choose_tuning(bags >= 40 * cus);
+  if (tbe->multi_feats.empty()) return choose_tuning(bags >= 40 * cus && num_indices >= 2500 * cus);
+  return choose_tuning(bags >= 40 * cus && (num_indices >= 640 * cus || bags >= 80 * cus));
+}
+
 // Whether a pooled call goes to the per-CU window kernel: the size heuristic
 // (or its override) and the limits of the kernel's packed window entries.
 static bool use_window_kernel(const tra_tbe* tbe, const Tuning& tune, bool nobag,
@@ -708,7 +720,7 @@ static bool fused_scan_possible(const tra_tbe* tbe, int32_t batch_size, int32_t 
                                 int64_t num_indices, int32_t pooling_mode, const void* lengths, const CallStream& c) {
   if (pooling_mode == TRA_POOL_NONE || batch_size <= 0 || tbe->num_features == 0) return false;
   if ((uintptr_t)lengths % 16 != 0) return false;
-  const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
+  const Tuning tune = tuning_of(tbe, batch_size, num_indices);
   if (!use_window_kernel(tbe, tune, false, batch_size)) return false;
   const int fused = g_ovr.fused_scan;
   if (fused >= 0) return fused != 0;
@@ -731,7 +743,7 @@ static bool small_fused_scan_possible(const tra_tbe* tbe, int32_t batch_size, in
                                       int64_t num_indices, int32_t pooling_mode, const void* lengths) {
   if (pooling_mode == TRA_POOL_NONE || batch_size <= 0 || tbe->num_features == 0) return false;
   if ((uintptr_t)lengths % 16 != 0 || g_ovr.fused_scan == 0) return false;
-  const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
+  const Tuning tune = tuning_of(tbe, batch_size, num_indices);
   if (use_window_kernel(tbe, tune, false, batch_size)) return false;
   return (int64_t)num_keys * batch_size <= kSmallFusedMaxLengths;
 }
@@ -744,7 +756,7 @@ int tra_tbe_launch_info(tra_tbe_t tbe, int32_t batch_size, int64_t num_indices,
     return TRA_ERR_INVALID_ARGUMENT;
   }
   const bool nobag = pooling_mode == TRA_POOL_NONE;
-  const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
+  const Tuning tune = tuning_of(tbe, batch_size, num_indices);
   const bool balanced = use_window_kernel(tbe, tune, nobag, batch_size);
   const CallStream c{nullptr, false, true};
   // lengths entry point: same decision as tra_tbe_forward_lengths (aligned lengths and no capture assumed)
@@ -1036,7 +1048,7 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
   {
     std::lock_guard<std::mutex> lock(tbe->geo_mutex);
     const int gen = g_ovr_gen.load(std::memory_order_relaxed);
-    const Tuning tune = choose_tuning(tbe->num_cus, tbe->classes.size(), (int64_t)tbe->num_features * batch_size, num_indices);
+    const Tuning tune = tuning_of(tbe, batch_size, num_indices);
     const int balanced = use_window_kernel(tbe, tune, nobag, batch_size) ? 1 : 0;
     const CallStream where{(hipStream_t)stream, one_stream, false};
     const int multi = balanced && use_one_launch(tbe, batch_size, num_indices, where) ? 1 : 0;
