@@ -8,7 +8,7 @@ import torch
 
 import oracle as O
 from helpers import bits_equal, make_table
-from test_tbe_gpu import DEV, build, _from_lengths
+from test_tbe_gpu import DEV, build, _from_lengths, _launch_text
 from torchrec_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -183,3 +183,30 @@ def test_table_beyond_four_gib(tuning, dtype, dim):
         _lib.check(l.tra_tbe_destroy(plan))
         outs.append(out)
     assert outs[0].abs().max() > 0 and torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("idt", [np.int32, np.int64])
+def test_one_class_line_to_the_window_kernel(idt, weighted):
+    """One launch class: the sixteen-lane kernel up to 40 bags per compute unit, rows of whole bytes in bags of 8 ids and
+    more up to 32; where a window would span more features than it can derive starts for, one launch of the
+    sixteen-lane kernel up to 16,384 lengths of few ids.  Both sides of each line against the oracle."""
+    rng = np.random.default_rng(77 + weighted)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    few, some = [0, 1, 2, 7], [9, 10]
+    for dtype, T, B, lens, kernel in (
+            (O.INT8, 8, 4 * cus, some, "tbe_pooled_kernel"), (O.INT8, 8, 4 * cus + 1, some, "tbe_pooled_cu_kernel"),
+            (O.INT8, 8, 4 * cus + 1, few, "tbe_pooled_kernel"), (O.INT4, 8, 4 * cus + 1, some, "tbe_pooled_kernel"),
+            (O.INT8, 8, 5 * cus, few, "tbe_pooled_cu_kernel"), (O.INT8, 200, 52, few, "tbe_pooled_kernel"),
+            (O.INT8, 240, 66, few, "tbe_pooled_kernel"), (O.INT8, 249, 66, few, "tbe_pooled_cu_kernel"),
+            (O.FP16, 128, 67, some, "tbe_pooled_cu_kernel")):
+        tbe, store = build(rng, [(dtype, 40, 16)] * T, list(range(T)), O.SUM, O.FP32, 16)
+        lengths = rng.choice(lens, T * B).astype(idt)
+        offsets = np.zeros(T * B + 1, dtype=idt)
+        offsets[1:] = np.cumsum(lengths)
+        ids = rng.integers(0, 40, int(offsets[-1])).astype(idt)
+        psw = rng.uniform(-1, 1, len(ids)).astype(np.float32) if weighted else None
+        text = _launch_text(tbe, B, len(ids), T)
+        assert kernel in text and ("scan" not in text) == (T * B <= 16384), (T, B, text)
+        want = O.tbe_forward(store, list(range(T)), B, ids, offsets, psw, O.SUM, O.FP32)
+        assert bits_equal(_from_lengths(tbe, ids, lengths, psw, B), want) == 0, (T, B)

@@ -649,6 +649,14 @@ int tra_tbe_destroy(tra_tbe_t tbe) {
   return TRA_OK;
 }
 
+// Largest number of features one window of the from-lengths kernel may span.
+constexpr int kMaxWindowFeatures = 32;
+// Lengths up to which the blocks of the sixteen-lane kernel sum the ones in front of their bags themselves.
+constexpr int64_t kSmallFusedMaxLengths = 16384;
+
+// A window of up to kMaxWindow bags spans kMaxWindow / B + 2 features at most.
+static bool windows_derive_starts(int32_t batch_size) { return batch_size > 0 && kMaxWindow / batch_size + 2 <= kMaxWindowFeatures; }
+
 // Ranking bags by length pays once every CU gets a few dozen bags; below that the sixteen-lane kernel is
 // faster, and with several launch classes it stays so for longer, being one launch for all of them.  Graph
 // replays of the whole call, us (sixteen-lane / window), ids a bag 3 and 20:
@@ -661,9 +669,23 @@ int tra_tbe_destroy(tra_tbe_t tbe) {
 //   150 features, two classes: 12 K bags of 20 ids 11.0 / 24.4, 33 K of 4 15.2 / 20.6, 33 K of 20 25.7 / 25.6 (rows in
 //   memory 27.3 / 29.1), 60 K of 20 44.3 / 43.2; with a cut fp32 row 33 K of 4 25.9 / 28.9, of 20 72.9 / 70.3
 //   136 features, seven classes: 60 K bags of 2.5 ids 24 / 59, 33 K of 20 40 / 93, rows in memory 43 / 105
+// One class of int8, fp16 or fp32 rows, bags of several ids: beyond 32 bags per compute unit (two blocks of the
+// sixteen-lane kernel) that kernel's further blocks wait for the first ones:
+//   8192 / 9216 bags of 20 ids, us: int8 128 columns 12.6 / 14.5 (windows 11.0 / 11.5), 256 17.0 / 20.4 (16.3 / 16.9);
+//   fp16 64 8.8 / 9.9 (8.2 / 8.3), 128 11.5 / 12.6 (11.4 / 11.9); fp32 64 11.1 / 12.1 (11.0 / 11.6)
+//   9216 weighted bags of 64-bit ids, of 3 and 20 ids: int8 64 7.1 / 6.9 and 11.2 / 10.7, 128 8.0 / 8.4 and 15.1 / 14.1;
+//   but int4 128 7.6 / 8.4 and 12.4 / 13.2, int2 64 7.5 / 9.8 and 12.1 / 16.8
+// Where a window spans too many features to derive its bags' starts a scan goes in front of it, which up to 16,384
+// lengths the sixteen-lane kernel does without: 10 - 12 K bags of 2 ids 6.3 / 9.6, of 20 11.9 / 14.7, of 80 26 / 26 (from
+// offsets, where neither has a scan, 5.7 / 5.3, 11.5 / 10.1, 26 / 22).
 static Tuning tuning_of(const tra_tbe* tbe, int32_t batch_size, int64_t num_indices) {
   const int64_t cus = tbe->num_cus, bags = (int64_t)tbe->num_features * batch_size;
-  if (tbe->classes.size() <= 1) return choose_tuning(bags >= 40 * cus);
+  if (tbe->classes.size() <= 1) {
+    if (!windows_derive_starts(batch_size))
+      return choose_tuning(bags >= 40 * cus && (num_indices >= 640 * cus || bags > kSmallFusedMaxLengths));
+    const bool bytes = !tbe->classes.empty() && bits_of(tbe->classes[0].dtype) >= 8;
+    return choose_tuning(bags >= 40 * cus || (bytes && bags > 32 * cus && num_indices >= 8 * bags));
+  }
   if (tbe->multi_feats.empty()) return choose_tuning(bags >= 40 * cus && num_indices >= 2500 * cus);
   return choose_tuning(bags >= 40 * cus && (num_indices >= 640 * cus || bags >= 80 * cus));
 }
@@ -707,9 +729,6 @@ static bool use_one_launch(const tra_tbe* tbe, int32_t batch_size, int64_t num_i
   return num_indices < 18000 * (int64_t)tbe->num_cus && (c.one_stream || (!c.described && captured(c.stream)));
 }
 
-// Largest number of features one window of the from-lengths kernel may span.
-constexpr int kMaxWindowFeatures = 32;
-
 // One launch for several classes derives its offsets itself up to as many lengths as one scan launch takes (its blocks
 // then sum 260 KB on average, about 4 us; the scan of more is two launches of 5 us each and the gaps).
 constexpr int64_t kOneLaunchMaxLengths = 131072;
@@ -724,8 +743,7 @@ static bool fused_scan_possible(const tra_tbe* tbe, int32_t batch_size, int32_t 
   if (!use_window_kernel(tbe, tune, false, batch_size)) return false;
   const int fused = g_ovr.fused_scan;
   if (fused >= 0) return fused != 0;
-  // A window of up to kMaxWindow bags spans kMaxWindow / B + 2 features at most.
-  if (kMaxWindow / batch_size + 2 > kMaxWindowFeatures) return false;
+  if (!windows_derive_starts(batch_size)) return false;
   // Every block of every launch sums the lengths in front of its window
   // (about 1.3 us + 1 us per 40k lengths, measured); a separate scan costs
   // about 7 us once.  Take whichever is less.
@@ -737,8 +755,6 @@ static bool fused_scan_possible(const tra_tbe* tbe, int32_t batch_size, int32_t 
 // A pooled call too small for the window kernel whose lengths are few enough
 // that every block of the sixteen-lane kernel can sum the ones in front of its
 // bags itself: one launch instead of a scan and a lookup.
-constexpr int64_t kSmallFusedMaxLengths = 16384;
-
 static bool small_fused_scan_possible(const tra_tbe* tbe, int32_t batch_size, int32_t num_keys,
                                       int64_t num_indices, int32_t pooling_mode, const void* lengths) {
   if (pooling_mode == TRA_POOL_NONE || batch_size <= 0 || tbe->num_features == 0) return false;
