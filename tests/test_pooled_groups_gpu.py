@@ -46,8 +46,8 @@ def test_group_widths(tuning, dtype, weighted):
         assert bits_equal(got, want) == 0, B
 
 
-# 32 and 64 lanes a bag, and what 64 cannot hold
-WIDE = {O.INT8: [100, 260, 264, 300, 504, 512, 1020, 1024, 1040], O.INT4: [264, 512, 520, 1024, 1032],
+# 32 and 64 lanes a bag, and what 64 cannot hold (int8 of 144 and 256: 32 where bags are few, else 16)
+WIDE = {O.INT8: [100, 144, 256, 260, 264, 300, 504, 512, 1020, 1024, 1040], O.INT4: [264, 512, 520, 1024, 1032],
         O.INT2: [272, 512, 1024, 1040], O.FP16: [130, 136, 256, 258, 512, 522], O.FP32: [65, 68, 128, 130, 256, 259, 516]}
 
 

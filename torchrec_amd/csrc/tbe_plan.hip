@@ -108,6 +108,8 @@ static Overrides g_ovr = overrides_from_env();
 // Bumped by tra_set_tuning: launch geometry remembered under an older value is recomputed.
 static std::atomic<int> g_ovr_gen{0};
 
+constexpr int kFewBags = 8;  // per compute unit
+
 // How the sixteen-lane kernel takes the columns of a row from `off` on: the first slice of them.
 struct GroupShape {
   int ne;  // columns per lane
@@ -122,10 +124,13 @@ struct GroupShape {
 // 10.9 / 10.2, 6400 bags 28.4 / 24.0; int8 300, 512 bags 10.5 / 8.3; int4 512, 6400 bags of 45 45.2 / 38.7; fp16 512
 // 55.6 / 50.3; fp32 256 53.3 / 48.8.  What is cut starts with a slice of half the most columns a lane can hold (int8 300:
 // 64 lanes of 4 columns 7.5 and 45.3 us at 512 bags of 20 and 6400 of 45, 32 of 8 8.3 and 43.1, 16 of 16 10.5 and 39.5).
-static GroupShape group_shape(int dtype, int dim, int off) {
+// few: the call has few bags (kFewBags).  int8 rows that need 16 columns of each of sixteen lanes go by 32 lanes then,
+// for a shorter chain per bag (us, 16 / 32 lanes: 192 columns, 128 bags of 3 5.4 / 4.7, of 20 8.9 / 7.2, 2048 bags
+// 5.9 / 5.4 and 10.2 / 9.0, but 3072 bags 6.0 / 6.3 and 10.4 / 10.6, 6400 bags of up to 45 16.5 / 18.5).
+static GroupShape group_shape(int dtype, int dim, int off, bool few) {
   const int bits = bits_of(dtype), left = dim - off;
   const int most = dtype == TRA_FP32 ? 4 : dtype == TRA_FP16 ? 8 : 16;
-  for (int log2 = 4; log2 <= 6; ++log2) {
+  for (int log2 = few && dtype == TRA_INT8 && dim > 128 ? 5 : 4; log2 <= 6; ++log2) {
     // (more than sixteen lanes, or a part of the row: with a header, the kernel's split kinds, whole dwords a lane)
     const int least = header_bytes(dtype) != 0 && (log2 > 4 || off > 0) ? 32 / bits : 1;
     for (int ne = least; ne <= most; ne *= 2)
@@ -248,6 +253,11 @@ constexpr int kGeometrySlots = 8;
 // are even (-1 %, +0.5 %), five gain 8 %, seven (of about 50 us) 9 %.
 constexpr size_t kForkMinClasses = 5;
 
+struct GroupSlices {
+  std::vector<GroupSlice> host;
+  GroupSlice* dev = nullptr;
+};
+
 struct tra_tbe {
   int device = 0;
   int num_cus = 256;  // compute units of the device (hipDeviceProp_t::multiProcessorCount)
@@ -285,8 +295,7 @@ struct tra_tbe {
   FeatureDesc* multi_descs_dev = nullptr;
   LookupArgs multi_base;
   // Column slices for the sixteen-lane kernel, in feature order.
-  std::vector<GroupSlice> group_slices;
-  GroupSlice* group_slices_dev = nullptr;
+  GroupSlices group_slices[2];  // [1]: calls of few bags (kFewBags), where they differ
   std::mutex geo_mutex;
   std::shared_ptr<const Geometry> geo[kGeometrySlots];
   int geo_next = 0;
@@ -421,29 +430,30 @@ int tra_tbe_create(const tra_table_spec* tables, int32_t num_tables,
       slice_lpr.push_back(bytes / cb);
     }
     // The sixteen-lane kernel's slices.
-    for (int off = 0; off < s.dim;) {
-      const GroupShape shape = group_shape(s.dtype, s.dim, off);
-      GroupSlice w;
-      w.table_offset = s.offset;
-      w.rows = s.rows;
-      w.rows32 = (uint32_t)std::min<int64_t>(s.rows, int64_t(1) << 31);
-      w.row_bytes = s.row_bytes;
-      w.cols = shape.cols;
-      w.out_col = col + off;
-      w.payload = header_bytes(s.dtype) + off * bits / 8;
-      w.key = feature_positions ? feature_positions[f] : f;
-      w.even = w.out_col % 2 == 0 ? 1 : 0;
-      w.first_slice = off == 0 ? 1 : 0;
-      w.lanes_log2 = (uint8_t)shape.lanes_log2;
-      // (near: row offset and place in the row are added in 32 bits)
-      const bool split = header_bytes(s.dtype) != 0 && (shape.cols < s.dim || shape.lanes_log2 > 4);
-      w.kind = group_kind(s.dtype, shape.ne, split ? kSplit : s.rows * s.row_bytes > 0xffffffffll ? kFar : kNear);
-      for (int part = 0; part < (1 << shape.lanes_log2) / 16; ++part) {
-        w.part = (uint8_t)part;
-        plan->group_slices.push_back(w);
+    for (const bool few : {false, true})
+      for (int off = 0; off < s.dim;) {
+        const GroupShape shape = group_shape(s.dtype, s.dim, off, few);
+        GroupSlice w;
+        w.table_offset = s.offset;
+        w.rows = s.rows;
+        w.rows32 = (uint32_t)std::min<int64_t>(s.rows, int64_t(1) << 31);
+        w.row_bytes = s.row_bytes;
+        w.cols = shape.cols;
+        w.out_col = col + off;
+        w.payload = header_bytes(s.dtype) + off * bits / 8;
+        w.key = feature_positions ? feature_positions[f] : f;
+        w.even = w.out_col % 2 == 0 ? 1 : 0;
+        w.first_slice = off == 0 ? 1 : 0;
+        w.lanes_log2 = (uint8_t)shape.lanes_log2;
+        // (near: row offset and place in the row are added in 32 bits)
+        const bool split = header_bytes(s.dtype) != 0 && (shape.cols < s.dim || shape.lanes_log2 > 4);
+        w.kind = group_kind(s.dtype, shape.ne, split ? kSplit : s.rows * s.row_bytes > 0xffffffffll ? kFar : kNear);
+        for (int part = 0; part < (1 << shape.lanes_log2) / 16; ++part) {
+          w.part = (uint8_t)part;
+          plan->group_slices[few].host.push_back(w);
+        }
+        off += shape.cols;
       }
-      off += shape.cols;
-    }
     col += s.dim;
   }
   // Classes: slices sorted by lanes-per-row; at most kMaxSub distinct values each.
@@ -563,11 +573,12 @@ int tra_tbe_create(const tra_table_spec* tables, int32_t num_tables,
     if (e == hipSuccess)
       e = hipMemcpy(plan->multi_descs_dev, ordered.data(), ordered.size() * sizeof(FeatureDesc), hipMemcpyHostToDevice);
   }
-  if (e == hipSuccess && !plan->group_slices.empty()) {
-    e = hipMalloc((void**)&plan->group_slices_dev, plan->group_slices.size() * sizeof(GroupSlice));
-    if (e == hipSuccess)
-      e = hipMemcpy(plan->group_slices_dev, plan->group_slices.data(), plan->group_slices.size() * sizeof(GroupSlice),
-                    hipMemcpyHostToDevice);
+  // (other lanes per bag are another number of descriptors)
+  if (plan->group_slices[1].host.size() == plan->group_slices[0].host.size()) plan->group_slices[1].host.clear();
+  for (GroupSlices& g : plan->group_slices) {
+    const size_t bytes = g.host.size() * sizeof(GroupSlice);
+    if (e == hipSuccess && bytes > 0) e = hipMalloc((void**)&g.dev, bytes);
+    if (e == hipSuccess && bytes > 0) e = hipMemcpy(g.dev, g.host.data(), bytes, hipMemcpyHostToDevice);
   }
   if (e == hipSuccess) e = hipMalloc((void**)&plan->err_dev, sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMemset(plan->err_dev, 0, sizeof(unsigned long long));
@@ -639,7 +650,8 @@ int tra_tbe_destroy(tra_tbe_t tbe) {
   if (tbe->slices_dev) (void)hipFree(tbe->slices_dev);
   if (tbe->feats_dev) (void)hipFree(tbe->feats_dev);
   if (tbe->cdescs_dev) (void)hipFree(tbe->cdescs_dev);
-  if (tbe->group_slices_dev) (void)hipFree(tbe->group_slices_dev);
+  for (const GroupSlices& g : tbe->group_slices)
+    if (g.dev) (void)hipFree(g.dev);
   if (tbe->multi_descs_dev) (void)hipFree(tbe->multi_descs_dev);
   if (tbe->err_dev) (void)hipFree(tbe->err_dev);
   if (tbe->side) (void)hipStreamDestroy(tbe->side);
@@ -697,6 +709,12 @@ static bool use_window_kernel(const tra_tbe* tbe, const Tuning& tune, bool nobag
   return !nobag && tune.balanced && batch_size <= (1 << kBagBits) && tbe->max_key_pos <= 32767 &&
          (int64_t)tbe->max_class_feats < (int64_t(1) << (32 - kBagBits)) &&
          (int64_t)tbe->max_class_feats * batch_size < (int64_t(1) << 31);
+}
+
+// The sixteen-lane kernel's slices for a call.
+static const GroupSlices& group_slices_of(const tra_tbe* tbe, int32_t batch_size) {
+  const bool few = (int64_t)tbe->num_features * batch_size <= kFewBags * (int64_t)tbe->num_cus;
+  return tbe->group_slices[few && tbe->group_slices[1].dev != nullptr];
 }
 
 // Whether launches on a stream are being captured into a graph (or the runtime cannot say).
@@ -787,7 +805,7 @@ int tra_tbe_launch_info(tra_tbe_t tbe, int32_t batch_size, int64_t num_indices,
   if (!nobag && (multi || !balanced)) {
     char line[120];
     snprintf(line, sizeof(line), "%s slices=%d%s", multi ? "tbe_pooled_multi_kernel" : "tbe_pooled_kernel",
-             (int)(multi ? tbe->multi_feats.size() : tbe->group_slices.size()), fused ? " from_lengths" : "");
+             (int)(multi ? tbe->multi_feats.size() : group_slices_of(tbe, batch_size).host.size()), fused ? " from_lengths" : "");
     text = line;
   }
   // In launch order; a plan with a second stream alternates between the two.
@@ -833,7 +851,7 @@ struct SequenceBounds {
 static GroupLaunch group_windows(const tra_tbe* tbe, int32_t batch_size) {
   GroupLaunch l{};
   constexpr int groups = kBlockThreads / 16;
-  const int64_t bags = (int64_t)tbe->group_slices.size() * batch_size;
+  const int64_t bags = (int64_t)group_slices_of(tbe, batch_size).host.size() * batch_size;
   const int64_t at_once = 4 * (int64_t)tbe->num_cus * groups;
   const int64_t per_group = std::min<int64_t>((bags + at_once - 1) / at_once, 16);
   l.per_group = (int)std::min<int64_t>(per_group, (batch_size + groups - 1) / groups);
@@ -1181,11 +1199,12 @@ static int forward_impl(tra_tbe_t tbe, const void* weights, const void* indices,
     a.pairs = (uintptr_t)out % 4 == 0 && out_stride % 2 == 0;
     a.bad_to_row0 = tbe->bad_to_row0.load(std::memory_order_relaxed) != 0;
     // (position weights: the launch arguments hold the layout of kMaxPos slices)
-    const size_t step = positions ? kMaxPos : tbe->group_slices.size();
-    for (size_t s0 = 0; s0 < tbe->group_slices.size(); s0 += step) {
-      const size_t n = std::min(step, tbe->group_slices.size() - s0);
-      const GroupSlice* slices = tbe->group_slices.data() + s0;
-      a.slices = tbe->group_slices_dev + s0;
+    const GroupSlices& all = group_slices_of(tbe, batch_size);
+    const size_t step = positions ? kMaxPos : all.host.size();
+    for (size_t s0 = 0; s0 < all.host.size(); s0 += step) {
+      const size_t n = std::min(step, all.host.size() - s0);
+      const GroupSlice* slices = all.host.data() + s0;
+      a.slices = all.dev + s0;
       GroupPositions p;
       if (positions) {
         const int rc = fill_positions(p.off, p.len, n, [&](size_t i) { return slices[i].key; });
