@@ -7,8 +7,9 @@
 namespace tra {
 
 // As tbe_pooled_cu_kernel, with blocks of all weight types and lane chunks in one grid: a block pools bags of one
-// sub-class and picks its body by it.  Lane chunks are at most 16 accumulators wide here, so that every body fits the
-// registers that sixteen waves leave each other.
+// sub-class and picks its body by it.  Lane chunks are at most 16 accumulators wide here: wider bodies would not fit the
+// 128 registers that sixteen waves leave each other.  With 32-bit ids they do, but for 4 registers with position weights;
+// with 64-bit ids 2 are kept in scratch memory without weights, 17 with per-sample and 24 with position weights.
 template <typename IdxT, int WEIGHTED, bool FROM_LENGTHS>
 __global__ __launch_bounds__(kCuThreads) void tbe_pooled_multi_kernel(const void* p_offsets, const FeatureDesc* p_cdescs,
                                                                       int32_t p_B, int32_t p_xcd_blocks,
