@@ -13,7 +13,8 @@ from torchrec_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
-# one lane's columns change at 16, 32, 64, 128 and 256; 100, 300 and 520 (int8), 200 (int4) are several slices
+# one lane's columns change at 16, 32, 64, 128 and 256; 100 (int8) and 200 (int4) go by 32 lanes, 264 (int4) by 64;
+# 300 and 520 (int8), 130 (fp16), 65 (fp32) are several slices
 DIMS = {O.INT8: [4, 16, 20, 32, 64, 72, 100, 128, 256, 300, 520], O.INT4: [8, 16, 40, 64, 104, 128, 200, 256, 264],
         O.INT2: [16, 32, 64, 80, 256, 272], O.FP16: [2, 16, 18, 64, 66, 128, 130, 256], O.FP32: [1, 16, 17, 33, 64, 65, 128]}
 

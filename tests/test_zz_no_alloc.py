@@ -77,7 +77,7 @@ def test_static_scratch_entry_two_calls_in_a_row():
     rows_f = [s[1] for s in specs]
     buf = ctypes.create_string_buffer(512)
     # call 1: 4 x 40000 bags: scan in tiles (partial sums in the scratch), window kernel from offsets
-    # call 2: 4 x 5000 bags of few ids: one-launch scan into the scratch, static kernel
+    # call 2: 4 x 5000 bags of few ids: one-launch scan into the scratch, sixteen-lane kernel
     # (a call of at most 16384 lengths would not touch the scratch at all: its one kernel
     # derives the bag starts itself)
     for B, max_len in ((40_000, 6), (5000, 5)):
@@ -112,12 +112,15 @@ def test_static_scratch_entry_under_graph_capture():
     rng = np.random.default_rng(99)
     specs = [(O.INT4, 3000, 64), (O.INT8, 2500, 64), (O.INT4, 2000, 64), (O.INT8, 1500, 64)]
     tbe, _ = _operator(rng, specs)
-    K, total_D, B = len(specs), 64 * len(specs), 6000
+    K, total_D, B = len(specs), 64 * len(specs), 5000
     assert K * B > 16384
     rows_f = [s[1] for s in specs]
     lib = _lib.lib()
     plan = tbe._get_plan(None)
     cap = K * B * 5
+    buf = ctypes.create_string_buffer(512)
+    _lib.check(lib.tra_tbe_launch_info(plan, B, cap, _lib.POOL_SUM, K, buf, 512))
+    assert b"scan" in buf.value and b"from_lengths" not in buf.value, buf.value  # (20,480 bags and more derive their starts)
     ti = torch.zeros(cap, dtype=torch.int32, device=DEV)
     tl = torch.zeros(K * B, dtype=torch.int32, device=DEV)
     out = torch.zeros(B, total_D, dtype=torch.float16, device=DEV)
