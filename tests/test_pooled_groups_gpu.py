@@ -211,3 +211,22 @@ def test_one_class_line_to_the_window_kernel(idt, weighted):
         assert kernel in text and ("scan" not in text) == (T * B <= 16384), (T, B, text)
         want = O.tbe_forward(store, list(range(T)), B, ids, offsets, psw, O.SUM, O.FP32)
         assert bits_equal(_from_lengths(tbe, ids, lengths, psw, B), want) == 0, (T, B)
+
+
+@pytest.mark.parametrize("T", [64, 65])
+def test_few_bags_take_one_launch_of_position_weights(T):
+    """int8 rows of 256 columns go by 32 lanes, two descriptors each, where bags are few, but not beyond the 128 that a
+    launch describes position weights for."""
+    rng = np.random.default_rng(T)
+    tbe, store = build(rng, [(O.INT8, 20, 256)] * T, list(range(T)), O.SUM, O.FP32, 16)
+    B = 3
+    assert f"slices={128 if T == 64 else T}" in _launch_text(tbe, B, 10, T)
+    lengths = rng.integers(0, 4, T * B).astype(np.int32)
+    offsets = np.zeros(T * B + 1, dtype=np.int32)
+    offsets[1:] = np.cumsum(lengths)
+    ids = rng.integers(0, 20, int(offsets[-1])).astype(np.int32)
+    table = rng.uniform(-1, 1, 6 * T).astype(np.float32)
+    place, key = np.arange(len(ids)) - np.repeat(offsets[:-1], lengths), np.repeat(np.arange(T * B) // B, lengths)
+    want = O.tbe_forward(store, list(range(T)), B, ids, offsets, table[6 * key + place], O.SUM, O.FP32)
+    pw = (torch.from_numpy(table).to(DEV), [6 * t for t in range(T)], [6] * T)
+    assert bits_equal(_from_lengths(tbe, ids, lengths, None, B, position_weights=pw), want) == 0

@@ -573,12 +573,19 @@ int tra_tbe_create(const tra_table_spec* tables, int32_t num_tables,
     if (e == hipSuccess)
       e = hipMemcpy(plan->multi_descs_dev, ordered.data(), ordered.size() * sizeof(FeatureDesc), hipMemcpyHostToDevice);
   }
-  // (other lanes per bag are another number of descriptors)
-  if (plan->group_slices[1].host.size() == plan->group_slices[0].host.size()) plan->group_slices[1].host.clear();
-  for (GroupSlices& g : plan->group_slices) {
-    const size_t bytes = g.host.size() * sizeof(GroupSlice);
-    if (e == hipSuccess && bytes > 0) e = hipMalloc((void**)&g.dev, bytes);
-    if (e == hipSuccess && bytes > 0) e = hipMemcpy(g.dev, g.host.data(), bytes, hipMemcpyHostToDevice);
+  // (other lanes per bag are another number of descriptors; beyond kMaxPos position weights would take more launches)
+  const size_t few_slices = plan->group_slices[1].host.size();
+  if (few_slices == plan->group_slices[0].host.size() || few_slices > kMaxPos) plan->group_slices[1].host.clear();
+  if (e == hipSuccess && !plan->group_slices[0].host.empty()) {
+    // (both sets in one buffer)
+    GroupSlices& few = plan->group_slices[1];
+    std::vector<GroupSlice> all = plan->group_slices[0].host;
+    all.insert(all.end(), few.host.begin(), few.host.end());
+    GroupSlice* dev = nullptr;
+    e = hipMalloc((void**)&dev, all.size() * sizeof(GroupSlice));
+    plan->group_slices[0].dev = dev;
+    if (e == hipSuccess) e = hipMemcpy(dev, all.data(), all.size() * sizeof(GroupSlice), hipMemcpyHostToDevice);
+    if (!few.host.empty()) few.dev = dev + plan->group_slices[0].host.size();
   }
   if (e == hipSuccess) e = hipMalloc((void**)&plan->err_dev, sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMemset(plan->err_dev, 0, sizeof(unsigned long long));
@@ -650,8 +657,7 @@ int tra_tbe_destroy(tra_tbe_t tbe) {
   if (tbe->slices_dev) (void)hipFree(tbe->slices_dev);
   if (tbe->feats_dev) (void)hipFree(tbe->feats_dev);
   if (tbe->cdescs_dev) (void)hipFree(tbe->cdescs_dev);
-  for (const GroupSlices& g : tbe->group_slices)
-    if (g.dev) (void)hipFree(g.dev);
+  if (tbe->group_slices[0].dev) (void)hipFree(tbe->group_slices[0].dev);
   if (tbe->multi_descs_dev) (void)hipFree(tbe->multi_descs_dev);
   if (tbe->err_dev) (void)hipFree(tbe->err_dev);
   if (tbe->side) (void)hipStreamDestroy(tbe->side);
