@@ -53,6 +53,9 @@ def _both_entries(tbe, ids, lengths, B, K, total_D):
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=DEV)
     args = (plan, _lib.ptr(tbe.weights_dev), _lib.ptr(ti), _lib.ptr(tl), 0, None, B, K, len(ids),
             _lib.POOL_SUM, _lib.FP16)
+    # (the runtime loads a kernel's code on its first launch, whichever entry that comes from)
+    _lib.check(lib.tra_tbe_forward_lengths(*args, out_ws.data_ptr(), total_D, ws.data_ptr(), stream))
+    out_ws.fill_(9.0)
     # the static entry allocates nothing: neither from the device (hipMemGetInfo) nor from torch's pools
     torch.cuda.synchronize()
     free_before, _ = torch.cuda.mem_get_info(DEV)
