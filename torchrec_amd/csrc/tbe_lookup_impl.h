@@ -958,47 +958,59 @@ struct PrefixSumAtOnce {
   const Vec* vin;
   int tid, nt, nvec, last;
 
-  template <int N>
-  __device__ __forceinline__ S steps(int k0) const {
+  template <int N, bool TWO>
+  __device__ __forceinline__ void steps(int k0, S& part, int nvec2, S& part2) const {
     Vec x[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) x[k] = vin[min((k0 + k) * nt + tid, last)];
-    S part = 0;
 #pragma unroll
     for (int k = 0; k < N; ++k) {
       S sum = 0;
 #pragma unroll
       for (int i = 0; i < V; ++i) sum += (S)x[k].v[i];
       part += (k0 + k) * nt + tid < nvec ? sum : (S)0;
+      if constexpr (TWO) part2 += (k0 + k) * nt + tid < nvec2 ? sum : (S)0;
     }
-    return part;
   }
-  // This thread's share of sum(lengths[0 .. p)); thread tid_ of nt_.
-  __device__ __forceinline__ S run(const IdxT* __restrict__ lengths, int64_t p, int tid_, int nt_) {
+  // The elements of [0, p) after the last whole 16-byte step: one per thread.
+  __device__ __forceinline__ S tail(const IdxT* __restrict__ lengths, int64_t p) const {
+    const int64_t whole = p / V * V, rest = p - whole;
+    const int64_t ti = whole + min((int64_t)tid, max(rest - 1, (int64_t)0));
+    const IdxT x = lengths[max(min(ti, p - 1), (int64_t)0)];
+    return (int64_t)tid < rest ? (S)x : (S)0;
+  }
+  // This thread's share of sum(lengths[0 .. p)) and, TWO, of sum(lengths[0 .. p2)), both in one go over the longer of
+  // the two; thread tid_ of nt_.
+  template <bool TWO>
+  __device__ __forceinline__ void run(const IdxT* __restrict__ lengths, int64_t p, int64_t p2, int tid_, int nt_,
+                                      S& part, S& part2) {
     tid = tid_;
     nt = nt_;
     vin = reinterpret_cast<const Vec*>(lengths);
     nvec = (int)(p / V);
-    last = max(nvec - 1, 0);
-    const int nk = (nvec + nt - 1) / nt;
-    // the elements after the last whole 16-byte step: one per thread
-    const int64_t rest = p - (int64_t)nvec * V;
-    const int64_t ti = (int64_t)nvec * V + min((int64_t)tid, max(rest - 1, (int64_t)0));
-    IdxT tail = lengths[max(min(ti, p - 1), (int64_t)0)];
-    if ((int64_t)tid >= rest) tail = 0;
-    S part = 0;
+    const int nvec2 = TWO ? (int)(p2 / V) : 0, most = max(nvec, nvec2);
+    last = max(most - 1, 0);
+    const int nk = (most + nt - 1) / nt;
+    const S tail1 = tail(lengths, p), tail2 = TWO ? tail(lengths, p2) : (S)0;
+    part = part2 = 0;
     int k0 = 0;
-    for (; nk - k0 > 16; k0 += 16) part += steps<16>(k0);
+    for (; nk - k0 > 16; k0 += 16) steps<16, TWO>(k0, part, nvec2, part2);
     const int r = nk - k0;
     if (r > 12)
-      part += steps<16>(k0);
+      steps<16, TWO>(k0, part, nvec2, part2);
     else if (r > 8)
-      part += steps<12>(k0);
+      steps<12, TWO>(k0, part, nvec2, part2);
     else if (r > 4)
-      part += steps<8>(k0);
+      steps<8, TWO>(k0, part, nvec2, part2);
     else if (r > 0)
-      part += steps<4>(k0);
-    return part + (S)tail;
+      steps<4, TWO>(k0, part, nvec2, part2);
+    part += tail1;
+    part2 += tail2;
+  }
+  __device__ __forceinline__ S run(const IdxT* __restrict__ lengths, int64_t p, int tid_, int nt_) {
+    S part, none;
+    run<false>(lengths, p, 0, tid_, nt_, part, none);
+    return part;
   }
 };
 
@@ -1023,6 +1035,11 @@ __device__ __forceinline__ int64_t wave_scan_incl(int64_t v) {
     if (ln >= off) v += o;
   }
   return v;
+}
+// A value that is the same in every lane, in scalar registers.
+__device__ __forceinline__ int32_t uniform(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t uniform(int64_t v) {
+  return (int64_t)(((uint64_t)(uint32_t)uniform((int32_t)(v >> 32)) << 32) | (uint32_t)uniform((int32_t)v));
 }
 // Lane 63's value of v, in every lane.
 __device__ __forceinline__ int32_t wave_last(int32_t v) { return __builtin_amdgcn_readlane(v, kWaveSize - 1); }
@@ -1081,6 +1098,13 @@ struct Window {
   __shared__ int s_taken;                                                                            \
   const Window<IdxT> name{s_start, s_len, s_ent, s_order, s_slot, s_hist, s_desc, s_red, s_wave_tot, &s_taken}
 
+// What a staged window's bag starts in LDS still lack: `add`, and from the sub-class's feature `second` on `second_add`.
+template <typename Sum>
+struct WindowStarts {
+  Sum add = 0, second_add = 0;
+  int second = INT32_MAX;
+};
+
 // The launch arguments that pooling reads, asked for together while the window is staged: fetched one behind the
 // other after the staging's barrier, as the compiler places them, they cost every wave a trip to memory each with
 // nothing else in flight (graph replays, us, without / with this: 26 int4 tables of 128 columns, 2048 samples
@@ -1090,15 +1114,14 @@ __device__ __forceinline__ void hold_pool_args(const LookupArgs& a) {
                "s"(a.mean), "s"(a.vec_store), "s"(a.out_fp16), "s"(a.bad_to_row0));
 }
 
-// Stages bags [q0, q0 + nb) of a sub-class and ranks them by length; returns what their starts in LDS still lack.
+// Stages bags [q0, q0 + nb) of a sub-class and ranks them by length.
 // FROM_LENGTHS: p_offsets points at the KJT's lengths instead of its offsets
 // and the block derives its bags' start positions itself: one block-wide sum
 // of everything in front of the window plus a scan of the window in LDS.
 template <typename IdxT, bool FROM_LENGTHS>
-__device__ __forceinline__ typename SumOf<IdxT>::type stage_window(const Window<IdxT> w, const LookupArgs& a,
-                                                                   const void* p_offsets, const FeatureDesc* p_cdescs,
-                                                                   int32_t p_B, const SubClass& sc, int q0, int nb,
-                                                                   int fi_lo) {
+__device__ __forceinline__ WindowStarts<typename SumOf<IdxT>::type> stage_window(
+    const Window<IdxT> w, const LookupArgs& a, const void* p_offsets, const FeatureDesc* p_cdescs, int32_t p_B,
+    const SubClass& sc, int q0, int nb, int fi_lo) {
   using Sum = typename SumOf<IdxT>::type;
 
   // Bag q0 + i of the window: where it sits in the offsets (or lengths) array.
@@ -1108,15 +1131,36 @@ __device__ __forceinline__ typename SumOf<IdxT>::type stage_window(const Window<
     b = q - fi * p_B;
     return (int64_t)feat_key_pos(a, sc, fi) * p_B + b;
   };
-  // What a bag's start in LDS still lacks (from lengths, small windows: the sum
-  // of everything in front of the window arrives last and is added on reading).
-  Sum front_add = 0;
+  WindowStarts<Sum> starts;
   if (threadIdx.x == 0) *w.taken = 0;
   // A window of at most 4 x 64 bags is staged, scanned and ranked by the
   // block's first wave alone, four consecutive bags per lane, with no block
   // barrier on the way; from lengths, the other fifteen waves meanwhile sum
   // the lengths in front of the window.  One barrier joins the two.
-  const bool solo = FROM_LENGTHS && nb <= 4 * kWaveSize && sc.key0 >= 0;
+  // The features' keys need not follow one another: a window whose bags lie in
+  // two runs has both runs' fronts summed in one go (graph replays, us, the
+  // general route for keys out of order / this: 26 int4 tables of 128 columns, 2048
+  // samples 31.1 / 29.2; 64 int8 tables of 64 columns, 300 samples 15.4 / 13.9, 40 of
+  // them, 1000 samples of 64-bit ids 26.8 / 24.2; a position-weighted call of 20
+  // features 22.8 / 21.3).
+  bool solo = FROM_LENGTHS && nb <= 4 * kWaveSize;
+  int key_lo = 0, key_second = 0;  // key positions of the window's first feature and of the second run's
+  if (solo) {
+    key_lo = feat_key_pos(a, sc, fi_lo);
+    if (sc.key0 < 0) {
+      const int fi_hi = (q0 + nb - 1) / p_B;
+      int before = key_lo;
+      for (int fi = fi_lo + 1; fi <= fi_hi; ++fi) {
+        const int key = feat_key_pos(a, sc, fi);
+        if (key != before + 1) {
+          solo = solo && starts.second == INT32_MAX;
+          starts.second = fi;
+          key_second = key;
+        }
+        before = key;
+      }
+    }
+  }
   if (solo) {
     const int wv = threadIdx.x / kWaveSize;
     const int ln = threadIdx.x & (kWaveSize - 1);
@@ -1125,8 +1169,11 @@ __device__ __forceinline__ typename SumOf<IdxT>::type stage_window(const Window<
       int fis[4], bs[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const int64_t bag = bag_of(min(4 * ln + k, nb - 1), fis[k], bs[k]);
-        given[k] = reinterpret_cast<const IdxT*>(p_offsets)[bag];
+        const int q = q0 + min(4 * ln + k, nb - 1);
+        fis[k] = q / p_B;
+        bs[k] = q - fis[k] * p_B;
+        const int key = fis[k] < starts.second ? key_lo + (fis[k] - fi_lo) : key_second + (fis[k] - starts.second);
+        given[k] = reinterpret_cast<const IdxT*>(p_offsets)[(int64_t)key * p_B + bs[k]];
       }
       {
         const int nfeat = min((q0 + nb - 1) / p_B - fi_lo + 1, kMaxWinFeat);
@@ -1189,16 +1236,32 @@ __device__ __forceinline__ typename SumOf<IdxT>::type stage_window(const Window<
         if (4 * ln + k < nb) w.order[w.hist[length_bin(len[k])] + slot[k]] = (uint16_t)(4 * ln + k);
     } else {
       PrefixSumAtOnce<IdxT> front_sum;
-      const Sum mine = front_sum.run(reinterpret_cast<const IdxT*>(p_offsets),
-                                     (int64_t)feat_key_pos(a, sc, fi_lo) * p_B + (q0 - fi_lo * p_B),
-                                     (int)threadIdx.x - kWaveSize, kCuThreads - kWaveSize);
+      const IdxT* lengths = reinterpret_cast<const IdxT*>(p_offsets);
+      const int64_t p = (int64_t)key_lo * p_B + (q0 - fi_lo * p_B);
+      const int tid = (int)threadIdx.x - kWaveSize, nt = kCuThreads - kWaveSize;
+      Sum mine, second;
+      if (starts.second == INT32_MAX) {
+        mine = front_sum.run(lengths, p, tid, nt);
+      } else {
+        front_sum.template run<true>(lengths, p, (int64_t)key_second * p_B, tid, nt, mine, second);
+        second = wave_last(wave_scan_incl(second));
+        if (ln == 0) w.wave_tot[wv] = second;
+      }
       hold_pool_args(a);
       const Sum front_w = wave_last(wave_scan_incl(mine));
       if (ln == 0) w.red[wv] = front_w;
     }
     lds_barrier();
 #pragma unroll
-    for (int v = 0; v < kCuWaves; ++v) front_add += w.red[v];
+    for (int v = 0; v < kCuWaves; ++v) starts.add += w.red[v];
+    if (starts.second != INT32_MAX) {
+      // (its bags' starts in LDS go on from the first run's)
+      starts.second_add = (Sum)-w.start[starts.second * p_B - q0];
+#pragma unroll
+      for (int v = 1; v < kCuWaves; ++v) starts.second_add += w.wave_tot[v];
+      starts.second_add = uniform(starts.second_add);
+    }
+    starts.add = uniform(starts.add);
     TRA_STAMP(2);
   } else {
     // The first bag of every thread is requested before anything else: the
@@ -1349,7 +1412,7 @@ __device__ __forceinline__ typename SumOf<IdxT>::type stage_window(const Window<
     TRA_STAMP(2);
   }
 
-  return front_add;
+  return starts;
 }
 
 // Which pooling bodies a kernel instance holds (see odd_lanes).
@@ -1359,7 +1422,8 @@ constexpr int kBodiesEven = 0;  // id blocks for powers of two from eight lanes,
 // Pools a staged window.  vec(): whether every lane's output slice is 16-byte aligned (asked where a bag is stored).
 template <int DTYPE, int CB, typename IdxT, int WEIGHTED, int U, int BODIES, typename Vec>
 __device__ __forceinline__ void pool_window(const Window<IdxT> win, const LookupArgs& a, const SubClass& sc, int nb,
-                                            int fi_lo, typename SumOf<IdxT>::type front_add, Vec&& vec) {
+                                            int fi_lo, const WindowStarts<typename SumOf<IdxT>::type> starts,
+                                            Vec&& vec) {
   constexpr int NE = CB * 8 / Traits<DTYPE>::kBits;
   constexpr bool ODD = BODIES == kBodiesOdd;
   const int lane = threadIdx.x & (kWaveSize - 1);
@@ -1387,7 +1451,7 @@ __device__ __forceinline__ void pool_window(const Window<IdxT> win, const Lookup
     const int fi = (int)(ent >> kBagBits);
     const int b = (int)(ent & ((1u << kBagBits) - 1));
     const FeatureDesc d = fi - fi_lo < kMaxWinFeat ? win.desc[fi - fi_lo] : a.cdescs[sc.first + fi];
-    const int64_t start = win.start[i] + (int64_t)front_add;
+    const int64_t start = win.start[i] + (int64_t)(fi < starts.second ? starts.add : starts.second_add);
     const int len = active ? max(win.len[i], 0) : 0;
     // The round's trip count.  Lengths below 192 have a sort bin each, so
     // the round's first bag is its longest; from 192 up a bin holds a range of
@@ -1483,8 +1547,8 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
   const int nb = min(sc.window, nb_all - q0);
 
   const int fi_lo = q0 / p_B;
-  const auto front_add = stage_window<IdxT, FROM_LENGTHS>(s_window, a, p_offsets, p_cdescs, p_B, sc, q0, nb, fi_lo);
-  pool_window<DTYPE, CB, IdxT, WEIGHTED, U, ODD ? kBodiesOdd : kBodiesEven>(s_window, a, sc, nb, fi_lo, front_add,
+  const auto starts = stage_window<IdxT, FROM_LENGTHS>(s_window, a, p_offsets, p_cdescs, p_B, sc, q0, nb, fi_lo);
+  pool_window<DTYPE, CB, IdxT, WEIGHTED, U, ODD ? kBodiesOdd : kBodiesEven>(s_window, a, sc, nb, fi_lo, starts,
                                                                              [&] { return a.vec_store != 0; });
 }
 

@@ -8,8 +8,8 @@ namespace tra {
 
 // As tbe_pooled_cu_kernel, with blocks of all weight types and lane chunks in one grid: a block pools bags of one
 // sub-class and picks its body by it.  Lane chunks are at most 16 accumulators wide here: wider bodies would not fit the
-// 128 registers that sixteen waves leave each other.  With 32-bit ids they do, but for 4 registers with position weights;
-// with 64-bit ids 2 are kept in scratch memory without weights, 17 with per-sample and 24 with position weights.
+// 128 registers that sixteen waves leave each other.  With 32-bit ids they do without weights; up to 6 registers are kept
+// in scratch memory with weights, with 64-bit ids up to 5 without, 15 with per-sample and 18 with position weights.
 template <typename IdxT, int WEIGHTED, bool FROM_LENGTHS>
 __global__ __launch_bounds__(kCuThreads) void tbe_pooled_multi_kernel(const void* p_offsets, const FeatureDesc* p_cdescs,
                                                                       int32_t p_B, int32_t p_xcd_blocks,
@@ -30,11 +30,11 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_multi_kernel(const void
   if (q0 >= nb_all) return;
   const int nb = min(sc.window, nb_all - q0);
   const int fi_lo = q0 / p_B;
-  const auto front_add = stage_window<IdxT, FROM_LENGTHS>(s_window, a, p_offsets, p_cdescs, p_B, sc, q0, nb, fi_lo);
+  const auto starts = stage_window<IdxT, FROM_LENGTHS>(s_window, a, p_offsets, p_cdescs, p_B, sc, q0, nb, fi_lo);
   const bool vec = (kind & kMultiVec) != 0;
 #define TRA_MULTI(D, CB)                                                                                       \
   case multi_kind(D, CB):                                                                                      \
-    pool_window<D, CB, IdxT, WEIGHTED, 4, kBodiesOdd>(s_window, a, sc, nb, fi_lo, front_add, [&] { return vec; }); \
+    pool_window<D, CB, IdxT, WEIGHTED, 4, kBodiesOdd>(s_window, a, sc, nb, fi_lo, starts, [&] { return vec; }); \
     break;
   switch (kind & ~kMultiVec) {
     TRA_MULTI(TRA_INT8, 16)
