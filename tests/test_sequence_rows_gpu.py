@@ -1,0 +1,80 @@
+"""The row ranges that a sequence collection hands out, against lookups of one key at a time."""
+import numpy as np
+import pytest
+import torch
+
+from torchrec_amd import KeyedJaggedTensor
+from torchrec_amd.modules.embedding_configs import DataType, EmbeddingConfig
+from torchrec_amd.quant import EmbeddingCollection as QuantEC
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def _collection(features, need_indices=False):
+    tables = [EmbeddingConfig(name="t%d" % i, embedding_dim=16, num_embeddings=97, feature_names=["f%d" % i],
+                              data_type=DataType.INT8) for i in range(features)]
+    module = QuantEC(tables, DEV, need_indices=need_indices, output_dtype=torch.float)
+    for op in module._emb_modules:
+        for payload, scale, bias in op.split_embedding_weights_with_scale_bias(2):
+            payload.view(torch.int32).random_(-(2**31), 2**31 - 1)
+            scale.uniform_(0.01, 0.02)
+            bias.uniform_(-1, 0)
+    return module
+
+
+# Ids per bag of each key; the collection's features among the keys (half of them and more: all ranges at once; fewer:
+# one by one), empty keys in front, between and behind, ids behind the last bag's, a negative length.
+@pytest.mark.parametrize("bags,used,tail", [
+    ([[1, 2]], [0], 0), ([[0, 0], [3, 1], [0, 0]], [0, 1, 2], 0), ([[4, 1], [0, 0], [2, 2], [1, 0]], [3, 0], 3),
+    ([[4, 1], [0, 5], [2, 2], [1, 0], [1, 1]], [2, 1], 2), ([[2, 1], [3, -1], [2, 2]], [0, 1, 2], 4),
+    ([[2, 1], [-4, 1], [2, 2]], [0, 1, 2], 9), ([[0, 0], [0, 0]], [1, 0], 1),
+])
+@pytest.mark.parametrize("counts_known", [False, True])
+@pytest.mark.parametrize("need_indices", [False, True])
+def test_row_ranges(bags, used, tail, counts_known, need_indices):
+    keys = [None] * len(bags)
+    for f, k in enumerate(used):
+        keys[k] = "f%d" % f
+    keys = [k or "unused%d" % i for i, k in enumerate(keys)]
+    module = _collection(len(used), need_indices)
+    per_key = [sum(b) for b in bags]
+    starts = np.concatenate([[0], np.cumsum(per_key)])
+    n = max(int(starts.max()), 0) + tail
+    ids = torch.randint(0, 97, (n,), device=DEV)
+    lengths = torch.tensor(sum(bags, []), device=DEV)
+    kjt = KeyedJaggedTensor(keys=keys, values=ids, lengths=lengths, length_per_key=per_key if counts_known else None)
+    out = module(kjt)
+    assert list(out) == ["f%d" % f for f in range(len(used))]
+    for f, k in enumerate(used):
+        jt = out["f%d" % f]
+        mine = ids[starts[k] : starts[k + 1]]
+        assert jt.values().shape == (mine.numel(), 16) and jt.values().is_contiguous()
+        assert jt.lengths().tolist() == bags[k]
+        if min(b for key in bags for b in key) >= 0:  # (else: which of the overlapping keys' rows are written is not said)
+            one = KeyedJaggedTensor(keys=["f%d" % i for i in range(len(used))], values=mine,
+                                    lengths=torch.tensor([mine.numel() if i == f else 0 for i in range(len(used))], device=DEV))
+            assert torch.equal(jt.values(), module(one)["f%d" % f].values())
+        assert (torch.equal(jt.weights(), mine)) if need_indices else jt.weights_or_none() is None
+
+
+def test_row_ranges_of_given_key_offsets():
+    module = _collection(2)
+    ids = torch.arange(8, device=DEV)
+    kjt = KeyedJaggedTensor(keys=["f0", "f1"], values=ids, lengths=torch.tensor([2, 1, 4, 1], device=DEV),
+                            offset_per_key=[0, 3, 8])
+    out = module(kjt)
+    assert [out[k].values().shape[0] for k in ("f0", "f1")] == [3, 5]
+    assert kjt.length_per_key_or_none() is None  # (nothing was added up for it)
+
+
+def test_rows_may_be_changed_in_place_with_a_gradient():
+    module = _collection(3)
+    kjt = KeyedJaggedTensor(keys=["f0", "f1", "f2"], values=torch.arange(9, device=DEV),
+                            lengths=torch.tensor([1, 2, 3, 0, 2, 1], device=DEV))
+    out = module(kjt)
+    before = out["f1"].values().clone()
+    scale = torch.full((1,), 2.0, device=DEV, requires_grad=True)
+    out["f1"].values().mul_(scale).sum().backward()
+    assert torch.allclose(scale.grad, before.sum())
+    assert not out["f0"].values().requires_grad

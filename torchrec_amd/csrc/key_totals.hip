@@ -76,7 +76,8 @@ struct MailSlot {
   int num_keys = 0;
 };
 static std::mutex g_mail_mutex;
-static int64_t* g_mail = nullptr;  // host address (the same pages are mapped into every GPU)
+static int64_t* g_mail = nullptr;      // host address (the same pages are mapped into every GPU)
+static int64_t* g_mail_dev = nullptr;  // their address there
 static uint64_t g_mail_used = 0;
 static MailSlot g_mail_slot[kMailSlots];
 
@@ -87,7 +88,14 @@ static int take_slot(int32_t* ticket) {
     const hipError_t e = hipHostMalloc(&p, sizeof(int64_t) * kMailSlots * kMailKeys,
                                        hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
     if (e != hipSuccess) return hip_fail(e, "hipHostMalloc(key totals)");
+    void* d = nullptr;
+    const hipError_t mapped = hipHostGetDevicePointer(&d, p, 0);
+    if (mapped != hipSuccess) {
+      (void)hipHostFree(p);
+      return hip_fail(mapped, "hipHostGetDevicePointer(totals)");
+    }
     g_mail = static_cast<int64_t*>(p);
+    g_mail_dev = static_cast<int64_t*>(d);
   }
   if (~g_mail_used == 0) {
     set_error("tra_key_totals_begin: %d calls are waiting for their totals already", kMailSlots);
@@ -122,13 +130,7 @@ int mail_open(hipStream_t s, int n, int32_t* ticket, int64_t** device) {
   int64_t* host = g_mail + (int64_t)slot * kMailKeys;
   for (int k = 0; k < n; ++k) host[k] = kMailEmpty;
   std::atomic_thread_fence(std::memory_order_release);
-  void* p = nullptr;
-  const hipError_t e = hipHostGetDevicePointer(&p, host, 0);
-  if (e != hipSuccess) {
-    mail_cancel(slot);
-    return hip_fail(e, "hipHostGetDevicePointer(totals)");
-  }
-  *device = static_cast<int64_t*>(p);
+  *device = g_mail_dev + (int64_t)slot * kMailKeys;
   g_mail_slot[slot].stream = s;
   g_mail_slot[slot].num_keys = n;
   *ticket = slot;

@@ -909,11 +909,24 @@ class EmbeddingCollection(EmbeddingCollectionInterface, ModuleNoCopyMixin, _Feat
             lookup = lookup[: offset_per_key[-1]]
         lengths_rows = torch.unbind(lengths, dim=0) if kjt_keys else ()
         need_indices = self._need_indices
+        names = self._flat_names()
+        # All keys' row ranges in one call where most of them are wanted: 0.3 us a range, a slice 0.9 us.  (Not as views
+        # of one function, which autograd does not let a caller change in place.)
+        rows = None
+        if kjt_keys and K <= 2 * len(order):
+            sizes = [end - start for start, end in zip(offset_per_key, offset_per_key[1:])]
+            behind = lookup.shape[0] - offset_per_key[K]
+            if offset_per_key[0] == 0 and behind >= 0 and min(sizes) >= 0:  # (lengths that are no partition: slices, which clip)
+                rows = lookup.unsafe_split_with_sizes([*sizes, behind] if behind else sizes)
+        if rows is not None and not need_indices:
+            of = JaggedTensor._of
+            return {name: of(rows[pos], lengths_rows[pos], None) for name, pos in zip(names, order)}
         feature_embeddings: Dict[str, JaggedTensor] = {}
-        for embedding_name, pos in zip(self._flat_names(), order):
+        for embedding_name, pos in zip(names, order):
             start, end = offset_per_key[pos], offset_per_key[pos + 1]
             feature_embeddings[embedding_name] = JaggedTensor._of(
-                lookup[start:end], lengths_rows[pos], indices[start:end] if need_indices else None
+                lookup[start:end] if rows is None else rows[pos], lengths_rows[pos],
+                indices[start:end] if need_indices else None,
             )
         return feature_embeddings
 
