@@ -3,6 +3,9 @@ import numpy as np
 import pytest
 import torch
 
+import oracle as O
+from helpers import bits_equal
+from test_tbe_gpu import build
 from torchrec_amd import KeyedJaggedTensor
 from torchrec_amd.modules.embedding_configs import DataType, EmbeddingConfig
 from torchrec_amd.quant import EmbeddingCollection as QuantEC
@@ -56,6 +59,31 @@ def test_row_ranges(bags, used, tail, counts_known, need_indices):
                                     lengths=torch.tensor([mine.numel() if i == f else 0 for i in range(len(used))], device=DEV))
             assert torch.equal(jt.values(), module(one)["f%d" % f].values())
         assert (torch.equal(jt.weights(), mine)) if need_indices else jt.weights_or_none() is None
+
+
+# One to sixteen 16-byte vectors of results per lane, rows that are and are not multiples of 16 bytes or of a line, lane
+# groups that leave lanes of the wave idle, a row in several column slices; tiles that begin at any row and end inside a
+# wave's step.
+@pytest.mark.parametrize("dtype,dims", [
+    (O.INT8, (4, 12, 32, 40, 72, 96, 104, 128, 192, 256, 1040)), (O.INT4, (8, 40, 64, 104, 128, 256, 512)),
+    (O.INT2, (16, 48, 64, 128, 256, 1024)), (O.FP16, (2, 8, 32, 36, 104, 128, 512)), (O.FP32, (1, 4, 36, 128, 256)),
+])
+@pytest.mark.parametrize("out", [O.FP16, O.FP32])
+def test_results_of_all_widths(dtype, dims, out):
+    rng = np.random.default_rng(int(dtype))
+    for dim in dims:
+        totals = [3, 0, 61, 1, 700, 5]
+        specs = [(dtype, 40 + 7 * t, dim) for t in range(3)]
+        ftm = [0, 0, 1, 1, 2, 2]
+        tbe, store = build(rng, specs, ftm, O.NONE, out, 16)
+        ids = np.concatenate([rng.integers(-1, specs[ftm[f]][1], n) for f, n in enumerate(totals)]).astype(np.int64)
+        starts = np.concatenate([[0], np.cumsum(totals)])
+        want = O.tbe_forward(store, ftm, 1, ids, starts, None, O.NONE, out)
+        guard = torch.full((ids.size + 40, dim), 7.0, dtype=torch.half if out == O.FP16 else torch.float, device=DEV)
+        tbe(indices=torch.from_numpy(ids).to(DEV), offsets=None, key_starts=starts.tolist(), out=guard)
+        got = guard.cpu().numpy()
+        assert bits_equal(got[: ids.size], want) == 0, dim
+        assert (got[ids.size :] == 7.0).all(), dim
 
 
 def test_row_ranges_of_given_key_offsets():

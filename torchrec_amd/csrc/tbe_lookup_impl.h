@@ -784,6 +784,29 @@ __device__ __forceinline__ void repool_bad_ids_as_row0(float (&acc)[NE], const L
 // (-0.5 to -1 us on the 13.6 MB output of the C2 workload).
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
+// Vector v (16 bytes) of a lane's NE outputs.
+template <int NE, bool FP16>
+__device__ __forceinline__ u32x4_t out_vector(const float (&acc)[NE], int v) {
+  u32x4_t x;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if constexpr (FP16) {
+      const uint32_t lo = __half_as_ushort(__float2half_rn(acc[8 * v + 2 * k]));
+      const uint32_t hi = __half_as_ushort(__float2half_rn(acc[8 * v + 2 * k + 1]));
+      x[k] = lo | (hi << 16);
+    } else {
+      x[k] = __builtin_bit_cast(uint32_t, acc[4 * v + k]);
+    }
+  }
+  return x;
+}
+
+// Where a wave puts vector k of lane's V in LDS: lane by lane, the vectors of neighbouring lanes in different banks.
+template <int V>
+__device__ __forceinline__ int stage_slot(int lane, int k) {
+  return lane * V + (k ^ (lane & (V - 1)));
+}
+
 template <int NE>
 __device__ __forceinline__ void finish_bag(float (&acc)[NE], const LookupArgs& a, int len,
                                            int64_t row_pos, int c, int lpr, int lane, bool active, bool vec) {

@@ -24,26 +24,46 @@ __device__ __forceinline__ void sequence_bounds(const LookupArgs& a, int ci, int
   n = last > first ? last - first : 0;
 }
 
-// Lane c's NE outputs of the row slice at `pos`.  Results are written once and read by a later kernel: as whole
-// lines with the non-temporal hint where a lane holds one or two 16-byte vectors (finish_bag exchanges two).
-template <int NE>
-__device__ __forceinline__ void store_row(float (&acc)[NE], const LookupArgs& a, int64_t pos, int c, int lpr, int lane,
-                                          bool active) {
-  if constexpr (NE == 8) {
-    if (a.vec_store && a.out_fp16) {
-      u32x4_t v;
+__device__ __forceinline__ int64_t from_lane(int64_t v, int lane) {
+  return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), lane) << 32) |
+                   (uint32_t)__builtin_amdgcn_readlane((int)v, lane));
+}
+
+// How a wave's outputs leave: whole rows as one piece, or a lane's columns for themselves (slices of a row, rows that do
+// not begin at multiples of 16 bytes).
+constexpr int kColumns = 0;
+constexpr int kRowsFp16 = 1;
+constexpr int kRowsFp32 = 2;
+constexpr int kAny = 3;  // one of them, decided where a row is stored
+
+// 16-byte vectors per lane of the room in LDS through which a wave's outputs leave.
+constexpr int kStageVectors = 4;
+
+// The outputs of a wave's consecutive rows as one piece, `rows` of them from `first` on: lane c of group g holds NE
+// columns of row g.  A lane with several 16-byte vectors would write a part of every line with each store
+// instruction; the wave's vectors change places in LDS first.
+template <int NE, bool FP16>
+__device__ __forceinline__ void store_rows(const float (&acc)[NE], u32x4_t* stage, unsigned char* first, int lpr,
+                                           int lane, int rows) {
+  constexpr int V = NE * (FP16 ? 2 : 4) / 16;
+  constexpr int kPasses = V > kStageVectors ? V / kStageVectors : 1;  // a part of the lanes each
+  constexpr int kLanes = kWaveSize / kPasses;
+  const int vectors = rows * lpr * V;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t lo = __half_as_ushort(__float2half_rn(acc[2 * k]));
-        const uint32_t hi = __half_as_ushort(__float2half_rn(acc[2 * k + 1]));
-        v[k] = lo | (hi << 16);
-      }
-      if (active)
-        __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(reinterpret_cast<__half*>(a.out) + pos + c * NE));
-      return;
+  for (int h = 0; h < kPasses; ++h) {
+    wave_lds_sync();
+    if (lane / kLanes == h)
+#pragma unroll
+      for (int k = 0; k < V; ++k) stage[stage_slot<V>(lane % kLanes, k)] = out_vector<NE, FP16>(acc, k);
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < V / kPasses; ++k) {
+      const int i = k * kWaveSize + lane;
+      const u32x4_t x = stage[stage_slot<V>(i / V, i % V)];
+      const int at = h * kLanes * V + i;
+      if (at < vectors) __builtin_nontemporal_store(x, reinterpret_cast<u32x4_t*>(first) + at);
     }
   }
-  finish_bag<NE>(acc, a, 0, pos, c, lpr, lane, active, a.vec_store != 0);
 }
 
 // A feature's ids are cut into tiles of sc.window consecutive ids; the tiles of
@@ -61,15 +81,27 @@ __device__ __forceinline__ void store_row(float (&acc)[NE], const LookupArgs& a,
 // Bound by memory: a 132-byte row costs two 128-byte lines, so 2.1 M int8 rows
 // of 128 columns with fp16 results move 1083 MB.  One row per lane group and
 // plain stores took 206 us; four in flight, and results that leave as whole
-// lines past the caches (store_row), 187 us = 5.8 TB/s, what a gather of random
+// lines past the caches, 187 us = 5.8 TB/s, what a gather of random
 // lines reaches (rows loaded with the non-temporal hint as well: 208 us).
+// Where the rows are in the caches the results are what counts (a fill writes
+// 6.9 TB/s), and how they leave: 1.8 M rows, us, lanes' vectors as they lie (two of
+// them exchanged by cross-lane reads) / whole rows of a wave through LDS:
+//   fp32 results: int8 128 columns 315 / 189, 64 84 / 78, 32 64 / 44, 104 234 / 187;
+//                 int4 64 162 / 97, int2 128 297 / 180, fp16 104 244 / 187, 32 73 / 51
+//   fp16 results: int4 32 57 / 28, 64 65 / 46, int2 128 159 / 95, int8 96 118 / 79,
+//                 128 89 / 84; slower only fp16 32 46 / 51
+// (Without the non-temporal hint int8 64 fp16 62 -> 92 us, fp16 128 92 -> 156 us.)
+// What describes the tile is scalar: 84 registers instead of 120, five waves a SIMD.
 template <int DTYPE, int CB, typename IdxT>
 __global__ __launch_bounds__(kBlockThreads) void tbe_nobag_kernel(const LookupArgs a) {
   constexpr int NE = CB * 8 / Traits<DTYPE>::kBits;
   constexpr int U = kSequenceUnroll;
   __shared__ int64_t s_starts[kMaxTotalKeys + 1];
+  constexpr int kStage = NE <= 4 ? 1 : kWaveSize * (NE < 16 ? NE / 4 : kStageVectors);  // vectors a wave puts by
+  __shared__ __align__(16) u32x4_t s_stage[kWavesPerBlock * kStage];
   const int lane = threadIdx.x & (kWaveSize - 1);
-  const int wave = threadIdx.x / kWaveSize;
+  const int wave = uniform((int)(threadIdx.x / kWaveSize));
+  u32x4_t* stage = s_stage + wave * kStage;
   if (a.bounds_kind == kBoundsTotals) {
     if (wave == 0) {
       const int64_t* totals = reinterpret_cast<const int64_t*>(a.offsets);
@@ -112,9 +144,9 @@ __global__ __launch_bounds__(kBlockThreads) void tbe_nobag_kernel(const LookupAr
       if (past != 0) {
         const int hit = __builtin_ctzll(past);
         fi = i0 + hit;
-        first = __shfl(f1, hit, kWaveSize);
-        n = __shfl(n1, hit, kWaveSize);
-        tile = t - before - __shfl(incl - tiles, hit, kWaveSize);
+        first = from_lane(f1, hit);
+        n = from_lane(n1, hit);
+        tile = t - before - __builtin_amdgcn_readlane(incl - tiles, hit);
         break;
       }
       before += wave_last(incl);
@@ -130,33 +162,67 @@ __global__ __launch_bounds__(kBlockThreads) void tbe_nobag_kernel(const LookupAr
     w.sel0 = mfma_byte_selector(lane, 0);
     w.sel1 = mfma_byte_selector(lane, 1);
     const int64_t col = (int64_t)d.payload_off * 8 / Traits<DTYPE>::kBits;
+    const bool whole_rows = a.vec_store != 0 && lpr * NE == d.dim && (!a.out_fp16 || NE >= 8);
     const int64_t begin = first + tile * tile_ids;
     const int64_t end = min(begin + tile_ids, first + n);
     // (a step's rows are dealt to the waves before the unroll, so a short tile still keeps all waves busy)
-    for (int64_t j0 = begin + wave * gpw + g; j0 - g < end; j0 += kWavesPerBlock * gpw * U) {
-      IdxT id[U];
-      bool active[U];
+    const auto walk = [&](auto how) {
+      constexpr int HOW = decltype(how)::value;
+      for (int64_t w0 = begin + wave * gpw; w0 < end; w0 += kWavesPerBlock * gpw * U) {
+        IdxT id[U];
+        bool active[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t j = j0 + u * (kWavesPerBlock * gpw);
-        active[u] = g < gpw && j < end;
-        id[u] = reinterpret_cast<const IdxT*>(a.indices)[active[u] ? j : end - 1];
+        for (int u = 0; u < U; ++u) {
+          const int64_t j = w0 + u * (kWavesPerBlock * gpw) + g;
+          active[u] = g < gpw && j < end;
+          id[u] = reinterpret_cast<const IdxT*>(a.indices)[active[u] ? j : end - 1];
+        }
+        RowBuf<CB> r[U];
+        int bad[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          bad[u] = fetch_row<DTYPE, CB, kUnweighted, IdxT>(r[u], id[u], (IdxT)0, (IdxT)0, a, w);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (bad[u] != 0 && active[u] && w.count_errors) atomicAdd(a.err_count, 1ull);
+          if (bad[u] != 0 && a.bad_to_row0 != 0) r[u].valid = 1;  // the row fetched for it is row 0
+          float acc[NE];
+#pragma unroll
+          for (int k = 0; k < NE; ++k) acc[k] = 0.0f;
+          if constexpr (NE > 16) __builtin_amdgcn_sched_barrier(0);
+          consume_row<DTYPE, CB, false>(acc, r[u], w);
+          const int64_t row = w0 + u * (kWavesPerBlock * gpw);  // of the wave's first group
+          const auto rows_as = [&](auto fp16) {
+            constexpr bool FP16 = decltype(fp16)::value;
+            unsigned char* at = reinterpret_cast<unsigned char*>(a.out) + row * d.dim * (FP16 ? 2 : 4);
+            if constexpr (NE * (FP16 ? 2 : 4) == 16) {
+              u32x4_t* mine = reinterpret_cast<u32x4_t*>(at) + lane;
+              if (active[u]) __builtin_nontemporal_store(out_vector<NE, FP16>(acc, 0), mine);
+            } else {
+              const int rows = (int)min(max(end - row, (int64_t)0), (int64_t)gpw);
+              store_rows<NE, FP16>(acc, stage, at, lpr, lane, rows);
+            }
+          };
+          if (HOW == kRowsFp16 || (HOW == kAny && whole_rows && a.out_fp16)) {
+            if constexpr (HOW == kRowsFp16 || HOW == kAny) rows_as(std::true_type());
+          } else if (HOW == kRowsFp32 || (HOW == kAny && whole_rows)) {
+            if constexpr (HOW == kRowsFp32 || HOW == kAny) rows_as(std::false_type());
+          } else if (active[u]) {
+            store_outputs<NE>(a, (row + g) * (int64_t)d.dim + col + c * NE, acc, a.vec_store != 0);
+          }
+        }
       }
-      RowBuf<CB> r[U];
-      int bad[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        bad[u] = fetch_row<DTYPE, CB, kUnweighted, IdxT>(r[u], id[u], (IdxT)0, (IdxT)0, a, w);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (bad[u] != 0 && active[u] && w.count_errors) atomicAdd(a.err_count, 1ull);
-        if (bad[u] != 0 && a.bad_to_row0 != 0) r[u].valid = 1;  // the row fetched for it is row 0
-        float acc[NE];
-#pragma unroll
-        for (int k = 0; k < NE; ++k) acc[k] = 0.0f;
-        consume_row<DTYPE, CB, false>(acc, r[u], w);
-        store_row<NE>(acc, a, (j0 + u * (kWavesPerBlock * gpw)) * (int64_t)d.dim + col, c, lpr, lane, active[u]);
-      }
+    };
+    // (Lanes of few columns have a loop for each kind of store: 64 int8 columns, 123 K rows 8.0 -> 7.7 us.  With more,
+    // one loop is better, the compiler keeps more rows apart: 128 int8 columns, 1.8 M rows 94 -> 84 us.)
+    if constexpr (NE >= 16) {
+      walk(std::integral_constant<int, kAny>());
+    } else if (NE >= 8 && whole_rows && a.out_fp16) {
+      if constexpr (NE >= 8) walk(std::integral_constant<int, kRowsFp16>());
+    } else if (NE >= 4 && whole_rows) {
+      if constexpr (NE >= 4) walk(std::integral_constant<int, kRowsFp32>());
+    } else {
+      walk(std::integral_constant<int, kColumns>());
     }
   }
 }
