@@ -1,0 +1,36 @@
+"""Results of the window kernel: one to sixteen 16-byte vectors per lane, lane groups of every kind, rows that begin off a
+16-byte boundary, both result types, SUM and MEAN; against the CPU oracle, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from helpers import bits_equal
+from test_tbe_gpu import _from_lengths, build
+
+pytestmark = pytest.mark.gpu
+
+
+# (lanes behind a wave's last whole group, rows of one lane, results of less than a vector a lane, several slices of a row)
+@pytest.mark.parametrize("dtype,dims", [
+    (O.INT8, (4, 32, 40, 72, 104, 128, 256, 1040)), (O.INT4, (8, 64, 104, 128, 512)), (O.INT2, (16, 48, 128, 256, 1024)),
+    (O.FP16, (2, 32, 36, 104, 512)), (O.FP32, (1, 4, 36, 256)),
+])
+@pytest.mark.parametrize("out", [O.FP16, O.FP32])
+@pytest.mark.parametrize("mode", [O.SUM, O.MEAN])
+@pytest.mark.parametrize("window", [0, 70])
+def test_results(tuning, dtype, dims, out, mode, window):
+    tuning(balanced=1, window=window)
+    for dim in dims:
+        for first in (dim, 4 if dtype != O.INT2 else 16):  # (the narrow feature in front shifts the others' columns)
+            rng = np.random.default_rng([int(dtype), dim, first])
+            B = 37
+            specs = [(dtype, 60, max(first, 8 if dtype == O.INT4 else first)), (dtype, 50, dim), (dtype, 70, dim)]
+            tbe, store = build(rng, specs, [0, 1, 2], mode, out, 16)
+            lengths = rng.choice([0, 1, 2, 9], 3 * B).astype(np.int64)
+            offsets = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+            ids = rng.integers(-1, 50, int(offsets[-1])).astype(np.int64)
+            want = O.tbe_forward(store, [0, 1, 2], B, ids, offsets, None, mode, out)
+            assert bits_equal(_from_lengths(tbe, ids, lengths, None, B), want) == 0, (dim, first)
+            got = tbe(indices=torch.from_numpy(ids).cuda(), offsets=torch.from_numpy(offsets).cuda()).cpu().numpy()
+            assert bits_equal(got, want) == 0, (dim, first)

@@ -771,17 +771,6 @@ __device__ __forceinline__ void repool_bad_ids_as_row0(float (&acc)[NE], const L
   }
 }
 
-// Finish one bag per lane group (MEAN scaling, rounding, store).  Lane c of the
-// group's lpr lanes holds the NE outputs at columns row_pos + c * NE.  Every
-// lane of the wave calls this; `active` says whether its group holds a bag.
-// Where a lane's outputs are two 16-byte vectors, storing them as they lie
-// would write every other 16 bytes of the group's row with each of the two
-// store instructions, i.e. half lines.  The lanes exchange vectors first, so
-// that store k writes the k-th half of the row in whole lines (lane c sends
-// bytes [(k * lpr + c) * 16, + 16) of the row, which lane (k * lpr + c) / 2
-// owns), and the stores carry the non-temporal hint: the output is written
-// once and read by a later kernel, and whole lines leave the L2 as they come
-// (-0.5 to -1 us on the 13.6 MB output of the C2 workload).
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 // Vector v (16 bytes) of a lane's NE outputs.
@@ -801,59 +790,96 @@ __device__ __forceinline__ u32x4_t out_vector(const float (&acc)[NE], int v) {
   return x;
 }
 
-// Where a wave puts vector k of lane's V in LDS: lane by lane, the vectors of neighbouring lanes in different banks.
+// Results leave a wave through LDS: where a lane holds V 16-byte vectors of a row, storing them as they lie would write
+// a part of every line with each store instruction.  Room per lane, in vectors:
+constexpr int kStageVectors = 4;
+// Where a wave puts vector k of lane's V: lane by lane, the vectors of neighbouring lanes in different banks.
 template <int V>
 __device__ __forceinline__ int stage_slot(int lane, int k) {
   return lane * V + (k ^ (lane & (V - 1)));
 }
 
+// LDS accesses of the lanes of one wave in order: what they have written is visible to its other lanes.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// A vector of a row of results.  Results are written once and read by a later kernel: with the non-temporal hint where
+// a store instruction writes whole lines of the row (`lines`), else they stay in the caches until the rest of the line
+// has come.
+__device__ __forceinline__ void store_vector(u32x4_t x, u32x4_t* to, bool lines) {
+  if (lines) {
+    __builtin_nontemporal_store(x, to);
+  } else {
+    // (fenced: the compiler makes one store of the two otherwise, without the hint)
+    asm volatile("" ::: "memory");
+    *to = x;
+    asm volatile("" ::: "memory");
+  }
+}
+
+// Lane c of a group holds NE columns of the group's row from `row` on, on 16-byte boundaries.  The lanes of a group change
+// their vectors in LDS, kStageVectors of each at a time, so that a store instruction writes whole runs of the row.
+// Calls of 213 K bags of two cached ids, us, vectors stored as they lie (two a lane exchanged by cross-lane reads, for
+// lane groups of powers of two) / this: fp32 results, int8 256 columns 102 / 55, int8 128 50 / 32, int4 128 49 / 32, 34
+// features of int8 128 and 256 90 / 59; fp16 results, int2 128 33 / 27, int8 256 49 / 48; 65 K bags of 20, int8 256 to
+// fp16 51 / 48, to fp32 57 / 49.  The hint, where a store writes less than a line of a row (without / with): int2 128 to
+// fp32 33 / 42, int4 64 to fp32 23 / 26, int8 40 - 104 to fp32 36 / 40; elsewhere: int8 256 to fp32 84 / 55, fp16 64 to
+// fp16 25.8 / 24.3.
+template <int NE, bool FP16>
+__device__ __forceinline__ void store_group_row(const float (&acc)[NE], u32x4_t* stage, unsigned char* row, int c,
+                                                int lpr, int lane, bool active) {
+  constexpr int V = NE * (FP16 ? 2 : 4) / 16;
+  const bool lines = V <= kStageVectors && (FP16 || lpr % 8 == 0);
+  if constexpr (V == 1) {
+    if (active) store_vector(out_vector<NE, FP16>(acc, 0), reinterpret_cast<u32x4_t*>(row) + c, lines);
+  } else {
+    // (Places in LDS are computed where they are used: kept through the pooling loop they would push its registers out.)
+    asm volatile("" : "+v"(lane), "+v"(c));
+    constexpr int P = V < kStageVectors ? V : kStageVectors;
+#pragma unroll
+    for (int h = 0; h < V; h += P) {
+      wave_lds_sync();
+#pragma unroll
+      for (int k = 0; k < P; ++k) stage[stage_slot<P>(lane, k)] = out_vector<NE, FP16>(acc, h + k);
+      wave_lds_sync();
+#pragma unroll
+      for (int k = 0; k < P; ++k) {
+        const int i = k * lpr + c;  // which of the group's vectors this lane stores
+        const int from = min(lane - c + i / P, kWaveSize - 1);  // (lanes behind the last whole group)
+        const u32x4_t x = stage[stage_slot<P>(from, i % P)];
+        if (active) store_vector(x, reinterpret_cast<u32x4_t*>(row) + (i / P * V + h + i % P), lines);
+      }
+    }
+  }
+}
+
+// Finish one bag per lane group (MEAN scaling, rounding, store).  Lane c of the
+// group's lpr lanes holds the NE outputs at columns row_pos + c * NE.  Every
+// lane of the wave calls this; `active` says whether its group holds a bag.
+// `stage`: the wave's room in LDS, 64 * kStageVectors vectors.
 template <int NE>
-__device__ __forceinline__ void finish_bag(float (&acc)[NE], const LookupArgs& a, int len,
+__device__ __forceinline__ void finish_bag(float (&acc)[NE], const LookupArgs& a, u32x4_t* stage, int len,
                                            int64_t row_pos, int c, int lpr, int lane, bool active, bool vec) {
   if (a.mean && len > 0) {
     const float inv = 1.0f / (float)len;
 #pragma unroll
     for (int i = 0; i < NE; ++i) acc[i] *= inv;
   }
-  if constexpr (NE == 16 || NE == 8) {
-    const bool two_vectors = vec && lpr >= 2 && (lpr & (lpr - 1)) == 0 &&
-                             (a.out_fp16 ? NE == 16 : NE == 8);  // wave-uniform
-    if (two_vectors) {
-      uint32_t v[2][4];
+  if (vec) {
+    unsigned char* row = reinterpret_cast<unsigned char*>(a.out) + row_pos * (a.out_fp16 ? 2 : 4);
+    if constexpr (NE >= 8) {
       if (a.out_fp16) {
-        if constexpr (NE == 16) {
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const uint32_t lo = __half_as_ushort(__float2half_rn(acc[8 * h + 2 * k]));
-              const uint32_t hi = __half_as_ushort(__float2half_rn(acc[8 * h + 2 * k + 1]));
-              v[h][k] = lo | (hi << 16);
-            }
-        }
-      } else {
-        if constexpr (NE == 8) {
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) v[h][k] = __builtin_bit_cast(uint32_t, acc[4 * h + k]);
-        }
+        store_group_row<NE, true>(acc, stage, row, c, lpr, lane, active);
+        return;
       }
-      unsigned char* row = reinterpret_cast<unsigned char*>(a.out) + row_pos * (a.out_fp16 ? 2 : 4);
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const int g = k * lpr + c;  // which 16 bytes of the row this lane stores
-        const int src = (lane - c) + (g >> 1);
-        u32x4_t x;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t x0 = (uint32_t)__shfl((int)v[0][i], src, kWaveSize);
-          const uint32_t x1 = (uint32_t)__shfl((int)v[1][i], src, kWaveSize);
-          x[i] = (g & 1) ? x1 : x0;
-        }
-        if (active) __builtin_nontemporal_store(x, reinterpret_cast<u32x4_t*>(row + (int64_t)g * 16));
+    }
+    if constexpr (NE >= 4) {
+      if (!a.out_fp16) {
+        store_group_row<NE, false>(acc, stage, row, c, lpr, lane, active);
+        return;
       }
-      return;
     }
   }
   if (active) store_outputs<NE>(a, row_pos + (int64_t)c * NE, acc, vec);
@@ -1072,11 +1098,6 @@ __device__ __forceinline__ int64_t wave_last(int64_t v) { return __shfl(v, kWave
 // every outstanding global load of the wave; the window kernel's prologue keeps
 // loads in flight across its barriers (nothing there is handed from wave to
 // wave through global memory).
-// The same inside one wave: LDS writes of its lanes are visible to its other lanes.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-  __builtin_amdgcn_wave_barrier();
-}
 __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
@@ -1108,6 +1129,7 @@ struct Window {
   Sum* red;
   Sum* wave_tot;
   int* taken;  // rounds that waves have asked for after their first
+  u32x4_t* stage;  // 64 * kStageVectors vectors of results per wave
 };
 #define TRA_WINDOW(IdxT, name)                                                                       \
   __shared__ int64_t s_start[kMaxWindow];                                                            \
@@ -1119,7 +1141,8 @@ struct Window {
   __shared__ FeatureDesc s_desc[kMaxWinFeat];                                                        \
   __shared__ typename SumOf<IdxT>::type s_red[kCuWaves], s_wave_tot[kCuWaves];                       \
   __shared__ int s_taken;                                                                            \
-  const Window<IdxT> name{s_start, s_len, s_ent, s_order, s_slot, s_hist, s_desc, s_red, s_wave_tot, &s_taken}
+  __shared__ u32x4_t s_stage[kCuWaves * kWaveSize * kStageVectors];                                  \
+  const Window<IdxT> name{s_start, s_len, s_ent, s_order, s_slot, s_hist, s_desc, s_red, s_wave_tot, &s_taken, s_stage}
 
 // What a staged window's bag starts in LDS still lack: `add`, and from the sub-class's feature `second` on `second_add`.
 template <typename Sum>
@@ -1524,7 +1547,8 @@ __device__ __forceinline__ void pool_window(const Window<IdxT> win, const Lookup
 #ifdef TRA_INSTRUMENT
     if (lane == 0) a.ts[((size_t)blockIdx.x * (blockDim.x / 64) + wave) * 8 + 5] = (unsigned long long)max_len;
 #endif
-    finish_bag<NE>(acc, a, len, (int64_t)b * a.out_stride + d.out_col, c, lpr, lane, active, vec());
+    finish_bag<NE>(acc, a, win.stage + uniform(wave) * (kWaveSize * kStageVectors), len, (int64_t)b * a.out_stride + d.out_col, c,
+                   lpr, lane, active, vec());
     TRA_STAMP(4);
     if (rounds <= kCuWaves) break;
     r = kCuWaves + __builtin_amdgcn_readfirstlane(lane == 0 ? atomicAdd(win.taken, 1) : 0);

@@ -150,7 +150,7 @@ static Tuning choose_tuning(bool balanced) {
   t.balanced = balanced ? 1 : 0;
   t.window = 0;
   t.unroll = 4;
-  t.lds_bytes = 48 * 1024;  // with the static arrays > half of a CU's LDS: one block per CU
+  t.lds_bytes = 0;  // (the static arrays are over half of a compute unit's LDS: one block each)
   if (g_ovr.balanced >= 0) t.balanced = g_ovr.balanced;
   if (g_ovr.window >= 0) t.window = g_ovr.window;
   if (g_ovr.unroll >= 0) t.unroll = g_ovr.unroll;

@@ -36,9 +36,6 @@ constexpr int kRowsFp16 = 1;
 constexpr int kRowsFp32 = 2;
 constexpr int kAny = 3;  // one of them, decided where a row is stored
 
-// 16-byte vectors per lane of the room in LDS through which a wave's outputs leave.
-constexpr int kStageVectors = 4;
-
 // The outputs of a wave's consecutive rows as one piece, `rows` of them from `first` on: lane c of group g holds NE
 // columns of row g.  A lane with several 16-byte vectors would write a part of every line with each store
 // instruction; the wave's vectors change places in LDS first.
