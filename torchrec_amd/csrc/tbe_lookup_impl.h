@@ -825,13 +825,13 @@ __device__ __forceinline__ void store_vector(u32x4_t x, u32x4_t* to, bool lines)
 // lane groups of powers of two) / this: fp32 results, int8 256 columns 102 / 55, int8 128 50 / 32, int4 128 49 / 32, 34
 // features of int8 128 and 256 90 / 59; fp16 results, int2 128 33 / 27, int8 256 49 / 48; 65 K bags of 20, int8 256 to
 // fp16 51 / 48, to fp32 57 / 49.  The hint, where a store writes less than a line of a row (without / with): int2 128 to
-// fp32 33 / 42, int4 64 to fp32 23 / 26, int8 40 - 104 to fp32 36 / 40; elsewhere: int8 256 to fp32 84 / 55, fp16 64 to
+// fp32 33 / 42, int4 64 to fp32 23 / 26, int8 40 - 104 to fp32 36 / 40, int2 48 - 112 to fp16 28 / 34; elsewhere: int8 256 to fp32 84 / 55, fp16 64 to
 // fp16 25.8 / 24.3.
 template <int NE, bool FP16>
 __device__ __forceinline__ void store_group_row(const float (&acc)[NE], u32x4_t* stage, unsigned char* row, int c,
                                                 int lpr, int lane, bool active) {
   constexpr int V = NE * (FP16 ? 2 : 4) / 16;
-  const bool lines = V <= kStageVectors && (FP16 || lpr % 8 == 0);
+  const bool lines = V <= kStageVectors && (lpr % 8 == 0 || (FP16 && V == 2 && lpr >= 2 && (lpr & (lpr - 1)) == 0));
   if constexpr (V == 1) {
     if (active) store_vector(out_vector<NE, FP16>(acc, 0), reinterpret_cast<u32x4_t*>(row) + c, lines);
   } else {
