@@ -261,3 +261,57 @@ def test_collection_remap_refuses_what_its_kernels_cannot_read(keys, given):
             setattr(module, name, bad(getattr(module, name)))
             with pytest.raises(AssertionError):
                 mcc(KeyedJaggedTensor(keys=keys, values=ids, **{given: bags}))
+
+
+def _hash(ids, size):
+    return (ids * 7 + 3) % size
+
+
+class _HashModule(torch.nn.Module):
+    def forward(self, ids, size):
+        return _hash(ids, size)
+
+
+# CPU tensors stand for a GPU's: what is asked of the features here is only where their ids are.
+class _OnDevice:
+    def __init__(self, values):
+        self._values = values
+
+    def values(self):
+        return self
+
+    is_cuda = True
+
+    def get_device(self):
+        return self._values.get_device()
+
+    def keys(self):
+        return ["f"]
+
+
+@pytest.mark.parametrize("hash_func", [None, _hash, _HashModule()], ids=["none", "function", "module"])
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda:0", marks=pytest.mark.gpu)])
+def test_input_hash(hash_func, device):
+    """An input hash may be any callable, a module too; ids are hashed before they are remapped."""
+    rng = np.random.default_rng(3)
+    sorted_ids, mapping = make_table(rng, 200, 150)
+    size = 10**9
+    dev = torch.device(device)
+    mc = MCHManagedCollisionModule(200, dev, input_hash_size=size, input_hash_func=hash_func).eval()
+    mc._mch_sorted_raw_ids.copy_(torch.from_numpy(sorted_ids))
+    mc._mch_remapped_ids_mapping.copy_(torch.from_numpy(mapping))
+    table = EmbeddingConfig(name="t", embedding_dim=8, num_embeddings=200, feature_names=["f"])
+    collection = ManagedCollisionCollection({"t": mc}, [table]).eval()
+    tables = collection._one_launch_tables(_OnDevice(mc._mch_sorted_raw_ids))
+    assert (tables is None) == (hash_func is not None)
+    # (7 * x + 3) % 10^9 = id: every other id is a known one
+    inverse = pow(7, -1, size)
+    known = rng.choice(sorted_ids[:150], 60)
+    raw = known if hash_func is None else (known - 3) * inverse % size
+    values = np.stack([raw, rng.integers(0, size, 60)], 1).reshape(-1)
+    kjt = KeyedJaggedTensor(keys=["f"], values=torch.from_numpy(values).to(dev),
+                            lengths=torch.full((40,), 3, dtype=torch.int64, device=dev))
+    got = collection(kjt).values().cpu().numpy()
+    want = ref_remap(values if hash_func is None else (values * 7 + 3) % size, sorted_ids, mapping, 199)
+    assert np.array_equal(got, want)
+    assert (want != 199).sum() >= 60

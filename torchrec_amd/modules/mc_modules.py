@@ -190,17 +190,16 @@ class ManagedCollisionCollection(nn.Module):
         sorted_ids, mappings, miss = [], [], []
         for config in self._embedding_configs:
             module = modules[config.name]
-            own = module.__dict__
-            if type(module) is not MCHManagedCollisionModule or own["training"] or own["_input_hash_func"] is not None:
+            if type(module) is not MCHManagedCollisionModule or module.training or module._input_hash_func is not None:
                 return None
-            buffers = own["_buffers"]
+            buffers = module._buffers
             ids, rows = buffers["_mch_sorted_raw_ids"], buffers["_mch_remapped_ids_mapping"]
             if ids.get_device() != dev or rows.get_device() != dev:
                 return None
             for _ in config.feature_names:
                 sorted_ids.append(ids)
                 mappings.append(rows)
-                miss.append(own["_output_global_offset"] + own["_zch_size"] - 1)
+                miss.append(module._output_global_offset + module._zch_size - 1)
         return sorted_ids, mappings, miss
 
     def forward(self, features: KeyedJaggedTensor) -> KeyedJaggedTensor:
