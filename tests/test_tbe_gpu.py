@@ -11,6 +11,7 @@ import torch
 
 import oracle as O
 from helpers import bits_equal, make_bags, make_table, weight_pair
+from torchrec_amd._lib import TorchrecAmdError
 from torchrec_amd.tbe import EmbeddingLocation, PoolingMode, SparseType
 from torchrec_amd.tbe.split_table_batched_embeddings_ops_inference import (
     IntNBitTableBatchedEmbeddingBagsCodegen as TBE,
@@ -1000,6 +1001,22 @@ def test_random_position_weights(tuning, seed):
         got = tbe(ti, torch.from_numpy(offsets).to(DEV), None, position_weights=pw)
     tag = (seed, specs, ftm, pooling, out_dtype, ra, idt.__name__, B, max_len, route, window, from_lengths, key_len)
     assert bits_equal(got.cpu().numpy(), want) == 0, tag
+
+
+@pytest.mark.parametrize("kind", ["buffer", "parameter"])
+def test_packed_weights_replaced_by_hand(kind):
+    """The packed weights may be replaced, by a parameter too; on another device they are refused."""
+    rng = np.random.default_rng(17)
+    specs = [(O.INT8, 100, 32), (O.INT4, 200, 64)]
+    tbe, store = build(rng, specs, [0, 1], O.SUM, O.FP32, 16)
+    lengths, offsets, ids = make_bags(rng, [100, 200], 9, 20)
+    same = tbe.weights_dev.clone()
+    tbe.weights_dev = same if kind == "buffer" else torch.nn.Parameter(same, requires_grad=False)
+    got, want = run_both(tbe, store, [0, 1], 9, ids, offsets, None, O.SUM, O.FP32)
+    assert bits_equal(got, want) == 0
+    tbe.weights_dev = same.cpu() if kind == "buffer" else torch.nn.Parameter(same.cpu(), requires_grad=False)
+    with pytest.raises(TorchrecAmdError, match="packed weights are on cpu"):
+        tbe(torch.from_numpy(ids).to(DEV), torch.from_numpy(offsets).to(DEV))
 
 
 def test_table_beyond_2_31_rows(tuning):

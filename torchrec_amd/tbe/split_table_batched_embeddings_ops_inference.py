@@ -454,7 +454,7 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(nn.Module):
             )
         if not self._weights_initialized:
             raise _lib.TorchrecAmdError("weights are not initialized (call initialize_weights())")
-        if self._buffers["weights_dev"].get_device() != dev.index:  # e.g. the buffer was replaced by hand
+        if self.weights_dev.device != dev:  # e.g. the buffer was replaced by hand
             raise _lib.TorchrecAmdError(f"packed weights are on {self.weights_dev.device}, the operator on {dev}")
         idt = indices.dtype
         if not indices.is_cuda:
