@@ -86,6 +86,30 @@ def test_results_of_all_widths(dtype, dims, out):
         assert (got[ids.size :] == 7.0).all(), dim
 
 
+# Ids enough for tiles of several rows a lane group (4 steps of `rows` rows); features that end at every place of a tile's
+# steps: in front of a wave's first row, inside its rows, behind them.
+@pytest.mark.parametrize("dtype,dim,rows", [(O.INT8, 1024, 4), (O.FP16, 512, 4), (O.INT4, 1024, 8), (O.INT8, 512, 4)])
+@pytest.mark.parametrize("out", [O.FP16, O.FP32])
+def test_steps_that_a_tile_does_not_fill(dtype, dim, rows, out):
+    rng = np.random.default_rng(dim + rows)
+    step = 4 * rows
+    totals = [step + 1, 0, 3, 2 * step - 1, rows, rows + 1, 3 * rows - 1, step]
+    totals.append(512 * step)
+    specs = [(dtype, 300, dim)]
+    ftm = [0] * len(totals)
+    tbe, store = build(rng, specs, ftm, O.NONE, out, 16)
+    ids = rng.integers(-1, 301, sum(totals)).astype(np.int32)
+    starts = np.concatenate([[0], np.cumsum(totals)]).astype(np.int32)
+    want = O.tbe_forward(store, ftm, 1, np.where(ids == 300, np.int32(-1), ids), starts, None, O.NONE, out)
+    guard = torch.full((ids.size + 40, dim), 7.0, dtype=torch.half if out == O.FP16 else torch.float, device=DEV)
+    tbe(indices=torch.from_numpy(ids).to(DEV), offsets=None, key_starts=starts.tolist(), out=guard)
+    got = guard.cpu().numpy()
+    assert bits_equal(got[: ids.size], want) == 0
+    assert (got[ids.size :] == 7.0).all()
+    # (ids outside the table are counted once a row, also in steps that are cut short)
+    assert tbe.out_of_range_count() == int((ids == 300).sum())
+
+
 def test_row_ranges_of_given_key_offsets():
     module = _collection(2)
     ids = torch.arange(8, device=DEV)
