@@ -86,9 +86,12 @@ __device__ __forceinline__ void store_rows(const float (&acc)[NE], u32x4_t* stag
 //   fp32 results: int8 128 columns 315 / 189, 64 84 / 78, 32 64 / 44, 104 234 / 187;
 //                 int4 64 162 / 97, int2 128 297 / 180, fp16 104 244 / 187, 32 73 / 51
 //   fp16 results: int4 32 57 / 28, 64 65 / 46, int2 128 159 / 95, int8 96 118 / 79,
-//                 128 89 / 84; slower only fp16 32 46 / 51
+//                 128 89 / 84
 // (Without the non-temporal hint int8 64 fp16 62 -> 92 us, fp16 128 92 -> 156 us.)
-// What describes the tile is scalar: 84 registers instead of 120, five waves a SIMD.
+// What describes the tile is scalar, so that more waves fit a SIMD: five instead of four with 16 int8 columns a lane in
+// 8-byte chunks, seven instead of four with 8 fp16 columns.
+// Slower than lanes' vectors as they lie and the tile in vector registers: fp16 rows of 16 and 32 columns to fp16, 32-bit
+// ids, 25.1 / 26.5 and 46 / 49 us (64-bit ids 27.5 / 26, 56 / 52); 123 K rows of int8 or int4 128 to fp16 9.5 / 9.8.
 template <int DTYPE, int CB, typename IdxT>
 __global__ __launch_bounds__(kBlockThreads) void tbe_nobag_kernel(const LookupArgs a) {
   constexpr int NE = CB * 8 / Traits<DTYPE>::kBits;
@@ -161,19 +164,28 @@ __global__ __launch_bounds__(kBlockThreads) void tbe_nobag_kernel(const LookupAr
     const int64_t col = (int64_t)d.payload_off * 8 / Traits<DTYPE>::kBits;
     const bool whole_rows = a.vec_store != 0 && lpr * NE == d.dim && (!a.out_fp16 || NE >= 8);
     const int64_t begin = first + tile * tile_ids;
-    const int64_t end = min(begin + tile_ids, first + n);
+    // Places in a tile, in 32 bits where lanes hold few columns: a 64-bit bound is compared in vector registers, there in
+    // those that the last row's load had used, so that every wave waited for its last store to end before it left (1.8 M
+    // rows, us, 64 / 32 bits: fp16 32 columns to fp16 52 / 49, 64 62 / 54, int8 64 62 / 56, 123 K rows of 64 7.5 / 7.0).
+    // With 16 columns 64 bits are better (int8 128 to fp16 84 / 90).
+    using Place = std::conditional_t<(NE <= kNarrowLane), int, int64_t>;
+    const Place ids = (Place)(min(begin + tile_ids, first + n) - begin);
+    const IdxT* in = reinterpret_cast<const IdxT*>(a.indices) + begin;
     // (a step's rows are dealt to the waves before the unroll, so a short tile still keeps all waves busy)
     const auto walk = [&](auto how) {
       constexpr int HOW = decltype(how)::value;
-      for (int64_t w0 = begin + wave * gpw; w0 < end; w0 += kWavesPerBlock * gpw * U) {
+      for (Place w0 = wave * gpw; w0 < ids; w0 += kWavesPerBlock * gpw * U) {
         IdxT id[U];
         bool active[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const int64_t j = w0 + u * (kWavesPerBlock * gpw) + g;
-          active[u] = g < gpw && j < end;
-          id[u] = reinterpret_cast<const IdxT*>(a.indices)[active[u] ? j : end - 1];
+          const Place j = w0 + u * (kWavesPerBlock * gpw) + g;
+          active[u] = g < gpw && j < ids;
+          id[u] = in[active[u] ? j : ids - 1];
         }
+        // (all ids are asked for before the first is looked at: left to the compiler, the last one's load waited for the
+        // first id; 1.8 M rows of 16 fp16 columns 27.5 / 26.5 us)
+        if constexpr (NE <= 4) __builtin_amdgcn_sched_barrier(0);
         RowBuf<CB> r[U];
         int bad[U];
 #pragma unroll
@@ -181,11 +193,12 @@ __global__ __launch_bounds__(kBlockThreads) void tbe_nobag_kernel(const LookupAr
           bad[u] = fetch_row<DTYPE, CB, kUnweighted, IdxT>(r[u], id[u], (IdxT)0, (IdxT)0, a, w);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
+          const Place place = w0 + u * (kWavesPerBlock * gpw);  // of the wave's first group
           // (a short tile fills a part of its only step: rows that it does not have are not exchanged in LDS.  Without / with
           // this, us: 3200 rows of int2 512 columns to fp16 10.0 / 6.5, to fp32 13.7 / 7.8, int4 256 to fp32 7.9 / 6.4; 31 K
           // rows of int8 192 to fp16 11.0 / 8.6, 96 7.7 / 6.5)
           if constexpr (NE >= 16)
-            if (w0 + u * (kWavesPerBlock * gpw) >= end) break;
+            if (place >= ids) break;
           if (bad[u] != 0 && active[u] && w.count_errors) atomicAdd(a.err_count, 1ull);
           if (bad[u] != 0 && a.bad_to_row0 != 0) r[u].valid = 1;  // the row fetched for it is row 0
           float acc[NE];
@@ -193,7 +206,7 @@ __global__ __launch_bounds__(kBlockThreads) void tbe_nobag_kernel(const LookupAr
           for (int k = 0; k < NE; ++k) acc[k] = 0.0f;
           if constexpr (NE > 16) __builtin_amdgcn_sched_barrier(0);
           consume_row<DTYPE, CB, false>(acc, r[u], w);
-          const int64_t row = w0 + u * (kWavesPerBlock * gpw);  // of the wave's first group
+          const int64_t row = begin + place;
           const auto rows_as = [&](auto fp16) {
             constexpr bool FP16 = decltype(fp16)::value;
             unsigned char* at = reinterpret_cast<unsigned char*>(a.out) + row * d.dim * (FP16 ? 2 : 4);
@@ -201,8 +214,7 @@ __global__ __launch_bounds__(kBlockThreads) void tbe_nobag_kernel(const LookupAr
               u32x4_t* mine = reinterpret_cast<u32x4_t*>(at) + lane;
               if (active[u]) __builtin_nontemporal_store(out_vector<NE, FP16>(acc, 0), mine);
             } else {
-              const int rows = (int)min(max(end - row, (int64_t)0), (int64_t)gpw);
-              store_rows<NE, FP16>(acc, stage, at, lpr, lane, rows);
+              store_rows<NE, FP16>(acc, stage, at, lpr, lane, (int)min(max(ids - place, (Place)0), (Place)gpw));
             }
           };
           if (HOW == kRowsFp16 || (HOW == kAny && whole_rows && a.out_fp16)) {
@@ -229,12 +241,18 @@ __global__ __launch_bounds__(kBlockThreads) void tbe_nobag_kernel(const LookupAr
   }
 }
 
+// fp32 results of eight columns a lane: LDS that leaves room for five blocks on a compute unit.  Seven, which the registers
+// allow, write 1.8 M rows of 64 fp16 columns in 84 us, five in 78, of 64 int8 columns in 84 and 79; fp16 results are better
+// with seven (54 and 58, 56 and 60 us).
+constexpr int kFiveBlocksLds = 18000;
+
 template <int DTYPE, int CB>
 static void launch_sequence_cb(const LookupArgs& a, bool idx64, int grid, hipStream_t stream) {
+  const int lds = CB * 8 / Traits<DTYPE>::kBits == 8 && !a.out_fp16 ? kFiveBlocksLds : 0;
   if (idx64)
-    hipLaunchKernelGGL((tbe_nobag_kernel<DTYPE, CB, int64_t>), dim3(grid), dim3(kBlockThreads), 0, stream, a);
+    hipLaunchKernelGGL((tbe_nobag_kernel<DTYPE, CB, int64_t>), dim3(grid), dim3(kBlockThreads), lds, stream, a);
   else
-    hipLaunchKernelGGL((tbe_nobag_kernel<DTYPE, CB, int32_t>), dim3(grid), dim3(kBlockThreads), 0, stream, a);
+    hipLaunchKernelGGL((tbe_nobag_kernel<DTYPE, CB, int32_t>), dim3(grid), dim3(kBlockThreads), lds, stream, a);
 }
 
 template <int DTYPE>
