@@ -1,5 +1,5 @@
-"""Bucketization by three launches and by two at the sizes where its tiles, groups of tiles, steps of ids and bitmap
-words begin and end, against the oracle: whole numbers, compared exactly."""
+"""Bucketization by four launches and by two at the sizes where its tiles, steps of ids and bitmap words
+begin and end, against the oracle: whole numbers, compared exactly."""
 import numpy as np
 import pytest
 import torch
@@ -24,9 +24,9 @@ def _lengths(how, n, rng):
 
 
 @pytest.mark.parametrize("F,B,W,how", [
-    (5, 3277, 3, "even"),     # 16385 lengths: the first count that takes three launches
+    (5, 3277, 3, "even"),     # 16385 lengths: the first count whose bounds come from launches of their own
     (4, 4096, 3, "even"),     # 16384: the last that takes two
-    (70, 300, 5, "even"),     # some hundred tiles, a dozen groups of them
+    (70, 300, 5, "even"),     # some hundred tiles
     (300, 80, 64, "even"),    # the most buckets
     (1, 20000, 1, "even"),    # one bucket
     (3, 6000, 7, "words"),

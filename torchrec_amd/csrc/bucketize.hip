@@ -364,7 +364,6 @@ __global__ __launch_bounds__(kBktThreads) void bucket_counts_kernel(
       lds_barrier();
     }
   }
-  if (ids == 0) lds_barrier();  // (the counters are clear)
   // new lengths, and the tile's total per bucket: a wave takes every fourth bucket
   T* out = reinterpret_cast<T*>(a.new_lengths);
   for (int p = wave; p < a.W; p += kBktWaves) {
