@@ -34,3 +34,26 @@ def test_results(tuning, dtype, dims, out, mode, window):
             assert bits_equal(_from_lengths(tbe, ids, lengths, None, B), want) == 0, (dim, first)
             got = tbe(indices=torch.from_numpy(ids).cuda(), offsets=torch.from_numpy(offsets).cuda()).cpu().numpy()
             assert bits_equal(got, want) == 0, (dim, first)
+
+
+# Lanes of 32 and 64 accumulators, which look up anew behind the pooling loop where a bag's results go: lane groups of every
+# kind (5, 6, 8, 16 and 64 lanes), more features in a window than its descriptors hold, waves of several rounds.
+@pytest.mark.parametrize("dtype,dim", [(O.INT4, 160), (O.INT4, 192), (O.INT4, 256), (O.INT4, 512), (O.INT4, 2080),
+                                       (O.INT2, 128), (O.INT2, 192), (O.INT2, 320), (O.INT2, 512)])
+@pytest.mark.parametrize("F,B", [(3, 211), (45, 5)])
+@pytest.mark.parametrize("weighted,idt", [(False, np.int32), (True, np.int64)])
+def test_wide_lanes(tuning, dtype, dim, F, B, weighted, idt):
+    tuning(balanced=1, window=256)
+    rng = np.random.default_rng([int(dtype), dim, F])
+    ftm = [f % 2 for f in range(F)]
+    for mode, out in ((O.SUM, O.FP16), (O.MEAN, O.FP32)):
+        tbe, store = build(rng, [(dtype, 60, dim), (dtype, 50, dim)], ftm, mode, out, 16)
+        lengths = rng.choice([0, 1, 3, 8, 17, 40], F * B).astype(idt)
+        offsets = np.concatenate([[0], np.cumsum(lengths)]).astype(idt)
+        ids = rng.integers(-1, 50, int(offsets[-1])).astype(idt)
+        psw = rng.random(len(ids)).astype(np.float32) if weighted else None
+        want = O.tbe_forward(store, ftm, B, ids, offsets, psw, mode, out)
+        assert bits_equal(_from_lengths(tbe, ids, lengths, psw, B), want) == 0
+        got = tbe(torch.from_numpy(ids).cuda(), torch.from_numpy(offsets).cuda(),
+                  None if psw is None else torch.from_numpy(psw).cuda()).cpu().numpy()
+        assert bits_equal(got, want) == 0

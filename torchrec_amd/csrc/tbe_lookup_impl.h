@@ -550,6 +550,9 @@ __device__ __forceinline__ int wave_max(int v) {
 #define TRA_STAMP(k)
 #endif
 
+constexpr int kNarrowLane = 8;  // accumulators per lane up to which one instance serves all widths (see odd_lanes)
+constexpr int kFewAccumulators = 16;  // per lane, up to which the compiler keeps the pooling loop's loads in flight by itself
+
 // ---- pooled lookup ----------------------------------------------------------
 
 // Pool one bag per lane group: ids [start, start + len), in order, into acc.
@@ -711,16 +714,22 @@ __device__ __forceinline__ int pool_bag_bulk(float (&acc)[NE], const LookupArgs&
     // compiler knows at the top of the loop that only the newest batch and
     // the id block are in flight and need not drain them before it reuses a
     // consumed buffer's registers.  The last, partial iteration follows below.
+    // (With 32 accumulators a lane a batch's loads are held in front of the batch consumed meanwhile: short of registers,
+    // the compiler puts each behind the row before it, and waits for it at once.  41 K bags of 20 ids of 1 M int4 rows of
+    // 256 columns 52.0 us, so 42.8.  With 64 it is better left to the compiler: 41 K position-weighted bags of 20 ids of 512
+    // cached int2 columns 109 us held, 86 not.)
     for (; it + 2 * U <= max_len; it += 2 * U) {
 #pragma unroll
       for (int u = 0; u < U; ++u)
         bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufB[u], id_of(it + U + u, U + u), start + it + U + u, last, a, w, weight_of(it + U + u, U + u));
+      if constexpr (NE == 2 * kFewAccumulators) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < U; ++u) consume_row<DTYPE, CB, (WEIGHTED != 0)>(acc, bufA[u], w);
       advance();
 #pragma unroll
       for (int u = 0; u < U; ++u)
         bad += fetch_row<DTYPE, CB, WEIGHTED, IdxT, true>(bufA[u], id_of(it + 2 * U + u, u), start + it + 2 * U + u, last, a, w, weight_of(it + 2 * U + u, u));
+      if constexpr (NE == 2 * kFewAccumulators) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < U; ++u) consume_row<DTYPE, CB, (WEIGHTED != 0)>(acc, bufB[u], w);
     }
@@ -1112,8 +1121,6 @@ __device__ __forceinline__ int feat_key_pos(const LookupArgs& a, const SubClass&
                                  : a.descs[a.feats[sc.first + fi]].feature;
 }
 
-constexpr int kNarrowLane = 8;  // accumulators per lane up to which one instance serves all widths (see odd_lanes)
-
 // A window's bags in LDS, in arrays of their own (so that the compiler can tell
 // accesses to one from accesses to another).
 template <typename IdxT>
@@ -1472,12 +1479,20 @@ __device__ __forceinline__ void pool_window(const Window<IdxT> win, const Lookup
                                             Vec&& vec) {
   constexpr int NE = CB * 8 / Traits<DTYPE>::kBits;
   constexpr bool ODD = BODIES == kBodiesOdd;
-  const int lane = threadIdx.x & (kWaveSize - 1);
-  const int wave = threadIdx.x / kWaveSize;
+  // Where a lane holds more than 16 accumulators, what the pooling loop does not need is found anew behind it (the lane's
+  // place in the wave, where its bag's results go): kept, it would push the loop's registers out.  Registers in scratch
+  // memory, int4 in 16-byte chunks, 32-bit ids from lengths, without, with per-sample and with position weights: 16, 16 and
+  // 24 with all of it kept, 4, 5 and 4 so.
+  constexpr bool kWide = NE > kFewAccumulators;
+  const auto lane_now = [&] {
+    if constexpr (!kWide) return (int)(threadIdx.x & (kWaveSize - 1));
+    int none = 0;
+    asm volatile("" : "+v"(none));
+    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, none));
+  };
+  const int wave = uniform((int)(threadIdx.x / kWaveSize));
   const int lpr = sc.lpr;
   const int gpw = kWaveSize / lpr;
-  const int g = lane / lpr;
-  const int c = lane - g * lpr;
   const int rounds = (nb + gpw - 1) / gpw;
   // Rounds are ordered longest first.  A wave's first one is dealt, in opposite
   // directions on neighbouring SIMDs' rows of waves; after that it takes the next
@@ -1490,12 +1505,18 @@ __device__ __forceinline__ void pool_window(const Window<IdxT> win, const Lookup
   // 30 ids of seven classes 358.8 / 358.6.
   const int four = wave >> 2;
   for (int r = four * 4 + ((four & 1) ? 3 - (wave & 3) : (wave & 3)); r < rounds;) {
-    const int pos = r * gpw + g;
-    const bool active = g < gpw && pos < nb;
-    const int i = win.order[active ? pos : r * gpw];
-    const uint32_t ent = win.ent[i];
-    const int fi = (int)(ent >> kBagBits);
-    const int b = (int)(ent & ((1u << kBagBits) - 1));
+    const auto bag_at = [&](int g, bool& active, int& i, int& fi, int& b) {
+      const int pos = r * gpw + g;
+      active = g < gpw && pos < nb;
+      i = win.order[active ? pos : r * gpw];
+      const uint32_t ent = win.ent[i];
+      fi = (int)(ent >> kBagBits);
+      b = (int)(ent & ((1u << kBagBits) - 1));
+    };
+    bool active;
+    int i, fi, b;
+    const int lane = lane_now(), g = lane / lpr, c = lane - g * lpr;
+    bag_at(g, active, i, fi, b);
     const FeatureDesc d = fi - fi_lo < kMaxWinFeat ? win.desc[fi - fi_lo] : a.cdescs[sc.first + fi];
     const int64_t start = win.start[i] + (int64_t)(fi < starts.second ? starts.add : starts.second_add);
     const int len = active ? max(win.len[i], 0) : 0;
@@ -1547,11 +1568,19 @@ __device__ __forceinline__ void pool_window(const Window<IdxT> win, const Lookup
 #ifdef TRA_INSTRUMENT
     if (lane == 0) a.ts[((size_t)blockIdx.x * (blockDim.x / 64) + wave) * 8 + 5] = (unsigned long long)max_len;
 #endif
-    finish_bag<NE>(acc, a, win.stage + uniform(wave) * (kWaveSize * kStageVectors), len, (int64_t)b * a.out_stride + d.out_col, c,
-                   lpr, lane, active, vec());
+    if constexpr (kWide) {
+      const int l = lane_now(), g2 = l / lpr, c2 = l - g2 * lpr;
+      bag_at(g2, active, i, fi, b);
+      const int out_col = fi - fi_lo < kMaxWinFeat ? win.desc[fi - fi_lo].out_col : a.cdescs[sc.first + fi].out_col;
+      finish_bag<NE>(acc, a, win.stage + wave * (kWaveSize * kStageVectors), active ? max(win.len[i], 0) : 0,
+                     (int64_t)b * a.out_stride + out_col, c2, lpr, l, active, vec());
+    } else {
+      finish_bag<NE>(acc, a, win.stage + wave * (kWaveSize * kStageVectors), len, (int64_t)b * a.out_stride + d.out_col, c,
+                     lpr, lane, active, vec());
+    }
     TRA_STAMP(4);
     if (rounds <= kCuWaves) break;
-    r = kCuWaves + __builtin_amdgcn_readfirstlane(lane == 0 ? atomicAdd(win.taken, 1) : 0);
+    r = kCuWaves + __builtin_amdgcn_readfirstlane(lane_now() == 0 ? atomicAdd(win.taken, 1) : 0);
   }
 }
 
