@@ -57,3 +57,23 @@ def test_wide_lanes(tuning, dtype, dim, F, B, weighted, idt):
         got = tbe(torch.from_numpy(ids).cuda(), torch.from_numpy(offsets).cuda(),
                   None if psw is None else torch.from_numpy(psw).cuda()).cpu().numpy()
         assert bits_equal(got, want) == 0
+
+
+# Blocks of one round to many times what their sixteen waves hold, numbers that leave some SIMDs a round more than others:
+# every round is pooled once.
+@pytest.mark.parametrize("dtype,dim,per_round", [(O.INT8, 256, 4), (O.INT8, 1024, 1), (O.FP16, 32, 8), (O.INT4, 512, 4)])
+@pytest.mark.parametrize("rounds", [1, 15, 16, 17, 18, 19, 20, 21, 33, 47])
+def test_every_round_once(tuning, dtype, dim, per_round, rounds):
+    tuning(balanced=1, window=rounds * per_round)
+    rng = np.random.default_rng([rounds, dim])
+    B = rounds * per_round + 3
+    tbe, store = build(rng, [(dtype, 60, dim), (dtype, 50, dim)], [0, 1], O.SUM, O.FP32, 16)
+    lengths = rng.choice([0, 1, 5, 30], 2 * B).astype(np.int32)
+    offsets = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    ids = rng.integers(0, 50, int(offsets[-1])).astype(np.int32)
+    want = O.tbe_forward(store, [0, 1], B, ids, offsets, None, O.SUM, O.FP32)
+    assert bits_equal(_from_lengths(tbe, ids, lengths, None, B), want) == 0
+    # (in place of the next call's results, so that a round left out shows)
+    out = torch.full((B, 2 * dim), float("nan"), device="cuda")
+    tbe(indices=torch.from_numpy(ids).cuda(), offsets=torch.from_numpy(offsets).cuda(), batch_size=B, out=out)
+    assert bits_equal(out.cpu().numpy(), want) == 0

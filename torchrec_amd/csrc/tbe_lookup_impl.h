@@ -898,10 +898,9 @@ __device__ __forceinline__ void finish_bag(float (&acc)[NE], const LookupArgs& a
 // consecutive bags (of one sub-class, possibly spanning features).  It ranks
 // them by length in LDS, longest first, and cuts the order into rounds of gpw
 // bags; a round is pooled by one wave, one bag per lane group, so the lane
-// groups that run in lock step hold bags of nearly equal length.  The first 16
-// rounds are dealt to the block's 16 waves in serpentine order over the four SIMDs
-// (waves w, w+4, w+8, w+12 share SIMD w & 3), the others taken as waves become
-// free.  A bag is still pooled whole and in id order by one lane group; there is no
+// groups that run in lock step hold bags of nearly equal length.  Rounds are
+// dealt to the four SIMDs in serpentine order (waves w, w+4, w+8, w+12 share SIMD
+// w & 3); a SIMD's waves take its rounds as they become free.  A bag is still pooled whole and in id order by one lane group; there is no
 // scratch memory, atomic or pre-pass.
 #ifndef TRA_CU_THREADS  // (measurement builds override these two)
 #define TRA_CU_THREADS 1024
@@ -1135,7 +1134,7 @@ struct Window {
   FeatureDesc* desc;
   Sum* red;
   Sum* wave_tot;
-  int* taken;  // rounds that waves have asked for after their first
+  int* taken;  // [4] rounds that a SIMD's waves have asked for after their first
   u32x4_t* stage;  // 64 * kStageVectors vectors of results per wave
 };
 #define TRA_WINDOW(IdxT, name)                                                                       \
@@ -1147,9 +1146,9 @@ struct Window {
   __shared__ int s_hist[kLenBins];                                                                   \
   __shared__ FeatureDesc s_desc[kMaxWinFeat];                                                        \
   __shared__ typename SumOf<IdxT>::type s_red[kCuWaves], s_wave_tot[kCuWaves];                       \
-  __shared__ int s_taken;                                                                            \
+  __shared__ int s_taken[4];                                                                            \
   __shared__ u32x4_t s_stage[kCuWaves * kWaveSize * kStageVectors];                                  \
-  const Window<IdxT> name{s_start, s_len, s_ent, s_order, s_slot, s_hist, s_desc, s_red, s_wave_tot, &s_taken, s_stage}
+  const Window<IdxT> name{s_start, s_len, s_ent, s_order, s_slot, s_hist, s_desc, s_red, s_wave_tot, s_taken, s_stage}
 
 // What a staged window's bag starts in LDS still lack: `add`, and from the sub-class's feature `second` on `second_add`.
 template <typename Sum>
@@ -1185,7 +1184,7 @@ __device__ __forceinline__ WindowStarts<typename SumOf<IdxT>::type> stage_window
     return (int64_t)feat_key_pos(a, sc, fi) * p_B + b;
   };
   WindowStarts<Sum> starts;
-  if (threadIdx.x == 0) *w.taken = 0;
+  if (threadIdx.x < 4) w.taken[threadIdx.x] = 0;
   // A window of at most 4 x 64 bags is staged, scanned and ranked by the
   // block's first wave alone, four consecutive bags per lane, with no block
   // barrier on the way; from lengths, the other fifteen waves meanwhile sum
@@ -1494,17 +1493,16 @@ __device__ __forceinline__ void pool_window(const Window<IdxT> win, const Lookup
   const int lpr = sc.lpr;
   const int gpw = kWaveSize / lpr;
   const int rounds = (nb + gpw - 1) / gpw;
-  // Rounds are ordered longest first.  A wave's first one is dealt, in opposite
-  // directions on neighbouring SIMDs' rows of waves; after that it takes the next
-  // one that nobody has: waves of equal work end at very different times (64
-  // rounds of the same length, four a wave: the first wave done after 190 us, the
-  // last after 340), and a compute unit that a part of its waves has left keeps
-  // fewer requests in flight.  Dealt throughout / taken, us: 131 K bags of 80 ids,
-  // int4 128 columns, 319.2 / 315.5; 31 K bags of up to 50 position-weighted ids of
-  // odd widths 24.8 / 23.7; 53 K bags of up to 40 ids 18.5 / 18.3; 262 K bags of
-  // 30 ids of seven classes 358.8 / 358.6.
-  const int four = wave >> 2;
-  for (int r = four * 4 + ((four & 1) ? 3 - (wave & 3) : (wave & 3)); r < rounds;) {
+  // Rounds are ordered longest first and dealt to the four SIMDs (waves w, w + 4, w + 8 and w + 12 share one) in alternating
+  // direction.  A wave's first one is fixed; after that it takes the next one of its SIMD that nobody has: waves of equal work
+  // end at very different times (64 rounds of the same length, four a wave: the first wave done after 190 us, the last after
+  // 340), and a compute unit that a part of its waves has left keeps fewer requests in flight.  One counter for all
+  // SIMDs gives rounds to the waves that are free first, and so two of four that are left to one SIMD.  us, fixed
+  // throughout / one counter / one a SIMD: bags of 80 cached ids, twenty rounds a block, weighted int4 512 columns
+  // 72.8 / 77.2 / 71.9, int8 256 44.8 / 47.9 / 44.4; bags of 20, forty rounds, int8 256 32.1 / 29.9 / 29.6, int2 512
+  // 92.5 / 83.7 / 84.1.
+  const auto round_of = [](int simd, int k) { return 4 * k + ((k & 1) ? 3 - simd : simd); };
+  for (int r = round_of(wave & 3, wave >> 2); r < rounds;) {
     const auto bag_at = [&](int g, bool& active, int& i, int& fi, int& b) {
       const int pos = r * gpw + g;
       active = g < gpw && pos < nb;
@@ -1568,19 +1566,23 @@ __device__ __forceinline__ void pool_window(const Window<IdxT> win, const Lookup
 #ifdef TRA_INSTRUMENT
     if (lane == 0) a.ts[((size_t)blockIdx.x * (blockDim.x / 64) + wave) * 8 + 5] = (unsigned long long)max_len;
 #endif
+    // (what hangs on the wave's number is computed here: kept through the loop it would push scalar registers out)
+    int w0 = wave;
+    asm volatile("" : "+s"(w0));
+    u32x4_t* stage = win.stage + w0 * (kWaveSize * kStageVectors);
     if constexpr (kWide) {
       const int l = lane_now(), g2 = l / lpr, c2 = l - g2 * lpr;
       bag_at(g2, active, i, fi, b);
       const int out_col = fi - fi_lo < kMaxWinFeat ? win.desc[fi - fi_lo].out_col : a.cdescs[sc.first + fi].out_col;
-      finish_bag<NE>(acc, a, win.stage + wave * (kWaveSize * kStageVectors), active ? max(win.len[i], 0) : 0,
-                     (int64_t)b * a.out_stride + out_col, c2, lpr, l, active, vec());
+      finish_bag<NE>(acc, a, stage, active ? max(win.len[i], 0) : 0, (int64_t)b * a.out_stride + out_col, c2, lpr, l, active,
+                     vec());
     } else {
-      finish_bag<NE>(acc, a, win.stage + wave * (kWaveSize * kStageVectors), len, (int64_t)b * a.out_stride + d.out_col, c,
-                     lpr, lane, active, vec());
+      finish_bag<NE>(acc, a, stage, len, (int64_t)b * a.out_stride + d.out_col, c, lpr, lane, active, vec());
     }
     TRA_STAMP(4);
     if (rounds <= kCuWaves) break;
-    r = kCuWaves + __builtin_amdgcn_readfirstlane(lane_now() == 0 ? atomicAdd(win.taken, 1) : 0);
+    const int next = lane_now() == 0 ? atomicAdd(win.taken + (w0 & 3), 1) : 0;
+    r = round_of(w0 & 3, kCuWaves / 4 + __builtin_amdgcn_readfirstlane(next));
   }
 }
 
