@@ -814,11 +814,10 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// A vector of a row of results.  Results are written once and read by a later kernel: with the non-temporal hint where
-// a store instruction writes whole lines of the row (`lines`), else they stay in the caches until the rest of the line
-// has come.
-__device__ __forceinline__ void store_vector(u32x4_t x, u32x4_t* to, bool lines) {
-  if (lines) {
+// A vector of a row of results.  Results are written once and read by a later kernel: with the non-temporal hint (`past`
+// the caches), or, where the rest of a line follows with another store instruction, into them until it has come.
+__device__ __forceinline__ void store_vector(u32x4_t x, u32x4_t* to, bool past) {
+  if (past) {
     __builtin_nontemporal_store(x, to);
   } else {
     // (fenced: the compiler makes one store of the two otherwise, without the hint)
@@ -833,16 +832,25 @@ __device__ __forceinline__ void store_vector(u32x4_t x, u32x4_t* to, bool lines)
 // Calls of 213 K bags of two cached ids, us, vectors stored as they lie (two a lane exchanged by cross-lane reads, for
 // lane groups of powers of two) / this: fp32 results, int8 256 columns 102 / 55, int8 128 50 / 32, int4 128 49 / 32, 34
 // features of int8 128 and 256 90 / 59; fp16 results, int2 128 33 / 27, int8 256 49 / 48; 65 K bags of 20, int8 256 to
-// fp16 51 / 48, to fp32 57 / 49.  The hint, where a store writes less than a line of a row (without / with): int2 128 to
-// fp32 33 / 42, int4 64 to fp32 23 / 26, int8 40 - 104 to fp32 36 / 40, int2 48 - 112 to fp16 28 / 34; elsewhere: int8 256 to fp32 84 / 55, fp16 64 to
-// fp16 25.8 / 24.3.
-template <int NE, bool FP16>
+// fp16 51 / 48, to fp32 57 / 49.
+// OWN: two vectors a lane in a group of no power of two are stored as they lie: 213 K bags of two ids to fp32, int8 104
+// 39.6 and through LDS 41.5, int4 104 39.8 and 41.4, fp16 104 37.8 and 39.7, 78 K bags of eight, int8 72 17.5 and 18.0.  (Not in the several-class kernel, whose bodies it
+// costs 4 to 10 registers in scratch memory: 60 K position-weighted bags of two ids 23.0 / 23.6.)
+// The hint pays where a store instruction writes whole lines of a row (int8 256 to fp32, without / with, 84 / 55), and below
+// that in groups of powers of two with two vectors a lane (two ids a bag, int4 64 to fp16 21.6 / 20.2, int4 32 17.8 / 17.2; eight,
+// int8 32 to fp32 12.8 / 11.9) and of four lanes with four fp16 vectors (int2 128, two ids 25.6 / 26.7, eight 18.3 / 16.8, 41 K
+// bags of 20 ids of 1 M rows 26.7 / 25.3), but not elsewhere: int2 128 to fp32 33 / 42, int4 64 to fp32 23 / 26, int2 64 to fp16
+// 21 / 30, int8 40 - 104 to fp32 36 / 40, int2 48 - 112 to fp16 28 / 34.
+template <int NE, bool FP16, bool OWN>
 __device__ __forceinline__ void store_group_row(const float (&acc)[NE], u32x4_t* stage, unsigned char* row, int c,
                                                 int lpr, int lane, bool active) {
   constexpr int V = NE * (FP16 ? 2 : 4) / 16;
-  const bool lines = V <= kStageVectors && (lpr % 8 == 0 || (FP16 && V == 2 && lpr >= 2 && (lpr & (lpr - 1)) == 0));
-  if constexpr (V == 1) {
-    if (active) store_vector(out_vector<NE, FP16>(acc, 0), reinterpret_cast<u32x4_t*>(row) + c, lines);
+  const bool two_to_n = (lpr & (lpr - 1)) == 0;
+  const bool past = (V <= kStageVectors && lpr % 8 == 0) || (V == 2 && two_to_n && lpr >= 2) || (FP16 && V == 4 && lpr == 4);
+  if (V == 1 || (OWN && V == 2 && lpr % 8 != 0 && !two_to_n)) {
+    if (active)
+#pragma unroll
+      for (int v = 0; v < V; ++v) store_vector(out_vector<NE, FP16>(acc, v), reinterpret_cast<u32x4_t*>(row) + c * V + v, past);
   } else {
     // (Places in LDS are computed where they are used: kept through the pooling loop they would push its registers out.)
     asm volatile("" : "+v"(lane), "+v"(c));
@@ -858,7 +866,7 @@ __device__ __forceinline__ void store_group_row(const float (&acc)[NE], u32x4_t*
         const int i = k * lpr + c;  // which of the group's vectors this lane stores
         const int from = min(lane - c + i / P, kWaveSize - 1);  // (lanes behind the last whole group)
         const u32x4_t x = stage[stage_slot<P>(from, i % P)];
-        if (active) store_vector(x, reinterpret_cast<u32x4_t*>(row) + (i / P * V + h + i % P), lines);
+        if (active) store_vector(x, reinterpret_cast<u32x4_t*>(row) + (i / P * V + h + i % P), past);
       }
     }
   }
@@ -868,7 +876,7 @@ __device__ __forceinline__ void store_group_row(const float (&acc)[NE], u32x4_t*
 // group's lpr lanes holds the NE outputs at columns row_pos + c * NE.  Every
 // lane of the wave calls this; `active` says whether its group holds a bag.
 // `stage`: the wave's room in LDS, 64 * kStageVectors vectors.
-template <int NE>
+template <int NE, bool OWN>
 __device__ __forceinline__ void finish_bag(float (&acc)[NE], const LookupArgs& a, u32x4_t* stage, int len,
                                            int64_t row_pos, int c, int lpr, int lane, bool active, bool vec) {
   if (a.mean && len > 0) {
@@ -880,13 +888,13 @@ __device__ __forceinline__ void finish_bag(float (&acc)[NE], const LookupArgs& a
     unsigned char* row = reinterpret_cast<unsigned char*>(a.out) + row_pos * (a.out_fp16 ? 2 : 4);
     if constexpr (NE >= 8) {
       if (a.out_fp16) {
-        store_group_row<NE, true>(acc, stage, row, c, lpr, lane, active);
+        store_group_row<NE, true, OWN>(acc, stage, row, c, lpr, lane, active);
         return;
       }
     }
     if constexpr (NE >= 4) {
       if (!a.out_fp16) {
-        store_group_row<NE, false>(acc, stage, row, c, lpr, lane, active);
+        store_group_row<NE, false, OWN>(acc, stage, row, c, lpr, lane, active);
         return;
       }
     }
@@ -1469,6 +1477,7 @@ __device__ __forceinline__ WindowStarts<typename SumOf<IdxT>::type> stage_window
 
 // Which pooling bodies a kernel instance holds (see odd_lanes).
 constexpr int kBodiesOdd = 1;   // id blocks of four for every lane group of four lanes or more
+constexpr int kBodiesMany = 2;  // the same, one body of several in a kernel
 constexpr int kBodiesEven = 0;  // id blocks for powers of two from eight lanes, for others where the registers allow
 
 // Pools a staged window.  vec(): whether every lane's output slice is 16-byte aligned (asked where a bag is stored).
@@ -1477,7 +1486,7 @@ __device__ __forceinline__ void pool_window(const Window<IdxT> win, const Lookup
                                             int fi_lo, const WindowStarts<typename SumOf<IdxT>::type> starts,
                                             Vec&& vec) {
   constexpr int NE = CB * 8 / Traits<DTYPE>::kBits;
-  constexpr bool ODD = BODIES == kBodiesOdd;
+  constexpr bool ODD = BODIES != kBodiesEven, kOwn = BODIES != kBodiesMany;
   // Where a lane holds more than 16 accumulators, what the pooling loop does not need is found anew behind it (the lane's
   // place in the wave, where its bag's results go): kept, it would push the loop's registers out.  Registers in scratch
   // memory, int4 in 16-byte chunks, 32-bit ids from lengths, without, with per-sample and with position weights: 16, 16 and
@@ -1574,10 +1583,10 @@ __device__ __forceinline__ void pool_window(const Window<IdxT> win, const Lookup
       const int l = lane_now(), g2 = l / lpr, c2 = l - g2 * lpr;
       bag_at(g2, active, i, fi, b);
       const int out_col = fi - fi_lo < kMaxWinFeat ? win.desc[fi - fi_lo].out_col : a.cdescs[sc.first + fi].out_col;
-      finish_bag<NE>(acc, a, stage, active ? max(win.len[i], 0) : 0, (int64_t)b * a.out_stride + out_col, c2, lpr, l, active,
+      finish_bag<NE, kOwn>(acc, a, stage, active ? max(win.len[i], 0) : 0, (int64_t)b * a.out_stride + out_col, c2, lpr, l, active,
                      vec());
     } else {
-      finish_bag<NE>(acc, a, stage, len, (int64_t)b * a.out_stride + d.out_col, c, lpr, lane, active, vec());
+      finish_bag<NE, kOwn>(acc, a, stage, len, (int64_t)b * a.out_stride + d.out_col, c, lpr, lane, active, vec());
     }
     TRA_STAMP(4);
     if (rounds <= kCuWaves) break;
@@ -1592,7 +1601,7 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_cu_kernel(
     const void* p_offsets, const FeatureDesc* p_cdescs, int32_t p_B, int32_t p_xcd_blocks,
     int32_t p_xcd_count, int32_t p_n_sub, int32_t p_window0, int32_t p_count0, int32_t p_key0,
     const LookupArgs a) {
-  extern __shared__ unsigned char tra_dyn_smem[];  // only its size matters (one block per CU)
+  extern __shared__ unsigned char tra_dyn_smem[];  // (room that a tuning override asks for, unused)
   TRA_WINDOW(IdxT, s_window);
 
   TRA_STAMP(0);
@@ -1665,7 +1674,7 @@ struct LaunchClass {
 
 struct LaunchParams {
   int grid;
-  int lds_bytes;  // dynamic LDS (sized so one block fits per CU)
+  int lds_bytes;  // window kernel: dynamic LDS beside its own 107 KB, which already leave a compute unit one block
   int unroll;     // rows per pipeline batch: 2, 4 or 8
   bool idx64;
   bool weighted;

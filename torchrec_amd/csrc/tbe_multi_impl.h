@@ -8,13 +8,14 @@ namespace tra {
 
 // As tbe_pooled_cu_kernel, with blocks of all weight types and lane chunks in one grid: a block pools bags of one
 // sub-class and picks its body by it.  Lane chunks are at most 16 accumulators wide here: wider bodies would not fit the
-// 128 registers that sixteen waves leave each other.  With 32-bit ids they do without weights; up to 6 registers are kept
-// in scratch memory with weights, with 64-bit ids up to 5 without, 15 with per-sample and 18 with position weights.
+// 128 registers that sixteen waves leave each other.  With 32-bit ids they do without weights; up to 4 registers are kept
+// in scratch memory with per-sample and 7 with position weights, with 64-bit ids up to 1 without, 9 with per-sample and 15
+// with position weights.
 template <typename IdxT, int WEIGHTED, bool FROM_LENGTHS>
 __global__ __launch_bounds__(kCuThreads) void tbe_pooled_multi_kernel(const void* p_offsets, const FeatureDesc* p_cdescs,
                                                                       int32_t p_B, int32_t p_xcd_blocks,
                                                                       int32_t p_xcd_count, const MultiArgs m) {
-  extern __shared__ unsigned char tra_dyn_smem[];  // only its size matters (one block per CU)
+  extern __shared__ unsigned char tra_dyn_smem[];  // (room that a tuning override asks for, unused)
   TRA_WINDOW(IdxT, s_window);
   const LookupArgs& a = m.common;
   int blk = blockIdx.x;
@@ -34,7 +35,7 @@ __global__ __launch_bounds__(kCuThreads) void tbe_pooled_multi_kernel(const void
   const bool vec = (kind & kMultiVec) != 0;
 #define TRA_MULTI(D, CB)                                                                                       \
   case multi_kind(D, CB):                                                                                      \
-    pool_window<D, CB, IdxT, WEIGHTED, 4, kBodiesOdd>(s_window, a, sc, nb, fi_lo, starts, [&] { return vec; }); \
+    pool_window<D, CB, IdxT, WEIGHTED, 4, kBodiesMany>(s_window, a, sc, nb, fi_lo, starts, [&] { return vec; }); \
     break;
   switch (kind & ~kMultiVec) {
     TRA_MULTI(TRA_INT8, 16)
