@@ -136,14 +136,6 @@ __device__ __forceinline__ int lanes_below(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-// Block barrier that orders LDS accesses only: loads and stores of global memory, through which the waves of a block
-// exchange nothing here, stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // The tile's bags: first bag and how many.
 __device__ __forceinline__ int64_t tile_bags(int tile, int f, int per_feature, int bags, int B, int& cnt) {
   const int b0 = (tile - f * per_feature) * bags;

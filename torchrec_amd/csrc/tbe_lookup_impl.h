@@ -1110,16 +1110,6 @@ __device__ __forceinline__ int64_t uniform(int64_t v) {
 __device__ __forceinline__ int32_t wave_last(int32_t v) { return __builtin_amdgcn_readlane(v, kWaveSize - 1); }
 __device__ __forceinline__ int64_t wave_last(int64_t v) { return __shfl(v, kWaveSize - 1, kWaveSize); }
 
-// Block barrier that orders LDS accesses only.  __syncthreads() also waits for
-// every outstanding global load of the wave; the window kernel's prologue keeps
-// loads in flight across its barriers (nothing there is handed from wave to
-// wave through global memory).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // Position of feature `fi` of a sub-class among the input keys: from the launch
 // arguments when the class is small enough, else from the descriptors.
 __device__ __forceinline__ int feat_key_pos(const LookupArgs& a, const SubClass& sc, int fi) {

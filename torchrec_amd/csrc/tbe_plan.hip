@@ -150,7 +150,7 @@ static Tuning choose_tuning(bool balanced) {
   t.balanced = balanced ? 1 : 0;
   t.window = 0;
   t.unroll = 4;
-  t.lds_bytes = 0;  // (the static arrays are over half of a compute unit's LDS: one block each)
+  t.lds_bytes = 0;  // (the window kernel's own 107 KB leave a compute unit one block; an override has 53 KB of room)
   if (g_ovr.balanced >= 0) t.balanced = g_ovr.balanced;
   if (g_ovr.window >= 0) t.window = g_ovr.window;
   if (g_ovr.unroll >= 0) t.unroll = g_ovr.unroll;

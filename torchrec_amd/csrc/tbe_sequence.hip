@@ -88,8 +88,9 @@ __device__ __forceinline__ void store_rows(const float (&acc)[NE], u32x4_t* stag
 //   fp16 results: int4 32 57 / 28, 64 65 / 46, int2 128 159 / 95, int8 96 118 / 79,
 //                 128 89 / 84
 // (Without the non-temporal hint int8 64 fp16 62 -> 92 us, fp16 128 92 -> 156 us.)
-// What describes the tile is scalar, so that more waves fit a SIMD: five instead of four with 16 int8 columns a lane in
-// 8-byte chunks, seven instead of four with 8 fp16 columns.
+// What describes the tile is scalar, so that more waves fit a SIMD: with eight columns a lane (int8 rows in 8-byte, fp16 in
+// 16-byte chunks) 63 to 69 registers instead of 118 to 122, seven waves instead of four; with sixteen of int8 or int4 it is
+// five before and after.
 // Slower than lanes' vectors as they lie and the tile in vector registers: fp16 rows of 16 and 32 columns to fp16, 32-bit
 // ids, 25.1 / 26.5 and 46 / 49 us (64-bit ids 27.5 / 26, 56 / 52); 123 K rows of int8 or int4 128 to fp16 9.5 / 9.8.
 template <int DTYPE, int CB, typename IdxT>

@@ -56,6 +56,14 @@ __device__ __forceinline__ void publish_total(int64_t v, int64_t* host) {
   __hip_atomic_store(host, v == kMailEmpty ? 0 : v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Block barrier that orders LDS accesses only.  __syncthreads() also waits for every outstanding global load of the wave;
+// where a block hands nothing from wave to wave through global memory, loads and stores stay in flight across this one.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 #define TRA_HIP(call)                                   \
   do {                                                  \
     hipError_t e__ = (call);                            \
