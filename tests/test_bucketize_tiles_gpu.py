@@ -58,6 +58,25 @@ def test_tiles(F, B, W, how, idt):
     assert np.array_equal(gu.cpu().numpy(), nu)
 
 
+# Ids, weights and places of more than 256 MB, whose blocks share a compute unit with fewer others, and of a little less.
+@pytest.mark.parametrize("mean", [3190, 3205])
+def test_more_than_the_cache_holds(mean):
+    rng = np.random.default_rng(mean)
+    F, B, W = 3, 700, 3
+    lengths = rng.integers(mean - 5, mean + 6, F * B)
+    n = int(lengths.sum())
+    assert (40 * n > 2**28) == (mean > 3200)
+    ids = rng.integers(0, 1000, n)
+    weights = rng.random(n).astype(np.float32)
+    block_sizes = np.full(F, 334)
+    nl, ni, nw, nu = O.bucketize(lengths, ids, block_sizes, W, weights, False, return_permute=True)
+    gl, gi, gw, _, gu, gb = ops._block_bucketize(
+        torch.from_numpy(lengths).to(DEV), torch.from_numpy(ids).to(DEV), False, True,
+        torch.from_numpy(block_sizes).to(DEV), W, torch.from_numpy(weights).to(DEV), False, want_buckets=True)
+    for got, want in ((gl, nl), (gi, ni), (gw, nw), (gu, nu), (gb, ids // 334)):
+        assert np.array_equal(got.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("F,B", [(3, 100), (40, 700)])
 @pytest.mark.parametrize("bad", [-1, 10**6])
 def test_lengths_that_are_no_partition(F, B, bad):

@@ -64,6 +64,7 @@ struct BucketArgs {
   int32_t keep;
 };
 constexpr int kBktOwnLengths = 16384;  // lengths up to which bucket_counts sums them itself
+constexpr size_t kBktSpareLds = 6000;  // beside the 30 KB of bucket_move's weighted 64-bit instances: four blocks a compute unit
 constexpr int kBktOwnCounts = 4096;    // tiles * buckets up to which bucket_move adds the counts itself
 
 // q = id / bs, r = id % bs of unsigned ids for one block size.  Below 2^32:
@@ -679,8 +680,13 @@ int tra_bucketize_ids(const void* lengths, const void* indices, int32_t is_i64, 
     hipLaunchKernelGGL(kernel, tiles, block, counters, s, a.lengths, a.tile_total, a.block_sizes, a.bags, a.per_feature,
                        a.B, a);
   };
+  // Weighted 64-bit ids whose places are wanted too, more bytes than the 256 MB of the memory-side cache: four blocks on a
+  // compute unit instead of the five that registers allow (us a call, five / four: 7.9 M ids, 2 buckets 104.5 / 101.0, 8
+  // buckets 91.1 / 88.4; but 5.2 M ids, 210 MB 73.5 / 75.3, and without places 74.3 / 75.6).
+  const int64_t moved = num_indices * (2 * (8 + 4) + 8 + (bucket_of != nullptr ? 8 : 0));
+  const size_t spare = is_i64 && weights && unbucketize_permute && moved > (int64_t(1) << 28) ? kBktSpareLds : 0;
   const auto move = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, tiles, block, 0, s, a.tile_first, a.tile_total, a.block_sizes, a.place, a.bucket_total,
+    hipLaunchKernelGGL(kernel, tiles, block, spare, s, a.tile_first, a.tile_total, a.block_sizes, a.place, a.bucket_total,
                        a.per_feature, a.tiles, a);
   };
   const auto launch = [&](auto id) {
