@@ -1014,6 +1014,11 @@ def test_packed_weights_replaced_by_hand(kind):
     tbe.weights_dev = same if kind == "buffer" else torch.nn.Parameter(same, requires_grad=False)
     got, want = run_both(tbe, store, [0, 1], 9, ids, offsets, None, O.SUM, O.FP32)
     assert bits_equal(got, want) == 0
+    assert bits_equal(_from_lengths(tbe, ids, lengths, None, 9), want) == 0
+    rows, of_rows = build(rng, specs[:1], [0], O.NONE, O.FP32, 16)
+    rows.weights_dev = rows.weights_dev.clone() if kind == "buffer" else torch.nn.Parameter(rows.weights_dev, requires_grad=False)
+    got = rows(torch.from_numpy(ids[: offsets[9]]).to(DEV), None, key_starts=[0, int(offsets[9])]).cpu().numpy()
+    assert bits_equal(got, O.tbe_forward(of_rows, [0], 9, ids[: offsets[9]], offsets[:10], None, O.NONE, O.FP32)) == 0
     tbe.weights_dev = same.cpu() if kind == "buffer" else torch.nn.Parameter(same.cpu(), requires_grad=False)
     with pytest.raises(TorchrecAmdError, match="packed weights are on cpu"):
         tbe(torch.from_numpy(ids).to(DEV), torch.from_numpy(offsets).to(DEV))

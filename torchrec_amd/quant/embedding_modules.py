@@ -539,7 +539,8 @@ class EmbeddingBagCollection(EmbeddingBagCollectionInterface, ModuleNoCopyMixin,
                 and v.is_contiguous()
                 and ln.is_contiguous()
                 and op._weights_initialized
-                and op._buffers["weights_dev"].get_device() == di
+                and (store := op._buffers.get("weights_dev")) is not None
+                and store.get_device() == di
                 # (where the first key order seen is kept for good: that it was the features' own)
                 and (
                     not getattr(self, MODULE_ATTR_CACHE_FEATURES_ORDER, False)
