@@ -833,9 +833,10 @@ __device__ __forceinline__ void store_vector(u32x4_t x, u32x4_t* to, bool past) 
 // lane groups of powers of two) / this: fp32 results, int8 256 columns 102 / 55, int8 128 50 / 32, int4 128 49 / 32, 34
 // features of int8 128 and 256 90 / 59; fp16 results, int2 128 33 / 27, int8 256 49 / 48; 65 K bags of 20, int8 256 to
 // fp16 51 / 48, to fp32 57 / 49.
-// OWN: two vectors a lane in a group of no power of two are stored as they lie: 213 K bags of two ids to fp32, int8 104
-// 39.6 and through LDS 41.5, int4 104 39.8 and 41.4, fp16 104 37.8 and 39.7, 78 K bags of eight, int8 72 17.5 and 18.0.  (Not in the several-class kernel, whose bodies it
-// costs 4 to 10 registers in scratch memory: 60 K position-weighted bags of two ids 23.0 / 23.6.)
+// OWN: two vectors of a lane that is alone, or in a group of no power of two, are stored as they lie: 213 K bags of two
+// ids to fp32, int8 104 39.6 and through LDS 41.5, int4 104 39.8 and 41.4, fp16 104 37.8 and 39.7, 78 K bags of eight, int8
+// 72 17.5 and 18.0.  (Not in the several-class kernel, whose bodies it costs 4 to 10 registers in scratch memory: 60 K
+// position-weighted bags of two ids 23.0 / 23.6.)
 // The hint pays where a store instruction writes whole lines of a row (int8 256 to fp32, without / with, 84 / 55), and below
 // that in groups of powers of two with two vectors a lane (two ids a bag, int4 64 to fp16 21.6 / 20.2, int4 32 17.8 / 17.2; eight,
 // int8 32 to fp32 12.8 / 11.9) and of four lanes with four fp16 vectors (int2 128, two ids 25.6 / 26.7, eight 18.3 / 16.8, 41 K
@@ -845,8 +846,8 @@ template <int NE, bool FP16, bool OWN>
 __device__ __forceinline__ void store_group_row(const float (&acc)[NE], u32x4_t* stage, unsigned char* row, int c,
                                                 int lpr, int lane, bool active) {
   constexpr int V = NE * (FP16 ? 2 : 4) / 16;
-  const bool two_to_n = (lpr & (lpr - 1)) == 0;
-  const bool past = (V <= kStageVectors && lpr % 8 == 0) || (V == 2 && two_to_n && lpr >= 2) || (FP16 && V == 4 && lpr == 4);
+  const bool two_to_n = lpr >= 2 && (lpr & (lpr - 1)) == 0;
+  const bool past = (V <= kStageVectors && lpr % 8 == 0) || (V == 2 && two_to_n) || (FP16 && V == 4 && lpr == 4);
   if (V == 1 || (OWN && V == 2 && lpr % 8 != 0 && !two_to_n)) {
     if (active)
 #pragma unroll
